@@ -940,21 +940,51 @@ constexpr bool cell_capable() {
 }
 
 // Second half of a split product: C = epilogue(sum of the partial planes, in split order).
+// What bounds it at the sizes that split (a few thousand to a few hundred thousand elements) is
+// memory latency, not bytes: a thread owns four consecutive rows of one column and has up to eight
+// planes' 16-byte loads in flight at once, so the whole launch is one or two round trips.
+// One element and one plane at a time it took 12.0 us for 2000 x 12, 11.1 us for 1000 x 64 and 9.4 us for
+// 1000 x 128 elements; it takes 4.9, 4.4 and 4.8 us.
+constexpr int kReduceBatch = 8;
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmArgs g) {
   const size_t plane = (size_t)g.ws_ld * g.N;
-  const size_t total = (size_t)g.M * g.N;
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (size_t)gridDim.x * 256) {
-    const int n = (int)(i / g.M), m = (int)(i % g.M);
+  const int quads = g.ws_ld / 4;  // a plane's columns are padded to whole quads
+  const size_t total = (size_t)quads * g.N;
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
+       i += (size_t)gridDim.x * blockDim.x) {
+    const int n = (int)(i / quads), m = (int)(i % quads) * 4;
     const float *p = g.ws_part + (size_t)n * g.ws_ld + m;
-    float acc = 0.f;
-    for (int s = 0; s < g.splits; ++s) acc += p[s * plane];
+    const int rows = min(4, g.M - m);
     float *cp = g.C + (size_t)n * g.ldc + m;
-    float v = g.alpha * acc;
-    if (g.beta != 0.f) v += g.beta * *cp;
-    if (g.bias) v += g.bias[m];
-    if (g.act == LH_ACT_TANH && m < g.act_rows) v = tanhf(v);
-    if (g.colmask) v *= (float)g.colmask[n];
-    *cp = v;
+    float old[4] = {0.f, 0.f, 0.f, 0.f}, bv[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if (g.beta != 0.f && r < rows) old[r] = cp[r];
+      if (g.bias && r < rows) bv[r] = g.bias[m + r];
+    }
+    const float cm = g.colmask ? (float)g.colmask[n] : 1.f;
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < g.splits; s0 += kReduceBatch) {
+      float4 v[kReduceBatch];
+#pragma unroll
+      for (int s = 0; s < kReduceBatch; ++s)  // past the last plane: that plane again, not added
+        v[s] = *reinterpret_cast<const float4 *>(p + (size_t)min(s0 + s, g.splits - 1) * plane);
+#pragma unroll
+      for (int s = 0; s < kReduceBatch; ++s) {
+        if (s0 + s >= g.splits) break;
+        acc[0] += v[s].x, acc[1] += v[s].y, acc[2] += v[s].z, acc[3] += v[s].w;
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if (r >= rows) break;
+      float o = g.alpha * acc[r];
+      if (g.beta != 0.f) o += g.beta * old[r];
+      if (g.bias) o += bv[r];
+      if (g.act == LH_ACT_TANH && m + r < g.act_rows) o = tanhf(o);
+      if (g.colmask) o *= cm;
+      cp[r] = o;
+    }
   }
 }
 
@@ -1060,10 +1090,12 @@ int launch_cfg(const GemmArgs &g0, bool ta, bool tx, bool vec, hipStream_t st) {
     else LH_GEMM_LAUNCH(false, true);
 #undef LH_GEMM_LAUNCH
     if (rc != LH_OK || g.splits == 1 || g.leave_partial) return rc;
-    const size_t total = (size_t)g.M * g.N;
-    const size_t blocks = (total + 1023) / 1024;  // four elements per thread
+    // four rows per thread; small products in single-wavefront workgroups, to reach more CUs
+    const size_t total = (size_t)(g.ws_ld / 4) * g.N;
+    const unsigned nt = total < 65536 ? 64 : 256;
+    const size_t blocks = (total + nt - 1) / nt;
     hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)(blocks < 8192 ? blocks : 8192)),
-                       dim3(256), 0, st, g);
+                       dim3(nt), 0, st, g);
     return lh::check_launch("lh_gemm_ws_f32 split reduction");
   }
   if constexpr (ALLOW_UNALIGNED) {

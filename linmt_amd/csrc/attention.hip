@@ -1,11 +1,10 @@
 // Attention core (Luong local-p, and the textbook global "general" variant): alignment position,
 // window indices, scores, max-subtracted exp, normalisation, Gaussian weighting and the context
-// vector in ONE kernel.  One workgroup (4 wavefronts) per column b:
+// vector in ONE kernel, one workgroup per column b:
 //   phase 1  v_p . tanh1[:,b]  -> sigmoid -> p_b -> window [lo,hi]           (block reduction)
-//   phase 2  score_j = hs_j . wa[:,b]; wavefront w takes slots j = w, w+4, ...  (DPP/shuffle sums)
-//   phase 3  max / exp / sum / Gaussian over the <= W slots, kept in LDS
-//   phase 4  ctx[:,b] = sum_j a_j hs_j, thread-per-row-quad; the second read of the window comes
-//            from L2 (the W x H window was just streamed by this very workgroup).
+//   phase 2  score_j = hs_j . wa[:,b]
+//   phase 3  max / exp / sum / Gaussian over the <= W slots
+//   phase 4  ctx[:,b] = sum_j a_j hs_j
 // The reference materialises the window (LoadInHSKernel) and launches eight kernels for this.
 #include "lh_common.h"
 
@@ -36,29 +35,24 @@ struct AttnArgs {
   int out_tanh;
 };
 
-template <bool VEC>
-__device__ __forceinline__ float dot_wave(const float *__restrict__ x, const float *__restrict__ y,
-                                          int H, int lane) {
-  float acc = 0.f;
-  if constexpr (VEC) {
-    for (int r = lane * 4; r < H; r += lh::kWave * 4) {
-      const float4 a = *reinterpret_cast<const float4 *>(x + r);
-      const float4 b = *reinterpret_cast<const float4 *>(y + r);
-      acc += a.x * b.x + a.y * b.y + a.z * b.z + a.w * b.w;
-    }
-  } else {
-    for (int r = lane; r < H; r += lh::kWave) acc += x[r] * y[r];
-  }
-  return lh::wave_sum(acc);
-}
+// Any window and alignment.  The time of a launch is the length of one workgroup's chain of
+// dependent memory round trips (a decoding or scoring step has at most a few columns per CU), so a
+// column gets 16 wavefronts, a wavefront has the rows of four slots in flight at once, every slot's
+// exponential is taken once, by the slot's own thread, and the context sum of a row is split over
+// as many groups of threads as the workgroup has left (their partial sums meet in LDS in group
+// order); its second read of the window comes from L2.
+// 128 columns of 1000 rows, 50 slots: 49.6 us with four wavefronts, a slot at a time; 22.4 us.
+constexpr int kWide = 1024;
+constexpr int kWideWaves = kWide / lh::kWave;
+constexpr int kSlotBatch = 4;
 
 template <bool VEC>
-__global__ __launch_bounds__(kThreads) void attn_core_kernel(const AttnArgs a) {
+__global__ __launch_bounds__(kWide) void attn_core_kernel(const AttnArgs a) {
   __shared__ float s_val[kMaxSlots];   // scores, then alignment weights
   __shared__ int s_tau[kMaxSlots];     // encoder timestep of slot j, -1 = no state to read
-  __shared__ int s_idx[kMaxSlots];     // source position of slot j, -1 = invalid slot
-  __shared__ float s_red[kWaves];
-  __shared__ float s_scalar[2];
+  __shared__ float s_red[kWideWaves];
+  __shared__ float4 s_ctx[kWide];
+  __shared__ int s_first;
 
   const int b = lh::xcd_contiguous(blockIdx.x, gridDim.x);  // a sentence's columns on one XCD
   const int tid = threadIdx.x, wave = tid / lh::kWave, lane = tid % lh::kWave;
@@ -75,8 +69,9 @@ __global__ __launch_bounds__(kThreads) void attn_core_kernel(const AttnArgs a) {
   if (D >= 0) {
     float part = 0.f;
     const float *t1 = a.tanh1 + (size_t)b * a.proj_col_stride;
-    for (int r = tid; r < H; r += kThreads) part += a.v_p[r] * t1[r];
-    const float dot = lh::block_sum<kWaves>(part, s_red);
+    if (tid < kThreads)  // the order of attn_core_regs_kernel: the position must not depend on the kernel
+      for (int r = tid; r < H; r += kThreads) part += a.v_p[r] * t1[r];
+    const float dot = lh::block_sum<kWideWaves>(part, s_red);
     const float sig = (float)(1.0 / (1.0 + exp(-1.0 * (double)dot)));
     p = (float)len * sig;
     lo = (0 > (int)p - D) ? 0 : ((int)p - D);
@@ -87,95 +82,166 @@ __global__ __launch_bounds__(kThreads) void attn_core_kernel(const AttnArgs a) {
     }
   }
 
-  // window indices (reference layout B x W, element (b,j) at b + B*j)
-  for (int j = tid; j < W; j += kThreads) {
-    int idx = -1;
-    if (m == 1 && lo + j <= hi) idx = lo + j;
-    a.indices[b + (size_t)B * j] = idx;
-    s_idx[j] = idx;
+  // window indices (reference layout B x W, element (b,j) at b + B*j); thread j owns slot j
+  static_assert(kMaxSlots <= kWide, "one thread per slot");
+  int idx = -1;
+  if (tid < W) {
+    if (m == 1 && lo + tid <= hi) idx = lo + tid;
+    a.indices[b + (size_t)B * tid] = idx;
     int tau = -1;
     if (idx >= 0) {
       tau = len - 1 - idx + off;
       if (tau < 0 || tau >= a.hs_steps) tau = -1;  // outside the caller's state buffer: zero vector
     }
-    s_tau[j] = tau;
+    s_tau[tid] = tau;
   }
   __syncthreads();
 
-  // scores
-  for (int j = wave; j < W; j += kWaves) {
-    const int tau = s_tau[j];
-    float sc = 0.f;
-    if (tau >= 0) sc = dot_wave<VEC>(hs_c + (size_t)tau * a.step_stride, wa, H, lane);
-    if (lane == 0) s_val[j] = sc;
+  // scores: wavefront w takes slots w, w + 16, ..., four at a time
+  for (int j0 = wave; j0 < W; j0 += kWideWaves * kSlotBatch) {
+    const float *row[kSlotBatch];
+    float acc[kSlotBatch];
+    bool live[kSlotBatch];
+#pragma unroll
+    for (int u = 0; u < kSlotBatch; ++u) {
+      const int j = j0 + u * kWideWaves;
+      const int tau = j < W ? s_tau[j] : -1;
+      live[u] = tau >= 0;
+      row[u] = hs_c + (size_t)(live[u] ? tau : 0) * a.step_stride;
+      acc[u] = 0.f;
+    }
+    if constexpr (VEC) {
+#pragma unroll 4
+      for (int r = lane * 4; r < H; r += lh::kWave * 4) {
+        const float4 y = *reinterpret_cast<const float4 *>(wa + r);
+#pragma unroll
+        for (int u = 0; u < kSlotBatch; ++u) {
+          if (!live[u]) continue;  // the same for the whole wavefront
+          const float4 x = *reinterpret_cast<const float4 *>(row[u] + r);
+          acc[u] += x.x * y.x + x.y * y.y + x.z * y.z + x.w * y.w;
+        }
+      }
+    } else {
+#pragma unroll 4
+      for (int r = lane; r < H; r += lh::kWave) {
+        const float y = wa[r];
+#pragma unroll
+        for (int u = 0; u < kSlotBatch; ++u)
+          if (live[u]) acc[u] += row[u][r] * y;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kSlotBatch; ++u) {
+      const float sc = lh::wave_sum(acc[u]);
+      const int j = j0 + u * kWideWaves;
+      if (lane == 0 && j < W) s_val[j] = live[u] ? sc : 0.f;
+    }
   }
   __syncthreads();
 
-  // normalisation: every thread reduces the (few) slots redundantly out of LDS
-  float mx = D >= 0 ? 0.f : -FLT_MAX;
-  for (int j = 0; j < W; ++j) {
-    if (s_idx[j] != -1 && s_val[j] > mx) mx = s_val[j];
-  }
-  float Z = 0.f;
-  for (int j = 0; j < W; ++j) {
-    if (s_idx[j] != -1) Z += expf(s_val[j] - mx);
-  }
-  __syncthreads();
-  const float sigma_sq = (float)((D * D) / 4.0);
-  for (int j = tid; j < W; j += kThreads) {
-    const int idx = s_idx[j];
+  // normalisation
+  const bool valid = tid < W && idx != -1;
+  const float val = valid ? s_val[tid] : 0.f;
+  const float floor_mx = D >= 0 ? 0.f : -FLT_MAX;
+  const float mx = lh::block_max<kWideWaves>(valid ? fmaxf(val, floor_mx) : floor_mx, s_red);
+  const float e = valid ? expf(val - mx) : 0.f;
+  const float Z = lh::block_sum<kWideWaves>(e, s_red);
+  if (tid < W) {
     float al = 0.f, g = 1.f;
-    if (idx != -1) {
-      const float e = expf(s_val[j] - mx);
+    if (valid) {
       if (D >= 0) {
+        const float sigma_sq = (float)((D * D) / 4.0);
         const float dlt = p - (float)idx;
         g = expf((-1.f * (dlt * dlt)) / (2.f * sigma_sq));
       }
       al = (Z != 0.f) ? (e / Z) * g : e;
     }
-    a.align[b + (size_t)B * j] = al;
-    a.cached_exp[j + (size_t)W * b] = g;
-    s_val[j] = al;
+    a.align[b + (size_t)B * tid] = al;
+    a.cached_exp[tid + (size_t)W * b] = g;
+    s_val[tid] = al;
   }
+  if (tid == 0) s_first = W;
   __syncthreads();
 
-  if (a.viterbi && tid == 0) {
-    float best = -1.f;
-    int best_idx = -1;
-    for (int j = 0; j < W; ++j) {
-      if (best < s_val[j]) {
-        best = s_val[j];
-        best_idx = s_idx[j];
-      }
-    }
-    a.viterbi[b] = best_idx;
+  if (a.viterbi) {
+    // the first slot of the largest weight (weights are >= 0, slots without a position weigh 0)
+    const float al = tid < W ? s_val[tid] : -1.f;
+    const float best = lh::block_max<kWideWaves>(fmaxf(al, -1.f), s_red);
+    if (tid < W && al == best) atomicMin(&s_first, tid);
+    __syncthreads();
+    const int first = best > -1.f ? s_first : W;
+    if (tid == (first < W ? first : 0)) a.viterbi[b] = first < W ? idx : -1;
   }
 
-  // context vector
+  // context vector: the rows (quads of them when aligned) of a column go to `lanes` threads,
+  // group g of the workgroup adds the slots j = g, g + groups, ...
   float *ctx = a.ctx + (size_t)b * H;
-  if constexpr (VEC) {
-    for (int r = tid * 4; r < H; r += kThreads * 4) {
-      float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-      for (int j = 0; j < W; ++j) {
+  const int units = VEC ? H / 4 : H;
+  const int lanes = min(kWide, (units + lh::kWave - 1) / lh::kWave * lh::kWave);
+  const int groups = kWide / lanes;
+  const int grp = tid / lanes;
+  for (int u0 = 0; u0 < units; u0 += lanes) {
+    const int unit = u0 + tid % lanes;
+    const bool mine = grp < groups && unit < units;
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (mine) {
+#pragma unroll 8
+      for (int j = grp; j < W; j += groups) {
         const int tau = s_tau[j];
-        if (tau < 0) continue;
         const float w = s_val[j];
-        const float4 v = *reinterpret_cast<const float4 *>(hs_c + (size_t)tau * a.step_stride + r);
-        acc.x += w * v.x; acc.y += w * v.y; acc.z += w * v.z; acc.w += w * v.w;
+        const float *x = hs_c + (size_t)max(tau, 0) * a.step_stride;
+        if constexpr (VEC) {
+          const float4 v = *reinterpret_cast<const float4 *>(x + (size_t)unit * 4);
+          acc.x = tau >= 0 ? acc.x + w * v.x : acc.x;
+          acc.y = tau >= 0 ? acc.y + w * v.y : acc.y;
+          acc.z = tau >= 0 ? acc.z + w * v.z : acc.z;
+          acc.w = tau >= 0 ? acc.w + w * v.w : acc.w;
+        } else {
+          const float v = x[unit];
+          acc.x = tau >= 0 ? acc.x + w * v : acc.x;
+        }
       }
-      *reinterpret_cast<float4 *>(ctx + r) = acc;
     }
-  } else {
-    for (int r = tid; r < H; r += kThreads) {
-      float acc = 0.f;
-      for (int j = 0; j < W; ++j) {
-        const int tau = s_tau[j];
-        if (tau < 0) continue;
-        acc += s_val[j] * hs_c[(size_t)tau * a.step_stride + r];
-      }
-      ctx[r] = acc;
+    if (groups > 1) {  // then every unit is covered by the first round
+      s_ctx[tid] = acc;
+      __syncthreads();
+      if (grp == 0 && mine)
+        for (int g = 1; g < groups; ++g) {
+          const float4 o = s_ctx[g * lanes + tid];
+          acc.x += o.x, acc.y += o.y, acc.z += o.z, acc.w += o.w;
+        }
+    }
+    if (grp == 0 && mine) {
+      if constexpr (VEC) *reinterpret_cast<float4 *>(ctx + (size_t)unit * 4) = acc;
+      else ctx[unit] = acc.x;
     }
   }
+}
+
+// Sums v[slot] over the 64 lanes of a wavefront for 32 slots at once: at every level a lane keeps
+// one half of its slots and hands the other half to its partner, 32 exchanges in place of 6 per
+// slot.  Lane l returns the sum of slot l / 2, added in the order of wave_sum.
+template <int HALF>
+__device__ __forceinline__ void fold_slots(float (&v)[32], int lane) {
+  const bool upper = (lane & (2 * HALF)) != 0;
+#pragma unroll
+  for (int i = 0; i < HALF; ++i) {
+    const float keep = upper ? v[i + HALF] : v[i];
+    const float send = upper ? v[i] : v[i + HALF];
+    v[i] = keep + __shfl_xor(send, 2 * HALF, lh::kWave);
+  }
+}
+__device__ __forceinline__ float wave_sum_slots(float (&v)[32], int lane) {
+  fold_slots<16>(v, lane);
+  fold_slots<8>(v, lane);
+  fold_slots<4>(v, lane);
+  fold_slots<2>(v, lane);
+  fold_slots<1>(v, lane);
+  return v[0] + __shfl_xor(v[0], 1, lh::kWave);
+}
+
+__device__ __forceinline__ float lane_value(float v, int lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
 // The same computation for windows of at most WCAP slots (local-p with D <= 10) and 16-byte
@@ -183,12 +249,15 @@ __global__ __launch_bounds__(kThreads) void attn_core_kernel(const AttnArgs a) {
 // (thread t holds rows 4t..4t+3 -- and 4(t+256).. when H > 1024 -- of every slot, all loads in
 // flight together), the scores are block-reduced from per-thread partial dot products, and the
 // context vector is accumulated from the same registers.
+// A launch lasts as long as one workgroup's chain of dependent steps (few columns per CU, the
+// columns of a sentence share their window in L2), so the chain is kept short: the window's bounds
+// live in scalar registers (no trip through LDS before its loads), lane j of every wavefront
+// normalises slot j by itself, and what all lanes need of it comes back as a lane read.
+// H = 1000, D = 10: 12 columns 16.0 -> 7.8 us, 64 columns 14.3 -> 7.0, 768 columns 21.4 -> 15.1.
 template <int NQ, int WCAP>
 __global__ __launch_bounds__(kThreads) void attn_core_regs_kernel(const AttnArgs a) {
-  __shared__ float s_part[kWaves][WCAP];
-  __shared__ float s_val[WCAP];
-  __shared__ int s_tau[WCAP];
-  __shared__ int s_idx[WCAP];
+  static_assert(WCAP <= 31, "wave_sum_slots, the bits of live");
+  __shared__ float s_part[kWaves][32];
   __shared__ float s_red[kWaves];
 
   const int b = lh::xcd_contiguous(blockIdx.x, gridDim.x);  // a sentence's columns on one XCD
@@ -242,113 +311,95 @@ __global__ __launch_bounds__(kThreads) void attn_core_regs_kernel(const AttnArgs
       a.sigma[b] = sig;
     }
   }
-  for (int j = tid; j < WCAP; j += kThreads) {
-    int idx = -1, tau = -1;
-    if (j < W) {
-      if (m == 1 && lo + j <= hi) idx = lo + j;
-      a.indices[b + (size_t)B * j] = idx;
-      if (idx >= 0) {
-        tau = len - 1 - idx + off;
-        if (tau < 0 || tau >= a.hs_steps) tau = -1;
-      }
-    }
-    s_idx[j] = idx;
-    s_tau[j] = tau;
-  }
-  __syncthreads();
+  // the window's slots: source position lo + j, encoder timestep tau0 - j
+  const int lo_s = __builtin_amdgcn_readfirstlane(lo);
+  const int slots = __builtin_amdgcn_readfirstlane(m == 1 ? min(W, hi - lo + 1) : 0);
+  const int tau0 = __builtin_amdgcn_readfirstlane(len - 1 + off) - lo_s;
+  const int steps = a.hs_steps;
+  // slots with a state to read (a timestep inside the caller's buffer): one run of them, as bits
+  const int j_lo = max(0, tau0 - steps + 1), j_hi = min(slots, tau0 + 1);
+  const unsigned live =
+      __builtin_amdgcn_readfirstlane(j_hi > j_lo ? ((2u << (j_hi - 1)) - 1u) & ~((1u << j_lo) - 1u) : 0u);
 
-  // the window, once
+  // The window, once.  A slot without a state to read loads a row that exists instead; its values
+  // are never used (no select per loaded register: they were most of this kernel's instructions).
+  int rows_at[NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) rows_at[q] = row_ok[q] ? (tid + q * kThreads) * 4 : 0;
+  auto slot_row = [&](const float *mem, int j) {
+    return mem + (size_t)min(max(tau0 - j, 0), steps - 1) * a.step_stride;
+  };
   float4 h[WCAP][NQ];
 #pragma unroll
   for (int j = 0; j < WCAP; ++j) {
-    const int tau = s_tau[j];  // the same for every thread: a scalar branch
+    const float *row = slot_row(hs_c, j);
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      h[j][q] = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (tau >= 0 && row_ok[q])
-        h[j][q] = *reinterpret_cast<const float4 *>(hs_c + (size_t)tau * a.step_stride +
-                                                    (size_t)(tid + q * kThreads) * 4);
-    }
+    for (int q = 0; q < NQ; ++q) h[j][q] = *reinterpret_cast<const float4 *>(row + rows_at[q]);
   }
   // scores: per-thread partial dot products, wavefront sums, then the four wavefronts in order
+  float part[32];
+#pragma unroll
+  for (int j = 0; j < 32; ++j) part[j] = 0.f;
 #pragma unroll
   for (int j = 0; j < WCAP; ++j) {
-    float sc = 0.f;
 #pragma unroll
-    for (int q = 0; q < NQ; ++q)
-      sc += h[j][q].x * w4[q].x + h[j][q].y * w4[q].y + h[j][q].z * w4[q].z + h[j][q].w * w4[q].w;
-    sc = lh::wave_sum(sc);
-    if (lane == 0) s_part[wave][j] = sc;
+    for (int q = 0; q < NQ; ++q) {
+      const float s = h[j][q].x * w4[q].x + h[j][q].y * w4[q].y + h[j][q].z * w4[q].z + h[j][q].w * w4[q].w;
+      part[j] += row_ok[q] ? s : 0.f;
+    }
   }
+  const float slot_sum = wave_sum_slots(part, lane);
+  if (lane % 2 == 0) s_part[wave][lane / 2] = slot_sum;
   if (a.ctx_mem) {
     // the scores are done with the window: the same registers take the window of ctx_mem, whose
     // loads fly while the scores are normalised
     const float *cm = a.ctx_mem + (size_t)col * a.col_stride;
 #pragma unroll
     for (int j = 0; j < WCAP; ++j) {
-      const int tau = s_tau[j];
+      const float *row = slot_row(cm, j);
 #pragma unroll
-      for (int q = 0; q < NQ; ++q) {
-        h[j][q] = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (tau >= 0 && row_ok[q])
-          h[j][q] = *reinterpret_cast<const float4 *>(cm + (size_t)tau * a.step_stride +
-                                                      (size_t)(tid + q * kThreads) * 4);
-      }
+      for (int q = 0; q < NQ; ++q) h[j][q] = *reinterpret_cast<const float4 *>(row + rows_at[q]);
     }
   }
   __syncthreads();
-  for (int j = tid; j < WCAP; j += kThreads) {
-    float sc = s_part[0][j];
+  // every wavefront normalises the whole window, lane j slot j
+  const bool valid = lane < slots;
+  float sc = 0.f;
+  if (lane < WCAP) {
+    sc = s_part[0][lane];
 #pragma unroll
-    for (int w = 1; w < kWaves; ++w) sc += s_part[w][j];
-    s_val[j] = s_tau[j] >= 0 ? sc : 0.f;
+    for (int w = 1; w < kWaves; ++w) sc += s_part[w][lane];
   }
-  __syncthreads();
-
-  float mx = D >= 0 ? 0.f : -FLT_MAX;
-  for (int j = 0; j < W; ++j) {
-    if (s_idx[j] != -1 && s_val[j] > mx) mx = s_val[j];
-  }
-  // one exponential per slot, taken by the slot's thread; the sum then runs over the slots in
-  // order as before
-  __shared__ float s_exp[WCAP];
-  for (int j = tid; j < WCAP; j += kThreads)
-    s_exp[j] = (j < W && s_idx[j] != -1) ? expf(s_val[j] - mx) : 0.f;
-  __syncthreads();
-  float Z = 0.f;
-  for (int j = 0; j < W; ++j) {
-    if (s_idx[j] != -1) Z += s_exp[j];
-  }
-  const float sigma_sq = (float)((D * D) / 4.0);
-  for (int j = tid; j < WCAP; j += kThreads) {
-    float al = 0.f, g = 1.f;
-    if (j < W) {
-      const int idx = s_idx[j];
-      if (idx != -1) {
-        const float e = s_exp[j];
-        if (D >= 0) {
-          const float dlt = p - (float)idx;
-          g = expf((-1.f * (dlt * dlt)) / (2.f * sigma_sq));
-        }
-        al = (Z != 0.f) ? (e / Z) * g : e;
-      }
-      a.align[b + (size_t)B * j] = al;
-      a.cached_exp[j + (size_t)W * b] = g;
+  const float val = lane < WCAP && ((live >> lane) & 1u) ? sc : 0.f;
+  const float floor_mx = D >= 0 ? 0.f : -FLT_MAX;
+  const float mx = lh::wave_max(valid ? fmaxf(val, floor_mx) : floor_mx);
+  const float e = valid ? expf(val - mx) : 0.f;
+  float Z = 0.f;  // in slot order
+#pragma unroll
+  for (int j = 0; j < WCAP; ++j) Z += lane_value(e, j);
+  float al = 0.f, g = 1.f;
+  if (valid) {
+    if (D >= 0) {
+      const float sigma_sq = (float)((D * D) / 4.0);
+      const float dlt = p - (float)(lo + lane);
+      g = expf((-1.f * (dlt * dlt)) / (2.f * sigma_sq));
     }
-    s_val[j] = al;
+    al = (Z != 0.f) ? (e / Z) * g : e;
   }
-  __syncthreads();
-
-  if (a.viterbi && tid == 0) {
-    float best = -1.f;
-    int best_idx = -1;
-    for (int j = 0; j < W; ++j) {
-      if (best < s_val[j]) {
-        best = s_val[j];
-        best_idx = s_idx[j];
-      }
+  if (wave == 0) {
+    if (lane < W) {
+      a.indices[b + (size_t)B * lane] = valid ? lo + lane : -1;
+      a.align[b + (size_t)B * lane] = al;
+      a.cached_exp[lane + (size_t)W * b] = g;
     }
-    a.viterbi[b] = best_idx;
+    if (a.viterbi) {
+      // the first slot of the largest weight (weights are >= 0, slots without a position weigh 0)
+      const float mine = lane < W ? al : -1.f;
+      const float best = lh::wave_max(fmaxf(mine, -1.f));
+      const unsigned long long at = __ballot(lane < W && mine == best);
+      const int first = at ? __ffsll(at) - 1 : -1;
+      if (lane == 0) a.viterbi[b] = best > -1.f && first >= 0 && first < slots ? lo + first : -1;
+    }
   }
 
   float *ctx = a.ctx + (size_t)b * H;
@@ -357,8 +408,9 @@ __global__ __launch_bounds__(kThreads) void attn_core_regs_kernel(const AttnArgs
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
     for (int j = 0; j < WCAP; ++j) {
-      if (s_tau[j] < 0) continue;  // the general kernel skips these slots too
-      const float w = s_val[j];
+      if (!((live >> j) & 1u)) continue;  // the general kernel skips these slots too
+      asm volatile("" ::: "memory");  // a scalar branch over four multiply-adds, not four selects
+      const float w = lane_value(al, j);
       acc.x += w * h[j][q].x; acc.y += w * h[j][q].y; acc.z += w * h[j][q].z; acc.w += w * h[j][q].w;
     }
     if (!row_ok[q]) continue;
@@ -415,8 +467,8 @@ extern "C" int lh_attn_core_fwd_f32(int H, int B, int D, int max_len, int hs_ste
     hipLaunchKernelGGL((attn_core_regs_kernel<1, kRegsSlots>), dim3(B), dim3(kThreads), 0, st, a);
   else if (vec && W <= kRegsSlots && H <= 8 * kThreads)
     hipLaunchKernelGGL((attn_core_regs_kernel<2, kRegsSlots>), dim3(B), dim3(kThreads), 0, st, a);
-  else if (vec) hipLaunchKernelGGL(attn_core_kernel<true>, dim3(B), dim3(kThreads), 0, st, a);
-  else hipLaunchKernelGGL(attn_core_kernel<false>, dim3(B), dim3(kThreads), 0, st, a);
+  else if (vec) hipLaunchKernelGGL(attn_core_kernel<true>, dim3(B), dim3(kWide), 0, st, a);
+  else hipLaunchKernelGGL(attn_core_kernel<false>, dim3(B), dim3(kWide), 0, st, a);
   return lh::check_launch("lh_attn_core_fwd_f32");
 }
 

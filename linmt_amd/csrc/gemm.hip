@@ -5,7 +5,7 @@
 // comes from X, its 2x32 operand from A), which makes the 32 lanes of an accumulator register hold
 // 32 consecutive m of one column n: stores to C are full 128-byte segments.
 //
-// Two kernels:
+// The kernels:
 //  * gemm_kernel (aligned operands, every tile configuration): 16-byte copies global -> registers
 //    -> LDS with no shuffles for either memory order (Stage); software pipeline two slabs deep;
 //    fragments read one group of 8 k ahead of the MFMAs that use them; the slab's staging work and
@@ -14,8 +14,9 @@
 //    time the matrix pipe stands still).  Products whose output has too few tiles split K across
 //    workgroups through partial planes in a caller workspace (splitk_reduce_kernel, or a consumer
 //    that adds the planes itself).  gate_gemm_cell_kernel is the same body with the LSTM cell as
-//    its epilogue.
-//  * gemm_generic_kernel (operands that are not 16-byte aligned): scalar loads, one tile shape.
+//    its epilogue, ragged::gemm_kernel the same body for operands at any float's address and with
+//    extents that are no multiple of 4.
+//  * gemm_generic_kernel (a ragged extent shorter than a copy or a tile): scalar loads, one tile shape.
 // WK > 1 splits every slab's k range over WK wavefront groups and reduces the partial
 // accumulators through LDS in a fixed order; deep slabs (BK 64/128) let one workgroup per CU hide
 // its own memory latency.  Workgroup ids are remapped so that each of the 8 XCDs (ids are dealt
@@ -25,6 +26,7 @@
 // (gemm_tuning.inc, regenerated by tune_gemm.py on the target GPU).
 #include "lh_common.h"
 
+#include <climits>
 #include <mutex>
 
 namespace {
@@ -56,6 +58,9 @@ struct GemmArgs {
   int splits, slabs_per_split;
   float *ws_part;
   int ws_ld;
+  // A (X) is contiguous along m (n) and that extent is no multiple of 4: the last row (column) of
+  // tiles is moved back to end with the operand, see gemm_body
+  int ragged_m, ragged_n;
   int leave_partial;  // host only: the caller sums the planes itself, no reduction launch
   // Gate product with the LSTM cell in its epilogue (gate_gemm_cell_kernel): M = 4 * cell_H rows
   // in gate order i, f, c', o; C (ldc) is a read-only addend to the pre-activations when beta = 1,
@@ -387,7 +392,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_generic_kernel(const G
 
 
 // =============================================================================================
-// Main kernel (16-byte aligned operands).  What shapes it:
+// Main kernel.  What shapes it:
 //   * On CDNA a VALU instruction and an MFMA do not overlap inside a SIMD: every non-MFMA vector
 //     instruction in the loop costs about four cycles of matrix-pipe time.  The loop therefore
 //     carries almost none.  Global addresses are a uniform base (scalar registers) plus
@@ -403,6 +408,25 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_generic_kernel(const G
 //     In both, lanes 0-31 take k = 8g+q and lanes 32-63 k = 8g+4+q for step q of group g: the K
 //     order inside a slab is a fixed permutation applied to both operands, which leaves the dot
 //     products unchanged.
+// RAGGED: operands need no alignment beyond a float's.  A 16-byte global load from any dword address
+// is one instruction here, and a wavefront's contiguous run only touches one more cache line.  What a
+// 16-byte unit must not do is reach past the operand, so where the contiguous extent is no
+// multiple of 4:
+//   * along m or n, the last tile is moved back to end with the operand (rows that the tile before
+//     it owns are computed again and not stored): the K loop knows nothing of it;
+//   * along k, the segment's last unit is loaded from up to three floats earlier and shifted into
+//     place on the masked path of the K tail, which the other slabs never take.
+// An output projection of 30003 words (M = 30003, K = 1000) at 84 columns took 128 us on the scalar
+// kernel and takes 64 us here, 48 columns 44 us, 12 columns 29 us.  Aligned operands keep kernels of their own: run through this
+// form the 128x96 gate product (768 columns) took 119 us instead of 107.
+typedef float unaligned_float4 __attribute__((ext_vector_type(4), aligned(4)));
+template <bool RAGGED>
+__device__ __forceinline__ float4 load4(const char *p) {
+  if constexpr (!RAGGED) return *reinterpret_cast<const float4 *>(p);
+  const unaligned_float4 t = *reinterpret_cast<const unaligned_float4 *>(p);
+  return make_float4(t.x, t.y, t.z, t.w);
+}
+
 __device__ __forceinline__ float4 keep_if(float4 w, bool c) {
   // per component: a select between two float4 objects makes the compiler pick an address
   w.x = c ? w.x : 0.f;
@@ -412,7 +436,17 @@ __device__ __forceinline__ float4 keep_if(float4 w, bool c) {
   return w;
 }
 
-template <int BD, int BK, int NT, bool KC>
+// The first `n` components of w, starting at its component 4 - n, and zeros (n <= 0: all zero).
+__device__ __forceinline__ float4 keep_last(float4 w, int n) {
+  float4 r;
+  r.x = n >= 4 ? w.x : (n == 3 ? w.y : (n == 2 ? w.z : (n == 1 ? w.w : 0.f)));
+  r.y = n >= 4 ? w.y : (n == 3 ? w.z : (n == 2 ? w.w : 0.f));
+  r.z = n >= 4 ? w.z : (n == 3 ? w.w : 0.f);
+  r.w = n >= 4 ? w.w : 0.f;
+  return r;
+}
+
+template <int BD, int BK, int NT, bool KC, bool RAGGED>
 struct Stage {
   static constexpr int KQ = BK / 4;
   // KC: 16-byte units per k-quad row.  A staging store walks k-quads first, and LDS takes 16-byte
@@ -433,6 +467,7 @@ struct Stage {
   float4 v[NU];
   unsigned goff[NU];  // byte offset of each unit from the slab origin
   unsigned ok;        // K-tail validity, one bit per unit
+  int ktail;          // RAGGED: k values in the K tail
 
   // unit u of the slab: (d, k) of its first element and its float offset in LDS
   static __device__ __forceinline__ int unit_d(int u) { return KC ? u / KQ : (u % (BD / 4)) * 4; }
@@ -464,25 +499,51 @@ struct Stage {
     }
   }
   // kn (< BK) = k values left in the segment: units past it re-read the slab origin and are
-  // zeroed before they reach LDS.
+  // zeroed before they reach LDS.  RAGGED: a unit along k that holds fewer than four of them is read
+  // from that many floats earlier; when it is the slab's first one the whole tail is addressed from
+  // four floats earlier (such a segment has at least four k values, so a slab lies before it).
+  static __device__ __forceinline__ int tail_back(int kn) { return RAGGED && KC && kn < 4 ? 4 : 0; }
   __device__ __forceinline__ void clamp_tail(int tid, int kn) {
-    ok = 0u;
+    if constexpr (RAGGED) {
+      ktail = kn;
+      const unsigned back = 4u * (unsigned)tail_back(kn);
 #pragma unroll
-    for (int i = 0; i < NU; ++i) {
-      const bool in = unit_k(tid + i * NT) < kn;
-      goff[i] = in ? goff[i] : 0u;
-      ok |= in ? (1u << i) : 0u;
+      for (int i = 0; i < NU; ++i) {
+        const int left = kn - unit_k(tid + i * NT);
+        unsigned off = goff[i] + back;
+        if (KC && left < 4) {
+          // a unit of a row past the tile's bound sits at the origin and stays there
+          const unsigned shift = 4u * (unsigned)(4 - left);
+          off = off >= shift ? off - shift : 0u;
+        }
+        goff[i] = left > 0 ? off : 0u;
+      }
+    } else {
+      ok = 0u;
+#pragma unroll
+      for (int i = 0; i < NU; ++i) {
+        const bool in = unit_k(tid + i * NT) < kn;
+        goff[i] = in ? goff[i] : 0u;
+        ok |= in ? (1u << i) : 0u;
+      }
     }
   }
   __device__ __forceinline__ void load(const float *__restrict__ base, int tid) {
     const char *b = reinterpret_cast<const char *>(base);
 #pragma unroll
     for (int i = 0; i < NU; ++i)
-      if (kExact || tid + i * NT < kUnits) v[i] = *reinterpret_cast<const float4 *>(b + goff[i]);
+      if (kExact || tid + i * NT < kUnits) v[i] = load4<RAGGED>(b + goff[i]);
   }
-  __device__ __forceinline__ void zero_tail() {
+  __device__ __forceinline__ void zero_tail(int tid) {
 #pragma unroll
-    for (int i = 0; i < NU; ++i) v[i] = keep_if(v[i], (ok >> i) & 1u);
+    for (int i = 0; i < NU; ++i) {
+      if constexpr (RAGGED) {
+        const int left = ktail - unit_k(tid + i * NT);
+        v[i] = keep_last(v[i], KC ? left : (left > 0 ? 4 : 0));
+      } else {
+        v[i] = keep_if(v[i], (ok >> i) & 1u);
+      }
+    }
   }
   __device__ __forceinline__ void store(float *__restrict__ buf, int tid) const {
 #pragma unroll
@@ -511,7 +572,7 @@ struct Stage {
 template <int BM, int BN, int WM, int WN, int WK, int BK, bool TA, bool TX>
 constexpr int smem2_floats() {
   constexpr int NT = 64 * WM * WN * WK;
-  return cmax(2 * (Stage<BM, BK, NT, TA>::kFloats + Stage<BN, BK, NT, !TX>::kFloats),
+  return cmax(2 * (Stage<BM, BK, NT, TA, false>::kFloats + Stage<BN, BK, NT, !TX, false>::kFloats),
               (WK - 1) * BM * BN);
 }
 
@@ -531,7 +592,7 @@ __device__ __forceinline__ int xcd_logical_id() {
   return xcd * per + (xcd < rem ? xcd : rem) + within;
 }
 
-template <int BM, int BN, int WM, int WN, int WK, int BK, bool TA, bool TX, bool CELL>
+template <int BM, int BN, int WM, int WN, int WK, int BK, bool TA, bool TX, bool CELL, bool RAGGED>
 __device__ __forceinline__ void gemm_body(const GemmArgs &g, const int logical) {
   constexpr int NT = 64 * WM * WN * WK;
   constexpr int TM = BM / WM, TN = BN / WN;
@@ -540,8 +601,8 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &g, const int logical) 
   constexpr int KPW = BK / WK;  // k values one wavefront group consumes per slab
   static_assert(KPW % 8 == 0, "a fragment group covers 8 k (4 per lane half)");
   constexpr int NG = KPW / 8;
-  using SA = Stage<BM, BK, NT, TA>;
-  using SX = Stage<BN, BK, NT, !TX>;
+  using SA = Stage<BM, BK, NT, TA, RAGGED>;
+  using SX = Stage<BN, BK, NT, !TX, RAGGED>;
   constexpr int kAF = SA::kFloats, kSlab = SA::kFloats + SX::kFloats;
   static_assert(smem2_floats<BM, BN, WM, WN, WK, BK, TA, TX>() * 4 <= 160 * 1024,
                 "LDS capacity of a CU");
@@ -552,8 +613,15 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &g, const int logical) 
   const int tile = splits == 1 ? logical : logical / splits;
   const int split = splits == 1 ? 0 : logical % splits;
   // CELL: m0 counts rows of ONE gate
-  const int m0 = (tile / g.tiles_n) * (CELL ? BM / 4 : BM);
-  const int n0 = (tile % g.tiles_n) * BN;
+  int m0 = (tile / g.tiles_n) * (CELL ? BM / 4 : BM);
+  int n0 = (tile % g.tiles_n) * BN;
+  // a tile that was moved back stores rows / columns from here on only (the host keeps the tile
+  // extent within a ragged operand's)
+  const int m_first = m0, n_first = n0;
+  if constexpr (RAGGED) {
+    if (!TA && g.ragged_m && m0 + BM > g.M) m0 = g.M - BM;
+    if (TX && g.ragged_n && n0 + BN > g.N) n0 = g.N - BN;
+  }
 
   const int tid = threadIdx.x;
   const int wave = tid / lh::kWave, lane = tid % lh::kWave;
@@ -629,6 +697,10 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &g, const int logical) 
       LH_KEEP_BRANCH();                                                            \
       sa.clamp_tail(tid, kleft);                                                   \
       sx.clamp_tail(tid, kleft);                                                   \
+      if constexpr (RAGGED) {                                                      \
+        pa -= SA::tail_back(kleft);                                                \
+        px -= SX::tail_back(kleft);                                                \
+      }                                                                            \
     }                                                                              \
     sa.load(pa, tid);                                                              \
     sx.load(px, tid);                                                              \
@@ -646,8 +718,8 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &g, const int logical) 
     float *sb = (BUF);        \
     if (tail) {               \
       LH_KEEP_BRANCH();       \
-      sa.zero_tail();         \
-      sx.zero_tail();         \
+      sa.zero_tail(tid);      \
+      sx.zero_tail(tid);      \
     }                         \
     sa.store(sb, tid);        \
     sx.store(sb + kAF, tid);  \
@@ -866,14 +938,14 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &g, const int logical) 
 #pragma unroll
     for (int b = 0; b < FM; ++b) {
       const int m = m0 + wm * TM + b * 32 + l32;
-      if (m >= g.M) continue;
+      if (m >= g.M || (RAGGED && m < m_first)) continue;
       const float bv = bias ? bias[m] : 0.f;
       const bool do_tanh = m < act_rows;
       const int nb = n0 + wn * TN + a * 32 + lhi * 4;
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
         const int n = nb + (j / 4) * 8 + (j % 4);
-        if (n >= g.N) continue;
+        if (n >= g.N || (RAGGED && n < n_first)) continue;
         float *cp = Cb + (size_t)n * ldc + m;
         float v = alpha * acc[a][b][j];
         if (use_beta) v += beta * *cp;
@@ -888,13 +960,20 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &g, const int logical) 
 
 template <int BM, int BN, int WM, int WN, int WK, int BK, bool TA, bool TX>
 __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_kernel(const GemmArgs g) {
-  gemm_body<BM, BN, WM, WN, WK, BK, TA, TX, false>(g, xcd_logical_id());
+  gemm_body<BM, BN, WM, WN, WK, BK, TA, TX, false, false>(g, xcd_logical_id());
 }
+
+namespace ragged {
+template <int BM, int BN, int WM, int WN, int WK, int BK, bool TA, bool TX>
+__global__ __launch_bounds__(64 * WM * WN * WK) void gemm_kernel(const GemmArgs g) {
+  gemm_body<BM, BN, WM, WN, WK, BK, TA, TX, false, true>(g, xcd_logical_id());
+}
+}  // namespace ragged
 
 // Stacked gate product W*[x; h; h~] (both operands as stored, no transposes) + LSTM cell.
 template <int BM, int BN, int WM, int WN, int WK, int BK>
 __global__ __launch_bounds__(64 * WM * WN * WK) void gate_gemm_cell_kernel(const GemmArgs g) {
-  gemm_body<BM, BN, WM, WN, WK, BK, false, false, true>(g, xcd_logical_id());
+  gemm_body<BM, BN, WM, WN, WK, BK, false, false, true, false>(g, xcd_logical_id());
 }
 
 // Several stacked gate products of one decoding step in ONE launch: everything that is known when
@@ -930,7 +1009,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gate_gemm_group_kernel(cons
   }
   if (tile < 0) return;
   const GemmArgs g = a.g[p];  // one copy into scalar registers: the K loop must not go back to memory
-  gemm_body<BM, BN, WM, WN, WK, BK, false, false, true>(g, tile);
+  gemm_body<BM, BN, WM, WN, WK, BK, false, false, true, false>(g, tile);
 }
 
 // Whether a configuration's LDS holds a whole tile, which the cell epilogue needs.
@@ -1001,7 +1080,7 @@ struct Config {
   X(4, 128, 64, 2, 2, 1, 32)                                                   \
   X(5, 64, 96, 2, 1, 2, 32)    /* stacked gate products at a few hundred columns */ \
   X(6, 64, 96, 2, 1, 2, 64)                                                    \
-  X(7, 64, 64, 2, 2, 1, 16)    /* also the only shape built for unaligned operands */ \
+  X(7, 64, 64, 2, 2, 1, 16)    /* also the only shape of the generic kernel */ \
   X(8, 64, 64, 2, 2, 1, 64)                                                    \
   X(9, 64, 64, 2, 2, 1, 128)                                                   \
   X(10, 32, 96, 1, 3, 2, 32)   /* M around 1000 */                             \
@@ -1044,6 +1123,12 @@ const Config kConfigs[] = {LH_GEMM_CONFIGS(LH_CFG_ENTRY)};
 #undef LH_CFG_ENTRY
 constexpr int kNumConfigs = sizeof(kConfigs) / sizeof(kConfigs[0]);
 constexpr int kUnalignedConfig = 7;
+// Configurations built for ragged operands as well: those that the cost model gives an aligned output
+// projection and its backward products at 5 to 2560 columns of 5000 to 30000 words, or one within
+// a few per cent of them.
+constexpr bool ragged_config(int c) {
+  return c == 0 || c == 3 || c == 7 || c == 12 || c == 15 || c == 18 || c == 24 || c == 32 || c == 35 || c == 36;
+}
 
 template <typename KernelT>
 int launch_kernel(KernelT kernel, int smem_bytes, dim3 grid, dim3 block, hipStream_t st,
@@ -1069,26 +1154,44 @@ int launch_kernel(KernelT kernel, int smem_bytes, dim3 grid, dim3 block, hipStre
   return lh::check_launch("lh_gemm_f32");
 }
 
-template <int BM, int BN, int WM, int WN, int WK, int BK, bool ALLOW_UNALIGNED>
-int launch_cfg(const GemmArgs &g0, bool ta, bool tx, bool vec, hipStream_t st) {
+// What takes a product: the scalar kernel, the main kernel for aligned operands, or its form for
+// ragged ones.
+enum Form { kGeneric, kRagged, kAligned };
+
+template <int BM, int BN, int WM, int WN, int WK, int BK, bool ALLOW_UNALIGNED, bool ALLOW_RAGGED>
+int launch_cfg(const GemmArgs &g0, bool ta, bool tx, Form form, hipStream_t st) {
   GemmArgs g = g0;
   g.tiles_m = (g.M + BM - 1) / BM;
   g.tiles_n = (g.N + BN - 1) / BN;
-  if (!vec) g.splits = 1;
+  if (form == kGeneric) g.splits = 1;
   int slabs = 0;
   for (int s = 0; s < g.nseg; ++s) slabs += (g.K[s] + BK - 1) / BK;
   g.slabs_per_split = (slabs + g.splits - 1) / g.splits;
   g.splits = (slabs + g.slabs_per_split - 1) / g.slabs_per_split;  // no empty share
   const dim3 grid(g.tiles_m * g.tiles_n * g.splits), block(64 * WM * WN * WK);
-  if (vec) {
-    int rc;
+  if (form != kGeneric) {
+    int rc = LH_OK;
+    if (form == kRagged) {
+      if constexpr (!ALLOW_RAGGED) {
+        return lh::fail_arg("lh_gemm_f32: internal error, ragged operands reached an aligned-only tile");
+      } else {
+#define LH_GEMM_LAUNCH(TA, TX)                                                              \
+  rc = launch_kernel(ragged::gemm_kernel<BM, BN, WM, WN, WK, BK, TA, TX>,                   \
+                     smem2_floats<BM, BN, WM, WN, WK, BK, TA, TX>() * 4, grid, block, st, g)
+        if (!ta && !tx) LH_GEMM_LAUNCH(false, false);
+        else if (ta) LH_GEMM_LAUNCH(true, false);
+        else LH_GEMM_LAUNCH(false, true);
+#undef LH_GEMM_LAUNCH
+      }
+    } else {
 #define LH_GEMM_LAUNCH(TA, TX)                                                              \
   rc = launch_kernel(gemm_kernel<BM, BN, WM, WN, WK, BK, TA, TX>,                           \
                      smem2_floats<BM, BN, WM, WN, WK, BK, TA, TX>() * 4, grid, block, st, g)
-    if (!ta && !tx) LH_GEMM_LAUNCH(false, false);
-    else if (ta) LH_GEMM_LAUNCH(true, false);
-    else LH_GEMM_LAUNCH(false, true);
+      if (!ta && !tx) LH_GEMM_LAUNCH(false, false);
+      else if (ta) LH_GEMM_LAUNCH(true, false);
+      else LH_GEMM_LAUNCH(false, true);
 #undef LH_GEMM_LAUNCH
+    }
     if (rc != LH_OK || g.splits == 1 || g.leave_partial) return rc;
     // four rows per thread; small products in single-wavefront workgroups, to reach more CUs
     const size_t total = (size_t)(g.ws_ld / 4) * g.N;
@@ -1110,11 +1213,11 @@ int launch_cfg(const GemmArgs &g0, bool ta, bool tx, bool vec, hipStream_t st) {
   return lh::fail_arg("lh_gemm_f32: internal error, unaligned operands reached an aligned-only tile");
 }
 
-int launch_index(int c, const GemmArgs &g, bool ta, bool tx, bool vec, hipStream_t st) {
+int launch_index(int c, const GemmArgs &g, bool ta, bool tx, Form form, hipStream_t st) {
   switch (c) {
 #define LH_CFG_CASE(I, BM, BN, WM, WN, WK, BK) \
   case I:                                      \
-    return launch_cfg<BM, BN, WM, WN, WK, BK, I == kUnalignedConfig>(g, ta, tx, vec, st);
+    return launch_cfg<BM, BN, WM, WN, WK, BK, I == kUnalignedConfig, ragged_config(I)>(g, ta, tx, form, st);
     LH_GEMM_CONFIGS(LH_CFG_CASE)
 #undef LH_CFG_CASE
     default: return lh::fail_arg("lh_gemm_f32: configuration %d does not exist", c);
@@ -1257,12 +1360,15 @@ float predict_us(const Tuning &t, const Config &k, int M, int N, const int *K, i
 // only_cell: restrict the choice to unsplit launches of configurations whose LDS holds a whole
 // tile (what the gate product with the cell in its epilogue can use).  *us (optional) receives
 // the predicted time of the choice.
-void pick_config(int M, int N, const int *K, int nseg, bool ta, bool tx, bool vec,
+// Ragged operands: max_bm / max_bn are the largest tile extents allowed (a ragged extent must hold a
+// whole tile), INT_MAX where the extent is a multiple of 4.
+void pick_config(int M, int N, const int *K, int nseg, bool ta, bool tx, Form form,
                  size_t workspace_bytes, int max_planes, int *config, int *splits,
-                 bool only_cell = false, float *us_out = nullptr) {
+                 bool only_cell = false, float *us_out = nullptr, int max_bm = INT_MAX,
+                 int max_bn = INT_MAX) {
   *splits = 1;
   if (us_out) *us_out = 0.f;
-  if (!vec) {
+  if (form == kGeneric) {
     *config = kUnalignedConfig;
     return;
   }
@@ -1274,7 +1380,9 @@ void pick_config(int M, int N, const int *K, int nseg, bool ta, bool tx, bool ve
   };
   static thread_local Memo memo[64];
   const int flags = 1 + (ta ? 2 : 0) + (tx ? 4 : 0) + 8 * nseg + 64 * (g_config_override + 1) +
-                    4096 * g_splits_override + 131072 * max_planes + (only_cell ? 1048576 : 0);
+                    4096 * g_splits_override + 131072 * max_planes + (only_cell ? 1048576 : 0) +
+                    (max_bm <= M ? 2097152 : 0) + (max_bn <= N ? 4194304 : 0) +
+                    (form == kRagged ? 8388608 : 0);
   int Kk[LH_GEMM_MAX_SEGS] = {0, 0, 0};
   for (int s = 0; s < nseg; ++s) Kk[s] = K[s];
   const unsigned h = ((unsigned)M * 2654435761u) ^ ((unsigned)N * 40503u) ^ ((unsigned)Kk[0] * 97u) ^
@@ -1295,6 +1403,7 @@ void pick_config(int M, int N, const int *K, int nseg, bool ta, bool tx, bool ve
   for (int c = 0; c < kNumConfigs; ++c) {
     if (g_config_override >= 0 && c != g_config_override) continue;
     if (only_cell && !cell_capable_index(c)) continue;
+    if (form == kRagged && (!ragged_config(c) || kConfigs[c].bm > max_bm || kConfigs[c].bn > max_bn)) continue;
     for (int want : kSplitChoices) {
       if (only_cell && want > 1) break;
       if (!only_cell && g_splits_override > 0) want = fit_splits(M, N, g_splits_override, workspace_bytes);
@@ -1310,14 +1419,15 @@ void pick_config(int M, int N, const int *K, int nseg, bool ta, bool tx, bool ve
       if (g_splits_override > 0 || (max_planes > 0 && want >= max_planes)) break;
     }
   }
-  if (best > 2.9e38f) *config = -1;  // only_cell: the override names a configuration that cannot
+  if (best > 2.9e38f) *config = -1;  // the override names a configuration that cannot run this
   if (us_out) *us_out = best;
   e = Memo{M, N, {Kk[0], Kk[1], Kk[2]}, flags, *config, *splits, workspace_bytes, best};
 }
 
 struct Prepared {
   GemmArgs g;
-  bool ta, tx, vec;
+  bool ta, tx;
+  Form form;
   int config;
 };
 
@@ -1333,7 +1443,7 @@ int prepare(int M, int N, const lh_gemm_seg *segs, int nseg, int transA, int tra
 
   GemmArgs &g = out->g;
   g = GemmArgs{};
-  bool vec = true;
+  bool vec = true, aligned = true;
   for (int s = 0; s < nseg; ++s) {
     const lh_gemm_seg &e = segs[s];
     if (!e.A || !e.X || e.K <= 0)
@@ -1348,14 +1458,21 @@ int prepare(int M, int N, const lh_gemm_seg *segs, int nseg, int transA, int tra
     g.lda[s] = e.lda;
     g.ldx[s] = e.ldx;
     g.K[s] = e.K;
-    // 16-byte loads need aligned bases / leading dimensions and a contiguous extent that is a
-    // multiple of 4 (the guards test only the first element of a float4).
     const int a_extent = transA ? e.K : M, x_extent = transX ? N : e.K;
-    // ... and the main kernel keeps per-thread byte offsets inside a slab in 32 bits.
+    // the main kernel keeps per-thread byte offsets inside a slab in 32 bits
     constexpr int kMaxLd = 1 << 22;
-    vec = vec && lh::aligned16(e.A) && lh::aligned16(e.X) && e.lda % 4 == 0 && e.ldx % 4 == 0 &&
-          a_extent % 4 == 0 && x_extent % 4 == 0 && e.lda < kMaxLd && e.ldx < kMaxLd;
+    vec = vec && e.lda < kMaxLd && e.ldx < kMaxLd;
+    aligned = aligned && lh::aligned16(e.A) && lh::aligned16(e.X) && e.lda % 4 == 0 &&
+              e.ldx % 4 == 0 && a_extent % 4 == 0 && x_extent % 4 == 0;
+    // a unit along k that is short of four values reaches back inside its row
+    if ((transA || !transX) && e.K < 4) vec = false;
   }
+  // A tile along a ragged m (n) moves back inside the operand: it must be at least a tile long.  The
+  // narrowest tiles are 32 wide; below that the scalar kernel runs a single row of tiles anyway.
+  const bool ragged_m = !transA && M % 4 != 0, ragged_n = transX && N % 4 != 0;
+  if ((ragged_m && M < 32) || (ragged_n && N < 32)) vec = false;
+  g.ragged_m = ragged_m ? 1 : 0;
+  g.ragged_n = ragged_n ? 1 : 0;
   for (int s = nseg; s < LH_GEMM_MAX_SEGS; ++s) {  // unused slots mirror segment 0 (never read)
     g.A[s] = g.A[0];
     g.X[s] = g.X[0];
@@ -1376,10 +1493,15 @@ int prepare(int M, int N, const lh_gemm_seg *segs, int nseg, int transA, int tra
   g.ldc = ldc;
   out->ta = transA != 0;
   out->tx = transX != 0;
-  out->vec = vec;
   if (!workspace || !lh::aligned16(workspace)) workspace_bytes = 0;
-  pick_config(M, N, g.K, nseg, transA != 0, transX != 0, vec, workspace_bytes, max_planes,
-              &out->config, &g.splits);
+  out->form = !vec ? kGeneric : (aligned ? kAligned : kRagged);
+  pick_config(M, N, g.K, nseg, transA != 0, transX != 0, out->form, workspace_bytes, max_planes,
+              &out->config, &g.splits, false, nullptr, ragged_m ? M : INT_MAX, ragged_n ? N : INT_MAX);
+  if (out->config < 0) {  // the configuration override does not fit a ragged operand
+    out->form = kGeneric;
+    out->config = kUnalignedConfig;
+    g.splits = 1;
+  }
   g.leave_partial = max_planes > 0 ? 1 : 0;
   g.ws_part = static_cast<float *>(workspace);
   g.ws_ld = plane_ld(M);
@@ -1398,7 +1520,7 @@ extern "C" int lh_gemm_ws_f32(int M, int N, const lh_gemm_seg *segs, int nseg, i
   const int rc = prepare(M, N, segs, nseg, transA, transX, alpha, beta, bias, act, act_rows,
                          colmask, C, ldc, workspace, workspace_bytes, 0, &p);
   if (rc != LH_OK) return rc;
-  return launch_index(p.config, p.g, p.ta, p.tx, p.vec, lh::as_stream(stream));
+  return launch_index(p.config, p.g, p.ta, p.tx, p.form, lh::as_stream(stream));
 }
 
 extern "C" int lh_gemm_planes_f32(int M, int N, const lh_gemm_seg *segs, int nseg, int transA,
@@ -1415,10 +1537,10 @@ extern "C" int lh_gemm_planes_f32(int M, int N, const lh_gemm_seg *segs, int nse
   const Config &k = kConfigs[p.config];
   int slabs = 0;
   for (int s = 0; s < p.g.nseg; ++s) slabs += (p.g.K[s] + k.bk - 1) / k.bk;
-  const int want = p.vec ? p.g.splits : 1;
+  const int want = p.form != kGeneric ? p.g.splits : 1;
   const int share = (slabs + want - 1) / want;
   *planes = (slabs + share - 1) / share;
-  return launch_index(p.config, p.g, p.ta, p.tx, p.vec, lh::as_stream(stream));
+  return launch_index(p.config, p.g, p.ta, p.tx, p.form, lh::as_stream(stream));
 }
 
 namespace {
@@ -1435,15 +1557,15 @@ int plan_cell(int H, int B, const lh_gemm_seg *segs, int nseg, bool has_addend, 
                          has_addend ? 2 : 3, p);
   if (rc != LH_OK) return rc;
   *fusable = false;
-  if (!p->vec || H % 4 != 0) return LH_OK;
+  if (p->form != kAligned || H % 4 != 0) return LH_OK;
   // Best unsplit launch that can carry the cell against the best launch of any kind followed by
   // the cell kernel (a launch of its own that reads the pre-activations, or S planes of them, back).
   int cfg_any, splits_any, cfg_cell, splits_cell;
   float us_any, us_cell;
   const size_t ws = workspace_bytes;
-  pick_config(4 * H, B, p->g.K, nseg, false, false, true, ws, has_addend ? 2 : 3, &cfg_any, &splits_any,
+  pick_config(4 * H, B, p->g.K, nseg, false, false, kAligned, ws, has_addend ? 2 : 3, &cfg_any, &splits_any,
               false, &us_any);
-  pick_config(4 * H, B, p->g.K, nseg, false, false, true, ws, has_addend ? 2 : 3, &cfg_cell,
+  pick_config(4 * H, B, p->g.K, nseg, false, false, kAligned, ws, has_addend ? 2 : 3, &cfg_cell,
               &splits_cell, true, &us_cell);
   if (cfg_cell < 0) return LH_OK;
   const float cell_us = kCellFixedUs + 28.f * (float)H * (float)B / kReduceBytesPerUs;
@@ -1646,7 +1768,7 @@ int plan_group(int H, int B, const lh_gate_problem *pr, int n, GroupArgs *a, int
     const int rc = prepare(4 * H, B, q.segs, q.nseg, 0, 0, 1.f, q.cell && q.addend ? 1.f : 0.f, nullptr,
                            LH_ACT_NONE, 4 * H, nullptr, C, ldc, nullptr, 0, 0, &pp);
     if (rc != LH_OK) return rc;
-    vec = vec && pp.vec && (q.cell || (lh::aligned16(q.out) && q.ld_out % 4 == 0));
+    vec = vec && pp.form == kAligned && (q.cell || (lh::aligned16(q.out) && q.ld_out % 4 == 0));
     GemmArgs &g = a->g[p];
     g = pp.g;
     a->cell[p] = q.cell ? 1 : 0;
@@ -1866,7 +1988,7 @@ extern "C" int lh_gemm_kernel_name(int M, int N, const lh_gemm_seg *segs, int ns
                          workspace_bytes, max_planes, &p);
   if (rc != LH_OK) return rc;
   const Config &k = kConfigs[p.config];
-  if (p.vec)
+  if (p.form != kGeneric)
     snprintf(name, name_cap, "gemm_kernel<%d, %d, %d, %d, %d, %d, %s, %s>", k.bm, k.bn, k.wm, k.wn,
              k.wk, k.bk, p.ta ? "true" : "false", p.tx ? "true" : "false");
   else

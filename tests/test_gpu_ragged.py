@@ -74,3 +74,72 @@ def test_ragged_products(lh, M, N, Ks, tA, tX, splits):
         L.lh_gemm_set_splits_override(0)
     generic = (not tA and M % 4 and M < 32) or (tX and N % 4 and N < 32) or ((tA or not tX) and min(Ks) < 4)
     assert all(n.startswith("gemm_generic" if generic else "gemm_kernel") for n in names), names
+
+
+@pytest.mark.parametrize("V", [13, 4097, 8191, 30003, 65533])
+@pytest.mark.parametrize("off", [0, 1])
+def test_ragged_columns(lh, V, off):
+    rng = np.random.default_rng(V + off)
+    B, K = 7, 13
+    z = rng.normal(0, 3, (V, B)).astype(np.float32)
+    z[:, 1] = np.round(z[:, 1])              # ties
+    z[:, 2] = 0.25                           # everything ties
+    z[V - 1, 3] = 40.0                       # the last row of the partial quad wins
+    if V > K:
+        z[5:, 4] = -np.inf                   # fewer finite rows than candidates
+    tgt = rng.integers(0, V, B).astype(np.int32)
+    tgt[0], tgt[4] = V - 1, 2
+    mask = np.array([1, 1, 0, 1, 1, 1, 1], np.int32)
+    dz, dt, dm = _odd(z, off), torch.from_numpy(tgt).cuda(), torch.from_numpy(mask).cuda()
+    z64 = z.astype(np.float64)
+    logp = z64 - scipy.special.logsumexp(z64, axis=0)
+    p = np.exp(logp)
+
+    def fresh():
+        return torch.full((V * B + 8,), 7.0, device="cuda")[1:]
+
+    out = fresh()
+    lh.softmax_fwd(dz, V, None, V, B, out, V)
+    got = out.cpu().numpy()
+    assert_close(got[:V * B].reshape(B, V).T, p, "probabilities", rtol=2e-6, atol=1e-9)
+    assert np.all(got[V * B:] == 7.0)
+
+    lt, loss = torch.zeros(B, dtype=torch.float64, device="cuda"), torch.zeros(1, dtype=torch.float64, device="cuda")
+    lh.logsoftmax_xent(dz, V, None, V, B, dt, dm, lt, loss)
+    # double exponentials, as in the strided kernel: only the fp32 logits bound the result
+    assert_close(lt.cpu().numpy(), logp[tgt, np.arange(B)], "log p", rtol=1e-12, atol=1e-12)
+    assert_close(loss.cpu().numpy()[0], (logp[tgt, np.arange(B)] * mask).sum(), "loss", rtol=1e-12, atol=1e-12)
+
+    out = fresh()
+    loss.zero_()
+    lh.softmax_xent_grad(dz, V, None, V, B, dt, dm, out, V, lt, loss)
+    got = out.cpu().numpy()
+    onehot = np.zeros((V, B))
+    onehot[tgt, np.arange(B)] = 1.0
+    assert_close(got[:V * B].reshape(B, V).T, (onehot - p) * mask, "output error", rtol=4e-6, atol=2e-7)
+    assert np.all(got[V * B:] == 7.0)
+
+    cl, ci = torch.empty(K * B, device="cuda"), torch.empty(K * B, dtype=torch.int32, device="cuda")
+    le = torch.empty(B, device="cuda")
+    lh.beam_topk(dz, V, None, V, B, K, 1, cl, ci, le)
+    gi, gl = ci.cpu().numpy().reshape(B, K), cl.cpu().numpy().reshape(B, K)
+    for b in range(B):
+        order = np.lexsort((np.arange(V), -z64[:, b]))[:K]
+        assert gi[b].tolist() == order.tolist(), f"column {b}"
+        finite = np.isfinite(logp[order, b])
+        assert np.array_equal(gl[b][~finite], logp[order, b][~finite])   # -inf
+        assert_close(gl[b][finite], logp[order, b][finite], f"column {b} scores", rtol=1e-5, atol=1e-5)
+    assert_close(le.cpu().numpy(), logp[1], "log p(<EOF>)", rtol=1e-5, atol=1e-5)
+
+
+def test_partial_nan_column(lh):
+    """A column of NaN holds no candidate: K rounds of arg-max over nothing, as the strided kernel gives."""
+    V, B, K = 4099, 2, 5
+    z = np.full((V, B), np.nan, np.float32)
+    z[:, 1] = np.arange(V) / V
+    cl, ci = torch.zeros(K * B, device="cuda"), torch.zeros(K * B, dtype=torch.int32, device="cuda")
+    le = torch.empty(B, device="cuda")
+    lh.beam_topk(_odd(z, 0), V, None, V, B, K, 1, cl, ci, le)
+    gi = ci.cpu().numpy().reshape(B, K)
+    assert gi[0].tolist() == [0x7fffffff] * K
+    assert gi[1].tolist() == [V - 1 - i for i in range(K)]

@@ -691,6 +691,10 @@ int lh_attn_core_bwd_f32(int H, int B, int D, int max_len, int hs_steps, const f
  * sumsq is read on the device, so no host synchronisation sits between norm and update.
  */
 #define LH_SUMSQ_WORKSPACE 1024
+/* dst[0:rows, 0:cols] = src[0:rows, 0:cols], both column-major (leading dimensions ld_dst, ld_src);
+ * the blocks must not overlap. */
+int lh_copy_block_f32(float *dst, long long ld_dst, const float *src, long long ld_src, long long rows,
+                      long long cols, lh_stream_t stream);
 int lh_grad_sumsq_f32(const float *g, long long rows, long long cols, long long ld, float scale,
                       double *workspace, double *accum, lh_stream_t stream);
 int lh_sgd_step_f32(float *theta, long long ld_theta, float *g, long long ld_g, long long rows,

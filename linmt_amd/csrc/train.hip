@@ -1,6 +1,8 @@
 // Training-side kernels: fused LSTM cell backward, attention backward, bias-gradient row sums,
 // deterministic embedding-gradient gather, gradient norm and the fused clip + SGD step.
 // All of them are HBM-bound passes: one coalesced read of every input, one write of every output.
+#include <algorithm>
+
 #include "lh_common.h"
 
 namespace {
@@ -383,6 +385,22 @@ __global__ __launch_bounds__(kAT) void attn_core_bwd_kernel(const AttnBwdArgs a)
 }
 
 // ---------------------------------------------------------------------------------------------
+// A rows x cols block of one column-major matrix into another: packs one gate's rows of a stacked
+// matrix together for a copy to the host, which then is one contiguous run.  The runtime's strided
+// copy to pageable host memory moves a column at a time: 7.1 ms for 1000 columns of 4 kB, 0.4 ms
+// this way.
+template <typename T>
+__global__ __launch_bounds__(256) void copy_block_kernel(T *__restrict__ dst, long long ld_dst,
+                                                         const T *__restrict__ src, long long ld_src,
+                                                         long long rows, long long cols) {
+  const long long n = rows * cols;
+  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) {
+    const long long c = i / rows, r = i - c * rows;
+    dst[c * ld_dst + r] = src[c * ld_src + r];
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
 // accum[0] += sum (scale * g)^2 over a rows x cols view.  Each thread sums runs of up to 64 squares
 // in float and adds the runs in double; a workgroup's threads are combined through a fixed-order
 // LDS fold, and the workgroups' partials by one more workgroup, again in a fixed order: the result
@@ -646,6 +664,26 @@ extern "C" int lh_attn_core_bwd_f32(int H, int B, int D, int max_len, int hs_ste
   if (vec) hipLaunchKernelGGL(attn_core_bwd_kernel<true>, dim3(B), dim3(kAT), 0, st, a);
   else hipLaunchKernelGGL(attn_core_bwd_kernel<false>, dim3(B), dim3(kAT), 0, st, a);
   return lh::check_launch("lh_attn_core_bwd_f32");
+}
+
+extern "C" int lh_copy_block_f32(float *dst, long long ld_dst, const float *src, long long ld_src,
+                                 long long rows, long long cols, lh_stream_t stream) {
+  if (rows <= 0 || cols < 0 || !dst || !src || ld_dst < rows || ld_src < rows)
+    return lh::fail_arg("lh_copy_block_f32: rows=%lld cols=%lld ld_dst=%lld ld_src=%lld or NULL pointer",
+                        rows, cols, ld_dst, ld_src);
+  if (cols == 0) return LH_OK;
+  const bool vec = rows % 4 == 0 && ld_dst % 4 == 0 && ld_src % 4 == 0 && lh::aligned16(dst) && lh::aligned16(src);
+  const long long units = vec ? rows / 4 * cols : rows * cols;
+  const unsigned blocks = (unsigned)std::min<long long>((units + 255) / 256, 65536);
+  hipStream_t st = lh::as_stream(stream);
+  if (vec)
+    hipLaunchKernelGGL(copy_block_kernel<float4>, dim3(blocks), dim3(256), 0, st,
+                       reinterpret_cast<float4 *>(dst), ld_dst / 4, reinterpret_cast<const float4 *>(src),
+                       ld_src / 4, rows / 4, cols);
+  else
+    hipLaunchKernelGGL(copy_block_kernel<float>, dim3(blocks), dim3(256), 0, st, dst, ld_dst, src, ld_src,
+                       rows, cols);
+  return lh::check_launch("lh_copy_block_f32");
 }
 
 extern "C" int lh_grad_sumsq_f32(const float *g, long long rows, long long cols, long long ld,

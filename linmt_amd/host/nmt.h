@@ -515,6 +515,11 @@ class NeuralMachineTranslation {
   // stream_, which is the ordering that sharing it requires.
   static constexpr size_t kGemmWorkspaceBytes = size_t(64) << 20;
   DeviceArray<char> gemm_workspace_;
+  // Rows x cols floats of a strided device matrix (leading dimension ld) <-> a contiguous host block,
+  // packed on the device through gemm_workspace_ so that the host copies are contiguous runs.
+  // Ordered on stream_; the host block is complete after Synchronize().
+  void DownloadBlock(const float *p_device, long long ld, int rows, int cols, float *host);
+  void UploadBlock(float *p_device, long long ld, int rows, int cols, const float *host);
   // the part of it the products launched right now may use (all of it on the single stream; one
   // slice per layer while the encoder's layers run side by side)
   char *gemm_ws_ptr_ = nullptr;

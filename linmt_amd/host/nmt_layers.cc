@@ -21,18 +21,13 @@ int GateIndex(char g) {  // stacked order i, f, c', o
 }
 
 // Host H x K column-major block <-> rows [gate*H, (gate+1)*H) of a stacked 4H x K device matrix.
-void UploadGateBlock(DeviceArray<float> &stack, int gate, int H, int K, const float *host,
-                     hipStream_t s) {
-  HipErrorWrapper(hipMemcpy2DAsync(stack.get() + (size_t)gate * H, sizeof(float) * 4 * H, host,
-                                   sizeof(float) * H, sizeof(float) * H, K, hipMemcpyHostToDevice, s),
-                  "parameter upload failed");
+void UploadGateBlock(NeuralMachineTranslation &M, DeviceArray<float> &stack, int gate, int H, int K,
+                     const float *host) {
+  M.UploadBlock(stack.get() + (size_t)gate * H, 4LL * H, H, K, host);
 }
-void DownloadGateBlock(const DeviceArray<float> &stack, int gate, int H, int K, float *host,
-                       hipStream_t s) {
-  HipErrorWrapper(hipMemcpy2DAsync(host, sizeof(float) * H, stack.get() + (size_t)gate * H,
-                                   sizeof(float) * 4 * H, sizeof(float) * H, K,
-                                   hipMemcpyDeviceToHost, s),
-                  "parameter download failed");
+void DownloadGateBlock(NeuralMachineTranslation &M, const DeviceArray<float> &stack, int gate, int H,
+                       int K, float *host) {
+  M.DownloadBlock(stack.get() + (size_t)gate * H, 4LL * H, H, K, host);
 }
 
 bool SetFlat(DeviceArray<float> &a, const float *host, size_t n, hipStream_t s) {
@@ -147,19 +142,19 @@ bool LstmLayer::SetParam(const std::string &name, const float *host, size_t n) {
   if (name.size() == 3 && name[0] == 'M' && name[1] == '_') {
     const int g = GateIndex(name[2]);
     if (g < 0 || n != (size_t)H * input_size_) return false;
-    UploadGateBlock(p_device_m_stack_, g, H, input_size_, host, s);
+    UploadGateBlock(*p_neural_mt_, p_device_m_stack_, g, H, input_size_, host);
     return true;
   }
   if (name.size() == 4 && name.compare(0, 3, "W_h") == 0) {
     const int g = GateIndex(name[3]);
     if (g < 0 || n != (size_t)H * H) return false;
-    UploadGateBlock(p_device_w_h_stack_, g, H, H, host, s);
+    UploadGateBlock(*p_neural_mt_, p_device_w_h_stack_, g, H, H, host);
     return true;
   }
   if (name.size() == 3 && name[0] == 'Q' && name[1] == '_') {
     const int g = GateIndex(name[2]);
     if (g < 0 || !feed_input_mode_ || n != (size_t)H * H) return false;
-    UploadGateBlock(p_device_q_stack_, g, H, H, host, s);
+    UploadGateBlock(*p_neural_mt_, p_device_q_stack_, g, H, H, host);
     return true;
   }
   if (name.size() == 3 && name[0] == 'b' && name[1] == '_') {
@@ -190,7 +185,7 @@ bool LstmLayer::GetParam(const std::string &name, std::vector<float> *out) {
   }
   if (!stack || g < 0) return false;
   out->resize((size_t)H * K);
-  DownloadGateBlock(*stack, g, H, K, out->data(), s);
+  DownloadGateBlock(*p_neural_mt_, *stack, g, H, K, out->data());
   HipErrorWrapper(hipStreamSynchronize(s), "parameter download failed");
   return true;
 }

@@ -35,6 +35,41 @@ void NeuralMachineTranslation::Gemm(int tag, int rows, int cols, const lh_gemm_s
                  what);
 }
 
+namespace {
+// Columns of `rows` floats that fit the staging buffer at a time.
+int StagedColumns(size_t bytes, int rows) {
+  return (int)std::max<size_t>(1, std::min<size_t>(bytes / sizeof(float) / rows, 1 << 20));
+}
+}  // namespace
+
+void NeuralMachineTranslation::DownloadBlock(const float *p_device, long long ld, int rows, int cols,
+                                             float *host) {
+  float *staged = reinterpret_cast<float *>(gemm_workspace_.get());
+  const int step = StagedColumns(gemm_workspace_.size(), rows);
+  for (int c = 0; c < cols; c += step) {
+    const int n = std::min(step, cols - c);
+    LhErrorWrapper(lh_copy_block_f32(staged, rows, p_device + (size_t)c * ld, ld, rows, n, stream_),
+                   "packing a block for the host");
+    HipErrorWrapper(hipMemcpyAsync(host + (size_t)c * rows, staged, sizeof(float) * (size_t)rows * n,
+                                   hipMemcpyDeviceToHost, stream_),
+                    "GPU memcpy D2H failed");
+  }
+}
+
+void NeuralMachineTranslation::UploadBlock(float *p_device, long long ld, int rows, int cols,
+                                           const float *host) {
+  float *staged = reinterpret_cast<float *>(gemm_workspace_.get());
+  const int step = StagedColumns(gemm_workspace_.size(), rows);
+  for (int c = 0; c < cols; c += step) {
+    const int n = std::min(step, cols - c);
+    HipErrorWrapper(hipMemcpyAsync(staged, host + (size_t)c * rows, sizeof(float) * (size_t)rows * n,
+                                   hipMemcpyHostToDevice, stream_),
+                    "GPU memcpy H2D failed");
+    LhErrorWrapper(lh_copy_block_f32(p_device + (size_t)c * ld, ld, staged, rows, rows, n, stream_),
+                   "unpacking a block from the host");
+  }
+}
+
 // A large product as a split product: both operands packed into the model's two scratch buffers by
 // one launch, then lh_gemm_split_f32.  false = not worthwhile or not expressible; the caller runs
 // the fp32 MFMA product.

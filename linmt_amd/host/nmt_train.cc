@@ -51,14 +51,11 @@ bool DownloadAll(const DeviceArray<float> &a, size_t n, std::vector<float> *out,
   return true;
 }
 
-bool DownloadGate(const DeviceArray<float> &stack, int gate, int H, int K, std::vector<float> *out,
-                  hipStream_t s) {
+bool DownloadGate(NeuralMachineTranslation &M, const DeviceArray<float> &stack, int gate, int H, int K,
+                  std::vector<float> *out) {
   out->resize((size_t)H * K);
-  HipErrorWrapper(hipMemcpy2DAsync(out->data(), sizeof(float) * H, stack.get() + (size_t)gate * H,
-                                   sizeof(float) * 4 * H, sizeof(float) * H, K,
-                                   hipMemcpyDeviceToHost, s),
-                  "gradient download failed");
-  HipErrorWrapper(hipStreamSynchronize(s), "gradient download failed");
+  M.DownloadBlock(stack.get() + (size_t)gate * H, 4LL * H, H, K, out->data());
+  M.Synchronize();
   return true;
 }
 
@@ -295,11 +292,11 @@ bool LstmLayer::GetGrad(const std::string &name, std::vector<float> *out) {
     return input_layer_mode_ &&
            DownloadAll(p_device_small_w_grad_, (size_t)input_size_ * w_grad_length_, out, s);
   if (name.size() == 3 && name[0] == 'M' && name[1] == '_' && GateIndex(name[2]) >= 0)
-    return DownloadGate(p_device_m_grad_, GateIndex(name[2]), H, input_size_, out, s);
+    return DownloadGate(*p_neural_mt_, p_device_m_grad_, GateIndex(name[2]), H, input_size_, out);
   if (name.size() == 4 && name.compare(0, 3, "W_h") == 0 && GateIndex(name[3]) >= 0)
-    return DownloadGate(p_device_w_h_grad_, GateIndex(name[3]), H, H, out, s);
+    return DownloadGate(*p_neural_mt_, p_device_w_h_grad_, GateIndex(name[3]), H, H, out);
   if (name.size() == 3 && name[0] == 'Q' && name[1] == '_' && feed_input_mode_ && GateIndex(name[2]) >= 0)
-    return DownloadGate(p_device_q_grad_, GateIndex(name[2]), H, H, out, s);
+    return DownloadGate(*p_neural_mt_, p_device_q_grad_, GateIndex(name[2]), H, H, out);
   if (name.size() == 3 && name[0] == 'b' && name[1] == '_' && GateIndex(name[2]) >= 0) {
     out->resize(H);
     p_device_b_grad_.Download(out->data(), H, s, (size_t)GateIndex(name[2]) * H);

@@ -147,6 +147,8 @@ SIGNATURES = {
                                       C.c_int, C.c_int, c_i32p, C.c_int, c_f32p, C.c_void_p]),
     "lh_softmax_xent_grad_f32": (C.c_int, [c_f32p, C.c_int, c_f32p, C.c_int, C.c_int, c_i32p,
                                            c_i32p, c_f32p, C.c_int, c_f64p, c_f64p, C.c_void_p]),
+    "lh_copy_block_f32": (C.c_int, [c_f32p, C.c_longlong, c_f32p, C.c_longlong, C.c_longlong, C.c_longlong,
+                                    C.c_void_p]),
     "lh_uniform_f32": (C.c_int, [c_f32p, C.c_longlong, C.c_ulonglong, C.c_void_p]),
     "lh_lstm_cell_bwd_f32": (C.c_int, [C.c_int, C.c_int, c_f32p, c_f32p, c_f32p, c_f32p, c_f32p,
                                        c_f32p, c_i32p, C.c_float, C.c_float, c_f32p, C.c_float,

@@ -1,7 +1,7 @@
 """Operands whose contiguous extent is no multiple of four floats or that start at an odd float: the
 products' moved-back last tiles and shifted K tails (lh_gemm_ws_f32), the vocabulary kernels' guarded
 last quad (lh_softmax_fwd_f32, lh_logsoftmax_xent_f32, lh_softmax_xent_grad_f32, lh_beam_topk_f32), and
-the reduction of split planes, against float64.
+the reduction of split planes, against float64; and copies of strided blocks.
 
 Tolerances: a product of K terms rounds K + 8 times at most, each by 2^-24 of the sum of magnitudes.
 """
@@ -143,3 +143,20 @@ def test_partial_nan_column(lh):
     gi = ci.cpu().numpy().reshape(B, K)
     assert gi[0].tolist() == [0x7fffffff] * K
     assert gi[1].tolist() == [V - 1 - i for i in range(K)]
+
+
+@pytest.mark.parametrize("rows,cols,ld_dst,ld_src", [(4, 1, 4, 16), (1000, 7, 1000, 4000), (37, 5, 37, 148),
+                                                     (8, 3, 9, 32), (1, 300, 1, 4)])
+@pytest.mark.parametrize("off", [0, 1])
+def test_copy_block(lh, rows, cols, ld_dst, ld_src, off):
+    """lh_copy_block_f32: exact, and nothing beside the block is written."""
+    rng = np.random.default_rng(rows)
+    src = torch.from_numpy(rng.random(ld_src * cols + off + 8, dtype=np.float32)).cuda()
+    dst = torch.full((ld_dst * cols + off + 8,), 7.0, device="cuda")
+    lh.check(lh.load().lh_copy_block_f32(dst[off:].data_ptr(), ld_dst, src[off:].data_ptr(), ld_src, rows, cols,
+                                         torch.cuda.current_stream().cuda_stream), "lh_copy_block_f32")
+    want = np.full(ld_dst * cols + off + 8, 7.0, np.float32)
+    s = src.cpu().numpy()
+    for c in range(cols):
+        want[off + c * ld_dst: off + c * ld_dst + rows] = s[off + c * ld_src: off + c * ld_src + rows]
+    assert np.array_equal(dst.cpu().numpy(), want)

@@ -697,6 +697,23 @@ int lh_copy_block_f32(float *dst, long long ld_dst, const float *src, long long 
                       long long cols, lh_stream_t stream);
 int lh_grad_sumsq_f32(const float *g, long long rows, long long cols, long long ld, float scale,
                       double *workspace, double *accum, lh_stream_t stream);
+/* The same two for many tensors in a few launches.  An item with norm >= 0 has its squares added to
+ * norms[norm] and is rescaled by it; norm < 0: neither.  Items that share a slot must follow one another.
+ * workspace holds lh_grad_sumsq_items_workspace(items, n) doubles. */
+typedef struct {
+  float *theta;
+  long long ld_theta;
+  float *grad;
+  long long ld_grad, rows, cols;
+  const int *col_index;
+  int norm;
+} lh_update_item;
+size_t lh_grad_sumsq_items_workspace(const lh_update_item *items, int n);
+int lh_grad_sumsq_items_f32(const lh_update_item *items, int n, float scale, double *workspace,
+                            double *norms, lh_stream_t stream);
+int lh_sgd_step_items_f32(const lh_update_item *items, int n, float learning_rate, float grad_scale,
+                          const double *norms, float norm_clip, float individual_clip,
+                          lh_stream_t stream);
 int lh_sgd_step_f32(float *theta, long long ld_theta, float *g, long long ld_g, long long rows,
                     long long cols, const int *col_index, float learning_rate, float grad_scale,
                     const double *sumsq, float norm_clip, float individual_clip,

@@ -385,6 +385,121 @@ __global__ __launch_bounds__(kAT) void attn_core_bwd_kernel(const AttnBwdArgs a)
 }
 
 // ---------------------------------------------------------------------------------------------
+// Norm and update of many tensors in a few launches: the items of a launch ride in its arguments, a
+// workgroup finds its item and takes kItemUnits units (quads of floats where the item allows them).
+// A tensor at a time they were 2 + 1 launches for every matrix and every gate of it, most of them too
+// small for the GPU, and read a float per thread with a 64-bit division for its place.
+// Four layers of 1000 hidden units, each gate clipped by itself (110 tensors, 110 M floats): 2.07 -> 0.43 ms
+// for norms and update, 5.1 TB/s; one layer of 256: 0.36 -> 0.04 ms.
+constexpr int kItems = 40;
+constexpr int kFoldNT = 256;
+constexpr int kItemUnits = 2048;  // eight units per thread
+
+struct ItemArgs {
+  struct Item {
+    float *theta, *grad;
+    const int *col_index;
+    long long units, rows, ld_theta, ld_grad;  // in units
+    int norm, vec;
+  } item[kItems];
+  int first_block[kItems + 1];
+  int n;
+};
+struct FoldArgs {
+  int first[kItems + 1], norm[kItems];
+  int n;
+};
+static_assert(sizeof(ItemArgs) <= 3600, "kernel arguments");
+
+__device__ __forceinline__ int item_of(const ItemArgs &a, int block) {
+  int i = 0;
+  while (block >= a.first_block[i + 1]) ++i;
+  return i;
+}
+
+// The units of a workgroup's share, eight per thread: fn(unit's offset in grad, in theta).
+template <typename T, typename F>
+__device__ __forceinline__ void each_unit(const ItemArgs::Item &it, int share, const F &fn) {
+  const long long u0 = (long long)share * kItemUnits + threadIdx.x;
+#pragma unroll
+  for (int k = 0; k < kItemUnits / 256; ++k) {
+    const long long u = u0 + k * 256;
+    if (u >= it.units) break;
+    long long c = 0, r = u;
+    if (u >= it.rows) {
+      if (it.units < (1LL << 31)) c = (long long)((unsigned)u / (unsigned)it.rows);
+      else c = u / it.rows;
+      r = u - c * it.rows;
+    }
+    fn(c * it.ld_grad + r, (it.col_index ? (long long)it.col_index[c] : c) * it.ld_theta + r);
+  }
+}
+
+__global__ __launch_bounds__(256) void sumsq_items_kernel(const ItemArgs a, float scale,
+                                                          double *__restrict__ partial) {
+  __shared__ double red[256 / lh::kWave];
+  const int i = item_of(a, blockIdx.x), share = blockIdx.x - a.first_block[i];
+  const ItemArgs::Item &it = a.item[i];
+  float f = 0.f;  // at most 32 squares in float, then double
+  if (it.vec)
+    each_unit<float4>(it, share, [&](long long og, long long) {
+      const float4 t = reinterpret_cast<const float4 *>(it.grad)[og];
+      const float x = scale * t.x, y = scale * t.y, z = scale * t.z, w = scale * t.w;
+      f += (x * x + y * y) + (z * z + w * w);
+    });
+  else
+    each_unit<float>(it, share, [&](long long og, long long) {
+      const float v = scale * it.grad[og];
+      f += v * v;
+    });
+  const double s = lh::block_sum<256 / lh::kWave>((double)f, red);
+  if (threadIdx.x == 0) partial[blockIdx.x] = s;
+}
+
+// one workgroup per run of items that share a slot
+__global__ __launch_bounds__(kFoldNT) void fold_items_kernel(const FoldArgs f, const double *partial,
+                                                             double *norms) {
+  __shared__ double red[kFoldNT / lh::kWave];
+  double s = 0.0;
+  for (int i = f.first[blockIdx.x] + threadIdx.x; i < f.first[blockIdx.x + 1]; i += kFoldNT) s += partial[i];
+  s = lh::block_sum<kFoldNT / lh::kWave>(s, red);
+  if (threadIdx.x == 0) norms[f.norm[blockIdx.x]] += s;
+}
+
+__global__ __launch_bounds__(256) void sgd_items_kernel(const ItemArgs a, float lr, float scale,
+                                                        const double *__restrict__ norms, float norm_clip,
+                                                        float individual_clip) {
+  const int i = item_of(a, blockIdx.x), share = blockIdx.x - a.first_block[i];
+  const ItemArgs::Item &it = a.item[i];
+  float f = 1.f;
+  if (it.norm >= 0) {
+    const float nrm = (float)sqrt(norms[it.norm]);
+    if (nrm > norm_clip) f = norm_clip / nrm;
+  }
+  auto step = [&](float &theta, float g) {
+    float v = scale * g;
+    v = f * v;
+    v = clampf(v, individual_clip);
+    theta += lr * v;
+  };
+  if (it.vec)
+    each_unit<float4>(it, share, [&](long long og, long long ot) {
+      float4 &g = reinterpret_cast<float4 *>(it.grad)[og];
+      float4 &t = reinterpret_cast<float4 *>(it.theta)[ot];
+      const float4 gv = g;
+      float4 tv = t;
+      step(tv.x, gv.x), step(tv.y, gv.y), step(tv.z, gv.z), step(tv.w, gv.w);
+      t = tv;
+      g = make_float4(0.f, 0.f, 0.f, 0.f);
+    });
+  else
+    each_unit<float>(it, share, [&](long long og, long long ot) {
+      step(it.theta[ot], it.grad[og]);
+      it.grad[og] = 0.f;
+    });
+}
+
+// ---------------------------------------------------------------------------------------------
 // A rows x cols block of one column-major matrix into another: packs one gate's rows of a stacked
 // matrix together for a copy to the host, which then is one contiguous run.  The runtime's strided
 // copy to pageable host memory moves a column at a time: 7.1 ms for 1000 columns of 4 kB, 0.4 ms
@@ -407,7 +522,6 @@ __global__ __launch_bounds__(256) void copy_block_kernel(T *__restrict__ dst, lo
 // depends on the shape of the launch only.  VEC: the view is one contiguous, 16-byte aligned run,
 // read as four-float vectors with four loads in flight per thread.
 constexpr int kNT = 1024;
-constexpr int kFoldNT = 256;
 template <bool VEC>
 __global__ __launch_bounds__(kNT) void sumsq_kernel(const float *__restrict__ g, long long rows,
                                                     long long cols, long long ld, float scale,
@@ -664,6 +778,97 @@ extern "C" int lh_attn_core_bwd_f32(int H, int B, int D, int max_len, int hs_ste
   if (vec) hipLaunchKernelGGL(attn_core_bwd_kernel<true>, dim3(B), dim3(kAT), 0, st, a);
   else hipLaunchKernelGGL(attn_core_bwd_kernel<false>, dim3(B), dim3(kAT), 0, st, a);
   return lh::check_launch("lh_attn_core_bwd_f32");
+}
+
+namespace {
+// Reads an item table into launches of at most kItems items; fn(args, blocks, partials before) for each.
+bool item_ok(const lh_update_item &it, bool need_theta) {
+  return it.rows > 0 && it.cols >= 0 && it.grad && it.ld_grad >= it.rows &&
+         (!need_theta || (it.theta && it.ld_theta >= it.rows));
+}
+long long item_units(const lh_update_item &it, bool *vec) {
+  *vec = it.rows % 4 == 0 && it.ld_grad % 4 == 0 && it.ld_theta % 4 == 0 && lh::aligned16(it.grad) &&
+         lh::aligned16(it.theta) && it.rows / 4 * it.cols < (1LL << 31);
+  return *vec ? it.rows / 4 * it.cols : it.rows * it.cols;
+}
+long long item_blocks(const lh_update_item &it) {
+  bool vec;
+  return (item_units(it, &vec) + kItemUnits - 1) / kItemUnits;
+}
+void add_item(ItemArgs &a, const lh_update_item &it) {
+  bool vec;
+  ItemArgs::Item &o = a.item[a.n];
+  o.theta = it.theta, o.grad = it.grad, o.col_index = it.col_index;
+  o.units = item_units(it, &vec);
+  o.vec = vec;
+  o.rows = vec ? it.rows / 4 : it.rows;
+  o.ld_theta = vec ? it.ld_theta / 4 : it.ld_theta;
+  o.ld_grad = vec ? it.ld_grad / 4 : it.ld_grad;
+  o.norm = it.norm;
+  a.first_block[a.n + 1] = a.first_block[a.n] + (int)item_blocks(it);
+  ++a.n;
+}
+}  // namespace
+
+extern "C" size_t lh_grad_sumsq_items_workspace(const lh_update_item *items, int n) {
+  size_t total = 1;
+  for (int i = 0; items && i < n; ++i)
+    if (item_ok(items[i], false)) total += (size_t)item_blocks(items[i]);
+  return total;
+}
+
+extern "C" int lh_grad_sumsq_items_f32(const lh_update_item *items, int n, float scale, double *workspace,
+                                       double *norms, lh_stream_t stream) {
+  if (n < 0 || (n && !items) || !workspace || !norms)
+    return lh::fail_arg("lh_grad_sumsq_items_f32: n=%d or NULL pointer", n);
+  for (int i = 0; i < n; ++i) {
+    if (!item_ok(items[i], false)) return lh::fail_arg("lh_grad_sumsq_items_f32: item %d", i);
+    for (int j = 0; j + 1 < i; ++j)
+      if (items[i].norm >= 0 && items[j].norm == items[i].norm && items[i - 1].norm != items[i].norm)
+        return lh::fail_arg("lh_grad_sumsq_items_f32: items %d and %d share a slot and are apart", j, i);
+  }
+  hipStream_t st = lh::as_stream(stream);
+  for (int i = 0; i < n;) {
+    ItemArgs a{};
+    FoldArgs f{};
+    for (; i < n && a.n < kItems; ++i) {
+      if (items[i].norm < 0 || items[i].cols == 0) continue;
+      if (!f.n || f.norm[f.n - 1] != items[i].norm) f.norm[f.n++] = items[i].norm;
+      add_item(a, items[i]);
+      f.first[f.n] = a.first_block[a.n];
+    }
+    if (!a.n) break;
+    hipLaunchKernelGGL(sumsq_items_kernel, dim3((unsigned)a.first_block[a.n]), dim3(256), 0, st, a, scale, workspace);
+    int rc = lh::check_launch("lh_grad_sumsq_items_f32");
+    if (rc != LH_OK) return rc;
+    hipLaunchKernelGGL(fold_items_kernel, dim3((unsigned)f.n), dim3(kFoldNT), 0, st, f, workspace, norms);
+    rc = lh::check_launch("lh_grad_sumsq_items_f32 (fold)");
+    if (rc != LH_OK) return rc;
+  }
+  return LH_OK;
+}
+
+extern "C" int lh_sgd_step_items_f32(const lh_update_item *items, int n, float learning_rate,
+                                     float grad_scale, const double *norms, float norm_clip,
+                                     float individual_clip, lh_stream_t stream) {
+  if (n < 0 || (n && !items)) return lh::fail_arg("lh_sgd_step_items_f32: n=%d or NULL pointer", n);
+  for (int i = 0; i < n; ++i) {
+    if (!item_ok(items[i], true)) return lh::fail_arg("lh_sgd_step_items_f32: item %d", i);
+    if (items[i].norm >= 0 && (!norms || !(norm_clip > 0.f)))
+      return lh::fail_arg("lh_sgd_step_items_f32: item %d needs norms and norm_clip > 0", i);
+  }
+  hipStream_t st = lh::as_stream(stream);
+  for (int i = 0; i < n;) {
+    ItemArgs a{};
+    for (; i < n && a.n < kItems; ++i)
+      if (items[i].cols) add_item(a, items[i]);
+    if (!a.n) break;
+    hipLaunchKernelGGL(sgd_items_kernel, dim3((unsigned)a.first_block[a.n]), dim3(256), 0, st, a, learning_rate,
+                       grad_scale, norms, norm_clip, individual_clip);
+    const int rc = lh::check_launch("lh_sgd_step_items_f32");
+    if (rc != LH_OK) return rc;
+  }
+  return LH_OK;
 }
 
 extern "C" int lh_copy_block_f32(float *dst, long long ld_dst, const float *src, long long ld_src,

@@ -772,31 +772,43 @@ void NeuralMachineTranslation::UpdateWeights() {
   if (items.size() > p_device_norms_.size()) p_device_norms_.Alloc(items.size() + 64);
   p_device_norms_.Zero(stream_);
   const float scale = 1.0f / (float)cfg_.minibatch_size_;  // ScaleGradients
-  if (mode == 1 || mode == 2) {
-    for (size_t i = 0; i < items.size(); ++i) {
-      const UpdateItem &it = items[i];
-      if (mode == 2 && !it.in_global_norm) continue;  // the embedding gradients are not in the norm
-      ProfileScope ps(profiler_, kTagUpdate, 4.0 * it.rows * it.cols);
-      LhErrorWrapper(lh_grad_sumsq_f32(it.grad, it.rows, it.cols, it.ld_grad, scale,
-                                       p_device_norm_workspace_.get(),
-                                       p_device_norms_.get() + (mode == 2 ? 0 : i), stream_),
-                     "CalculateGlobalNorm");
-    }
-  }
+  // one slot per item, or one for all but the embedding gradients, which the global norm leaves out
+  std::vector<lh_update_item> table, live;
+  double elements = 0, live_elements = 0;
   for (size_t i = 0; i < items.size(); ++i) {
     const UpdateItem &it = items[i];
-    const double *nrm = mode == 2 ? p_device_norms_.get() : (mode == 1 ? p_device_norms_.get() + i : nullptr);
-    if (it.frozen) {
-      // the gradient is dropped, row block by row block (columns are ld_grad apart)
-      HipErrorWrapper(hipMemset2DAsync(it.grad, sizeof(float) * it.ld_grad, 0, sizeof(float) * it.rows,
-                                       (size_t)it.cols, stream_),
-                      "UpdateParams: clearing a frozen group's gradient failed");
-      continue;
+    const int norm = mode == 2 ? (it.in_global_norm ? 0 : -1) : (mode == 1 ? (int)i : -1);
+    const lh_update_item entry{it.theta, it.ld_theta, it.grad, it.ld_grad, it.rows, it.cols, it.col_index, norm};
+    if (norm >= 0) {
+      table.push_back(entry);
+      elements += (double)it.rows * it.cols;
     }
-    ProfileScope ps(profiler_, kTagUpdate, 16.0 * it.rows * it.cols);
-    LhErrorWrapper(lh_sgd_step_f32(it.theta, it.ld_theta, it.grad, it.ld_grad, it.rows, it.cols,
-                                   it.col_index, cfg_.learning_rate_, scale, nrm, cfg_.norm_clip_,
-                                   mode == 3 ? cfg_.individual_norm_clip_threshold_ : 0.f, stream_),
+    if (!it.frozen) {
+      live.push_back(entry);
+      if (mode == 2) live.back().norm = 0;  // ... but not the rescaling
+      live_elements += (double)it.rows * it.cols;
+    }
+  }
+  if (!table.empty()) {
+    const size_t need = lh_grad_sumsq_items_workspace(table.data(), (int)table.size());
+    if (need > p_device_norm_workspace_.size()) p_device_norm_workspace_.Alloc(need);
+    ProfileScope ps(profiler_, kTagUpdate, 4.0 * elements);
+    LhErrorWrapper(lh_grad_sumsq_items_f32(table.data(), (int)table.size(), scale,
+                                           p_device_norm_workspace_.get(), p_device_norms_.get(), stream_),
+                   "CalculateGlobalNorm");
+  }
+  for (const UpdateItem &it : items) {
+    if (!it.frozen) continue;
+    // the gradient is dropped, row block by row block (columns are ld_grad apart)
+    HipErrorWrapper(hipMemset2DAsync(it.grad, sizeof(float) * it.ld_grad, 0, sizeof(float) * it.rows,
+                                     (size_t)it.cols, stream_),
+                    "UpdateParams: clearing a frozen group's gradient failed");
+  }
+  if (!live.empty()) {
+    ProfileScope ps(profiler_, kTagUpdate, 16.0 * live_elements);
+    LhErrorWrapper(lh_sgd_step_items_f32(live.data(), (int)live.size(), cfg_.learning_rate_, scale,
+                                         p_device_norms_.get(), cfg_.norm_clip_,
+                                         mode == 3 ? cfg_.individual_norm_clip_threshold_ : 0.f, stream_),
                    "UpdateParams");
   }
   double ss = 0;

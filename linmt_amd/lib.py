@@ -31,6 +31,11 @@ class GemmSeg(C.Structure):
                 ("K", C.c_int)]
 
 
+class UpdateItem(C.Structure):
+    _fields_ = [("theta", C.c_void_p), ("ld_theta", C.c_longlong), ("grad", C.c_void_p), ("ld_grad", C.c_longlong),
+                ("rows", C.c_longlong), ("cols", C.c_longlong), ("col_index", C.c_void_p), ("norm", C.c_int)]
+
+
 class GateProblem(C.Structure):
     _fields_ = [("segs", GemmSeg * LH_GEMM_MAX_SEGS), ("nseg", C.c_int), ("cell", C.c_int),
                 ("addend", C.c_void_p), ("ld_addend", C.c_int), ("addend_col", C.c_void_p),
@@ -169,6 +174,10 @@ SIGNATURES = {
                                        c_f32p, c_f32p, C.c_void_p]),
     "lh_grad_sumsq_f32": (C.c_int, [c_f32p, C.c_longlong, C.c_longlong, C.c_longlong, C.c_float,
                                     c_f64p, c_f64p, C.c_void_p]),
+    "lh_grad_sumsq_items_workspace": (C.c_size_t, [C.c_void_p, C.c_int]),
+    "lh_grad_sumsq_items_f32": (C.c_int, [C.c_void_p, C.c_int, C.c_float, C.c_void_p, C.c_void_p, C.c_void_p]),
+    "lh_sgd_step_items_f32": (C.c_int, [C.c_void_p, C.c_int, C.c_float, C.c_float, C.c_void_p, C.c_float,
+                                        C.c_float, C.c_void_p]),
     "lh_sgd_step_f32": (C.c_int, [c_f32p, C.c_longlong, c_f32p, C.c_longlong, C.c_longlong,
                                   C.c_longlong, c_i32p, C.c_float, C.c_float, c_f64p, C.c_float,
                                   C.c_float, C.c_void_p]),

@@ -367,6 +367,10 @@ class SoftmaxLayer : public BaseLossLayer {
   bool split_dirty_ = true;
   void BuildSplitWeights();
   void ComputeLogitsSplit(float *p_device_h_t, int minibatch);
+  // scoring: logits and log-probabilities of a group of steps (kept between calls, grow-only)
+  DeviceArray<float> loss_logits_;
+  DeviceArray<double> loss_logp_;
+  void LossAllSteps(const float *p_device_h_t_all, int steps);
   DeviceArray<float> p_device_outputdist_;           // V x B logits / probabilities (one step)
   DeviceArray<double> p_device_logp_tgt_, p_device_loss_, p_device_train_perplexity_;
   DeviceArray<int> p_device_output_vocab_indices_, p_device_output_vocab_indices_01_;

@@ -342,6 +342,9 @@ void NeuralMachineTranslation::ForwardTeacherForced(const int *p_host_source, in
     attention_layer_.projected_memory_ = false;  // a decoding batch's memory is not this pass's
   }
   softmax_layer_.p_device_loss_.Zero(stream_);
+  // Scoring reads nothing back per step: with every allocated column in use the steps' states are one
+  // matrix, and the output projection runs over many steps at a time.
+  const bool all_steps_loss = per_step_loss && B == cfg_.minibatch_size_;
 
   if (seq2seq) RunSourceSide(source_length, B);
   {
@@ -390,7 +393,7 @@ void NeuralMachineTranslation::ForwardTeacherForced(const int *p_host_source, in
     }
     softmax_layer_.SetHTPtr(t, top);
     softmax_layer_.BackPropPreprocessGpu(top, (int)step);
-    if (!per_step_loss) continue;
+    if (!per_step_loss || all_steps_loss) continue;
     // ComputeLossGpu without the per-step host read-back: accumulate on the device
     softmax_layer_.ComputeLogits(top, B);
     ProfileScope px(profiler_, kTagXent, 4.0 * cfg_.target_vocab_size_ * B);
@@ -402,6 +405,10 @@ void NeuralMachineTranslation::ForwardTeacherForced(const int *p_host_source, in
                                softmax_layer_.p_device_logp_tgt_.get(),
                                softmax_layer_.p_device_loss_.get(), stream_),
         "GetError loss");
+  }
+  if (all_steps_loss) {
+    const float *tops = attention ? attention_layer_.final_all_.get() : UpwardState(TargetLayer(L - 1), 0);
+    softmax_layer_.LossAllSteps(tops, target_length);
   }
 }
 

@@ -1404,6 +1404,9 @@ void pick_config(int M, int N, const int *K, int nseg, bool ta, bool tx, Form fo
     if (g_config_override >= 0 && c != g_config_override) continue;
     if (only_cell && !cell_capable_index(c)) continue;
     if (form == kRagged && (!ragged_config(c) || kConfigs[c].bm > max_bm || kConfigs[c].bn > max_bn)) continue;
+    // Wavefronts that split K are for vocabularies (an extent in the thousands, where they are worth up
+    // to 2x); smaller ragged products keep one chain of K per tile, as on the scalar kernel.
+    if (form == kRagged && kConfigs[c].wk > 1 && M < 1024 && N < 1024 && Kk[0] + Kk[1] + Kk[2] < 1024) continue;
     for (int want : kSplitChoices) {
       if (only_cell && want > 1) break;
       if (!only_cell && g_splits_override > 0) want = fit_splits(M, N, g_splits_override, workspace_bytes);

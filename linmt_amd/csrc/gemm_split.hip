@@ -131,9 +131,19 @@ struct SplitArgs {
 // WK wavefront groups share a tile: a slab is 16*WK deep and group wk takes its k-groups 2wk, 2wk+1
 // (a product with few tiles is bound by the chain slab -> fragments -> MFMAs -> barrier of one
 // workgroup; WK shortens that chain).  The groups' partial tiles are added up through LDS.
+//
+// DA (one wavefront along n): a fragment of A belongs to one wavefront alone, and its 32 rows x 16 k are
+// two contiguous 512-byte runs of a plane, so the wavefront loads it from memory straight into the
+// registers the MFMA reads, four slabs ahead; only X goes through LDS.  With A staged too, the 128x96
+// gate product was LDS-bound (139 KB a slab, 1086 cycles of the CU's LDS pipe beside 1152 of MFMAs).
+// H = 1000, 768 columns, K = 2000: 74.6 -> 70.5 us (1.05 PFLOP/s of bf16 products).
+// A thread's share of X is then a whole number of units, the surplus past the slab loading zeros from
+// past the descriptor's end into LDS nobody reads: a guarded load would put a branch, and a wait for
+// every load before it, into the loop.
 template <int BM, int BN, int WK>
-constexpr int split_lds_bytes(bool cell) {
-  const int stages = 2 * 6 * WK * (BM + BN) * 16, tile = (cell || WK > 1) ? BN * (BM + 4) * 4 : 0;
+constexpr int split_lds_bytes(bool cell, bool da, int nt) {
+  const int ux = 6 * WK * BN, staged = da ? (ux + nt - 1) / nt * nt : ux + 6 * WK * BM;
+  const int stages = 2 * staged * 16, tile = (cell || WK > 1) ? BN * (BM + 4) * 4 : 0;
   return stages > tile ? stages : tile;
 }
 
@@ -150,10 +160,12 @@ __attribute__((amdgpu_waves_per_eu(split_waves_per_simd<BM, BN, WK, CELL>()))) v
   constexpr int NT = 64 * WM * WN * WK, TM = BM / WM, TN = BN / WN, FM = TM / 32, FN = TN / 32;
   static_assert(FM >= 1 && FN >= 1 && TM % 32 == 0 && TN % 32 == 0, "wave tile = 32x32 MFMA tiles");
   constexpr int KGL = 2 * WK;                         // k-groups of a slab
-  constexpr int UA = 3 * KGL * BM, UX = 3 * KGL * BN;  // 16-byte units of a slab: planes x k-groups x rows
-  constexpr int NUA = (UA + NT - 1) / NT, NUX = (UX + NT - 1) / NT;
-  constexpr bool kExactA = UA % NT == 0, kExactX = UX % NT == 0;
-  constexpr int STAGE = UA + UX;
+  constexpr bool DA = WN == 1;
+  // 16-byte units of a staged slab: planes x k-groups x rows
+  constexpr int UA = DA ? 0 : 3 * KGL * BM, UX = 3 * KGL * BN;
+  constexpr int NUA = DA ? 1 : (UA + NT - 1) / NT, NUX = (UX + NT - 1) / NT;
+  constexpr bool kExactA = !DA && UA % NT == 0, kExactX = DA || UX % NT == 0;
+  constexpr int STAGE = DA ? NUX * NT : UA + UX;
   static_assert(!CELL || BM % (4 * kGateRows) == 0, "a cell tile holds whole groups of 8 rows per gate");
   extern __shared__ u4v lds[];
   const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
@@ -174,14 +186,15 @@ __attribute__((amdgpu_waves_per_eu(split_waves_per_simd<BM, BN, WK, CELL>()))) v
   // Scalar slab origins + per-thread byte offsets that never change: no vector ALU in the loop.
   unsigned oa[NUA], ox[NUX];
 #pragma unroll
-  for (int i = 0; i < NUA; ++i) {
-    const int u = (tid + i * NT) % UA, p = u / (KGL * BM), kgl = (u / BM) % KGL, r = u % BM;
+  for (int i = 0; i < (DA ? 0 : NUA); ++i) {
+    const int u = (tid + i * NT) % (DA ? 1 : UA), p = u / (KGL * BM), kgl = (u / BM) % KGL, r = u % BM;
     oa[i] = (unsigned)((p * g.KG + kgl) * g.Mp + r) * 16u;
   }
 #pragma unroll
   for (int i = 0; i < NUX; ++i) {
     const int u = (tid + i * NT) % UX, p = u / (KGL * BN), kgl = (u / BN) % KGL, r = u % BN;
     ox[i] = (unsigned)((p * g.KG + kgl) * g.Np + r) * 16u;
+    if (DA && tid + i * NT >= UX) ox[i] = 0xFFFFFFF0u;
   }
   // Buffer loads: the descriptor and the slab origin are scalars, the unit offset a 32-bit vector
   // register -- nothing to compute per load.  (The host keeps a packed operand below 4 GiB.)
@@ -194,12 +207,23 @@ __attribute__((amdgpu_waves_per_eu(split_waves_per_simd<BM, BN, WK, CELL>()))) v
   const unsigned step_a = (unsigned)KGL * g.Mp * 16u, step_x = (unsigned)KGL * g.Np * 16u;
   const int slabs = g.KG / KGL;
   u4v ra[2][NUA], rx[2][NUX];
+  u4v da[DA ? 4 : 1][3][FM];  // fragments of A of four slabs
+  const unsigned od = (unsigned)((2 * wk + lhi) * g.Mp + wm * TM + l32) * 16u;
+  const unsigned plane_a = (unsigned)g.KG * g.Mp * 16u;
+  auto direct = [&](u4v (&q)[3][FM], int sn) {
+    const unsigned so = (unsigned)min(sn, slabs - 1) * step_a;
+#pragma unroll
+    for (int p = 0; p < 3; ++p)
+#pragma unroll
+      for (int f = 0; f < FM; ++f)
+        q[p][f] = __builtin_amdgcn_raw_buffer_load_b128(res_a, od + f * 512u, so + p * plane_a, 0);
+  };
 
   auto loads = [&](u4v (&qa)[NUA], u4v (&qx)[NUX], int sn) {
     const unsigned s = min(sn, slabs - 1);  // past the end: a harmless re-read of the last slab
     const unsigned sa = s * step_a, sx = s * step_x;
 #pragma unroll
-    for (int i = 0; i < NUA; ++i)
+    for (int i = 0; i < (DA ? 0 : NUA); ++i)
       if (kExactA || tid + i * NT < UA) qa[i] = __builtin_amdgcn_raw_buffer_load_b128(res_a, oa[i], sa, 0);
 #pragma unroll
     for (int i = 0; i < NUX; ++i)
@@ -208,7 +232,7 @@ __attribute__((amdgpu_waves_per_eu(split_waves_per_simd<BM, BN, WK, CELL>()))) v
   auto stores = [&](int stage, const u4v (&qa)[NUA], const u4v (&qx)[NUX]) {
     u4v *w = lds + stage * STAGE;
 #pragma unroll
-    for (int i = 0; i < NUA; ++i)
+    for (int i = 0; i < (DA ? 0 : NUA); ++i)
       if (kExactA || tid + i * NT < UA) w[tid + i * NT] = qa[i];
 #pragma unroll
     for (int i = 0; i < NUX; ++i)
@@ -217,18 +241,20 @@ __attribute__((amdgpu_waves_per_eu(split_waves_per_simd<BM, BN, WK, CELL>()))) v
   const int fa0 = (2 * wk + lhi) * BM + wm * TM + l32, fx0 = UA + (2 * wk + lhi) * BN + wn * TN + l32;
   // One slab: its fragments, the next slab from the staging registers to the other LDS stage, the
   // loads of the slab after the next two, 6 MFMAs per 32x32 tile (smallest terms first), barrier.
-  auto body = [&](int stage, u4v (&qa)[NUA], u4v (&qx)[NUX], int sn) {
+  auto body = [&](int stage, u4v (&qa)[NUA], u4v (&qx)[NUX], int sn, u4v (&qd)[3][FM], int sd) {
     const u4v *b = lds + stage * STAGE;
     bf16x8 fa[3][FM], fx[3][FN];
 #pragma unroll
     for (int p = 0; p < 3; ++p) {
 #pragma unroll
-      for (int f = 0; f < FM; ++f) fa[p][f] = __builtin_bit_cast(bf16x8, b[fa0 + p * KGL * BM + f * 32]);
+      for (int f = 0; f < FM; ++f)
+        fa[p][f] = __builtin_bit_cast(bf16x8, DA ? qd[p][f] : b[fa0 + p * KGL * BM + f * 32]);
 #pragma unroll
       for (int f = 0; f < FN; ++f) fx[p][f] = __builtin_bit_cast(bf16x8, b[fx0 + p * KGL * BN + f * 32]);
     }
     stores(stage ^ 1, qa, qx);
     loads(qa, qx, sn);
+    if constexpr (DA) __builtin_amdgcn_sched_barrier(0);  // all of that ahead of the MFMAs, not behind them
     constexpr int PA[6] = {2, 1, 0, 1, 0, 0}, PX[6] = {0, 1, 2, 0, 1, 0};
 #pragma unroll
     for (int t = 0; t < 6; ++t)
@@ -239,19 +265,47 @@ __attribute__((amdgpu_waves_per_eu(split_waves_per_simd<BM, BN, WK, CELL>()))) v
           // operands swapped on purpose: consecutive m in consecutive lanes of every accumulator
           acc[a][bb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fx[PX[t]][a], fa[PA[t]][bb], acc[a][bb],
                                                                0, 0, 0);
+    if constexpr (DA) {
+      __builtin_amdgcn_sched_barrier(0);
+      direct(qd, sd);
+    }
     __syncthreads();
   };
   loads(ra[0], rx[0], 0);
   loads(ra[1], rx[1], 1);
+  if constexpr (DA) {
+    // in this order: a wait in the loop must allow for what is in flight on its first pass too
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      direct(da[i], i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
   stores(0, ra[0], rx[0]);
   loads(ra[0], rx[0], 2);
   __syncthreads();
-  int s = 0;
-  for (; s + 1 < slabs; s += 2) {
-    body(0, ra[1], rx[1], s + 3);
-    body(1, ra[0], rx[0], s + 4);
+  if constexpr (DA) {
+    int s = 0;  // KG is a multiple of 16, so slabs is one of 4 for WK <= 2
+    for (; s + 4 <= slabs; s += 4) {
+      body(0, ra[1], rx[1], s + 3, da[0], s + 4);
+      body(1, ra[0], rx[0], s + 4, da[1], s + 5);
+      body(0, ra[1], rx[1], s + 5, da[2], s + 6);
+      body(1, ra[0], rx[0], s + 6, da[3], s + 7);
+    }
+    if constexpr (WK > 2) {
+      if (s < slabs) body(0, ra[1], rx[1], s + 3, da[0], s + 4);
+      if (s + 1 < slabs) body(1, ra[0], rx[0], s + 4, da[1], s + 5);
+      if (s + 2 < slabs) body(0, ra[1], rx[1], s + 5, da[2], s + 6);
+    }
+  } else {
+    int s = 0;
+    for (; s + 1 < slabs; s += 2) {
+      body(0, ra[1], rx[1], s + 3, da[0], 0);
+      body(1, ra[0], rx[0], s + 4, da[0], 0);
+    }
+    if (s < slabs) body(0, ra[1], rx[1], s + 3, da[0], 0);
   }
-  if (s < slabs) body(0, ra[1], rx[1], s + 3);
 
   constexpr int LDS_M = BM + 4;
   float *const S = reinterpret_cast<float *>(lds);  // the tile as S[n][m]; the slab stages are dead
@@ -409,7 +463,7 @@ thread_local int g_split_override = -1;
 
 template <int BM, int BN, int WM, int WN, int WK, bool CELL>
 int launch_split(SplitArgs &g, hipStream_t s, const char *what) {
-  static_assert(split_lds_bytes<BM, BN, WK>(CELL) <= 160 * 1024, "LDS capacity of a CU");
+  static_assert(split_lds_bytes<BM, BN, WK>(CELL, WN == 1, 64 * WM * WN * WK) <= 160 * 1024, "LDS capacity of a CU");
   static_assert(64 * WM * WN * WK <= 1024, "workgroup size");
   const int tiles_m = CELL ? (4 * g.M + BM - 1) / BM : (g.M + BM - 1) / BM;
   g.tiles_n = (g.N + BN - 1) / BN;
@@ -420,7 +474,7 @@ int launch_split(SplitArgs &g, hipStream_t s, const char *what) {
   if (tiles_m * BM > g.Mp || g.KG % (2 * WK))
     return lh::fail_arg("%s: %d row tiles of %d exceed the %d padded rows, or %d k-groups are not whole slabs",
                         what, tiles_m, BM, g.Mp, g.KG);
-  constexpr int bytes = split_lds_bytes<BM, BN, WK>(CELL);
+  constexpr int bytes = split_lds_bytes<BM, BN, WK>(CELL, WN == 1, 64 * WM * WN * WK);
   static thread_local bool raised[64] = {};
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return lh::fail_arg("%s: hipGetDevice", what);

@@ -1572,6 +1572,17 @@ int plan_cell(int H, int B, const lh_gemm_seg *segs, int nseg, bool has_addend, 
               &splits_cell, true, &us_cell);
   if (cfg_cell < 0) return LH_OK;
   const float cell_us = kCellFixedUs + 28.f * (float)H * (float)B / kReduceBytesPerUs;
+  // A short product with tiles for a quarter of the CUs: the table's fixed costs are those of a full
+  // chip, where the deep slab pays for its LDS traffic; alone on its CU it is two slabs and done.
+  // 256 hidden units, K = 256, 5 and 32 columns: 32x32 tiles in 128-deep slabs 5.5 us, the table's
+  // choice (64x32, 32-deep) 6.8 us.
+  constexpr int kShortConfig = 15;
+  int depth = 0;
+  for (int s = 0; s < nseg; ++s) depth += p->g.K[s];
+  if (g_config_override < 0 && depth <= 256 && ((H + 7) / 8) * ((B + 31) / 32) <= kCUs / 4) {
+    cfg_cell = kShortConfig;
+    us_cell = 0.f;
+  }
   // a configuration override (tuning, tests) asks for the fused form whenever the tile can hold it
   if (g_config_override >= 0 || us_cell <= us_any + cell_us) {
     *fusable = true;

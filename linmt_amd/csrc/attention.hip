@@ -189,7 +189,8 @@ __global__ __launch_bounds__(kWide) void attn_core_kernel(const AttnArgs a) {
       for (int j = grp; j < W; j += groups) {
         const int tau = s_tau[j];
         const float w = s_val[j];
-        const float *x = hs_c + (size_t)max(tau, 0) * a.step_stride;
+        // a slot without a state reads column 0's first one, which exists, and drops it
+        const float *x = tau >= 0 ? hs_c + (size_t)tau * a.step_stride : a.hs;
         if constexpr (VEC) {
           const float4 v = *reinterpret_cast<const float4 *>(x + (size_t)unit * 4);
           acc.x = tau >= 0 ? acc.x + w * v.x : acc.x;
@@ -268,7 +269,6 @@ __global__ __launch_bounds__(kThreads) void attn_core_regs_kernel(const AttnArgs
   const int m = a.mask01[b];
   const int col = a.hs_col ? a.hs_col[b] : b;
   const float *wa = a.wa + (size_t)b * a.wa_col_stride;
-  const float *hs_c = a.hs + (size_t)col * a.col_stride;
 
   // everything that does not depend on the window position is requested first
   float4 w4[NQ], oadd[NQ], obias[NQ];
@@ -326,13 +326,15 @@ __global__ __launch_bounds__(kThreads) void attn_core_regs_kernel(const AttnArgs
   int rows_at[NQ];
 #pragma unroll
   for (int q = 0; q < NQ; ++q) rows_at[q] = row_ok[q] ? (tid + q * kThreads) * 4 : 0;
+  // (A column without any such slot, a padded one say, may carry any entry of hs_col: column 0's rows then.)
+  const size_t col_at = live ? (size_t)col * a.col_stride : 0;
   auto slot_row = [&](const float *mem, int j) {
-    return mem + (size_t)min(max(tau0 - j, 0), steps - 1) * a.step_stride;
+    return mem + col_at + (size_t)min(max(tau0 - j, 0), steps - 1) * a.step_stride;
   };
   float4 h[WCAP][NQ];
 #pragma unroll
   for (int j = 0; j < WCAP; ++j) {
-    const float *row = slot_row(hs_c, j);
+    const float *row = slot_row(a.hs, j);
 #pragma unroll
     for (int q = 0; q < NQ; ++q) h[j][q] = *reinterpret_cast<const float4 *>(row + rows_at[q]);
   }
@@ -353,10 +355,9 @@ __global__ __launch_bounds__(kThreads) void attn_core_regs_kernel(const AttnArgs
   if (a.ctx_mem) {
     // the scores are done with the window: the same registers take the window of ctx_mem, whose
     // loads fly while the scores are normalised
-    const float *cm = a.ctx_mem + (size_t)col * a.col_stride;
 #pragma unroll
     for (int j = 0; j < WCAP; ++j) {
-      const float *row = slot_row(cm, j);
+      const float *row = slot_row(a.ctx_mem, j);
 #pragma unroll
       for (int q = 0; q < NQ; ++q) h[j][q] = *reinterpret_cast<const float4 *>(row + rows_at[q]);
     }

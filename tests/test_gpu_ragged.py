@@ -161,3 +161,27 @@ def test_copy_block(lh, rows, cols, ld_dst, ld_src, off):
     for c in range(cols):
         want[off + c * ld_dst: off + c * ld_dst + rows] = s[off + c * ld_src: off + c * ld_src + rows]
     assert np.array_equal(dst.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("H,D,W", [(64, 10, 21), (1500, 3, 7), (100, -1, 40), (68, 20, 41)])
+def test_padded_columns_read_no_column_of_their_own(lh, H, D, W):
+    """A column with mask 0, or whose window lies outside the caller's steps, may carry any hs_col entry: it
+    reads nothing through it.  NaN behind every column that is not such a column's neighbour shows a use."""
+    rng = np.random.default_rng(H)
+    S, B = 40, 4
+    hs = rng.normal(0, 1, (S, 2, H)).astype(np.float32)      # two columns of states
+    wa, t1, vp = (rng.normal(0, 0.1, n).astype(np.float32) for n in ((B, H), (B, H), H))
+    hs_col = np.array([1, 1 << 20, 0, 1 << 20], np.int32)     # columns 1 and 3 point nowhere
+    info = np.array([S, S, S, S, 0, 0, 0, 5 * S], np.int32)   # lengths, offsets: column 3 lies past the steps
+    mask = np.array([1, 0, 1, 1], np.int32)
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    f = lambda n: torch.full((n,), float("nan"), device="cuda")     # noqa: E731
+    p, sg, al, ce, ctx = f(B), f(B), f(B * W), f(B * W), f(B * H)
+    idx = torch.zeros(B * W, dtype=torch.int32, device="cuda")
+    lh.attn_core_fwd(H, B, D, W, S, d(t1), d(vp), d(wa), d(hs), 2 * H, H, d(hs_col), d(info), d(mask), p, sg, idx, al,
+                     ce, ctx)
+    got, w, at = ctx.cpu().numpy().reshape(B, H), al.cpu().numpy().reshape(W, B), idx.cpu().numpy().reshape(W, B)
+    assert np.all(got[1] == 0) and np.all(got[3] == 0) and np.all(at[:, 1] == -1)
+    for b in (0, 2):
+        want = sum(w[j, b].astype(np.float64) * hs[S - 1 - at[j, b], hs_col[b]] for j in range(W) if at[j, b] >= 0)
+        assert np.abs(got[b] - want).max() <= 2.0 ** -22 * W * np.abs(hs).max()

@@ -125,7 +125,7 @@ __global__ __launch_bounds__(kT, (NV <= 8 ? 8 : 4)) void softmax_fwd_kernel(cons
   }
 }
 
-// Generic fallback: any V / alignment, column re-read twice.
+// Columns too long for the registers: re-read twice.
 __global__ __launch_bounds__(kT) void softmax_fwd_generic_kernel(const float *logits, int ldl,
                                                                  const float *bias, int V, float *p,
                                                                  int ldp) {

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <cstdint>
 #include <cstdio>
 #include <cstdlib>
 #include <stdexcept>
@@ -58,10 +59,15 @@ class DeviceArray {
 
   void Alloc(size_t n) {
     Free();
-    n_ = n;
     if (n == 0) return;
-    HipErrorWrapper(hipMalloc(reinterpret_cast<void **>(&p_), n * sizeof(T)),
-                    "GPU memory allocation failed");
+    if (n > SIZE_MAX / sizeof(T)) throw LinmtError("GPU memory allocation failed: size out of range");
+    const hipError_t e = hipMalloc(reinterpret_cast<void **>(&p_), n * sizeof(T));
+    if (e != hipSuccess) {
+      p_ = nullptr;              // an array that has no buffer holds no elements
+      (void)hipGetLastError();   // reported here, not by the next launch check
+      HipErrorWrapper(e, "GPU memory allocation failed");
+    }
+    n_ = n;
   }
   // Grow-only: keeps the buffer when it already holds n elements (contents are not kept otherwise).
   void Reserve(size_t n) {

@@ -73,6 +73,19 @@ class DeviceArray {
   void Reserve(size_t n) {
     if (n > n_) Alloc(n);
   }
+  // The same for memory the caller can do without: false (and an empty array) when there is none.
+  bool TryReserve(size_t n) {
+    if (n <= n_) return true;
+    Free();
+    if (n > SIZE_MAX / sizeof(T)) return false;
+    if (hipMalloc(reinterpret_cast<void **>(&p_), n * sizeof(T)) != hipSuccess) {
+      p_ = nullptr;
+      (void)hipGetLastError();
+      return false;
+    }
+    n_ = n;
+    return true;
+  }
   void Free() {
     if (p_) (void)hipFree(p_);
     p_ = nullptr;

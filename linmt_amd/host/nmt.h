@@ -14,6 +14,7 @@
 //     sentence s owns columns [s*beam,(s+1)*beam); beam selection, back-pointers and the state swap
 //     stay on the device, the host only reads the per-step (token, back-pointer, score) history.
 #pragma once
+#include <algorithm>
 #include <functional>
 #include <map>
 #include <memory>
@@ -367,10 +368,21 @@ class SoftmaxLayer : public BaseLossLayer {
   bool split_dirty_ = true;
   void BuildSplitWeights();
   void ComputeLogitsSplit(float *p_device_h_t, int minibatch);
-  // scoring: logits and log-probabilities of a group of steps (kept between calls, grow-only)
+  // scoring: logits and log-probabilities of a group of steps (kept between calls, grow-only; a training
+  // model has dz_chunk_ for them)
   DeviceArray<float> loss_logits_;
   DeviceArray<double> loss_logp_;
   void LossAllSteps(const float *p_device_h_t_all, int steps);
+  // Steps a group: groups of about equal size and at most 2^27 logits (512 MiB), halved until fits(steps a
+  // group) has memory for them.  1 takes no memory and fits is not asked: the model has one step's buffers.
+  template <typename Fits>
+  static int LossGroupSteps(size_t logits_per_step, int steps, Fits &&fits) {
+    for (size_t most = std::max<size_t>(1, ((size_t)1 << 27) / logits_per_step);; most = std::max<size_t>(1, most / 2)) {
+      const int groups = (int)((steps + most - 1) / most), per = (steps + groups - 1) / groups;
+      if (per == 1 || fits(per)) return per;
+      most = (size_t)per;
+    }
+  }
   DeviceArray<float> p_device_outputdist_;           // V x B logits / probabilities (one step)
   DeviceArray<double> p_device_logp_tgt_, p_device_loss_, p_device_train_perplexity_;
   DeviceArray<int> p_device_output_vocab_indices_, p_device_output_vocab_indices_01_;

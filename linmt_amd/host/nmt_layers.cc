@@ -777,24 +777,31 @@ void SoftmaxLayer::ComputeLogitsSplit(float *p_device_h_t, int minibatch) {
 // The loss of `steps` steps whose top states lie side by side, added to p_device_loss_.  A step of its
 // own has too few columns for the output projection's wide tiles and splits K behind a reduction
 // launch (128 columns of 30000 words: 77 + 5 us, then 8 + 5 for the loss); together they take
-// 61 + 3.  Steps go in equal groups of at most 2^27 logits (512 MiB).
+// 61 + 3.  The logits of a group of steps go to a training model's dz_chunk_, which is idle here, or to
+// memory of their own while there is some.
 void SoftmaxLayer::LossAllSteps(const float *p_device_h_t_all, int steps) {
   NeuralMachineTranslation &M = *p_neural_mt_;
   const int H = lstm_size_, V = output_vocab_size_, B = current_minibatch_;
-  const size_t most = std::max<size_t>(1, ((size_t)1 << 27) / ((size_t)V * B));
-  const int groups = (int)((steps + most - 1) / most), per = (steps + groups - 1) / groups;
-  loss_logits_.Reserve((size_t)V * B * per);
-  loss_logp_.Reserve((size_t)B * per);
+  float *logits = dz_chunk_.get();
+  double *logp = p_device_logp_tgt_.get();
+  int per = std::min(steps, chunk_steps_);
+  if (!logits) {
+    per = LossGroupSteps((size_t)V * B, steps, [&](int n) {
+      return loss_logits_.TryReserve((size_t)V * B * n) && loss_logp_.TryReserve((size_t)B * n);
+    });
+    logits = per == 1 ? p_device_outputdist_.get() : loss_logits_.get();
+    if (per > 1) logp = loss_logp_.get();
+  }
   for (int t = 0; t < steps; t += per) {
     const int N = B * std::min(per, steps - t);
     lh_gemm_seg seg{p_device_d_.get(), V, p_device_h_t_all + (size_t)H * B * t, H, H};
-    M.Gemm(kTagLogitsGemm, V, N, &seg, 1, 0, 0, 0.f, p_device_b_d_.get(), LH_ACT_NONE, nullptr,
-           loss_logits_.get(), V, "SoftmaxLayer::LossAllSteps logits");
+    M.Gemm(kTagLogitsGemm, V, N, &seg, 1, 0, 0, 0.f, p_device_b_d_.get(), LH_ACT_NONE, nullptr, logits, V,
+           "SoftmaxLayer::LossAllSteps logits");
     ProfileScope px(M.profiler_, kTagXent, 4.0 * V * N);
-    LhErrorWrapper(lh_logsoftmax_xent_f32(loss_logits_.get(), V, nullptr, V, N,
+    LhErrorWrapper(lh_logsoftmax_xent_f32(logits, V, nullptr, V, N,
                                           p_device_output_vocab_indices_.get() + (size_t)B * t,
                                           p_device_output_vocab_indices_01_.get() + (size_t)B * t,
-                                          loss_logp_.get(), p_device_loss_.get(), M.stream_),
+                                          logp, p_device_loss_.get(), M.stream_),
                    "SoftmaxLayer::LossAllSteps");
   }
 }

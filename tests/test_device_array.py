@@ -1,6 +1,7 @@
 """DeviceArray (host/hip_util.h) when an allocation fails: it holds no elements, says so on every later use, and
 the failure is not left behind for the next launch check.  The size asked for is larger than any device, so the
-allocation fails with and without a GPU."""
+allocation fails with and without a GPU.  And what scoring makes of memory it does not get (SoftmaxLayer::
+LossGroupSteps, host/nmt.h): smaller groups of steps, at last one step in the buffers the model has."""
 import os
 import subprocess
 import tempfile
@@ -39,19 +40,59 @@ int main() {
   a.Zero(nullptr);                                  // nothing to clear
   EXPECT(Throws([&] { a.Alloc(SIZE_MAX / 2); }));   // the byte count must not wrap round
   EXPECT(a.size() == 0);
+  EXPECT(a.TryReserve(0));
+  EXPECT(!a.TryReserve(huge) && a.size() == 0 && a.get() == nullptr);
+  EXPECT(!a.TryReserve(SIZE_MAX / 2));
+  EXPECT(!gpu || hipGetLastError() == hipSuccess);
+  return 0;
+}
+"""
+
+GROUPS = r"""
+#include "linmt_amd/host/nmt.h"
+using namespace linmt;
+
+int main() {
+  // logits a step, steps, steps that fit, expected steps a group
+  const long long cases[][4] = {{100, 7, 1000, 7},            // all at once
+                                {(1 << 27) / 3, 7, 1000, 3},  // three groups of at most 2^27 logits: 3, 3, 1
+                                {7680000, 41, 1000, 14},      // 17 fit: 14, 14, 13
+                                {7680000, 41, 8, 7},          // 14 do not, half of them do
+                                {7680000, 41, 6, 3}, {7680000, 41, 2, 1}, {7680000, 41, 0, 1},
+                                {1LL << 28, 41, 1000, 1},     // one step is more than a group may have
+                                {(1LL << 26) + 1, 5, 1000, 1}, {100, 1, 0, 1}, {1LL << 40, 1, 0, 1}};
+  for (auto &c : cases) {
+    long long asked = 0;
+    const int per = SoftmaxLayer::LossGroupSteps((size_t)c[0], (int)c[1], [&](int n) {
+      asked = n;
+      return n <= c[2];
+    });
+    if (per != c[3] || (per > 1 && asked != per)) {
+      printf("%lld logits, %lld steps, %lld fit: %d (expected %lld)\n", c[0], c[1], c[2], per, c[3]);
+      return 1;
+    }
+  }
   return 0;
 }
 """
 
 
-def test_failed_allocation_leaves_an_empty_array():
+def _run(source):
     with tempfile.TemporaryDirectory() as d:
-        src, exe = os.path.join(d, "device_array.cc"), os.path.join(d, "device_array")
+        src, exe = os.path.join(d, "program.cc"), os.path.join(d, "program")
         with open(src, "w") as f:
-            f.write(SOURCE)
+            f.write(source)
+        lib = os.path.join(ROOT, "linmt_amd")
         subprocess.run(["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I", ROOT, "-I", "/opt/rocm/include", src,
-                        "-o", exe, "-L", "/opt/rocm/lib", "-lamdhip64", "-Wl,-rpath,/opt/rocm/lib",
-                        "-L", os.path.join(ROOT, "linmt_amd"), "-llinmt_hip",
-                        "-Wl,-rpath," + os.path.join(ROOT, "linmt_amd")], check=True)
+                        "-o", exe, "-L", lib, "-llinmt_host", "-llinmt_hip", "-Wl,-rpath," + lib,
+                        "-L", "/opt/rocm/lib", "-lamdhip64", "-Wl,-rpath,/opt/rocm/lib"], check=True)
         r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
         assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_failed_allocation_leaves_an_empty_array():
+    _run(SOURCE)
+
+
+def test_scoring_takes_smaller_groups_when_memory_is_short():
+    _run(GROUPS)

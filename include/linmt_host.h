@@ -207,7 +207,9 @@ void *lnmt_model_stream(lnmt_model *m);
  * On a model created for training the same switch makes the large batched products of a minibatch
  * (weight gradients accumulated over all steps, the output projection and its two backward products,
  * the layer-major input products) split products, both operands packed per call; the per-step
- * products keep the fp32 MFMA path (min_columns == 1 there takes every product: a test aid). */
+ * products keep the fp32 MFMA path (min_columns == 1 there takes every product: a test aid).  Scoring
+ * on such a model: the layer-major input products as in training, the output projection in fp32 (it
+ * goes by the columns of one step, however many steps run together). */
 int lnmt_set_split_products(lnmt_model *m, int on, int min_columns);
 /* Measurement and test aids of the decode path, process-wide, all 0 by default (no counterpart in
  * the reference).  Each switches one part back to the form it replaced, with the same results up

@@ -523,6 +523,10 @@ class NeuralMachineTranslation {
   // layer-major input products) this way, packing both operands on the fly into these buffers;
   // worthwhile while the packing is a small part of the product (both extents in the thousands).
   DeviceArray<unsigned> split_scratch_a_, split_scratch_x_;
+  // ... by this rule (split_min_columns_ == 1, a test aid, takes every product)
+  bool SplitProductPays(int rows, int cols, double k_sum) const {
+    return split_min_columns_ == 1 || (2.0 * rows * cols * k_sum >= 2e10 && 160.0 * (1.0 / rows + 1.0 / cols) <= 0.2);
+  }
   bool GemmAsSplitProduct(int tag, int rows, int cols, const lh_gemm_seg *segs, int nseg, int trans_a,
                           int trans_x, float beta, const float *bias, int act, const int *colmask,
                           float *C, int ldc, const char *what, int act_rows);
@@ -550,6 +554,10 @@ class NeuralMachineTranslation {
   void Gemm(int tag, int rows, int cols, const lh_gemm_seg *segs, int nseg, int trans_a, int trans_x,
             float beta, const float *bias, int act, const int *colmask, float *C, int ldc,
             const char *what, int act_rows = -1);  // act_rows < 0: the activation covers every row
+  // the same on the fp32 MFMA kernels whatever split_products_ says
+  void GemmFp32(int tag, int rows, int cols, const lh_gemm_seg *segs, int nseg, int trans_a, int trans_x,
+                float beta, const float *bias, int act, const int *colmask, float *C, int ldc,
+                const char *what, int act_rows = -1);
   // The plain product for a consumer that adds partial sums itself (the LSTM cell kernel takes
   // three addends).  Returns the number of addends n and fills addend[0..n): either {C} with
   // C = beta * C + product, or the partial planes of a split product preceded by C when beta = 1.

@@ -778,7 +778,8 @@ void SoftmaxLayer::ComputeLogitsSplit(float *p_device_h_t, int minibatch) {
 // own has too few columns for the output projection's wide tiles and splits K behind a reduction
 // launch (128 columns of 30000 words: 77 + 5 us, then 8 + 5 for the loss); together they take
 // 61 + 3.  The logits of a group of steps go to a training model's dz_chunk_, which is idle here, or to
-// memory of their own while there is some.
+// memory of their own while there is some.  Split products stay what they are for a step by itself:
+// grouping alone does not switch scoring over to them.
 void SoftmaxLayer::LossAllSteps(const float *p_device_h_t_all, int steps) {
   NeuralMachineTranslation &M = *p_neural_mt_;
   const int H = lstm_size_, V = output_vocab_size_, B = current_minibatch_;
@@ -792,11 +793,12 @@ void SoftmaxLayer::LossAllSteps(const float *p_device_h_t_all, int steps) {
     logits = per == 1 ? p_device_outputdist_.get() : loss_logits_.get();
     if (per > 1) logp = loss_logp_.get();
   }
+  const auto gemm = M.SplitProductPays(V, B, H) ? &NeuralMachineTranslation::Gemm : &NeuralMachineTranslation::GemmFp32;
   for (int t = 0; t < steps; t += per) {
     const int N = B * std::min(per, steps - t);
     lh_gemm_seg seg{p_device_d_.get(), V, p_device_h_t_all + (size_t)H * B * t, H, H};
-    M.Gemm(kTagLogitsGemm, V, N, &seg, 1, 0, 0, 0.f, p_device_b_d_.get(), LH_ACT_NONE, nullptr, logits, V,
-           "SoftmaxLayer::LossAllSteps logits");
+    (M.*gemm)(kTagLogitsGemm, V, N, &seg, 1, 0, 0, 0.f, p_device_b_d_.get(), LH_ACT_NONE, nullptr, logits, V,
+              "SoftmaxLayer::LossAllSteps logits", -1);
     ProfileScope px(M.profiler_, kTagXent, 4.0 * V * N);
     LhErrorWrapper(lh_logsoftmax_xent_f32(logits, V, nullptr, V, N,
                                           p_device_output_vocab_indices_.get() + (size_t)B * t,

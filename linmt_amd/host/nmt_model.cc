@@ -27,6 +27,13 @@ void NeuralMachineTranslation::Gemm(int tag, int rows, int cols, const lh_gemm_s
       GemmAsSplitProduct(tag, rows, cols, segs, nseg, trans_a, trans_x, beta, bias, act, colmask, C, ldc,
                          what, act_rows))
     return;
+  GemmFp32(tag, rows, cols, segs, nseg, trans_a, trans_x, beta, bias, act, colmask, C, ldc, what, act_rows);
+}
+
+void NeuralMachineTranslation::GemmFp32(int tag, int rows, int cols, const lh_gemm_seg *segs, int nseg,
+                                        int trans_a, int trans_x, float beta, const float *bias, int act,
+                                        const int *colmask, float *C, int ldc, const char *what,
+                                        int act_rows) {
   ProfileScope ps(profiler_, tag, gemm_ws_bytes_, 0, rows, cols, segs, nseg, trans_a, trans_x);
   LhErrorWrapper(lh_gemm_ws_f32(rows, cols, segs, nseg, trans_a, trans_x, 1.f, beta, bias, act,
                                 act_rows < 0 ? rows : act_rows,
@@ -87,10 +94,7 @@ bool NeuralMachineTranslation::GemmAsSplitProduct(int tag, int rows, int cols, c
   }
   // packing costs about 10 bytes of traffic per operand element against 2*rows*cols*K flop:
   // 160 * (1/rows + 1/cols) is its share of the product's time at the rates of this GPU
-  // (split_min_columns_ == 1, a test aid, takes every product)
-  if (split_min_columns_ != 1 &&
-      (2.0 * rows * cols * k_sum < 2e10 || 160.0 * (1.0 / rows + 1.0 / cols) > 0.2))
-    return false;
+  if (!SplitProductPays(rows, cols, k_sum)) return false;
   const int total = lh_split_kgroups_padded(groups);
   const size_t a_bytes = lh_split_bytes(rows, total), x_bytes = lh_split_bytes(cols, total);
   if (a_bytes >= (size_t(1) << 32) || x_bytes >= (size_t(1) << 32)) return false;

@@ -83,3 +83,14 @@ def test_training_model_scores_in_its_own_buffers(host):
     want, bound = _expected(m, P, tout, H, B)
     assert abs(got - want.sum()) <= bound.sum() and abs(trained - want.sum()) <= bound.sum()
     m.close()
+
+
+def test_grouping_does_not_switch_scoring_to_split_products(host):
+    """A step's output projection (64 columns) stays an fp32 product with split products on, so the projection
+    of many steps does; nothing else of this minibatch is large enough for them."""
+    H, V, B, T = 1024, 16000, 64, 20
+    m, P, tin, tout = _language_model(host, np.random.default_rng(2), H, V, B, T, training=dict(grad_clip_mode=0))
+    want = m.get_error(None, tin, tout, None)
+    m.set_split_products(True)
+    assert m.get_error(None, tin, tout, None) == want
+    m.close()

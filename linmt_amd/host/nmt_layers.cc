@@ -781,6 +781,7 @@ void SoftmaxLayer::ComputeLogitsSplit(float *p_device_h_t, int minibatch) {
 // memory of their own while there is some.  Split products stay what they are for a step by itself:
 // grouping alone does not switch scoring over to them.
 void SoftmaxLayer::LossAllSteps(const float *p_device_h_t_all, int steps) {
+  if (steps < 1) return;
   NeuralMachineTranslation &M = *p_neural_mt_;
   const int H = lstm_size_, V = output_vocab_size_, B = current_minibatch_;
   float *logits = dz_chunk_.get();

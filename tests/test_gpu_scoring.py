@@ -94,3 +94,10 @@ def test_grouping_does_not_switch_scoring_to_split_products(host):
     m.set_split_products(True)
     assert m.get_error(None, tin, tout, None) == want
     m.close()
+
+
+def test_empty_target(host):
+    m, P, tin, tout = _language_model(host, np.random.default_rng(3), 16, 20, 4, 1)
+    assert m.get_error(None, tin[:, :0], tout[:, :0], None) == 0.0
+    assert m.get_error(None, tin, tout, None) < 0.0
+    m.close()

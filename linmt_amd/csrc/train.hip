@@ -389,7 +389,9 @@ __global__ __launch_bounds__(kBT) void attn_core_bwd_kernel(const AttnBwdArgs a)
           at[u] = (size_t)max(tau, 0) * a.step_stride + r;
           rj[u] = j < W ? s_r[j] : 0.f, aj[u] = j < W ? s_al[j] : 0.f;
           h[u].load(hs_c + at[u]);
-          d[u].load(dhs_c + at[u]);
+          // a slot without a state reads the states' first row again and drops it: the same row of dhs
+          // may be another group's to write at this moment
+          d[u].load((live[u] ? dhs_c : hs_c) + at[u]);
         }
 #pragma unroll
         for (int u = 0; u < kSlotBatch; ++u) {

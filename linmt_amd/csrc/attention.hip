@@ -35,23 +35,21 @@ struct AttnArgs {
   int out_tanh;
 };
 
-// Any window and alignment.  The time of a launch is the length of one workgroup's chain of
-// dependent memory round trips (a decoding or scoring step has at most a few columns per CU), so a
-// column gets 16 wavefronts, a wavefront has the rows of four slots in flight at once, every slot's
+// Any window and alignment.  With at most a few columns per CU a launch lasts as long as one workgroup's
+// chain of dependent memory round trips, so a column gets up to 16 wavefronts (NT threads), a wavefront has
+// the rows of two slots in flight at once (four were slower at every count of columns), every slot's
 // exponential is taken once, by the slot's own thread, and the context sum of a row is split over
 // as many groups of threads as the workgroup has left (their partial sums meet in LDS in group
-// order); its second read of the window comes from L2.
-// 128 columns of 1000 rows, 50 slots: 49.6 us with four wavefronts, a slot at a time; 22.4 us.
-constexpr int kWide = 1024;
-constexpr int kWideWaves = kWide / lh::kWave;
-constexpr int kSlotBatch = 4;
+// order); its second read of the window comes from L2.  Position and weights do not depend on NT.
+constexpr int kSlotBatch = 2;
 
-template <bool VEC>
-__global__ __launch_bounds__(kWide) void attn_core_kernel(const AttnArgs a) {
+template <bool VEC, int NT>
+__global__ __launch_bounds__(NT) void attn_core_kernel(const AttnArgs a) {
+  constexpr int kNW = NT / lh::kWave;
   __shared__ float s_val[kMaxSlots];   // scores, then alignment weights
   __shared__ int s_tau[kMaxSlots];     // encoder timestep of slot j, -1 = no state to read
-  __shared__ float s_red[kWideWaves];
-  __shared__ float4 s_ctx[kWide];
+  __shared__ float s_red[kNW];
+  __shared__ float4 s_ctx[NT];
   __shared__ int s_first;
 
   const int b = lh::xcd_contiguous(blockIdx.x, gridDim.x);  // a sentence's columns on one XCD
@@ -71,7 +69,7 @@ __global__ __launch_bounds__(kWide) void attn_core_kernel(const AttnArgs a) {
     const float *t1 = a.tanh1 + (size_t)b * a.proj_col_stride;
     if (tid < kThreads)  // the order of attn_core_regs_kernel: the position must not depend on the kernel
       for (int r = tid; r < H; r += kThreads) part += a.v_p[r] * t1[r];
-    const float dot = lh::block_sum<kWideWaves>(part, s_red);
+    const float dot = lh::block_sum<kNW>(part, s_red);
     const float sig = (float)(1.0 / (1.0 + exp(-1.0 * (double)dot)));
     p = (float)len * sig;
     lo = (0 > (int)p - D) ? 0 : ((int)p - D);
@@ -82,8 +80,7 @@ __global__ __launch_bounds__(kWide) void attn_core_kernel(const AttnArgs a) {
     }
   }
 
-  // window indices (reference layout B x W, element (b,j) at b + B*j); thread j owns slot j
-  static_assert(kMaxSlots <= kWide, "one thread per slot");
+  // window indices (reference layout B x W, element (b,j) at b + B*j); thread j owns slot j (W <= NT)
   int idx = -1;
   if (tid < W) {
     if (m == 1 && lo + tid <= hi) idx = lo + tid;
@@ -98,20 +95,20 @@ __global__ __launch_bounds__(kWide) void attn_core_kernel(const AttnArgs a) {
   __syncthreads();
 
   // scores: wavefront w takes slots w, w + 16, ..., four at a time
-  for (int j0 = wave; j0 < W; j0 += kWideWaves * kSlotBatch) {
+  for (int j0 = wave; j0 < W; j0 += kNW * kSlotBatch) {
     const float *row[kSlotBatch];
     float acc[kSlotBatch];
     bool live[kSlotBatch];
 #pragma unroll
     for (int u = 0; u < kSlotBatch; ++u) {
-      const int j = j0 + u * kWideWaves;
+      const int j = j0 + u * kNW;
       const int tau = j < W ? s_tau[j] : -1;
       live[u] = tau >= 0;
       row[u] = hs_c + (size_t)(live[u] ? tau : 0) * a.step_stride;
       acc[u] = 0.f;
     }
     if constexpr (VEC) {
-#pragma unroll 4
+#pragma unroll 2
       for (int r = lane * 4; r < H; r += lh::kWave * 4) {
         const float4 y = *reinterpret_cast<const float4 *>(wa + r);
 #pragma unroll
@@ -122,7 +119,7 @@ __global__ __launch_bounds__(kWide) void attn_core_kernel(const AttnArgs a) {
         }
       }
     } else {
-#pragma unroll 4
+#pragma unroll 2
       for (int r = lane; r < H; r += lh::kWave) {
         const float y = wa[r];
 #pragma unroll
@@ -133,7 +130,7 @@ __global__ __launch_bounds__(kWide) void attn_core_kernel(const AttnArgs a) {
 #pragma unroll
     for (int u = 0; u < kSlotBatch; ++u) {
       const float sc = lh::wave_sum(acc[u]);
-      const int j = j0 + u * kWideWaves;
+      const int j = j0 + u * kNW;
       if (lane == 0 && j < W) s_val[j] = live[u] ? sc : 0.f;
     }
   }
@@ -143,9 +140,9 @@ __global__ __launch_bounds__(kWide) void attn_core_kernel(const AttnArgs a) {
   const bool valid = tid < W && idx != -1;
   const float val = valid ? s_val[tid] : 0.f;
   const float floor_mx = D >= 0 ? 0.f : -FLT_MAX;
-  const float mx = lh::block_max<kWideWaves>(valid ? fmaxf(val, floor_mx) : floor_mx, s_red);
+  const float mx = lh::block_max<kNW>(valid ? fmaxf(val, floor_mx) : floor_mx, s_red);
   const float e = valid ? expf(val - mx) : 0.f;
-  const float Z = lh::block_sum<kWideWaves>(e, s_red);
+  const float Z = lh::block_sum<kNW>(e, s_red);
   if (tid < W) {
     float al = 0.f, g = 1.f;
     if (valid) {
@@ -166,7 +163,7 @@ __global__ __launch_bounds__(kWide) void attn_core_kernel(const AttnArgs a) {
   if (a.viterbi) {
     // the first slot of the largest weight (weights are >= 0, slots without a position weigh 0)
     const float al = tid < W ? s_val[tid] : -1.f;
-    const float best = lh::block_max<kWideWaves>(fmaxf(al, -1.f), s_red);
+    const float best = lh::block_max<kNW>(fmaxf(al, -1.f), s_red);
     if (tid < W && al == best) atomicMin(&s_first, tid);
     __syncthreads();
     const int first = best > -1.f ? s_first : W;
@@ -177,15 +174,15 @@ __global__ __launch_bounds__(kWide) void attn_core_kernel(const AttnArgs a) {
   // group g of the workgroup adds the slots j = g, g + groups, ...
   float *ctx = a.ctx + (size_t)b * H;
   const int units = VEC ? H / 4 : H;
-  const int lanes = min(kWide, (units + lh::kWave - 1) / lh::kWave * lh::kWave);
-  const int groups = kWide / lanes;
+  const int lanes = min(NT, (units + lh::kWave - 1) / lh::kWave * lh::kWave);
+  const int groups = NT / lanes;
   const int grp = tid / lanes;
   for (int u0 = 0; u0 < units; u0 += lanes) {
     const int unit = u0 + tid % lanes;
     const bool mine = grp < groups && unit < units;
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
     if (mine) {
-#pragma unroll 8
+#pragma unroll 4
       for (int j = grp; j < W; j += groups) {
         const int tau = s_tau[j];
         const float w = s_val[j];
@@ -433,6 +430,12 @@ __global__ __launch_bounds__(kThreads) void attn_core_regs_kernel(const AttnArgs
 
 constexpr int kRegsSlots = 21;  // the reference's default window: D = 10
 
+template <int NT>
+void launch_general(const AttnArgs &a, bool vec, hipStream_t st) {
+  if (vec) hipLaunchKernelGGL((attn_core_kernel<true, NT>), dim3(a.B), dim3(NT), 0, st, a);
+  else hipLaunchKernelGGL((attn_core_kernel<false, NT>), dim3(a.B), dim3(NT), 0, st, a);
+}
+
 }  // namespace
 
 extern "C" int lh_attn_core_fwd_f32(int H, int B, int D, int max_len, int hs_steps,
@@ -468,8 +471,11 @@ extern "C" int lh_attn_core_fwd_f32(int H, int B, int D, int max_len, int hs_ste
     hipLaunchKernelGGL((attn_core_regs_kernel<1, kRegsSlots>), dim3(B), dim3(kThreads), 0, st, a);
   else if (vec && W <= kRegsSlots && H <= 8 * kThreads)
     hipLaunchKernelGGL((attn_core_regs_kernel<2, kRegsSlots>), dim3(B), dim3(kThreads), 0, st, a);
-  else if (vec) hipLaunchKernelGGL(attn_core_kernel<true>, dim3(B), dim3(kWide), 0, st, a);
-  else hipLaunchKernelGGL(attn_core_kernel<false>, dim3(B), dim3(kWide), 0, st, a);
+  // Any other: as many wavefronts per column as leave every column resident (256 CUs of 32 wavefronts).
+  // Past 2048 columns none of the three does; eight wavefronts then tail off best.
+  else if (B <= 512) launch_general<1024>(a, vec, st);
+  else if (B <= 1024 || B > 2048 || W > 256) launch_general<512>(a, vec, st);
+  else launch_general<256>(a, vec, st);
   return lh::check_launch("lh_attn_core_fwd_f32");
 }
 

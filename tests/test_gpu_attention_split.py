@@ -45,3 +45,37 @@ def test_backward_slots_without_a_state(lh, orc, H, B, S, D):
         tau = S - 1 - index[index >= 0]      # left-padded: timestep of source position i
         idle = np.setdiff1d(np.arange(S), tau)
         assert np.array_equal(got[0][1][idle, b], dhs0.reshape(S, B, H)[idle, b])
+
+
+@pytest.mark.parametrize("H,D,S", [(64, 20, 50), (38, -1, 30), (132, 130, 300), (512, -1, 60)])
+@pytest.mark.parametrize("B", [512, 513, 1024, 1025, 2048, 2049])
+def test_forward_at_the_column_counts_of_the_split(lh, orc, H, D, S, B):
+    """A column has 16 wavefronts up to 512 columns, 8 up to 1024 and past 2048 (or for windows of more than 256
+    slots), 4 between.  Against the oracle; and what does not depend on the split (position, window, weights)
+    has the bits it has among 512 columns."""
+    rng = np.random.default_rng(H + B)
+    W, cols = 2 * D + 1 if D >= 0 else S, 40
+    hs, v_p = uni(rng, S * cols * H, s=0.5), uni(rng, H, s=0.1)
+    tanh1, wa = np.tanh(uni(rng, H, B)), uni(rng, H, B, s=0.1)
+    lens = rng.integers(1, S + 1, size=B)
+    lens[:2], lens[-1] = (S, 1), S
+    bi, mask = np.concatenate([lens, S - lens]).astype(np.int32), (rng.random(B) < 0.9).astype(np.int32)
+    mask[0] = mask[-1] = 1
+    hs_col = rng.integers(0, cols, B).astype(np.int32)
+
+    def run(n):
+        f = lambda k: torch.full((k,), float("nan"), device="cuda")  # noqa: E731
+        p, sg, al, ce, ctx = f(n), f(n), f(n * W), f(n * W), f(n * H)
+        ix, vt = (torch.zeros(k, dtype=torch.int32, device="cuda") for k in (n * W, n))
+        lh.attn_core_fwd(H, n, D, S, S, dev(tanh1[:, :n]), dev(v_p), dev(wa[:, :n]), dev(hs), cols * H, H, dev(hs_col[:n]),
+                         dev(np.concatenate([bi[:n], bi[B:B + n]])), dev(mask[:n]), p, sg, ix, al, ce, ctx, vt)
+        return dict(p_t=host(p, (n,)), indices=host(ix, (n, W)), align=host(al, (n, W)), viterbi=host(vt, (n,)),
+                    ctx=host(ctx, (H, n)))
+
+    got, few = run(B), run(512)
+    want = orc.attn_core_fwd(H, B, D, S, S, tanh1, v_p, wa, hs, cols * H, H, hs_col, bi, mask)
+    assert np.array_equal(got["indices"], want["indices"])
+    for name in ("align", "ctx") + (("p_t",) if D >= 0 else ()):
+        assert_close(got[name], want[name], name)
+    for name in ("p_t", "indices", "align", "viterbi"):
+        assert np.array_equal(got[name][:512], few[name], equal_nan=True), name

@@ -267,24 +267,22 @@ struct AttnBwdArgs {
 };
 
 // A launch lasts as long as one workgroup's chain of memory round trips (one column each, a minibatch
-// has fewer columns than the GPU has room for): 16 wavefronts per column, a wavefront with four
-// slots' rows in flight for the scores; then the rows of a column go to `lanes` threads and the slots are
-// dealt to the groups of them a workgroup holds, four slots' reads ahead of their writes.  The
+// has fewer columns than the GPU has room for): NT threads per column, a wavefront with BATCH slots'
+// rows in flight for the scores; then the rows of a column go to `lanes` threads and the slots are
+// dealt to the groups of them a workgroup holds, BATCH slots' reads ahead of their writes.  The
 // groups' partial sums of hsum meet in LDS in group order.
-// Window of 21: 64 columns of 1000 rows 23.0 -> 16.9 us, 256 columns of 2048 rows 56.7 -> 30.7.
-constexpr int kBT = 1024;
-constexpr int kBW = kBT / lh::kWave;
-constexpr int kSlotBatch = 4;
-
-template <bool VEC>
-__global__ __launch_bounds__(kBT) void attn_core_bwd_kernel(const AttnBwdArgs a) {
+// Four wavefronts with a slot at a time -> now: window of 21, 64 columns of 1000 rows 15.8 -> 10.8 us, 256
+// columns of 2048 rows 41.7 -> 30.5; window of 5, 512 columns of 256 rows 6.0 -> 5.7.
+template <bool VEC, int NT, int BATCH>
+__global__ __launch_bounds__(NT) void attn_core_bwd_kernel(const AttnBwdArgs a) {
+  constexpr int kBW = NT / lh::kWave;
   __shared__ int s_tau[kMaxSlots];
   __shared__ float s_das[kMaxSlots];  // d alignment score
   __shared__ float s_al[kMaxSlots];
   __shared__ float s_r[kMaxSlots];
   __shared__ float s_red[kBW];
   constexpr int VW = VEC ? 4 : 1;
-  __shared__ float s_sum[kBT * VW];
+  __shared__ float s_sum[NT * VW];
 
   const int b = blockIdx.x, tid = threadIdx.x, wave = tid / lh::kWave, lane = tid % lh::kWave;
   const int H = a.H, B = a.B, W = a.W, D = a.D;
@@ -295,7 +293,7 @@ __global__ __launch_bounds__(kBT) void attn_core_bwd_kernel(const AttnBwdArgs a)
   float *dhs_c = a.dhs + (size_t)b * a.col_stride;
 
   // thread j owns slot j
-  static_assert(kMaxSlots <= kBT, "one thread per slot");
+  static_assert(kMaxSlots <= NT, "one thread per slot");
   int idx = -1;
   float al = 0.f, g = 1.f;
   if (tid < W) {
@@ -313,12 +311,12 @@ __global__ __launch_bounds__(kBT) void attn_core_bwd_kernel(const AttnBwdArgs a)
   __syncthreads();
 
   // d score_j = dctx . hs_j
-  for (int j0 = wave; j0 < W; j0 += kBW * kSlotBatch) {
-    const float *row[kSlotBatch];
-    float acc[kSlotBatch];
-    bool live[kSlotBatch];
+  for (int j0 = wave; j0 < W; j0 += kBW * BATCH) {
+    const float *row[BATCH];
+    float acc[BATCH];
+    bool live[BATCH];
 #pragma unroll
-    for (int u = 0; u < kSlotBatch; ++u) {
+    for (int u = 0; u < BATCH; ++u) {
       const int j = j0 + u * kBW;
       const int tau = j < W ? s_tau[j] : -1;
       live[u] = tau >= 0;
@@ -330,7 +328,7 @@ __global__ __launch_bounds__(kBT) void attn_core_bwd_kernel(const AttnBwdArgs a)
       Vec<VW> y;
       y.load(dctx + r);
 #pragma unroll
-      for (int u = 0; u < kSlotBatch; ++u) {
+      for (int u = 0; u < BATCH; ++u) {
         if (!live[u]) continue;  // the same for the whole wavefront
         Vec<VW> x;
         x.load(row[u] + r);
@@ -341,7 +339,7 @@ __global__ __launch_bounds__(kBT) void attn_core_bwd_kernel(const AttnBwdArgs a)
       }
     }
 #pragma unroll
-    for (int u = 0; u < kSlotBatch; ++u) {
+    for (int u = 0; u < BATCH; ++u) {
       const float v = lh::wave_sum(acc[u]);
       const int j = j0 + u * kBW;
       if (lane == 0 && j < W) s_das[j] = live[u] ? v : 0.f;
@@ -365,8 +363,8 @@ __global__ __launch_bounds__(kBT) void attn_core_bwd_kernel(const AttnBwdArgs a)
 
   const float pcoef = dp * sg * (1.f - sg) * (float)len;
   const int units = (H + VW - 1) / VW;  // VEC: H % 4 == 0
-  const int lanes = min(kBT, (units + lh::kWave - 1) / lh::kWave * lh::kWave);
-  const int groups = kBT / lanes, grp = tid / lanes;
+  const int lanes = min(NT, (units + lh::kWave - 1) / lh::kWave * lh::kWave);
+  const int groups = NT / lanes, grp = tid / lanes;
   for (int u0 = 0; u0 < units; u0 += lanes) {
     const int unit = u0 + tid % lanes, r = unit * VW;
     const bool mine = grp < groups && unit < units;
@@ -376,13 +374,13 @@ __global__ __launch_bounds__(kBT) void attn_core_bwd_kernel(const AttnBwdArgs a)
     if (mine) {
       dc.load(dctx + r);
       wv.load(wa + r);
-      for (int j0 = grp; j0 < W; j0 += groups * kSlotBatch) {
-        Vec<VW> h[kSlotBatch], d[kSlotBatch];
-        size_t at[kSlotBatch];
-        float rj[kSlotBatch], aj[kSlotBatch];
-        bool live[kSlotBatch];
+      for (int j0 = grp; j0 < W; j0 += groups * BATCH) {
+        Vec<VW> h[BATCH], d[BATCH];
+        size_t at[BATCH];
+        float rj[BATCH], aj[BATCH];
+        bool live[BATCH];
 #pragma unroll
-        for (int u = 0; u < kSlotBatch; ++u) {
+        for (int u = 0; u < BATCH; ++u) {
           const int j = j0 + u * groups;
           const int tau = j < W ? s_tau[j] : -1;
           live[u] = tau >= 0;
@@ -394,7 +392,7 @@ __global__ __launch_bounds__(kBT) void attn_core_bwd_kernel(const AttnBwdArgs a)
           d[u].load((live[u] ? dhs_c : hs_c) + at[u]);
         }
 #pragma unroll
-        for (int u = 0; u < kSlotBatch; ++u) {
+        for (int u = 0; u < BATCH; ++u) {
           if (!live[u]) continue;
 #pragma unroll
           for (int i = 0; i < VW; ++i) hsum.v[i] += h[u].v[i] * rj[u];
@@ -821,8 +819,16 @@ extern "C" int lh_attn_core_bwd_f32(int H, int B, int D, int max_len, int hs_ste
                    lh::aligned16(v_p) && lh::aligned16(u) && lh::aligned16(w) &&
                    hs_step_stride % 4 == 0 && hs_col_stride % 4 == 0;
   hipStream_t st = lh::as_stream(stream);
-  if (vec) hipLaunchKernelGGL(attn_core_bwd_kernel<true>, dim3(B), dim3(kBT), 0, st, a);
-  else hipLaunchKernelGGL(attn_core_bwd_kernel<false>, dim3(B), dim3(kBT), 0, st, a);
+  // Sixteen wavefronts pay for slots to give them and while every column has a CU to itself.  Against
+  // eight, 1000 rows: 10.8 / 12.8 us (21 slots, 64 columns), 18.3 / 20.4 (21, 256); 7.1 / 6.6 (5 slots, 64
+  // columns), 12.3 / 10.5 (5, 512); 256 rows, 21 slots, 384 columns 9.5 / 8.2.
+  if (W > 8 && B <= 256) {
+    if (vec) hipLaunchKernelGGL((attn_core_bwd_kernel<true, 1024, 2>), dim3(B), dim3(1024), 0, st, a);
+    else hipLaunchKernelGGL((attn_core_bwd_kernel<false, 1024, 2>), dim3(B), dim3(1024), 0, st, a);
+  } else {
+    if (vec) hipLaunchKernelGGL((attn_core_bwd_kernel<true, 512, 1>), dim3(B), dim3(512), 0, st, a);
+    else hipLaunchKernelGGL((attn_core_bwd_kernel<false, 512, 1>), dim3(B), dim3(512), 0, st, a);
+  }
   return lh::check_launch("lh_attn_core_bwd_f32");
 }
 

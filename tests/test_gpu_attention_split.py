@@ -12,10 +12,12 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("H,B,S,D", [(36, 6, 40, 10), (510, 5, 30, 10), (516, 5, 30, 3), (1003, 4, 12, 10),
-                                     (2048, 5, 30, 10), (4200, 3, 9, 2), (1000, 4, 70, -1)])
+                                     (2048, 5, 30, 10), (4200, 3, 9, 2), (1000, 4, 70, -1), (40, 3, 300, 255),
+                                     (36, 257, 300, 255), (64, 256, 20, 4), (64, 257, 20, 4), (1000, 300, 9, 3)])
 def test_backward_slots_without_a_state(lh, orc, H, B, S, D):
     """Sentences shorter than the window and columns without a word: slot j of one group is live while slots of
-    the others are not.  Rows of dhs that no slot points at keep their bits."""
+    the others are not.  Rows of dhs that no slot points at keep their bits.  Sixteen wavefronts a column up to
+    256 columns with more than 8 slots, else eight."""
     rng = np.random.default_rng(H + S)
     lens = rng.integers(1, S + 1, size=B)
     lens[:3] = S, 1, 2

@@ -1563,6 +1563,8 @@ int plan_cell(int H, int B, const lh_gemm_seg *segs, int nseg, bool has_addend, 
   if (p->form != kAligned || H % 4 != 0) return LH_OK;
   // Best unsplit launch that can carry the cell against the best launch of any kind followed by
   // the cell kernel (a launch of its own that reads the pre-activations, or S planes of them, back).
+  // 64 to 640 hidden units, 1 to 3 segments, 1 to 64 columns: on average as fast as the best of a sweep over
+  // the configurations and both ways, 22 % behind it at worst (640 units, 2 segments, 32 columns).
   int cfg_any, splits_any, cfg_cell, splits_cell;
   float us_any, us_cell;
   const size_t ws = workspace_bytes;
@@ -1572,17 +1574,6 @@ int plan_cell(int H, int B, const lh_gemm_seg *segs, int nseg, bool has_addend, 
               &splits_cell, true, &us_cell);
   if (cfg_cell < 0) return LH_OK;
   const float cell_us = kCellFixedUs + 28.f * (float)H * (float)B / kReduceBytesPerUs;
-  // A short product with tiles for a quarter of the CUs: the table's fixed costs are those of a full
-  // chip, where the deep slab pays for its LDS traffic; alone on its CU it is two slabs and done.
-  // 256 hidden units, K = 256, 5 and 32 columns: 32x32 tiles in 128-deep slabs 5.5 us, the table's
-  // choice (64x32, 32-deep) 6.8 us.
-  constexpr int kShortConfig = 15;
-  int depth = 0;
-  for (int s = 0; s < nseg; ++s) depth += p->g.K[s];
-  if (g_config_override < 0 && depth <= 256 && ((H + 7) / 8) * ((B + 31) / 32) <= kCUs / 4) {
-    cfg_cell = kShortConfig;
-    us_cell = 0.f;
-  }
   // a configuration override (tuning, tests) asks for the fused form whenever the tile can hold it
   if (g_config_override >= 0 || us_cell <= us_any + cell_us) {
     *fusable = true;

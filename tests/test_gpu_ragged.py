@@ -72,8 +72,7 @@ def test_ragged_products(lh, M, N, Ks, tA, tX, splits):
     finally:
         L.lh_gemm_set_config_override(-1)
         L.lh_gemm_set_splits_override(0)
-    tile = 32 if max(M, N, sum(Ks)) >= 1024 else 64   # the narrowest one the rule allows
-    generic = (not tA and M % 4 and M < tile) or (tX and N % 4 and N < tile) or ((tA or not tX) and min(Ks) < 4)
+    generic = (not tA and M % 4 and M < 32) or (tX and N % 4 and N < 32) or ((tA or not tX) and min(Ks) < 4)
     assert all(n.startswith("gemm_generic" if generic else "gemm_kernel") for n in names), names
 
 

@@ -225,8 +225,9 @@ int lh_gate_gemm_group_plan(int H, int B, const lh_gate_problem *problems, int n
 int lh_gate_gemm_group_f32(int H, int B, const lh_gate_problem *problems, int n_problems,
                            lh_stream_t stream);
 /* Name of the kernel instance lh_gemm_ws_f32 (max_planes = 0) or lh_gemm_planes_f32 would launch
- * for this problem (tile shape and operand flags), as profilers print it; no counterpart in the
- * reference.  Pointers in `segs` are only inspected for alignment; workspace_bytes = 0 describes
+ * for this problem (tile shape and operand flags), as profilers print it: gemm_kernel<...> of eight
+ * arguments for aligned operands, of nine, the last one true, for ragged ones, gemm_generic_kernel<...> for
+ * what neither takes; no counterpart in the reference.  Pointers in `segs` are only inspected for alignment; workspace_bytes = 0 describes
  * lh_gemm_f32 / lh_gemm_act_rows_f32. */
 int lh_gemm_kernel_name(int M, int N, const lh_gemm_seg *segs, int nseg, int transA, int transX,
                         size_t workspace_bytes, int max_planes, char *name, int name_cap);

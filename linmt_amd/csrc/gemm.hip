@@ -14,8 +14,8 @@
 //    time the matrix pipe stands still).  Products whose output has too few tiles split K across
 //    workgroups through partial planes in a caller workspace (splitk_reduce_kernel, or a consumer
 //    that adds the planes itself).  gate_gemm_cell_kernel is the same body with the LSTM cell as
-//    its epilogue, ragged::gemm_kernel the same body for operands at any float's address and with
-//    extents that are no multiple of 4.
+//    its epilogue, gemm_kernel<..., true> (a ninth template argument) the same body for operands at any
+//    float's address and with extents that are no multiple of 4.
 //  * gemm_generic_kernel (a ragged extent shorter than a copy or a tile): scalar loads, one tile shape.
 // WK > 1 splits every slab's k range over WK wavefront groups and reduces the partial
 // accumulators through LDS in a fixed order; deep slabs (BK 64/128) let one workgroup per CU hide
@@ -963,12 +963,13 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_kernel(const GemmArgs 
   gemm_body<BM, BN, WM, WN, WK, BK, TA, TX, false, false>(g, xcd_logical_id());
 }
 
-namespace ragged {
-template <int BM, int BN, int WM, int WN, int WK, int BK, bool TA, bool TX>
+// A kernel of its own for ragged operands, told apart by name.
+template <int BM, int BN, int WM, int WN, int WK, int BK, bool TA, bool TX, bool RAGGED>
 __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_kernel(const GemmArgs g) {
+  static_assert(RAGGED, "aligned operands: the kernel above");
   gemm_body<BM, BN, WM, WN, WK, BK, TA, TX, false, true>(g, xcd_logical_id());
 }
-}  // namespace ragged
+using GemmKernel = void (*)(GemmArgs);  // picks one of the two by the template arguments given
 
 // Stacked gate product W*[x; h; h~] (both operands as stored, no transposes) + LSTM cell.
 template <int BM, int BN, int WM, int WN, int WK, int BK>
@@ -1179,7 +1180,7 @@ int launch_cfg(const GemmArgs &g0, bool ta, bool tx, Form form, hipStream_t st) 
         return lh::fail_arg("lh_gemm_f32: internal error, ragged operands reached an aligned-only tile");
       } else {
 #define LH_GEMM_LAUNCH(TA, TX)                                                              \
-  rc = launch_kernel(ragged::gemm_kernel<BM, BN, WM, WN, WK, BK, TA, TX>,                   \
+  rc = launch_kernel((GemmKernel)gemm_kernel<BM, BN, WM, WN, WK, BK, TA, TX, true>,         \
                      smem2_floats<BM, BN, WM, WN, WK, BK, TA, TX>() * 4, grid, block, st, g)
         if (!ta && !tx) LH_GEMM_LAUNCH(false, false);
         else if (ta) LH_GEMM_LAUNCH(true, false);
@@ -1188,7 +1189,7 @@ int launch_cfg(const GemmArgs &g0, bool ta, bool tx, Form form, hipStream_t st) 
       }
     } else {
 #define LH_GEMM_LAUNCH(TA, TX)                                                              \
-  rc = launch_kernel(gemm_kernel<BM, BN, WM, WN, WK, BK, TA, TX>,                           \
+  rc = launch_kernel((GemmKernel)gemm_kernel<BM, BN, WM, WN, WK, BK, TA, TX>,               \
                      smem2_floats<BM, BN, WM, WN, WK, BK, TA, TX>() * 4, grid, block, st, g)
       if (!ta && !tx) LH_GEMM_LAUNCH(false, false);
       else if (ta) LH_GEMM_LAUNCH(true, false);
@@ -1272,7 +1273,7 @@ int occupancy_cfg(bool ta, bool tx, int *blocks_per_cu, int *lds_bytes) {
   do {                                                                                            \
     constexpr int bytes = smem2_floats<BM, BN, WM, WN, WK, BK, TA, TX>() * 4;                     \
     *lds_bytes = bytes;                                                                           \
-    auto kernel = gemm_kernel<BM, BN, WM, WN, WK, BK, TA, TX>;                                    \
+    GemmKernel kernel = gemm_kernel<BM, BN, WM, WN, WK, BK, TA, TX>;                              \
     if (bytes > 64 * 1024)                                                                        \
       (void)hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, \
                                 bytes);                                                           \
@@ -1994,8 +1995,8 @@ extern "C" int lh_gemm_kernel_name(int M, int N, const lh_gemm_seg *segs, int ns
   if (rc != LH_OK) return rc;
   const Config &k = kConfigs[p.config];
   if (p.form != kGeneric)
-    snprintf(name, name_cap, "gemm_kernel<%d, %d, %d, %d, %d, %d, %s, %s>", k.bm, k.bn, k.wm, k.wn,
-             k.wk, k.bk, p.ta ? "true" : "false", p.tx ? "true" : "false");
+    snprintf(name, name_cap, "gemm_kernel<%d, %d, %d, %d, %d, %d, %s, %s%s>", k.bm, k.bn, k.wm, k.wn,
+             k.wk, k.bk, p.ta ? "true" : "false", p.tx ? "true" : "false", p.form == kRagged ? ", true" : "");
   else
     snprintf(name, name_cap, "gemm_generic_kernel<%d, %d, %d, %d, %d, %d, %s, %s, false>", k.bm,
              k.bn, k.wm, k.wn, k.wk, k.bk, p.ta ? "true" : "false", p.tx ? "true" : "false");

@@ -24,11 +24,29 @@ def _odd(a, off):
     return view
 
 
-# M, N, Ks, transA, transX
+# M, N, Ks, transA, transX.  Tails of 1, 2 and 3 past whole slabs of 16 to 128 k, in one segment and in two, with
+# either operand or both contiguous along k; tiles moved back along m, along n and along both.
 SHAPES = [(33, 5, (4,), False, False), (35, 33, (19, 5), False, True), (63, 40, (130,), False, False),
           (129, 97, (67, 18), True, False), (131, 3, (5,), True, False), (257, 129, (33,), False, True),
           (1003, 84, (250, 131), False, False), (31, 30, (9,), False, False), (40, 31, (7,), False, True),
-          (34, 34, (3,), True, False), (5001, 12, (256,), False, False), (256, 130, (5001,), True, False)]
+          (34, 34, (3,), True, False), (5001, 12, (256,), False, False), (256, 130, (5001,), True, False),
+          (131, 40, (129,), True, False), (70, 45, (130, 67), True, False), (133, 50, (131, 259), False, False),
+          (129, 131, (257, 18), False, True), (1001, 1027, (35,), False, True), (130, 70, (66, 129, 5), True, False)]
+RAGGED_CONFIGS = {0, 3, 7, 12, 15, 18, 24, 32, 35, 36}
+
+
+def _kernel(M, N, Ks, tA, tX, off, tile):
+    """What takes the product: 'aligned', 'ragged' or 'generic'; tile = (config, BM, BN) or None for any."""
+    extents = ([M] if not tA else list(Ks)) + ([N] if tX else list(Ks))
+    if off == 0 and all(e % 4 == 0 for e in extents):
+        return "aligned"
+    ragged_m, ragged_n = not tA and M % 4 != 0, tX and N % 4 != 0
+    if (ragged_m and M < 32) or (ragged_n and N < 32) or ((tA or not tX) and min(Ks) < 4):
+        return "generic"
+    if tile is None:
+        return "ragged"
+    cfg, bm, bn = tile
+    return "ragged" if cfg in RAGGED_CONFIGS and not (ragged_m and bm > M) and not (ragged_n and bn > N) else "generic"
 
 
 @pytest.mark.parametrize("splits", [0, 3])
@@ -49,7 +67,7 @@ def test_ragged_products(lh, M, N, Ks, tA, tX, splits):
     limit = (sum(Ks) + 8) * 2.0 ** -24 * (mag + np.abs(C0) + np.abs(bias[:, None]))
     ws = torch.full((4 << 20,), float("nan"), device="cuda")
     n_cfg = L.lh_gemm_set_config_override(-1)
-    names = set()
+    ran = set()
     try:
         L.lh_gemm_set_splits_override(splits)
         for cfg in [-1] + list(range(n_cfg)):
@@ -57,8 +75,16 @@ def test_ragged_products(lh, M, N, Ks, tA, tX, splits):
             for off in (0, 1, 3):
                 segs = [(_odd(A, off), A.shape[0], _odd(X, off), X.shape[0], K)
                         for A, X, K in zip(As, Xs, Ks)]
-                if cfg < 0:
-                    names.add(lh.gemm_kernel_name(M, N, segs, transA=tA, transX=tX, workspace_bytes=16 << 20))
+                name = lh.gemm_kernel_name(M, N, segs, transA=tA, transX=tX, workspace_bytes=16 << 20)
+                info = lh.gemm_config_info(cfg, tA, tX) if cfg >= 0 else None
+                form = _kernel(M, N, Ks, tA, tX, off, (cfg, info["BM"], info["BN"]) if info else None)
+                assert (form == "generic") == name.startswith("gemm_generic_kernel<"), (name, cfg, off)
+                assert (form == "ragged") == (name.startswith("gemm_kernel<") and name.count(",") == 8), (name, cfg, off)
+                if cfg >= 0 and form != "generic":
+                    assert name.startswith("gemm_kernel<%d, %d, %d, %d, %d, %d," % tuple(
+                        info[k] for k in ("BM", "BN", "WM", "WN", "WK", "BK"))), (name, cfg)
+                    if form == "ragged":
+                        ran.add(cfg)
                 ldc = M + 3                       # three guard rows behind every column
                 out = np.full((ldc, N), 7.0, np.float32)
                 out[:M] = C0
@@ -72,8 +98,8 @@ def test_ragged_products(lh, M, N, Ks, tA, tX, splits):
     finally:
         L.lh_gemm_set_config_override(-1)
         L.lh_gemm_set_splits_override(0)
-    generic = (not tA and M % 4 and M < 32) or (tX and N % 4 and N < 32) or ((tA or not tX) and min(Ks) < 4)
-    assert all(n.startswith("gemm_generic" if generic else "gemm_kernel") for n in names), names
+    if min(M, N) >= 129 and min(Ks) >= 4:     # large enough for every ragged configuration
+        assert ran == RAGGED_CONFIGS, ran
 
 
 @pytest.mark.parametrize("V", [13, 4097, 8191, 30003, 65533])

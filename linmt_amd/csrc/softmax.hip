@@ -7,8 +7,8 @@
 // hand back probabilities.  Columns that are not 16-byte aligned or whose length is no multiple of 4
 // take the RAGGED form of the same kernels: 16-byte accesses at dword alignment (one instruction
 // each here) and a guarded last quad.  Its exponentials are expf / exp where the aligned form
-// multiplies and takes v_exp_f32.  Columns longer than 65536 rows take a generic strided kernel that
-// re-reads the column (from L2) instead.
+// multiplies and takes v_exp_f32.  Columns longer than 65536 rows and short ragged ones take a generic
+// strided kernel that re-reads the column (from L2) instead.
 // Log-softmax and the top 13 of 84 columns of 30003 rows: 107 us in the strided kernel, 12 us here.
 #include "lh_common.h"
 
@@ -125,7 +125,7 @@ __global__ __launch_bounds__(kT, (NV <= 8 ? 8 : 4)) void softmax_fwd_kernel(cons
   }
 }
 
-// Columns too long for the registers: re-read twice.
+// Columns too long for the registers, and short ragged ones: re-read twice.
 __global__ __launch_bounds__(kT) void softmax_fwd_generic_kernel(const float *logits, int ldl,
                                                                  const float *bias, int V, float *p,
                                                                  int ldp) {
@@ -342,7 +342,8 @@ constexpr int kIdNone = 0x7fffffff;
 //   fast path: tau = K-th largest of G group maxima (G = 16 wavefronts for K <= 16, else 64
 //     quarter-wavefronts): K groups hold an element >= tau.  Values only, a few instructions per
 //     element; the list has a few dozen entries on ordinary logits.
-//   exact path (list overflow: massive ties, winners packed into one group): per-thread bests with
+//   exact path (a long list: fewer than K well-filled groups, massive ties, winners packed into one
+//     group): per-thread bests with
 //     ids, the K best of each wavefront's 64 thread-bests, tau = K-th best of those 16*K survivors
 //     as a (value, id) pair.  Never more than K*NV*4 <= kListCap elements pass it.
 constexpr int kListCap = 4096;
@@ -442,6 +443,7 @@ __device__ __forceinline__ void beam_topk_body(
     logp_eof[b] = score_of(z);
   }
 
+  const int longest = min(64 + 16 * K, kT);  // list that the fast path ranks
   // ---- fast path: threshold from group maxima ----------------------------------------------
   {
     const int G = K <= 16 ? kNW : 64;
@@ -458,10 +460,14 @@ __device__ __forceinline__ void beam_topk_body(
       if (rank == K - 1) s_tau_v = mine;
     }
     __syncthreads();
-    collect<NV>(x, tid, V, s_tau_v, kIdNone, l_v, l_id, &s_count);  // every element >= tau
+    // Groups that are empty or hold a row or two (a column of up to K groups' rows: 3072 for 13 candidates) make a
+    // threshold that much of the column passes.  Ranking a list against itself takes 0.1 us an entry, the exact
+    // path 1.5 us a candidate: 12 columns of 3001 rows, 13 candidates, 819 us and 18.
+    if (s_tau_v != kNegInf || V <= longest) collect<NV>(x, tid, V, s_tau_v, kIdNone, l_v, l_id, &s_count);  // every element >= tau
+    else if (tid == 0) s_count = kListCap + 1;
     __syncthreads();
   }
-  if (s_count > kListCap) {
+  if (s_count > longest) {
     // ---- exact path ---------------------------------------------------------------------------
     // thread best; a thread without a finite value gets a unique id above every vocabulary id so
     // that the order stays strict
@@ -629,6 +635,11 @@ int pick_nv(int V) {
     if (V <= kT * 4 * nv) return nv;
   return 0;
 }
+// A short ragged column stays with the strided kernel, which reads it from L1 again at no cost: 501 rows, 768
+// columns, strided / registers: softmax 6.3 / 7.5 us, output error 9.4 / 10.7; 1501 rows 7.9 / 8.2 and 11.0 /
+// 11.3; 2001 rows 8.7 / 8.3 and 11.8 / 11.5.  Top 4 of 501 rows 21 / 27 us, of 1001 rows 22 / 13.
+constexpr int kShortRagged = 1536, kShortRaggedTopK = 768;
+int ragged_nv(int V, bool ragged, int shortest) { return ragged && V <= shortest ? 0 : pick_nv(V); }
 bool quads_ok(const float *base, int ld, const float *bias, int V) {
   return V % 4 == 0 && ld % 4 == 0 && lh::aligned16(base) && lh::aligned16(bias);
 }
@@ -638,8 +649,10 @@ bool quads_ok(const float *base, int ld, const float *bias, int V) {
   case 2 * NV + RAGGED:                                                                   \
     hipLaunchKernelGGL((KERNEL<NV, RAGGED != 0>), grid, block, 0, st, __VA_ARGS__);       \
     break;
-#define LH_COLUMN_LAUNCH(KERNEL, GENERIC, NVSEL, ISRAGGED, ...)                          \
-  switch (2 * (NVSEL) + ((NVSEL) && (ISRAGGED) ? 1 : 0)) {                               \
+#define LH_COLUMN_LAUNCH(KERNEL, GENERIC, SHORTEST, ISRAGGED, ...)                        \
+  const bool ragged = ISRAGGED;                                                           \
+  const int nv = ragged_nv(V, ragged, SHORTEST);                                          \
+  switch (2 * nv + (nv && ragged ? 1 : 0)) {                                              \
     LH_COLUMN_CASE(KERNEL, 2, 0, __VA_ARGS__)                                             \
     LH_COLUMN_CASE(KERNEL, 4, 0, __VA_ARGS__)                                             \
     LH_COLUMN_CASE(KERNEL, 8, 0, __VA_ARGS__)                                             \
@@ -660,7 +673,7 @@ extern "C" int lh_softmax_fwd_f32(const float *logits, int ldl, const float *bia
                         ldp);
   hipStream_t st = lh::as_stream(stream);
   const dim3 grid(B), block(kT);
-  LH_COLUMN_LAUNCH(softmax_fwd_kernel, softmax_fwd_generic_kernel, pick_nv(V), !(quads_ok(logits, ldl, bias, V) && quads_ok(p, ldp, nullptr, V)),
+  LH_COLUMN_LAUNCH(softmax_fwd_kernel, softmax_fwd_generic_kernel, kShortRagged, !(quads_ok(logits, ldl, bias, V) && quads_ok(p, ldp, nullptr, V)),
                    logits, ldl, bias, V, p, ldp)
   return lh::check_launch("lh_softmax_fwd_f32");
 }
@@ -681,7 +694,7 @@ extern "C" int lh_logsoftmax_xent_f32(const float *logits, int ldl, const float 
     return lh::fail_arg("lh_logsoftmax_xent_f32: V=%d B=%d ldl=%d or NULL pointer", V, B, ldl);
   hipStream_t st = lh::as_stream(stream);
   const dim3 grid(B), block(kT);
-  LH_COLUMN_LAUNCH(logsoftmax_tgt_kernel, logsoftmax_tgt_generic_kernel, pick_nv(V), !quads_ok(logits, ldl, bias, V),
+  LH_COLUMN_LAUNCH(logsoftmax_tgt_kernel, logsoftmax_tgt_generic_kernel, kShortRagged, !quads_ok(logits, ldl, bias, V),
                    logits, ldl, bias, V, tgt0, logp_tgt)
   int rc = lh::check_launch("lh_logsoftmax_xent_f32");
   if (rc != LH_OK) return rc;
@@ -699,7 +712,7 @@ extern "C" int lh_softmax_xent_grad_f32(const float *logits, int ldl, const floa
                         ldl, ldz);
   hipStream_t st = lh::as_stream(stream);
   const dim3 grid(B), block(kT);
-  LH_COLUMN_LAUNCH(softmax_xent_grad_kernel, softmax_xent_grad_generic_kernel, pick_nv(V), !(quads_ok(logits, ldl, bias, V) && quads_ok(dz, ldz, nullptr, V)),
+  LH_COLUMN_LAUNCH(softmax_xent_grad_kernel, softmax_xent_grad_generic_kernel, kShortRagged, !(quads_ok(logits, ldl, bias, V) && quads_ok(dz, ldz, nullptr, V)),
                    logits, ldl, bias, V, tgt0, mask01, dz, ldz, logp_tgt)
   int rc = lh::check_launch("lh_softmax_xent_grad_f32");
   if (rc != LH_OK) return rc;
@@ -750,7 +763,7 @@ extern "C" int lh_beam_topk_f32(const float *logits, int ldl, const float *bias,
     return lh::fail_arg("lh_beam_topk_f32: K=%d outside [1,min(%d,V=%d)]", K, LH_BEAM_MAX_K, V);
   hipStream_t st = lh::as_stream(stream);
   const dim3 grid(B), block(kT);
-  LH_COLUMN_LAUNCH(beam_topk_kernel, beam_topk_generic_kernel, pick_nv(V), !quads_ok(logits, ldl, bias, V),
+  LH_COLUMN_LAUNCH(beam_topk_kernel, beam_topk_generic_kernel, kShortRaggedTopK, !quads_ok(logits, ldl, bias, V),
                    logits, ldl, bias, V, K, eof_id, cand_logp, cand_id, logp_eof)
   return lh::check_launch("lh_beam_topk_f32");
 }

@@ -102,7 +102,9 @@ def test_ragged_products(lh, M, N, Ks, tA, tX, splits):
         assert ran == RAGGED_CONFIGS, ran
 
 
-@pytest.mark.parametrize("V", [13, 4097, 8191, 30003, 65533])
+# 768 and 1536 rows: the last a short ragged column may have; up to 3072 rows fill fewer wavefronts than there are
+# candidates
+@pytest.mark.parametrize("V", [13, 501, 767, 769, 1535, 1537, 3001, 3073, 4097, 8191, 30003, 65533])
 @pytest.mark.parametrize("off", [0, 1])
 def test_ragged_columns(lh, V, off):
     rng = np.random.default_rng(V + off)
@@ -158,9 +160,39 @@ def test_ragged_columns(lh, V, off):
     assert_close(le.cpu().numpy(), logp[1], "log p(<EOF>)", rtol=1e-5, atol=1e-5)
 
 
-def test_partial_nan_column(lh):
+@pytest.mark.parametrize("K", [1, 4, 16, 17, 64])
+@pytest.mark.parametrize("V", [100, 128, 129, 500, 769, 772, 1088, 1092, 2000, 3073, 3076, 4096, 4100])
+def test_candidates_of_short_columns(lh, V, K):
+    """Columns that fill few or partly filled groups: nothing of them, all of them or the K best pass the first
+    threshold.  Aligned and ragged; ties, one value everywhere, few finite values, winners packed together."""
+    rng = np.random.default_rng(V * 100 + K)
+    B = 6
+    z = rng.normal(0, 3, (V, B)).astype(np.float32)
+    z[:, 1] = np.round(z[:, 1])
+    z[:, 2] = -1.5
+    z[max(1, K - 1):, 3] = -np.inf           # fewer finite rows than candidates
+    z[:, 4] = np.sort(z[:, 4])               # the winners in one wavefront, at the end
+    z[:, 5] = np.sort(z[:, 5])[::-1]         # ... at the start
+    z64 = z.astype(np.float64)
+    logp = z64 - scipy.special.logsumexp(z64, axis=0)
+    cl, ci = torch.full((K * B,), 7.0, device="cuda"), torch.full((K * B,), -7, dtype=torch.int32, device="cuda")
+    le = torch.empty(B, device="cuda")
+    for off in (0, 1):
+        lh.beam_topk(_odd(z, off), V, None, V, B, K, 1, cl, ci, le)
+        gi, gl = ci.cpu().numpy().reshape(B, K), cl.cpu().numpy().reshape(B, K)
+        for b in range(B):
+            order = np.lexsort((np.arange(V), -z64[:, b]))[:K]
+            assert gi[b].tolist() == order.tolist(), f"column {b} offset {off}"
+            want = logp[order, b]
+            finite = np.isfinite(want)
+            assert np.array_equal(gl[b][~finite], want[~finite])
+            assert_close(gl[b][finite], want[finite], f"column {b} scores", rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("V", [515, 1027, 2051, 4099])
+def test_partial_nan_column(lh, V):
     """A column of NaN holds no candidate: K rounds of arg-max over nothing, as the strided kernel gives."""
-    V, B, K = 4099, 2, 5
+    B, K = 2, 5
     z = np.full((V, B), np.nan, np.float32)
     z[:, 1] = np.arange(V) / V
     cl, ci = torch.zeros(K * B, device="cuda"), torch.zeros(K * B, dtype=torch.int32, device="cuda")

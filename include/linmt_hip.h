@@ -692,15 +692,16 @@ int lh_attn_core_bwd_f32(int H, int B, int D, int max_len, int hs_steps, const f
  * sumsq is read on the device, so no host synchronisation sits between norm and update.
  */
 #define LH_SUMSQ_WORKSPACE 1024
-/* dst[0:rows, 0:cols] = src[0:rows, 0:cols], both column-major (leading dimensions ld_dst, ld_src);
- * the blocks must not overlap. */
-int lh_copy_block_f32(float *dst, long long ld_dst, const float *src, long long ld_src, long long rows,
-                      long long cols, lh_stream_t stream);
 int lh_grad_sumsq_f32(const float *g, long long rows, long long cols, long long ld, float scale,
                       double *workspace, double *accum, lh_stream_t stream);
-/* The same two for many tensors in a few launches.  An item with norm >= 0 has its squares added to
- * norms[norm] and is rescaled by it; norm < 0: neither.  Items that share a slot must follow one another.
- * workspace holds lh_grad_sumsq_items_workspace(items, n) doubles. */
+int lh_sgd_step_f32(float *theta, long long ld_theta, float *g, long long ld_g, long long rows,
+                    long long cols, const int *col_index, float learning_rate, float grad_scale,
+                    const double *sumsq, float norm_clip, float individual_clip,
+                    lh_stream_t stream);
+/* The same two for many tensors in a few launches, which is what UpdateWeights calls.  An item with
+ * norm >= 0 has its squares added to norms[norm] and is rescaled by it; norm < 0: neither.  Items that
+ * share a slot must follow one another.  workspace holds lh_grad_sumsq_items_workspace(items, n) doubles,
+ * fewer than sum(rows * cols) / 2048 + n + 2 of them. */
 typedef struct {
   float *theta;
   long long ld_theta;
@@ -715,10 +716,10 @@ int lh_grad_sumsq_items_f32(const lh_update_item *items, int n, float scale, dou
 int lh_sgd_step_items_f32(const lh_update_item *items, int n, float learning_rate, float grad_scale,
                           const double *norms, float norm_clip, float individual_clip,
                           lh_stream_t stream);
-int lh_sgd_step_f32(float *theta, long long ld_theta, float *g, long long ld_g, long long rows,
-                    long long cols, const int *col_index, float learning_rate, float grad_scale,
-                    const double *sumsq, float norm_clip, float individual_clip,
-                    lh_stream_t stream);
+/* dst[0:rows, 0:cols] = src[0:rows, 0:cols], both column-major (leading dimensions ld_dst, ld_src);
+ * the blocks must not overlap. */
+int lh_copy_block_f32(float *dst, long long ld_dst, const float *src, long long ld_src, long long rows,
+                      long long cols, lh_stream_t stream);
 
 #ifdef __cplusplus
 }

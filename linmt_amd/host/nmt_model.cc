@@ -186,7 +186,22 @@ void NeuralMachineTranslation::InitModel() {
   softmax_layer_.Init(this, B, T);
   if (cfg_.train_mode_) {
     softmax_layer_.InitTraining();
-    p_device_norm_workspace_.Alloc(LH_SUMSQ_WORKSPACE);
+    // norms of every gradient, at the most words a minibatch can have: at least 2048 floats per partial sum
+    size_t floats = softmax_layer_.p_device_d_grad_.size() + softmax_layer_.p_device_b_d_grad_.size(), tensors = 2;
+    for (int side = seq2seq ? 0 : 1; side < 2; ++side)
+      for (int l = 0; l < L; ++l) {
+        LstmLayer &Ly = side == 0 ? SourceLayer(l) : TargetLayer(l);
+        floats += Ly.p_device_w_h_grad_.size() + Ly.p_device_b_grad_.size() + Ly.p_device_m_grad_.size() +
+                  Ly.p_device_q_grad_.size() + Ly.p_device_small_w_grad_.size();
+        tensors += 4 * 4 + 1;  // each gate of the stacked ones may be a tensor
+      }
+    if (cfg_.attention_mode_ && seq2seq) {
+      const AttentionLayer &A = attention_layer_;
+      floats += A.p_device_w_a_grad_.size() + A.p_device_w_p_grad_.size() + A.p_device_v_p_grad_.size() +
+                A.p_device_output_bias_grad_.size() + A.p_device_w_c_p1_grad_.size() + A.p_device_w_c_p2_grad_.size();
+      tensors += 6;
+    }
+    p_device_norm_workspace_.Alloc(floats / 2048 + tensors + 1);
     p_device_norms_.Alloc(512);
   }
   // wiring that does not change between minibatches: h_below and h~ pointers
@@ -973,14 +988,14 @@ void NeuralMachineTranslation::DecodeBatch(const std::vector<std::vector<int>> &
     }
   } one_stream{models};
   if (n_models > 1) {
-    while (ensemble_events_.size() < (size_t)n_models + 1) {
+    while (ensemble_events_.size() + 1 < (size_t)n_models) {
       hipEvent_t e;
       HipErrorWrapper(hipEventCreateWithFlags(&e, hipEventDisableTiming), "ensemble event creation failed");
       ensemble_events_.push_back(e);
     }
     for (int k = 1; k < n_models; ++k) {
-      HipErrorWrapper(hipEventRecord(ensemble_events_[k], models[k]->stream_), "ensemble event record failed");
-      HipErrorWrapper(hipStreamWaitEvent(stream_, ensemble_events_[k], 0), "ensemble wait failed");
+      HipErrorWrapper(hipEventRecord(ensemble_events_[k - 1], models[k]->stream_), "ensemble event record failed");
+      HipErrorWrapper(hipStreamWaitEvent(stream_, ensemble_events_[k - 1], 0), "ensemble wait failed");
       models[k]->stream_ = models[k]->profiler_.stream_ = stream_;
     }
   }

@@ -791,8 +791,7 @@ void NeuralMachineTranslation::UpdateWeights() {
   }
   if (!table.empty()) {
     const size_t need = lh_grad_sumsq_items_workspace(table.data(), (int)table.size());
-    // the embedding gradients' share varies with the minibatch's words: grow with room to spare
-    if (need > p_device_norm_workspace_.size()) p_device_norm_workspace_.Alloc(need + need / 4);
+    if (need > p_device_norm_workspace_.size()) throw LinmtError("CalculateGlobalNorm: workspace too small");
     ProfileScope ps(profiler_, kTagUpdate, 4.0 * elements);
     LhErrorWrapper(lh_grad_sumsq_items_f32(table.data(), (int)table.size(), scale,
                                            p_device_norm_workspace_.get(), p_device_norms_.get(), stream_),

@@ -472,7 +472,9 @@ extern "C" int lh_attn_core_fwd_f32(int H, int B, int D, int max_len, int hs_ste
   else if (vec && W <= kRegsSlots && H <= 8 * kThreads)
     hipLaunchKernelGGL((attn_core_regs_kernel<2, kRegsSlots>), dim3(B), dim3(kThreads), 0, st, a);
   // Any other: as many wavefronts per column as leave every column resident (256 CUs of 32 wavefronts).
-  // Past 2048 columns none of the three does; eight wavefronts then tail off best.
+  // Past 2048 columns none of the three does; eight wavefronts then tail off best.  1000 rows, 60 slots, with
+  // sixteen / eight / four wavefronts: 512 columns 22 / 25 / 34 us, 768 columns 36 / 33 / 38, 1536 columns
+  // 68 / 77 / 67, 3072 columns 121 / 113 / 127; four wavefronts with a slot at a time 38, 41, 63 and 119.
   else if (B <= 512) launch_general<1024>(a, vec, st);
   else if (B <= 1024 || B > 2048 || W > 256) launch_general<512>(a, vec, st);
   else launch_general<256>(a, vec, st);

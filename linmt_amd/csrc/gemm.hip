@@ -16,7 +16,8 @@
 //    that adds the planes itself).  gate_gemm_cell_kernel is the same body with the LSTM cell as
 //    its epilogue, gemm_kernel<..., true> (a ninth template argument) the same body for operands at any
 //    float's address and with extents that are no multiple of 4.
-//  * gemm_generic_kernel (a ragged extent shorter than a copy or a tile): scalar loads, one tile shape.
+//  * gemm_generic_kernel (a ragged extent shorter than a copy or a tile, one slab of k): scalar loads, one
+//    tile shape.
 // WK > 1 splits every slab's k range over WK wavefront groups and reduces the partial
 // accumulators through LDS in a fixed order; deep slabs (BK 64/128) let one workgroup per CU hide
 // its own memory latency.  Workgroup ids are remapped so that each of the 8 XCDs (ids are dealt
@@ -1471,6 +1472,9 @@ int prepare(int M, int N, const lh_gemm_seg *segs, int nseg, int transA, int tra
     // a unit along k that is short of four values reaches back inside its row
     if ((transA || !transX) && e.K < 4) vec = false;
   }
+  // One 16-deep slab is all the scalar kernel has to do, too: 30003 x 1000, K = 16, 29.6 us there and 37.7
+  // here, 130 x 33 5.7 and 6.1, 1002 x 1000 6.4 and 6.2; at K = 18 40 and 43, 6.5 and 6.2, 7.3 and 6.8.
+  if (!aligned && nseg == 1 && segs[0].K <= 16) vec = false;
   // A tile along a ragged m (n) moves back inside the operand: it must be at least a tile long.  The
   // narrowest tiles are 32 wide; below that the scalar kernel runs a single row of tiles anyway.
   const bool ragged_m = !transA && M % 4 != 0, ragged_n = transX && N % 4 != 0;

@@ -26,7 +26,8 @@ def _odd(a, off):
 
 # M, N, Ks, transA, transX.  Tails of 1, 2 and 3 past whole slabs of 16 to 128 k, in one segment and in two, with
 # either operand or both contiguous along k; tiles moved back along m, along n and along both.
-SHAPES = [(33, 5, (4,), False, False), (35, 33, (19, 5), False, True), (63, 40, (130,), False, False),
+SHAPES = [(33, 5, (4,), False, False), (33, 5, (17,), False, False), (131, 3, (18,), True, False),
+          (63, 34, (16,), False, True), (35, 33, (19, 5), False, True), (63, 40, (130,), False, False),
           (129, 97, (67, 18), True, False), (131, 3, (5,), True, False), (257, 129, (33,), False, True),
           (1003, 84, (250, 131), False, False), (31, 30, (9,), False, False), (40, 31, (7,), False, True),
           (34, 34, (3,), True, False), (5001, 12, (256,), False, False), (256, 130, (5001,), True, False),
@@ -42,6 +43,8 @@ def _kernel(M, N, Ks, tA, tX, off, tile):
         return "aligned"
     ragged_m, ragged_n = not tA and M % 4 != 0, tX and N % 4 != 0
     if (ragged_m and M < 32) or (ragged_n and N < 32) or ((tA or not tX) and min(Ks) < 4):
+        return "generic"
+    if len(Ks) == 1 and Ks[0] <= 16:
         return "generic"
     if tile is None:
         return "ragged"
@@ -98,7 +101,7 @@ def test_ragged_products(lh, M, N, Ks, tA, tX, splits):
     finally:
         L.lh_gemm_set_config_override(-1)
         L.lh_gemm_set_splits_override(0)
-    if min(M, N) >= 129 and min(Ks) >= 4:     # large enough for every ragged configuration
+    if min(M, N) >= 129 and min(Ks) > 16:     # large enough for every ragged configuration
         assert ran == RAGGED_CONFIGS, ran
 
 

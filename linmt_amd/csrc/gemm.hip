@@ -16,6 +16,7 @@
 //    that adds the planes itself).  gate_gemm_cell_kernel is the same body with the LSTM cell as
 //    its epilogue, gemm_kernel<..., true> (a ninth template argument) the same body for operands at any
 //    float's address and with extents that are no multiple of 4.
+//    Tiles of eight 32x32 blocks (products of few columns) run its streamed form, stream_body.
 //  * gemm_generic_kernel (a ragged extent shorter than a copy or a tile, one slab of k): scalar loads, one
 //    tile shape.
 // WK > 1 splits every slab's k range over WK wavefront groups and reduces the partial
@@ -570,11 +571,125 @@ struct Stage {
   }
 };
 
-template <int BM, int BN, int WM, int WN, int WK, int BK, bool TA, bool TX>
+// ---- streamed form --------------------------------------------------------------------------
+// One 32x32 block of C per wavefront, and every wavefront on its own: it reads the k it multiplies
+// (CK of every slab) into a ring of LDS stages that no other wavefront touches, straight from
+// memory (global_load_lds, no register and no LDS store of its own in between), and the K loop has
+// no barrier.  All eight wavefronts share the sum over the partial blocks and the epilogue, and the cell's
+// inputs are requested behind the first slabs.
+// What bounds these products is not bandwidth but what a workgroup does between its loads and its MFMAs:
+// with one workgroup per CU nothing else hides a staging store, a barrier or the wavefront that sums
+// eight partial tiles alone.  4000 x 64, K = 1000 / 2000 (weights from HBM): 11.3 / 17.0 us staged, 9.4 / 14.3
+// streamed; transposed 11.2 / 17.4 and 10.1 / 16.5.  A fixed part of 4.0 instead of 5.6 us (an empty launch:
+// 2.8), and 0.63 us per slab of 128 k where the MFMAs alone take 0.47 at the 2.16 GHz the card runs here.
+// Deeper rings (5 stages: 14.3), fragments read a slab ahead (15.2), 16 wavefronts (15.9) and four of 32 k each
+// (15.6) gave nothing.  Shapes of 8 k per wavefront and slab stay staged except the 32x32 one: their 32-byte runs along k
+// cost more than the stores (32x64, full CUs: 0.0108 us per k and workgroup against 0.0087).
+constexpr int kRingStages = 4;
+template <int BM, int BN, int WM, int WN, int WK, int BK>
+constexpr bool streamed() {
+  // eight wavefronts, a 32 x 32 block each, 16 k of every slab (8 where all of them share one block)
+  return BM == 32 * WM && BN == 32 * WN && WK >= 4 && WM * WN * WK == 8 && BK >= (WK == 8 ? 64 : 16 * WK);
+}
+// Floats from one column to the next of a partial tile in LDS: a quarter of the rows (a gate's share
+// of the tile) as padding puts the columns a wavefront reads at once on distinct banks.
+template <int BM>
+constexpr int spread_ld() {
+  return BM + BM / 4;
+}
+
+template <int BM, int BN, int WM, int WN, int WK, int BK, bool TA, bool TX, bool RAGGED>
 constexpr int smem2_floats() {
   constexpr int NT = 64 * WM * WN * WK;
+  if constexpr (!RAGGED && streamed<BM, BN, WM, WN, WK, BK>())
+    return cmax(kRingStages * WM * WN * BK * 64, WK * BN * spread_ld<BM>());
   return cmax(2 * (Stage<BM, BK, NT, TA, false>::kFloats + Stage<BN, BK, NT, !TX, false>::kFloats),
               (WK - 1) * BM * BN);
+}
+
+// A wavefront's CK x 32 piece of one operand in its ring stage.  A load writes 64 consecutive
+// 16-byte units, one per lane, so what the layout can choose is which unit a lane fetches:
+//  * contiguous along d: rows of 32 floats, one per k; the k of a group of 8 in the order 0 4 2 6 1 5 3 7,
+//    which puts the two k of one MFMA step (k and k + 4, lanes 0-31 and 32-63) into neighbouring rows:
+//    a fragment read is 64 consecutive floats;
+//  * contiguous along k: rows of CK floats, one per d, their units permuted (XOR with bits of d) so
+//    that the 16 lanes of one phase of a 16-byte read meet all banks.
+template <int CK, bool KC>
+struct Piece {
+  static constexpr int U = CK / 4;       // KC: units per row
+  static constexpr int kLoads = CK / 8;  // wavefront loads per piece
+  static constexpr int kFloats = CK * 32;
+  unsigned goff[kLoads];
+
+  static __device__ __forceinline__ int swap02(int k) { return (k & ~5) | ((k & 1) << 2) | ((k >> 2) & 1); }
+  static __device__ __forceinline__ int swizzle(int d) { return (d / (16 / U)) % U; }
+  static __device__ __forceinline__ int unit_d(int u) { return KC ? u / U : (u % 8) * 4; }
+  static __device__ __forceinline__ int unit_k(int u) {
+    return KC ? ((u % U) ^ swizzle(u / U)) * 4 : swap02(u / 8);
+  }
+  // dn = rows/columns of the operand from the tile origin on, first = this wavefront's first of them
+  __device__ __forceinline__ void set_ld(int ld, int lane, int first, int dn) {
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      const int u = lane + i * 64;
+      const int d = first + unit_d(u), k = unit_k(u);
+      const unsigned off = KC ? (unsigned)(d * ld + k) * 4u : (unsigned)(k * ld + d) * 4u;
+      goff[i] = d < dn ? off : 0u;
+    }
+  }
+  template <int GQ>
+  __device__ __forceinline__ void set_ld_gates(int ld, int lane, int first, int H, int rows_left) {
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      const int u = lane + i * 64;
+      const int d = first + unit_d(u), k = unit_k(u);
+      const int r = d % GQ, row = (d / GQ) * H + r;
+      const unsigned off = KC ? (unsigned)(row * ld + k) * 4u : (unsigned)(k * ld + row) * 4u;
+      goff[i] = r < rows_left ? off : 0u;
+    }
+  }
+  static __device__ __forceinline__ void load_unit(const float *base, unsigned off, unsigned lds) {
+    // No register receives the data, so nothing the compiler allocates can meet the load in
+    // flight; its addresses are read when it is issued.  Completion: wait_loads below.
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :
+                 : "s"(lds), "v"(off), "s"(base)
+                 : "memory", "m0");
+  }
+  __device__ __forceinline__ void load(const float *base, unsigned lds) const {
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) load_unit(base, goff[i], lds + 1024u * i);
+  }
+  // The same where the segment ends behind the kn-th k: units past it fetch the first k's instead
+  // (their fragments are zeroed).
+  __device__ __forceinline__ void load_tail(const float *base, unsigned lds, int ld, int lane, int kn) const {
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      const int k = unit_k(lane + i * 64);
+      const unsigned back = (KC ? (unsigned)k : (unsigned)(k * ld)) * 4u;
+      load_unit(base, k < kn ? goff[i] : (goff[i] >= back ? goff[i] - back : 0u), lds + 1024u * i);
+    }
+  }
+  static __device__ __forceinline__ void read_frag(const float *piece, int grp, int l32, int lhi, float (&out)[4]) {
+    if constexpr (KC) {
+      const float4 t = *reinterpret_cast<const float4 *>(piece + (l32 * U + ((2 * grp + lhi) ^ swizzle(l32))) * 4);
+      out[0] = t.x, out[1] = t.y, out[2] = t.z, out[3] = t.w;
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) out[q] = piece[(8 * grp + swap02(q) + lhi) * 32 + l32];
+    }
+  }
+};
+
+// At most N of this wavefront's loads still in flight; its LDS reads have returned.
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(N) : "memory");
+}
+
+template <int BM, int BN, int WM, int WN, int WK, int BK, bool TA, bool TX>
+constexpr int smem2_floats() {
+  return smem2_floats<BM, BN, WM, WN, WK, BK, TA, TX, false>();
 }
 
 // The rare paths of the K loop (a new K segment, a short last slab) are a few dozen selects each.
@@ -593,6 +708,250 @@ __device__ __forceinline__ int xcd_logical_id() {
   return xcd * per + (xcd < rem ? xcd : rem) + within;
 }
 
+// The streamed form of gemm_body.
+template <int BM, int BN, int WM, int WN, int WK, int BK, bool TA, bool TX, bool CELL>
+__device__ __forceinline__ void stream_body(const GemmArgs &g, const int m0, const int n0, const int split,
+                                            const int splits) {
+  constexpr int NT = 64 * WM * WN * WK;
+  constexpr int CK = BK / WK, NG = CK / 8;
+  constexpr int NB = kRingStages;
+  static_assert(NB == 4, "the waits of the K loop");
+  using PA = Piece<CK, TA>;
+  using PX = Piece<CK, !TX>;
+  constexpr int kStage = PA::kFloats + PX::kFloats;  // floats of one wavefront's stage
+  constexpr int kLoads = PA::kLoads + PX::kLoads;
+  constexpr int GQ = BM / 4;
+
+  const int tid = threadIdx.x, lane = tid % lh::kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / lh::kWave);
+  const int wk = wave / (WM * WN), wmn = wave % (WM * WN);
+  const int wm = wmn % WM, wn = wmn / WM;
+  const int l32 = lane % 32, lhi = lane / 32;
+  float *const ring = smem + wave * NB * kStage;
+  const unsigned ring_lds = (unsigned)(size_t)(__attribute__((address_space(3))) float *)ring;
+
+  const int M = g.M, N = g.N;
+  const int slabs0 = (g.K[0] + BK - 1) / BK;
+  const int slabs1 = g.nseg > 1 ? (g.K[1] + BK - 1) / BK : 0;
+  const int slabs2 = g.nseg > 2 ? (g.K[2] + BK - 1) / BK : 0;
+  const int first = split * g.slabs_per_split;
+  const int total = min(g.slabs_per_split, slabs0 + slabs1 + slabs2 - first);
+  int lseg = 0, k0 = first;  // segment and (below) k of the next slab to request
+  if (k0 >= slabs0) {
+    k0 -= slabs0;
+    lseg = 1;
+    if (k0 >= slabs1) {
+      k0 -= slabs1;
+      lseg = 2;
+    }
+  }
+  k0 *= BK;
+  int cseg = lseg, ck = k0;  // the same of the slab to multiply
+  // (an array indexed by a variable would move the arguments to memory)
+  auto pick = [](int seg, auto v0, auto v1, auto v2) __attribute__((always_inline)) {
+    return seg == 0 ? v0 : (seg == 1 ? v1 : v2);
+  };
+#define LH_SEG(FIELD, SEG) pick(SEG, g.FIELD[0], g.FIELD[1], g.FIELD[2])
+
+  PA pa;
+  PX px;
+  bool new_seg = true;
+  const float *a = nullptr, *x = nullptr;  // this wavefront's first k of the next slab
+  int step_a = 0, step_x = 0, lda = 0, ldx = 0, Ks = 0;
+  unsigned put = ring_lds;  // stage the next slab goes to
+  auto request = [&]() __attribute__((always_inline)) {
+    if (new_seg) {
+      LH_KEEP_BRANCH();
+      Ks = LH_SEG(K, lseg);
+      if (lda != LH_SEG(lda, lseg) || ldx != LH_SEG(ldx, lseg)) {
+        LH_KEEP_BRANCH();
+        lda = LH_SEG(lda, lseg), ldx = LH_SEG(ldx, lseg);
+        if constexpr (CELL) pa.template set_ld_gates<GQ>(lda, lane, 32 * wm, g.cell_H, g.cell_H - m0);
+        else pa.set_ld(lda, lane, 32 * wm, M - m0);
+        px.set_ld(ldx, lane, 32 * wn, N - n0);
+      }
+      const int k = k0 + wk * CK;
+      a = LH_SEG(A, lseg) + (TA ? (size_t)m0 * lda + k : (size_t)k * lda + m0);
+      x = LH_SEG(X, lseg) + (!TX ? (size_t)n0 * ldx + k : (size_t)k * ldx + n0);
+      step_a = TA ? BK : BK * lda;
+      step_x = !TX ? BK : BK * ldx;
+    }
+    const int kn = Ks - k0 - wk * CK;
+    if (kn < CK) {
+      LH_KEEP_BRANCH();
+      if (kn <= 0) {  // nothing left for this wavefront: any valid address, nothing is multiplied
+        a = LH_SEG(A, lseg) + (TA ? (size_t)m0 * lda : (size_t)m0);
+        x = LH_SEG(X, lseg) + (!TX ? (size_t)n0 * ldx : (size_t)n0);
+      }
+      pa.load_tail(a, put, lda, lane, kn);
+      px.load_tail(x, put + PA::kFloats * 4u, ldx, lane, kn);
+    } else {
+      pa.load(a, put);
+      px.load(x, put + PA::kFloats * 4u);
+    }
+    put = put + kStage * 4u == ring_lds + NB * kStage * 4u ? ring_lds : put + kStage * 4u;
+    a += step_a;
+    x += step_x;
+    k0 += BK;
+    new_seg = k0 >= Ks;
+    if (new_seg) {
+      ++lseg;
+      k0 = 0;
+    }
+  };
+
+  floatx16 acc;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) acc[j] = 0.f;
+  int issued = min(total, NB - 1);
+  for (int i = 0; i < issued; ++i) request();
+
+  // What the cell reads from memory, requested behind the first slabs: the epilogue would wait a
+  // memory latency for it, two with addend_col.
+  float ep_add[4] = {0.f, 0.f, 0.f, 0.f}, ep_bias[4] = {0.f, 0.f, 0.f, 0.f}, ep_c = 0.f;
+  int ep_mask = 0;
+  bool ep_ok = false;
+  if constexpr (CELL) {
+    static_assert(GQ * BN <= NT, "one cell per thread");
+    const int r = m0 + tid % GQ, n = n0 + tid / GQ;
+    ep_ok = tid < GQ * BN && r < g.cell_H && n < N;
+    if (ep_ok && !g.pre_out) {
+      int col = n;
+      if (g.addend_col) col = min(max(g.addend_col[n], 0), g.addend_ncols - 1);
+      const float *ad = g.C + (size_t)col * g.ldc + r;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        if (g.beta != 0.f) ep_add[q] = ad[(size_t)q * g.cell_H];
+        ep_bias[q] = g.bias[q * g.cell_H + r];
+      }
+      ep_c = g.c_prev[(size_t)n * g.cell_H + r];
+      ep_mask = g.colmask[n];
+    }
+  }
+
+  const float *get = ring;
+  int cK = LH_SEG(K, cseg);
+  for (int s = 0; s < total; ++s) {
+    const int behind = issued - 1 - s;  // slabs requested after this one
+    if (behind >= 2) wait_loads<kLoads * 2>();
+    else if (behind == 1) wait_loads<kLoads>();
+    else wait_loads<0>();
+    float fa[NG][4], fx[NG][4];
+#pragma unroll
+    for (int grp = 0; grp < NG; ++grp) {
+      PA::read_frag(get, grp, l32, lhi, fa[grp]);
+      PX::read_frag(get + PA::kFloats, grp, l32, lhi, fx[grp]);
+    }
+    // the stage this goes to was read in the last round, and those reads have returned
+    if (issued < total) {
+      request();
+      ++issued;
+    }
+    const int kn = cK - ck - wk * CK;
+    if (kn < CK) {
+      LH_KEEP_BRANCH();
+#pragma unroll
+      for (int grp = 0; grp < NG; ++grp)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const bool in = 8 * grp + 4 * lhi + q < kn;
+          fa[grp][q] = in ? fa[grp][q] : 0.f;
+          fx[grp][q] = in ? fx[grp][q] : 0.f;
+        }
+    }
+#pragma unroll
+    for (int grp = 0; grp < NG; ++grp)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fx[grp][q], fa[grp][q], acc, 0, 0, 0);
+    get = get + kStage == ring + NB * kStage ? ring : get + kStage;
+    ck += BK;
+    if (ck >= cK) {
+      LH_KEEP_BRANCH();
+      ck = 0;
+      ++cseg;
+      if (s + 1 < total) cK = LH_SEG(K, cseg);
+    }
+  }
+#undef LH_SEG
+
+  // Every wavefront puts its partial block into LDS as S[wk][n][m] once all of them have left
+  // their rings, then every thread sums the WK values of its own elements, in the order of wk,
+  // and takes them through the epilogue.
+  constexpr int LDS_N = spread_ld<BM>();
+  constexpr int kPlane = LDS_N * BN;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 16; ++j)
+    smem[wk * kPlane + (wn * 32 + lhi * 4 + (j / 4) * 8 + (j % 4)) * LDS_N + wm * 32 + l32] = acc[j];
+  __syncthreads();
+  if constexpr (CELL) {
+    if (!ep_ok) return;
+    const int H = g.cell_H;
+    const int rl = tid % GQ, nl = tid / GQ;
+    const int r = m0 + rl, n = n0 + nl;
+    float pre[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float *src = smem + nl * LDS_N + q * GQ + rl;
+      pre[q] = src[0];
+#pragma unroll
+      for (int p = 1; p < WK; ++p) pre[q] += src[p * kPlane];
+    }
+    if (g.pre_out) {
+      float *o = g.pre_out + (size_t)n * g.pre_ld + r;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) o[(size_t)q * H] = pre[q];
+      return;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) pre[q] = (g.beta != 0.f ? pre[q] + ep_add[q] : pre[q]) + ep_bias[q];
+    float c, h;
+    const float mask = (float)(ep_mask & 1);
+    if (g.sigmoid_f64 && !(ep_mask & LH_MASK_F32_GATES))
+      lh::lstm_cell_point<true>(pre[0], pre[1], pre[2], pre[3], ep_c, mask, g.cell_clip, c, h);
+    else
+      lh::lstm_cell_point<false>(pre[0], pre[1], pre[2], pre[3], ep_c, mask, g.cell_clip, c, h);
+    const size_t o = (size_t)n * H + r;
+    g.c_out[o] = c;
+    g.h_out[o] = h;
+    if (g.gates_out) {
+      float *go = g.gates_out + (size_t)n * 4 * H + r;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) go[(size_t)q * H] = pre[q];  // the cell left i, f, g, o there
+    }
+    if (g.h_drop) g.h_drop[o] = ((float)(g.drop_mask[o] < g.keep) * (1.0f / g.keep)) * h;
+  } else {
+    // a split product stores the bare partial sums in its plane of the workspace
+    const bool partial = splits > 1;
+    const float alpha = partial ? 1.f : g.alpha, beta = partial ? 0.f : g.beta;
+    const int *const colmask = partial ? nullptr : g.colmask;
+    const float *const bias = partial ? nullptr : g.bias;
+    const int act_rows = partial || g.act != LH_ACT_TANH ? 0 : g.act_rows;
+    float *const Cb = partial ? g.ws_part + (size_t)split * g.ws_ld * N : g.C;
+    const int ldc = partial ? g.ws_ld : g.ldc;
+    static_assert(BM * BN % NT == 0, "whole elements per thread");
+#pragma unroll
+    for (int i = 0; i < BM * BN / NT; ++i) {
+      const int idx = tid + i * NT;
+      const int ml = idx % BM, nl = idx / BM;
+      const int m = m0 + ml, n = n0 + nl;
+      if (m >= M || n >= N) continue;
+      const float *src = smem + nl * LDS_N + ml;
+      float sum = src[0];
+#pragma unroll
+      for (int p = 1; p < WK; ++p) sum += src[p * kPlane];
+      float *cp = Cb + (size_t)n * ldc + m;
+      float v = alpha * sum;
+      if (beta != 0.f) v += beta * *cp;
+      if (bias) v += bias[m];
+      if (m < act_rows) v = tanhf(v);
+      if (colmask) v *= (float)colmask[n];
+      *cp = v;
+    }
+  }
+}
+
 template <int BM, int BN, int WM, int WN, int WK, int BK, bool TA, bool TX, bool CELL, bool RAGGED>
 __device__ __forceinline__ void gemm_body(const GemmArgs &g, const int logical) {
   constexpr int NT = 64 * WM * WN * WK;
@@ -602,6 +961,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &g, const int logical) 
   constexpr int KPW = BK / WK;  // k values one wavefront group consumes per slab
   static_assert(KPW % 8 == 0, "a fragment group covers 8 k (4 per lane half)");
   constexpr int NG = KPW / 8;
+  constexpr bool kStream = !RAGGED && streamed<BM, BN, WM, WN, WK, BK>();
   using SA = Stage<BM, BK, NT, TA, RAGGED>;
   using SX = Stage<BN, BK, NT, !TX, RAGGED>;
   constexpr int kAF = SA::kFloats, kSlab = SA::kFloats + SX::kFloats;
@@ -637,6 +997,11 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &g, const int logical) 
     for (int b = 0; b < FM; ++b)
 #pragma unroll
       for (int j = 0; j < 16; ++j) acc[a][b][j] = 0.f;
+
+  if constexpr (kStream) {
+    stream_body<BM, BN, WM, WN, WK, BK, TA, TX, CELL>(g, m0, n0, split, splits);
+    return;
+  }
 
   SA sa;
   SX sx;
@@ -1088,13 +1453,13 @@ struct Config {
   X(10, 32, 96, 1, 3, 2, 32)   /* M around 1000 */                             \
   X(11, 32, 96, 1, 3, 2, 128)                                                  \
   X(12, 32, 64, 1, 2, 4, 32)   /* skinny */                                    \
-  X(13, 32, 64, 1, 2, 4, 128)                                                  \
+  X(13, 32, 64, 1, 2, 4, 64)                                                   \
   X(14, 32, 32, 1, 1, 8, 64)   /* very skinny */                               \
   X(15, 32, 32, 1, 1, 8, 128)                                                  \
   X(16, 128, 32, 4, 1, 1, 16)                                                  \
   X(17, 128, 32, 4, 1, 1, 64)                                                  \
   X(18, 64, 32, 2, 1, 4, 32)                                                   \
-  X(19, 64, 32, 2, 1, 4, 128)                                                  \
+  X(19, 64, 32, 2, 1, 4, 64)                                                   \
   X(20, 128, 128, 2, 2, 1, 64) /* deep slabs: one workgroup per CU hides its own latency */ \
   X(21, 128, 64, 2, 2, 1, 64)                                                  \
   X(22, 128, 128, 2, 2, 2, 64) /* ... or two wavefronts per SIMD inside the workgroup */ \
@@ -1182,7 +1547,7 @@ int launch_cfg(const GemmArgs &g0, bool ta, bool tx, Form form, hipStream_t st) 
       } else {
 #define LH_GEMM_LAUNCH(TA, TX)                                                              \
   rc = launch_kernel((GemmKernel)gemm_kernel<BM, BN, WM, WN, WK, BK, TA, TX, true>,         \
-                     smem2_floats<BM, BN, WM, WN, WK, BK, TA, TX>() * 4, grid, block, st, g)
+                     smem2_floats<BM, BN, WM, WN, WK, BK, TA, TX, true>() * 4, grid, block, st, g)
         if (!ta && !tx) LH_GEMM_LAUNCH(false, false);
         else if (ta) LH_GEMM_LAUNCH(true, false);
         else LH_GEMM_LAUNCH(false, true);
@@ -1415,7 +1780,9 @@ void pick_config(int M, int N, const int *K, int nseg, bool ta, bool tx, Form fo
       if (max_planes > 0 && want > max_planes) want = max_planes;
       if (want > 1 && fit_splits(M, N, want, workspace_bytes) < want) break;
       int S;
-      const float us = predict_us(table[c], kConfigs[c], M, N, K, nseg, want, max_planes > 0, &S);
+      float us = predict_us(table[c], kConfigs[c], M, N, K, nseg, want, max_planes > 0, &S);
+      // an override asks for this many shares: too few slabs for them only where no other choice has enough
+      if (g_splits_override > 0 && S < want) us += 1.0e6f;
       if (us < best) {
         best = us;
         *config = c;

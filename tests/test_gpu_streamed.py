@@ -1,0 +1,64 @@
+"""Products on the streamed tiles (eight wavefronts, a 32x32 block each, operands loaded straight into LDS)
+against float64: the edges of tiles and slabs, segments that end inside a slab or within a wavefront's share of
+one, segments of unlike leading dimensions, K split over workgroups."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+CONFIGS = [13, 14, 15, 19]
+
+
+@pytest.fixture()
+def lh():
+    from linmt_amd import lib
+    lib.load()
+    yield lib
+    lib.load().lh_gemm_set_config_override(-1)
+    lib.load().lh_gemm_set_splits_override(0)
+
+
+def operand(torch, rows, cols, pad, seed):
+    """rows x cols column-major with leading dimension rows + pad; what lies between is NaN: never to be used."""
+    g = torch.Generator("cuda").manual_seed(seed)
+    full = torch.full((cols, rows + pad), float("nan"), device="cuda")
+    full[:, :rows] = torch.randn(cols, rows, device="cuda", generator=g)
+    return full, full[:, :rows].T.double()
+
+
+@pytest.mark.parametrize("config", CONFIGS)
+@pytest.mark.parametrize("tA,tX", [(False, False), (True, False), (False, True)], ids=["NN", "TN", "NT"])
+@pytest.mark.parametrize("M,N,Ks,splits", [
+    (4, 4, (4,), 1),              # one unit of everything
+    (32, 32, (8,), 1),            # less than a wavefront's share of a slab
+    (36, 20, (64,), 1),           # one row unit past a tile, one slab of the shallow tiles
+    (64, 64, (132, 20), 1),       # a segment that ends in the first wavefront's share, then a short one
+    (100, 68, (16, 512, 60), 1),  # four slabs in flight and the ring round more than once
+    (1000, 64, (1000, 1000), 1),
+    (200, 36, (1000,), 4),        # K split over workgroups
+    (200, 36, (260, 20), 2),
+])
+def test_streamed_product_matches_float64(lh, config, tA, tX, M, N, Ks, splits):
+    import torch
+    segs, want, bound = [], 0, 0
+    for i, K in enumerate(Ks):
+        pad = 4 * (i + 1)
+        a, a64 = operand(torch, K if tA else M, M if tA else K, pad, 10 * i)
+        x, x64 = operand(torch, N if tX else K, K if tX else N, pad + 4, 10 * i + 1)
+        a64, x64 = (a64.T if tA else a64), (x64.T if tX else x64)
+        segs.append((a, a.shape[1], x, x.shape[1], K))
+        want = want + a64 @ x64
+        bound = bound + a64.abs() @ x64.abs()
+    bias = torch.randn(M, device="cuda")
+    old = torch.randn(N, M, device="cuda")
+    out = old.clone()
+    ws = torch.empty(16 * M * N, device="cuda")
+    lib = lh.load()
+    lib.lh_gemm_set_config_override(config)
+    lib.lh_gemm_set_splits_override(splits)
+    lh.gemm(M, N, segs, out, M, transA=tA, transX=tX, beta=1.0, bias=bias, workspace=ws)
+    torch.cuda.synchronize()
+    want = want + old.T.double() + bias.double()[:, None]
+    # K products and their sum in fp32, in any order, plus the two addends: (K + 3) roundings of the sum of
+    # magnitudes at most
+    bound = (sum(Ks) + 3) * 2.0 ** -24 * (bound + old.T.double().abs() + bias.double().abs()[:, None])
+    assert bool(((out.T.double() - want).abs() <= bound).all())

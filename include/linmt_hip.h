@@ -186,6 +186,33 @@ int lh_gate_gemm_lstm_cell_train_f32(int H, int B, const lh_gemm_seg *segs, int 
                                      float cell_clip, float *gates, float *c, float *h,
                                      const float *next_drop_mask, float keep, float *h_drop,
                                      size_t workspace_bytes, lh_stream_t stream);
+/* The same product and cell on gate matrices laid out for it (no counterpart in the reference).  A tile of
+ * a stacked 4H x K matrix holds a few rows of each gate, which are short runs of memory (8 rows: 32 bytes);
+ * lh_gate_pack_f32 writes a copy in which they are one run: for every 8 cells (the last block padded with
+ * zeros) K rows of 32 floats, float 4r + q of row k = gate q of cell r.  A caller packs once per change of
+ * the weights, and uses the copy where lh_gate_gemm_lstm_cell_packed_plan says that it is the faster way
+ * (*faster; segs, workspace_bytes and has_addend as for lh_gate_gemm_lstm_cell_plan, with the matrices as
+ * stored; few columns, H and K multiples of 4, 16-byte aligned operands).
+ * lh_gate_gemm_lstm_cell_packed_f32: A of a segment is a packed matrix (16-byte aligned; lda is not read);
+ * everything else as for lh_gate_gemm_lstm_cell_f32 and, with gates / h_drop (both optional),
+ * lh_gate_gemm_lstm_cell_train_f32.  It does not look at the plan's advice: any B runs. */
+#define LH_GATE_PACK_MAX 4
+typedef struct lh_gate_pack_source {
+  const float *src; /* 4H x K, leading dimension ld */
+  int ld;
+  int K;
+  float *dst; /* lh_gate_pack_floats(H, K) floats */
+} lh_gate_pack_source;
+size_t lh_gate_pack_floats(int H, int K);
+int lh_gate_pack_f32(int H, const lh_gate_pack_source *src, int n, lh_stream_t stream);
+int lh_gate_gemm_lstm_cell_packed_plan(int H, int B, const lh_gemm_seg *segs, int nseg, int has_addend,
+                                       size_t workspace_bytes, int *faster, char *name, int name_cap);
+int lh_gate_gemm_lstm_cell_packed_f32(int H, int B, const lh_gemm_seg *segs, int nseg, const float *addend,
+                                      int ld_addend, const int *addend_col, int addend_ncols,
+                                      const float *bias4h, const float *c_prev, const int *mask01,
+                                      int sigmoid_f64, float cell_clip, float *gates, float *c, float *h,
+                                      const float *next_drop_mask, float keep, float *h_drop,
+                                      lh_stream_t stream);
 /* Several stacked gate products of one step in ONE launch (no counterpart in the reference, which
  * issues every layer's 8-12 SGEMMs one after the other, src/node_input_to_hidden.h:297-556,
  * src/node_hidden_to_hidden.h:248-386).  While decoding, what a step needs from the previous one is

@@ -709,7 +709,10 @@ __device__ __forceinline__ int xcd_logical_id() {
 }
 
 // The streamed form of gemm_body.
-template <int BM, int BN, int WM, int WN, int WK, int BK, bool TA, bool TX, bool CELL>
+// PACKED: A is a gate matrix as lh_gate_pack_f32 lays it out: for every 8 cells K rows of 32 floats, row k
+// holding the four gates of each of the cells at that k.
+constexpr int kPackCells = 8, kPackRows = 4 * kPackCells;
+template <int BM, int BN, int WM, int WN, int WK, int BK, bool TA, bool TX, bool CELL, bool PACKED>
 __device__ __forceinline__ void stream_body(const GemmArgs &g, const int m0, const int n0, const int split,
                                             const int splits) {
   constexpr int NT = 64 * WM * WN * WK;
@@ -757,6 +760,8 @@ __device__ __forceinline__ void stream_body(const GemmArgs &g, const int m0, con
   PX px;
   bool new_seg = true;
   const float *a = nullptr, *x = nullptr;  // this wavefront's first k of the next slab
+  // PACKED: this wavefront's group of cells (a tile may reach past the last one)
+  const int cells = PACKED ? min(m0 / kPackCells + wm, (g.cell_H - 1) / kPackCells) : 0;
   int step_a = 0, step_x = 0, lda = 0, ldx = 0, Ks = 0;
   unsigned put = ring_lds;  // stage the next slab goes to
   auto request = [&]() __attribute__((always_inline)) {
@@ -766,12 +771,14 @@ __device__ __forceinline__ void stream_body(const GemmArgs &g, const int m0, con
       if (lda != LH_SEG(lda, lseg) || ldx != LH_SEG(ldx, lseg)) {
         LH_KEEP_BRANCH();
         lda = LH_SEG(lda, lseg), ldx = LH_SEG(ldx, lseg);
-        if constexpr (CELL) pa.template set_ld_gates<GQ>(lda, lane, 32 * wm, g.cell_H, g.cell_H - m0);
+        if constexpr (PACKED) pa.set_ld(lda, lane, 0, kPackRows);
+        else if constexpr (CELL) pa.template set_ld_gates<GQ>(lda, lane, 32 * wm, g.cell_H, g.cell_H - m0);
         else pa.set_ld(lda, lane, 32 * wm, M - m0);
         px.set_ld(ldx, lane, 32 * wn, N - n0);
       }
       const int k = k0 + wk * CK;
-      a = LH_SEG(A, lseg) + (TA ? (size_t)m0 * lda + k : (size_t)k * lda + m0);
+      if constexpr (PACKED) a = LH_SEG(A, lseg) + ((size_t)cells * Ks + k) * kPackRows;
+      else a = LH_SEG(A, lseg) + (TA ? (size_t)m0 * lda + k : (size_t)k * lda + m0);
       x = LH_SEG(X, lseg) + (!TX ? (size_t)n0 * ldx + k : (size_t)k * ldx + n0);
       step_a = TA ? BK : BK * lda;
       step_x = !TX ? BK : BK * ldx;
@@ -780,7 +787,7 @@ __device__ __forceinline__ void stream_body(const GemmArgs &g, const int m0, con
     if (kn < CK) {
       LH_KEEP_BRANCH();
       if (kn <= 0) {  // nothing left for this wavefront: any valid address, nothing is multiplied
-        a = LH_SEG(A, lseg) + (TA ? (size_t)m0 * lda : (size_t)m0);
+        a = LH_SEG(A, lseg) + (PACKED ? (size_t)cells * Ks * kPackRows : (TA ? (size_t)m0 * lda : (size_t)m0));
         x = LH_SEG(X, lseg) + (!TX ? (size_t)n0 * ldx : (size_t)n0);
       }
       pa.load_tail(a, put, lda, lane, kn);
@@ -893,7 +900,8 @@ __device__ __forceinline__ void stream_body(const GemmArgs &g, const int m0, con
     float pre[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const float *src = smem + nl * LDS_N + q * GQ + rl;
+      const int ml = PACKED ? (rl / kPackCells) * kPackRows + (rl % kPackCells) * 4 + q : q * GQ + rl;
+      const float *src = smem + nl * LDS_N + ml;
       pre[q] = src[0];
 #pragma unroll
       for (int p = 1; p < WK; ++p) pre[q] += src[p * kPlane];
@@ -999,7 +1007,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &g, const int logical) 
       for (int j = 0; j < 16; ++j) acc[a][b][j] = 0.f;
 
   if constexpr (kStream) {
-    stream_body<BM, BN, WM, WN, WK, BK, TA, TX, CELL>(g, m0, n0, split, splits);
+    stream_body<BM, BN, WM, WN, WK, BK, TA, TX, CELL, false>(g, m0, n0, split, splits);
     return;
   }
 
@@ -1343,6 +1351,47 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gate_gemm_cell_kernel(const
   gemm_body<BM, BN, WM, WN, WK, BK, false, false, true, false>(g, xcd_logical_id());
 }
 
+// The same on packed gate matrices (lda = 32).  A tile of 32 rows takes 8 rows of each gate: 32-byte runs of the
+// stored matrix, of which a CU fetches whole 64-byte halves of lines: 1.5 times the bytes of the whole product,
+// and 50 GB/s per CU (13 TB/s in all) is what the L2s deliver.  Packed, they are one 128-byte line.
+// 1000 hidden units, K = 1000 / 2000: 64 columns 12.7 / 20.6 us streamed from the stored matrix, 10.3 / 16.1 packed
+// (staged, the way before: 12.7 / 20.3); 12 columns 11.5 / 17.6 and 9.5 / 14.7; 128 columns 16.5 / 27.3 (64-byte runs)
+// and 15.6 / 25.4.
+template <int BM, int BN, int WM, int WN, int WK, int BK>
+__global__ __launch_bounds__(64 * WM * WN * WK) void gate_gemm_packed_kernel(const GemmArgs g) {
+  const int logical = xcd_logical_id();
+  stream_body<BM, BN, WM, WN, WK, BK, false, false, true, true>(g, (logical / g.tiles_n) * (BM / 4),
+                                                                (logical % g.tiles_n) * BN, 0, 1);
+}
+
+// 4H x K stacked gate matrix (gates H rows apart) -> ceil(H / 8) blocks of K x 32 (see stream_body).
+// Through LDS, so that both sides are whole lines: 32 rows of a gate in, 32 floats of a block out.  Two
+// matrices of 4000 x 1000 take 20.5 us (3.1 TB/s), once per change of the weights.
+struct PackArgs {
+  const float *src[LH_GATE_PACK_MAX];
+  float *dst[LH_GATE_PACK_MAX];
+  int ld[LH_GATE_PACK_MAX], K[LH_GATE_PACK_MAX];
+  int H;
+};
+constexpr int kPackK = 8;  // k per workgroup
+__global__ __launch_bounds__(256) void gate_pack_kernel(const PackArgs p) {
+  // a workgroup: 32 cells (four blocks) of kPackK k
+  __shared__ float t[kPackK][4][33];
+  const int mat = blockIdx.z, H = p.H, K = p.K[mat];
+  const int c0 = blockIdx.x * 32, k0 = blockIdx.y * kPackK;
+  if (k0 >= K) return;  // the grid covers the deepest matrix
+  for (int i = threadIdx.x; i < kPackK * 4 * 32; i += 256) {
+    const int c = i % 32, q = i / 32 % 4, k = i / 128;
+    t[k][q][c] = c0 + c < H && k0 + k < K ? p.src[mat][(size_t)(k0 + k) * p.ld[mat] + (size_t)q * H + c0 + c] : 0.f;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < kPackK * 4 * 32; i += 256) {
+    const int r = i % kPackRows, k = i / kPackRows % kPackK, b = i / (kPackRows * kPackK);
+    if (c0 + b * kPackCells < H && k0 + k < K)
+      p.dst[mat][((size_t)(c0 / kPackCells + b) * K + k0 + k) * kPackRows + r] = t[k][r % 4][b * kPackCells + r / 4];
+  }
+}
+
 // Several stacked gate products of one decoding step in ONE launch: everything that is known when
 // the step starts -- each layer's recurrent product W_h h_{t-1}, and the first layer's whole
 // pre-activation with its cell -- so that the GPU sees a few thousand tiles at once instead of a
@@ -1611,6 +1660,44 @@ int launch_cell_cfg(const GemmArgs &g0, hipStream_t st) {
   }
 }
 
+// Configurations of the packed gate product: the streamed ones.
+bool packed_config(int c) {
+  switch (c) {
+#define LH_CFG_CASE(I, BM, BN, WM, WN, WK, BK) \
+  case I: return streamed<BM, BN, WM, WN, WK, BK>();
+    LH_GEMM_CONFIGS(LH_CFG_CASE)
+#undef LH_CFG_CASE
+    default: return false;
+  }
+}
+
+template <int BM, int BN, int WM, int WN, int WK, int BK>
+int launch_packed_cfg(const GemmArgs &g0, hipStream_t st) {
+  if constexpr (streamed<BM, BN, WM, WN, WK, BK>()) {
+    GemmArgs g = g0;
+    g.tiles_m = (g.cell_H + BM / 4 - 1) / (BM / 4);
+    g.tiles_n = (g.N + BN - 1) / BN;
+    g.splits = 1;
+    g.slabs_per_split = 0;
+    for (int s = 0; s < g.nseg; ++s) g.slabs_per_split += (g.K[s] + BK - 1) / BK;
+    return launch_kernel(gate_gemm_packed_kernel<BM, BN, WM, WN, WK, BK>,
+                         smem2_floats<BM, BN, WM, WN, WK, BK, false, false>() * 4, dim3(g.tiles_m * g.tiles_n),
+                         dim3(64 * WM * WN * WK), st, g);
+  } else {
+    return lh::fail_arg("lh_gate_gemm_lstm_cell_packed_f32: internal error, configuration %dx%d", BM, BN);
+  }
+}
+
+int launch_packed_index(int c, const GemmArgs &g, hipStream_t st) {
+  switch (c) {
+#define LH_CFG_CASE(I, BM, BN, WM, WN, WK, BK) \
+  case I: return launch_packed_cfg<BM, BN, WM, WN, WK, BK>(g, st);
+    LH_GEMM_CONFIGS(LH_CFG_CASE)
+#undef LH_CFG_CASE
+    default: return lh::fail_arg("lh_gate_gemm_lstm_cell_packed_f32: configuration %d does not exist", c);
+  }
+}
+
 int launch_cell_index(int c, const GemmArgs &g, hipStream_t st) {
   switch (c) {
 #define LH_CFG_CASE(I, BM, BN, WM, WN, WK, BK) \
@@ -1794,6 +1881,18 @@ void pick_config(int M, int N, const int *K, int nseg, bool ta, bool tx, Form fo
   if (best > 2.9e38f) *config = -1;  // the override names a configuration that cannot run this
   if (us_out) *us_out = best;
   e = Memo{M, N, {Kk[0], Kk[1], Kk[2]}, flags, *config, *splits, workspace_bytes, best};
+}
+
+// The packed gate product's configuration and predicted time (fifth table).
+void pick_packed(int H, int B, const int *K, int nseg, int *config, float *us) {
+  *config = -1;
+  *us = 3.0e38f;
+  for (int c = 0; c < kNumConfigs; ++c) {
+    if ((g_config_override >= 0 && c != g_config_override) || !packed_config(c)) continue;
+    int S;
+    const float t = predict_us(kTuning[4][c], kConfigs[c], 4 * H, B, K, nseg, 1, false, &S);
+    if (t < *us) *us = t, *config = c;
+  }
 }
 
 struct Prepared {
@@ -2055,6 +2154,110 @@ int gate_gemm_lstm_cell(int H, int B, const lh_gemm_seg *segs, int nseg, const f
   return launch_cell_index(p.config, g, lh::as_stream(stream));
 }
 }  // namespace
+
+// ---- gate products on packed gate matrices -----------------------------------------------------
+extern "C" size_t lh_gate_pack_floats(int H, int K) {
+  return H > 0 && K > 0 ? (size_t)((H + kPackCells - 1) / kPackCells) * kPackRows * (size_t)K : 0;
+}
+
+extern "C" int lh_gate_pack_f32(int H, const lh_gate_pack_source *src, int n, lh_stream_t stream) {
+  if (H <= 0 || !src || n < 1 || n > LH_GATE_PACK_MAX)
+    return lh::fail_arg("lh_gate_pack_f32: H=%d sources=%d (at most %d)", H, n, LH_GATE_PACK_MAX);
+  PackArgs p{};
+  p.H = H;
+  int deepest = 0;
+  for (int i = 0; i < n; ++i) {
+    if (!src[i].src || !src[i].dst || src[i].K <= 0 || src[i].ld < 4 * H)
+      return lh::fail_arg("lh_gate_pack_f32: source %d: src=%p dst=%p K=%d ld=%d (at least 4H)", i,
+                          (const void *)src[i].src, (void *)src[i].dst, src[i].K, src[i].ld);
+    p.src[i] = src[i].src, p.dst[i] = src[i].dst, p.ld[i] = src[i].ld, p.K[i] = src[i].K;
+    deepest = src[i].K > deepest ? src[i].K : deepest;
+  }
+  const unsigned gy = (unsigned)((deepest + kPackK - 1) / kPackK);
+  if (gy > 65535) return lh::fail_arg("lh_gate_pack_f32: K=%d is too deep", deepest);
+  hipLaunchKernelGGL(gate_pack_kernel, dim3((unsigned)((H + 31) / 32), gy, (unsigned)n), dim3(256), 0,
+                     lh::as_stream(stream), p);
+  return lh::check_launch("lh_gate_pack_f32");
+}
+
+extern "C" int lh_gate_gemm_lstm_cell_packed_plan(int H, int B, const lh_gemm_seg *segs, int nseg,
+                                                  int has_addend, size_t workspace_bytes, int *faster,
+                                                  char *name, int name_cap) {
+  if (!faster) return lh::fail_arg("lh_gate_gemm_lstm_cell_packed_plan: faster is NULL");
+  *faster = 0;
+  if (name && name_cap > 0) name[0] = 0;
+  Prepared p;
+  bool f = false;
+  const int rc = plan_cell(H, B, segs, nseg, has_addend != 0, nullptr, 0, workspace_bytes, &p, &f);
+  if (rc != LH_OK || p.form != kAligned || H % 4 != 0) return rc;
+  // Against what runs without packing: the fused launch, or the product and the cell kernel behind it.
+  int c, S, c0 = p.config;
+  float us, us0;
+  pick_packed(H, B, p.g.K, nseg, &c, &us);
+  if (c < 0) return LH_OK;
+  pick_config(4 * H, B, p.g.K, nseg, false, false, kAligned, workspace_bytes, has_addend ? 2 : 3, &c0, &S, f, &us0);
+  if (!f) us0 += kCellFixedUs + 28.f * (float)H * (float)B / kReduceBytesPerUs;
+  if (us > us0) return LH_OK;
+  *faster = 1;
+  if (name && name_cap > 0) {
+    const Config &k = kConfigs[c];
+    snprintf(name, name_cap, "gate_gemm_packed_kernel<%d, %d, %d, %d, %d, %d>", k.bm, k.bn, k.wm, k.wn, k.wk, k.bk);
+  }
+  return LH_OK;
+}
+
+extern "C" int lh_gate_gemm_lstm_cell_packed_f32(int H, int B, const lh_gemm_seg *segs, int nseg,
+                                                 const float *addend, int ld_addend, const int *addend_col,
+                                                 int addend_ncols, const float *bias4h, const float *c_prev,
+                                                 const int *mask01, int sigmoid_f64, float cell_clip,
+                                                 float *gates, float *c, float *h, const float *next_drop_mask,
+                                                 float keep, float *h_drop, lh_stream_t stream) {
+  const char *const what = "lh_gate_gemm_lstm_cell_packed_f32";
+  if (H <= 0 || B <= 0 || !segs || nseg < 1 || nseg > LH_GEMM_MAX_SEGS)
+    return lh::fail_arg("%s: H=%d B=%d segments=%d", what, H, B, nseg);
+  if (!bias4h || !c_prev || !mask01 || !c || !h) return lh::fail_arg("%s: a required pointer is NULL", what);
+  if (addend && ld_addend < 4 * H) return lh::fail_arg("%s: ld_addend=%d < 4H=%d", what, ld_addend, 4 * H);
+  if (addend_col && (!addend || addend_ncols < 1))
+    return lh::fail_arg("%s: addend_col needs addend and addend_ncols >= 1", what);
+  if (h_drop && (!next_drop_mask || !(keep > 0.f)))
+    return lh::fail_arg("%s: h_drop needs next_drop_mask and keep > 0", what);
+  GemmArgs g{};
+  for (int s = 0; s < LH_GEMM_MAX_SEGS; ++s) {
+    const lh_gemm_seg &e = segs[s < nseg ? s : 0];
+    if (!e.A || !e.X || e.K <= 0 || e.K % 4 != 0 || e.ldx < e.K || e.ldx % 4 != 0 || e.ldx >= 1 << 22 ||
+        !lh::aligned16(e.A) || !lh::aligned16(e.X))
+      return lh::fail_arg("%s: segment %d: A=%p X=%p K=%d ldx=%d (16-byte aligned, multiples of 4)", what, s,
+                          (const void *)e.A, (const void *)e.X, e.K, e.ldx);
+    g.A[s] = e.A, g.X[s] = e.X, g.lda[s] = kPackRows, g.ldx[s] = e.ldx, g.K[s] = e.K;
+  }
+  // other workgroups still read the operands while one writes its cells
+  for (int s = 0; s < nseg; ++s) {
+    const float *x0 = segs[s].X, *x1 = x0 + (size_t)segs[s].ldx * B;
+    const float *outs[4] = {c, h, h_drop, gates};
+    for (int o = 0; o < 4; ++o)
+      if (outs[o] && outs[o] < x1 && x0 < outs[o] + (size_t)(o == 3 ? 4 : 1) * H * B)
+        return lh::fail_arg("%s: an output overlaps operand X of segment %d", what, s);
+  }
+  int config;
+  float us;
+  pick_packed(H, B, g.K, nseg, &config, &us);
+  if (config < 0) return lh::fail_arg("%s: the configuration override names none of its configurations", what);
+  g.nseg = nseg;
+  g.M = 4 * H, g.N = B;
+  g.beta = addend ? 1.f : 0.f;
+  g.C = const_cast<float *>(addend);
+  g.ldc = ld_addend;
+  g.bias = bias4h;
+  g.colmask = mask01;
+  g.cell_H = H;
+  g.c_prev = c_prev, g.c_out = c, g.h_out = h;
+  g.cell_clip = cell_clip;
+  g.sigmoid_f64 = sigmoid_f64;
+  g.addend_col = addend_col, g.addend_ncols = addend_ncols;
+  g.gates_out = gates;
+  g.drop_mask = next_drop_mask, g.h_drop = h_drop, g.keep = keep;
+  return launch_packed_index(config, g, lh::as_stream(stream));
+}
 
 // ---- grouped gate products ----------------------------------------------------------------------
 namespace {

@@ -5,7 +5,8 @@ configuration list:   python linmt_amd/csrc/tune_gemm.py > linmt_amd/csrc/gemm_t
 and rebuild.  For every configuration and operand layout it times a product whose tiles give each
 CU exactly one workgroup, and one that gives each CU as many as fit at once, at two depths K; the
 table holds the fixed and per-k cost of both, which is all the cost model in gemm.hip uses; a
-fourth block does the same for the stacked gate product that ends in the LSTM cell.
+fourth block does the same for the stacked gate product that ends in the LSTM cell, a fifth for that
+product on packed gate matrices.
 """
 import sys
 
@@ -57,7 +58,7 @@ def main():
     print("// {workgroups resident per CU, then (fixed us, us per k) with one workgroup per CU and")
     print("//  with the CU full}, by operand layout (NN, TN, NT) and configuration.")
     print(f"static_assert(kNumConfigs == {n_cfg}, \"gemm_tuning.inc is stale: rerun tune_gemm.py\");")
-    print("const Tuning kTuning[4][kNumConfigs] = {")
+    print("const Tuning kTuning[5][kNumConfigs] = {")
     try:
         for lay, (tA, tX) in (("NN", (False, False)), ("TN", (True, False)), ("NT", (False, True))):
             print(f"    {{  // {lay}")
@@ -83,35 +84,46 @@ def main():
                 sys.stdout.flush()
             print("    },")
         # the stacked gate product with the LSTM cell in its epilogue (a tile = BM/4 rows of each gate)
-        print("    {  // NN with the cell epilogue (zeros: the configuration's LDS cannot hold a tile)")
         bias, ones = torch.zeros(4 * 12288, device="cuda"), torch.ones(8192, dtype=torch.int32, device="cuda")
-        for cfg in range(n_cfg):
-            info = lh.gemm_config_info(cfg, False, False)
-            occ = max(1, info["occupancy"])
-            L.lh_gemm_set_config_override(cfg)
-            fits = []
-            for per_cu in (1, occ):
-                tm, tn = 16 * per_cu, 16
-                while tm * info["BM"] > 12288:
-                    tm //= 2
-                    tn *= 2
-                H, B = info["BM"] // 4 * tm, info["BN"] * tn
-                ts = []
-                for K in KS:
-                    segs = [(a, 4 * H, x, K, K)]
-                    if not lh.gate_gemm_lstm_cell_plan(H, B, segs)[0]:
+        for packed in (False, True):
+            print("    {  // packed gate matrices with the cell epilogue (zeros: not a configuration of that kernel)"
+                  if packed else
+                  "    {  // NN with the cell epilogue (zeros: the configuration's LDS cannot hold a tile)")
+            for cfg in range(n_cfg):
+                info = lh.gemm_config_info(cfg, False, False)
+                occ = max(1, info["occupancy"])
+                L.lh_gemm_set_config_override(cfg)
+                fits = []
+                for per_cu in (1, occ):
+                    tm, tn = 16 * per_cu, 16
+                    while tm * info["BM"] > 12288:
+                        tm //= 2
+                        tn *= 2
+                    H, B = info["BM"] // 4 * tm, info["BN"] * tn
+                    ts = []
+                    for K in KS:
+                        segs = [(a, 32 if packed else 4 * H, x, K, K)]
+                        if packed:
+                            call = lh.gate_gemm_lstm_cell_packed
+                            try:
+                                call(H, B, segs, bias, c, ones, c, c[H * B:])
+                            except lh.LinmtHipError:
+                                break
+                        else:
+                            call = lh.gate_gemm_lstm_cell
+                            if not lh.gate_gemm_lstm_cell_plan(H, B, segs)[0]:
+                                break
+                        ts.append(timeit(lambda: call(H, B, segs, bias, c, ones, c, c[H * B:])))
+                    if len(ts) < 2:
                         break
-                    ts.append(timeit(lambda: lh.gate_gemm_lstm_cell(H, B, segs, bias, c, ones, c, c[H * B:])))
-                if len(ts) < 2:
-                    break
-                slope = (ts[1] - ts[0]) / (KS[1] - KS[0])
-                fits += [max(0.0, ts[0] - slope * KS[0]), slope]
-            if len(fits) < 4:
-                fits, occ = [0.0] * 4, 0
-            print(f"        {{{occ}, {fits[0]:.2f}f, {fits[1]:.5f}f, {fits[2]:.2f}f, {fits[3]:.5f}f}},"
-                  f"  // {cfg}: {info['BM']}x{info['BN']} wk{info['WK']} bk{info['BK']}")
-            sys.stdout.flush()
-        print("    },")
+                    slope = (ts[1] - ts[0]) / (KS[1] - KS[0])
+                    fits += [max(0.0, ts[0] - slope * KS[0]), slope]
+                if len(fits) < 4:
+                    fits, occ = [0.0] * 4, 0
+                print(f"        {{{occ}, {fits[0]:.2f}f, {fits[1]:.5f}f, {fits[2]:.2f}f, {fits[3]:.5f}f}},"
+                      f"  // {cfg}: {info['BM']}x{info['BN']} wk{info['WK']} bk{info['BK']}")
+                sys.stdout.flush()
+            print("    },")
     finally:
         L.lh_gemm_set_config_override(-1)
     print("};")

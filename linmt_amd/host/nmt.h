@@ -207,6 +207,13 @@ class LstmLayer {
   int split_kgroups_ = 0;  // k-groups of both operands, padding included
   bool split_dirty_ = true;
   void BuildSplitWeights();
+  // The stacked gate matrices as the packed gate product reads them (lh_gate_pack_f32), a copy beside the
+  // stored ones: made by the first step that runs faster on it, made anew after a change of the weights.
+  // M is not among them where it never is an operand of a step's product (the input layer).  A model whose
+  // memory does not hold the copies runs on the stored matrices.
+  DeviceArray<float> packed_m_, packed_w_h_, packed_q_;
+  bool packed_dirty_ = true, packed_possible_ = true;
+  bool PackGates();  // false: no memory
   void ForwardPropInputAllSteps(int steps);
   void ForwardPropInputSteps(int first, int steps);
   void BuildEmbeddingFold();

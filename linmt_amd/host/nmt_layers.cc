@@ -137,7 +137,7 @@ bool LstmLayer::SetParam(const std::string &name, const float *host, size_t n) {
   hipStream_t s = p_neural_mt_->stream_;
   const int H = lstm_size_;
   if (name == "W" || name[0] == 'M') mw_fold_dirty_ = true;
-  split_dirty_ = true;
+  split_dirty_ = packed_dirty_ = true;
   if (name == "W") return input_layer_mode_ && SetFlat(p_device_w_, host, n, s);
   if (name.size() == 3 && name[0] == 'M' && name[1] == '_') {
     const int g = GateIndex(name[2]);
@@ -238,6 +238,34 @@ void LstmLayer::BuildSplitWeights() {
   split_dirty_ = false;
 }
 
+bool LstmLayer::PackGates() {
+  if (!packed_possible_) return false;
+  if (!packed_dirty_) return true;
+  const int H = lstm_size_;
+  DeviceArray<float> *to[3] = {&packed_m_, &packed_w_h_, &packed_q_};
+  DeviceArray<float> *from[3] = {&p_device_m_stack_, &p_device_w_h_stack_, &p_device_q_stack_};
+  const int K[3] = {input_layer_mode_ ? 0 : input_size_, H, feed_input_mode_ ? H : 0};
+  lh_gate_pack_source src[3];
+  int n = 0;
+  for (int i = 0; i < 3; ++i) {
+    if (!K[i]) continue;
+    const size_t floats = lh_gate_pack_floats(H, K[i]);
+    if (to[i]->size() != floats) {
+      try {
+        to[i]->Alloc(floats);
+      } catch (const std::exception &) {
+        for (DeviceArray<float> *a : to) a->Free();
+        packed_possible_ = false;
+        return false;
+      }
+    }
+    src[n++] = lh_gate_pack_source{from[i]->get(), 4 * H, K[i], to[i]->get()};
+  }
+  LhErrorWrapper(lh_gate_pack_f32(H, src, n, p_neural_mt_->stream_), "LstmLayer::PackGates");
+  packed_dirty_ = false;
+  return true;
+}
+
 // ForwardProp of a target node whose step runs on split products: the packed input of the layer
 // is complete (h_{t-1}, h~_{t-1} packed at the start of the step, h of the layer below written as
 // planes by that layer's kernel); one launch does the product, the cell and the planes of h for
@@ -322,6 +350,34 @@ void LstmNode::ForwardProp() {
   if (feed) segs[nseg++] = {L.p_device_q_stack_.get(), 4 * H, p_device_h_tild_, H, H};
   const bool drop_out = M.apply_dropout_ && L.out_dropout_;
   const float cell_clip = M.cfg_.clip_cell_mode_ ? M.cfg_.cell_clip_threshold_ : 0.f;
+
+  // Product and cell in ONE kernel on packed gate matrices, where that is the faster way (few columns).
+  if (!(x && L.input_layer_mode_)) {
+    int faster = 0;
+    char name[160] = {0};
+    LhErrorWrapper(lh_gate_gemm_lstm_cell_packed_plan(H, B, segs, nseg, beta != 0.f, M.gemm_ws_bytes_, &faster,
+                                                      name, sizeof(name)),
+                   "lh_gate_gemm_lstm_cell_packed_plan");
+    if (faster && !(folded && (p_device_gates_ || drop_out)) && L.PackGates()) {
+      double k = 0;
+      for (int i = 0; i < nseg; ++i) {
+        k += segs[i].K;
+        segs[i].A = segs[i].A == L.p_device_m_stack_.get()     ? L.packed_m_.get()
+                    : segs[i].A == L.p_device_w_h_stack_.get() ? L.packed_w_h_.get()
+                                                               : L.packed_q_.get();
+      }
+      ProfileScope ps(M.profiler_, kTagGateGemm, name, 2.0 * 4 * H * (double)B * k);
+      LhErrorWrapper(lh_gate_gemm_lstm_cell_packed_f32(
+                         H, B, segs, nseg, beta != 0.f ? (folded ? L.mw_fold_.get() : pre) : nullptr, 4 * H,
+                         folded ? p_device_input_vocab_indices_ : nullptr, folded ? L.vocab_size_ : 0,
+                         L.p_device_b_stack_.get(), p_device_c_t_prev_, p_device_input_vocab_indices_01_,
+                         feed ? 1 : 0, cell_clip, p_device_gates_, p_device_c_t_, p_device_h_t_,
+                         drop_out ? p_device_out_dropout_mask_ : nullptr, drop_out ? M.cfg_.dropout_rate_ : 1.f,
+                         drop_out ? p_device_h_t_dropped_ : nullptr, s),
+                     "LstmNode::ForwardPropGpu packed gate product with cell");
+      return;
+    }
+  }
 
   // Product and cell in ONE kernel whenever the product runs unsplit; in the inference form (no
   // gate values kept, no dropout) the folded embedding table is read by that kernel too, the

@@ -36,6 +36,10 @@ class UpdateItem(C.Structure):
                 ("rows", C.c_longlong), ("cols", C.c_longlong), ("col_index", C.c_void_p), ("norm", C.c_int)]
 
 
+class GatePackSource(C.Structure):
+    _fields_ = [("src", c_f32p), ("ld", C.c_int), ("K", C.c_int), ("dst", c_f32p)]
+
+
 class GateProblem(C.Structure):
     _fields_ = [("segs", GemmSeg * LH_GEMM_MAX_SEGS), ("nseg", C.c_int), ("cell", C.c_int),
                 ("addend", C.c_void_p), ("ld_addend", C.c_int), ("addend_col", C.c_void_p),
@@ -85,6 +89,14 @@ SIGNATURES = {
                                                    c_f32p, C.c_int, c_f32p, c_f32p, c_i32p, C.c_int,
                                                    C.c_float, c_f32p, c_f32p, c_f32p, c_f32p,
                                                    C.c_float, c_f32p, C.c_size_t, C.c_void_p]),
+    "lh_gate_pack_floats": (C.c_size_t, [C.c_int, C.c_int]),
+    "lh_gate_pack_f32": (C.c_int, [C.c_int, C.POINTER(GatePackSource), C.c_int, C.c_void_p]),
+    "lh_gate_gemm_lstm_cell_packed_plan": (C.c_int, [C.c_int, C.c_int, C.POINTER(GemmSeg), C.c_int, C.c_int,
+                                                     C.c_size_t, C.POINTER(C.c_int), C.c_char_p, C.c_int]),
+    "lh_gate_gemm_lstm_cell_packed_f32": (C.c_int, [C.c_int, C.c_int, C.POINTER(GemmSeg), C.c_int, c_f32p,
+                                                    C.c_int, c_i32p, C.c_int, c_f32p, c_f32p, c_i32p,
+                                                    C.c_int, C.c_float, c_f32p, c_f32p, c_f32p, c_f32p,
+                                                    C.c_float, c_f32p, C.c_void_p]),
     "lh_gate_gemm_group_plan": (C.c_int, [C.c_int, C.c_int, C.POINTER(GateProblem), C.c_int,
                                           C.POINTER(C.c_int), C.c_char_p, C.c_int]),
     "lh_gate_gemm_group_f32": (C.c_int, [C.c_int, C.c_int, C.POINTER(GateProblem), C.c_int,
@@ -345,6 +357,38 @@ def gate_gemm_lstm_cell_train(H, B, segs, bias4h, c_prev, mask01, c, h, gates=No
                                                   _ptr(h), _ptr(next_drop_mask), keep, _ptr(h_drop),
                                                   workspace_bytes, _stream(stream)),
           "lh_gate_gemm_lstm_cell_train_f32")
+
+
+def gate_pack_floats(H, K):
+    return load().lh_gate_pack_floats(H, K)
+
+
+def gate_pack(H, sources, stream=None):
+    """sources: (stacked 4H x K matrix, ld, K, destination) per matrix."""
+    arr = (GatePackSource * len(sources))()
+    for i, (src, ld, K, dst) in enumerate(sources):
+        arr[i].src, arr[i].ld, arr[i].K, arr[i].dst = src.data_ptr(), ld, K, dst.data_ptr()
+    check(load().lh_gate_pack_f32(H, arr, len(sources), _stream(stream)), "lh_gate_pack_f32")
+
+
+def gate_gemm_lstm_cell_packed_plan(H, B, segs, has_addend=False, workspace_bytes=0):
+    """(faster, kernel instance name) for lh_gate_gemm_lstm_cell_packed_f32 on this problem."""
+    f, buf = C.c_int(), C.create_string_buffer(128)
+    check(load().lh_gate_gemm_lstm_cell_packed_plan(H, B, _segs(segs), len(segs), int(has_addend),
+                                                    workspace_bytes, C.byref(f), buf, 128),
+          "lh_gate_gemm_lstm_cell_packed_plan")
+    return bool(f.value), buf.value.decode()
+
+
+def gate_gemm_lstm_cell_packed(H, B, segs, bias4h, c_prev, mask01, c, h, addend=None, ld_addend=0,
+                               addend_col=None, addend_ncols=0, sigmoid_f64=False, cell_clip=0.0, gates=None,
+                               next_drop_mask=None, keep=1.0, h_drop=None, stream=None):
+    check(load().lh_gate_gemm_lstm_cell_packed_f32(H, B, _segs(segs), len(segs), _ptr(addend), ld_addend,
+                                                   _ptr(addend_col), addend_ncols, _ptr(bias4h), _ptr(c_prev),
+                                                   _ptr(mask01), int(sigmoid_f64), cell_clip, _ptr(gates),
+                                                   _ptr(c), _ptr(h), _ptr(next_drop_mask), keep, _ptr(h_drop),
+                                                   _stream(stream)),
+          "lh_gate_gemm_lstm_cell_packed_f32")
 
 
 def _gate_problems(problems):

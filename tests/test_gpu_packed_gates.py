@@ -1,0 +1,109 @@
+"""Gate products on packed gate matrices: the layout of lh_gate_pack_f32, the product with its cell
+against float64 and against the kernel on the stored matrix, and a model whose weights change
+between two passes."""
+import numpy as np
+import pytest
+
+from tests.conftest import assert_close
+
+pytestmark = pytest.mark.gpu
+
+CONFIGS = [-1, 13, 14, 15, 19]
+
+
+@pytest.fixture()
+def lh():
+    from linmt_amd import lib
+    lib.load()
+    yield lib
+    lib.load().lh_gemm_set_config_override(-1)
+
+
+def _packed(lh, torch, H, W, Ks):
+    P = [torch.full((lh.gate_pack_floats(H, K),), float("nan"), device="cuda") for K in Ks]
+    lh.gate_pack(H, [(w, w.shape[1], K, p) for w, K, p in zip(W, Ks, P)])
+    return P
+
+
+@pytest.mark.parametrize("H,Ks", [(4, (4,)), (8, (20,)), (36, (36, 12)), (100, (100, 8, 4)), (1000, (1000, 1000))])
+def test_pack_layout(lh, H, Ks):
+    import torch
+    W = [torch.randn(K, 4 * H + 4, device="cuda") for K in Ks]  # column-major, ld = 4H + 4
+    for w, K, p in zip(W, Ks, _packed(lh, torch, H, W, Ks)):
+        blocks = (H + 7) // 8
+        cells = torch.zeros(K, 4, blocks * 8, device="cuda")
+        cells[:, :, :H] = w[:, :4 * H].view(K, 4, H)
+        want = cells.view(K, 4, blocks, 8).permute(2, 0, 3, 1)
+        assert torch.equal(want.flatten(), p)
+
+
+@pytest.mark.parametrize("config", CONFIGS)
+@pytest.mark.parametrize("H,B,Ks", [(4, 1, (4,)), (36, 33, (36,)), (64, 32, (132, 20)), (100, 65, (16, 100, 60)),
+                                    (1000, 12, (1000, 1000))])
+def test_packed_gate_product_with_cell(lh, config, H, B, Ks):
+    """All of the cell's forms: an addend by column, gate values and the dropped copy kept."""
+    import torch
+    torch.manual_seed(H + B)
+    dev = dict(device="cuda")
+    W = [torch.randn(K, 4 * H, **dev) / K ** 0.5 for K in Ks]
+    X = [torch.randn(B, K, **dev) for K in Ks]
+    table, col = torch.randn(7, 4 * H, **dev), torch.randint(0, 7, (B,), dtype=torch.int32, **dev)
+    bias, c_prev, drop = torch.randn(4 * H, **dev), torch.randn(B, H, **dev), torch.rand(B, H, **dev)
+    mask = (torch.rand(B, **dev) > 0.2).int()
+    pre = sum(x.double() @ w.double() for w, x in zip(W, X)) + table.double()[col.long()] + bias.double()
+    i, f, g, o = pre.view(B, 4, H).unbind(1)
+    i, f, g, o = torch.sigmoid(i), torch.sigmoid(f), torch.tanh(g), torch.sigmoid(o)
+    c = (f * c_prev.double() + i * g)
+    h = (o * torch.tanh(c)) * mask[:, None]
+    c = c * mask[:, None]
+    segs = [(p, 32, x, K, K) for p, x, K in zip(_packed(lh, torch, H, W, Ks), X, Ks)]
+    got_c, got_h, got_d = (torch.full((B, H), float("nan"), **dev) for _ in range(3))
+    gates = torch.full((B, 4 * H), float("nan"), **dev)
+    lh.load().lh_gemm_set_config_override(config)
+    lh.gate_gemm_lstm_cell_packed(H, B, segs, bias, c_prev, mask, got_c, got_h, addend=table, ld_addend=4 * H,
+                                  addend_col=col, addend_ncols=7, gates=gates, next_drop_mask=drop, keep=0.8,
+                                  h_drop=got_d)
+    torch.cuda.synchronize()
+    # a pre-activation rounds K + 3 times, by 2^-24 of the sum of magnitudes; the cell's derivatives are below 1 in
+    # i, f, o (times |c_prev| or 1) and g, and its own functions round a few times more
+    mags = sum(x.abs().double() @ w.abs().double() for w, x in zip(W, X)) + table.abs().max() + bias.abs().max()
+    tol = ((sum(Ks) + 3) * 2.0 ** -24 * mags.max().item() + 1e-6) * (1 + c_prev.abs().max().item())
+    for name, got, want in (("c", got_c, c), ("h", got_h, h), ("gates", gates, torch.cat([i, f, g, o], 1)),
+                            ("h_drop", got_d, (drop < 0.8).double() / 0.8 * h)):
+        assert (got.double() - want).abs().max().item() <= tol, name
+
+
+@pytest.mark.parametrize("B", [3, 64])
+def test_weights_set_between_passes_reach_the_packed_copy(lh, B):
+    """A model that has packed its gates must pack them anew when a matrix is set and after an update."""
+    import torch
+    from linmt_amd import host
+    rng = np.random.default_rng(B)
+    H, V, S = 256, 50, 6
+    any_matrix = torch.empty(4 * H * H, device="cuda")
+    assert lh.gate_gemm_lstm_cell_packed_plan(H, B, [(any_matrix, 4 * H, any_matrix, H, H)] * 2)[0]
+    kw = dict(longest_sentence=S + 4, attention_mode=0, minibatch_size=B)
+    u = lambda *s: rng.uniform(-0.3, 0.3, size=s).astype(np.float32)  # noqa: E731
+    P = {"softmax.D": u(V, H), "softmax.b_d": u(V)}
+    for side in ("src", "tgt"):
+        P[side + ".0.W"] = u(H, V)
+        for layer in range(2):
+            for g in "ifco":
+                P[f"{side}.{layer}.W_h{g}"], P[f"{side}.{layer}.M_{g}"], P[f"{side}.{layer}.b_{g}"] = u(H, H), u(H, H), u(H)
+    src, ti, to = (rng.integers(0, V, (B, S)).astype(np.int32) for _ in range(3))
+    info = np.concatenate([np.full(B, S), np.zeros(B)]).astype(np.int32)
+    unique = [np.unique(a).astype(np.int32) for a in (src, ti)]
+    m = host.Model(2, H, V, V, training=dict(learning_rate=0.5, grad_clip_mode=0), **kw)
+    m.set_params(P)
+    first = m.compute_gradients(src, ti, to, info, *unique)
+    m.update_weights()
+    P["src.1.W_hf"] = u(H, H)
+    m.set_params({"src.1.W_hf": P["src.1.W_hf"]})
+    second = m.compute_gradients(src, ti, to, info, *unique)
+    fresh = host.Model(2, H, V, V, **kw)
+    shapes = {n: a.shape for n, a in P.items()}
+    fresh.set_params({n: np.asfortranarray(m.get_param(n, s)) for n, s in shapes.items()})
+    want = fresh.get_error(src, ti, to, info)
+    assert abs(first - second) > 1e-2
+    assert_close(second, want, "loss with the weights as they are now", rtol=1e-6, atol=1e-4)
+    m.close(), fresh.close()

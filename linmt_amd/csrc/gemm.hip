@@ -608,18 +608,19 @@ constexpr int smem2_floats() {
               (WK - 1) * BM * BN);
 }
 
-// A wavefront's CK x 32 piece of one operand in its ring stage.  A load writes 64 consecutive
+// A wavefront's CK x BD piece of one operand in its ring stage.  A load writes 64 consecutive
 // 16-byte units, one per lane, so what the layout can choose is which unit a lane fetches:
 //  * contiguous along d: rows of 32 floats, one per k; the k of a group of 8 in the order 0 4 2 6 1 5 3 7,
 //    which puts the two k of one MFMA step (k and k + 4, lanes 0-31 and 32-63) into neighbouring rows:
 //    a fragment read is 64 consecutive floats;
 //  * contiguous along k: rows of CK floats, one per d, their units permuted (XOR with bits of d) so
 //    that the 16 lanes of one phase of a 16-byte read meet all banks.
-template <int CK, bool KC>
+template <int CK, bool KC, int BD = 32>
 struct Piece {
   static constexpr int U = CK / 4;       // KC: units per row
-  static constexpr int kLoads = CK / 8;  // wavefront loads per piece
-  static constexpr int kFloats = CK * 32;
+  static_assert(KC || BD == 32, "rows of k");
+  static constexpr int kFloats = CK * BD;
+  static constexpr int kLoads = kFloats / 256;  // wavefront loads per piece
   unsigned goff[kLoads];
 
   static __device__ __forceinline__ int swap02(int k) { return (k & ~5) | ((k & 1) << 2) | ((k >> 2) & 1); }
@@ -681,6 +682,26 @@ struct Piece {
     }
   }
 };
+
+// The cell of row r, column n from its pre-activations, and everything it leaves.
+__device__ __forceinline__ void store_cell(const GemmArgs &g, float (&pre)[4], float c_prev, int colmask, int r, int n) {
+  const int H = g.cell_H;
+  float c, h;
+  const float mask = (float)(colmask & 1);
+  if (g.sigmoid_f64 && !(colmask & LH_MASK_F32_GATES))
+    lh::lstm_cell_point<true>(pre[0], pre[1], pre[2], pre[3], c_prev, mask, g.cell_clip, c, h);
+  else
+    lh::lstm_cell_point<false>(pre[0], pre[1], pre[2], pre[3], c_prev, mask, g.cell_clip, c, h);
+  const size_t o = (size_t)n * H + r;
+  g.c_out[o] = c;
+  g.h_out[o] = h;
+  if (g.gates_out) {
+    float *go = g.gates_out + (size_t)n * 4 * H + r;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) go[(size_t)q * H] = pre[q];  // the cell left i, f, g, o there
+  }
+  if (g.h_drop) g.h_drop[o] = ((float)(g.drop_mask[o] < g.keep) * (1.0f / g.keep)) * h;
+}
 
 // At most N of this wavefront's loads still in flight; its LDS reads have returned.
 template <int N>
@@ -915,21 +936,7 @@ __device__ __forceinline__ void stream_body(const GemmArgs &g, const int m0, con
     }
 #pragma unroll
     for (int q = 0; q < 4; ++q) pre[q] = (g.beta != 0.f ? pre[q] + ep_add[q] : pre[q]) + ep_bias[q];
-    float c, h;
-    const float mask = (float)(ep_mask & 1);
-    if (g.sigmoid_f64 && !(ep_mask & LH_MASK_F32_GATES))
-      lh::lstm_cell_point<true>(pre[0], pre[1], pre[2], pre[3], ep_c, mask, g.cell_clip, c, h);
-    else
-      lh::lstm_cell_point<false>(pre[0], pre[1], pre[2], pre[3], ep_c, mask, g.cell_clip, c, h);
-    const size_t o = (size_t)n * H + r;
-    g.c_out[o] = c;
-    g.h_out[o] = h;
-    if (g.gates_out) {
-      float *go = g.gates_out + (size_t)n * 4 * H + r;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) go[(size_t)q * H] = pre[q];  // the cell left i, f, g, o there
-    }
-    if (g.h_drop) g.h_drop[o] = ((float)(g.drop_mask[o] < g.keep) * (1.0f / g.keep)) * h;
+    store_cell(g, pre, ep_c, ep_mask, r, n);
   } else {
     // a split product stores the bare partial sums in its plane of the workspace
     const bool partial = splits > 1;
@@ -1393,6 +1400,204 @@ __global__ __launch_bounds__(256) void gate_pack_kernel(const PackArgs p) {
   }
 }
 
+// ---- narrow form: packed gate product of at most a few 16-column blocks ------------------------
+// A tile of 16 rows (four cells) x 16 FC columns; the eight wavefronts share its k, 32 of every slab of 256
+// each, streamed like stream_body's.  What bounds a gate product of few columns is reading the weights: 32-row
+// tiles are 125 workgroups at 1000 hidden units, which leaves half the CUs idle, and the 32x32 MFMA multiplies
+// 32 columns whatever there are; these are 250 workgroups with the 16x16x4 MFMA at the same rate per column.
+// 1000 hidden units, K = 1000 / 2000, with cell: 12 columns 9.5 / 14.7 us on 32x32 tiles, 6.8 / 9.9 (16 and 32 MB of
+// weights, 5.3 TB/s beyond the fixed part); 32 columns 10.1 / 15.3 and 8.6 / 12.3; 256 hidden units, 12 columns, K = 512
+// 6.7 and 4.5.  At 2048 hidden units both read the weights at the same rate (16.8 us, K = 2048).
+constexpr int kNarrowK = 32, kNarrowSlab = 8 * kNarrowK, kNarrowCells = 4;
+constexpr int kNarrowLd = 20;  // floats between the columns of a partial block in LDS
+template <int FC>
+constexpr int narrow_stages() {
+  return FC == 1 ? 4 : 3;
+}
+template <int FC>
+constexpr int narrow_smem_floats() {
+  return cmax(narrow_stages<FC>() * kNarrowSlab * 16 * (1 + FC), 8 * 16 * FC * kNarrowLd);
+}
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+template <int FC>
+__global__ __launch_bounds__(512) void gate_gemm_narrow_kernel(const GemmArgs g) {
+  constexpr int CK = kNarrowK, SLAB = kNarrowSlab, NB = narrow_stages<FC>(), BN = 16 * FC;
+  using PX = Piece<CK, true, 16>;
+  constexpr int kA = CK * 16, kStage = kA + FC * PX::kFloats;  // floats
+  constexpr int kLoadsA = kA / 256, kLoads = kLoadsA + FC * PX::kLoads;
+  const int logical = xcd_logical_id();
+  const int cell0 = (logical / g.tiles_n) * kNarrowCells, n0 = (logical % g.tiles_n) * BN;
+  const int tid = threadIdx.x, lane = tid % lh::kWave;
+  const int wk = __builtin_amdgcn_readfirstlane(tid / lh::kWave);
+  const int l16 = lane % 16, lq = lane / 16;
+  float *const ring = smem + wk * NB * kStage;
+  const unsigned ring_lds = (unsigned)(size_t)(__attribute__((address_space(3))) float *)ring;
+  const int N = g.N, H = g.cell_H;
+  auto pick = [](int seg, auto v0, auto v1, auto v2) __attribute__((always_inline)) {
+    return seg == 0 ? v0 : (seg == 1 ? v1 : v2);
+  };
+#define LH_SEG(FIELD, SEG) pick(SEG, g.FIELD[0], g.FIELD[1], g.FIELD[2])
+
+  // A unit of the ring's A rows: row `pos` of 16 floats is k = 16 (pos / 16) + 4 (pos % 4) + pos / 4 % 4, so that the
+  // four k of one MFMA step (4 apart, one per quarter of the wavefront) are neighbouring rows.
+  auto a_k = [](int u) __attribute__((always_inline)) { return (u / 64) * 16 + 4 * (u / 4 % 4) + u / 16 % 4; };
+  unsigned aoff[kLoadsA];
+#pragma unroll
+  for (int i = 0; i < kLoadsA; ++i) {
+    const int u = lane + i * 64;
+    aoff[i] = (unsigned)(a_k(u) * kPackRows + (u % 4) * 4) * 4u;
+  }
+  PX px[FC];
+  int lseg = 0, k0 = 0, Ks = 0, ldx = 0;
+  bool new_seg = true;
+  const float *a = nullptr, *x = nullptr;
+  unsigned put = ring_lds;
+  auto request = [&]() __attribute__((always_inline)) {
+    if (new_seg) {
+      LH_KEEP_BRANCH();
+      Ks = LH_SEG(K, lseg);
+      if (ldx != LH_SEG(ldx, lseg)) {
+        LH_KEEP_BRANCH();
+        ldx = LH_SEG(ldx, lseg);
+#pragma unroll
+        for (int c = 0; c < FC; ++c) px[c].set_ld(ldx, lane, 16 * c, N - n0);
+      }
+      const int k = k0 + wk * CK;
+      a = LH_SEG(A, lseg) + ((size_t)(cell0 / kPackCells) * Ks + k) * kPackRows + cell0 % kPackCells * 4;
+      x = LH_SEG(X, lseg) + (size_t)n0 * ldx + k;
+    }
+    const int kn = Ks - k0 - wk * CK;
+    if (kn < CK) {
+      LH_KEEP_BRANCH();
+      if (kn <= 0) {
+        a = LH_SEG(A, lseg) + (size_t)(cell0 / kPackCells) * Ks * kPackRows + cell0 % kPackCells * 4;
+        x = LH_SEG(X, lseg) + (size_t)n0 * ldx;
+      }
+#pragma unroll
+      for (int i = 0; i < kLoadsA; ++i) {
+        const int k = a_k(lane + i * 64);
+        PX::load_unit(a, k < kn ? aoff[i] : aoff[i] - (unsigned)(k * kPackRows) * 4u, put + 1024u * i);
+      }
+#pragma unroll
+      for (int c = 0; c < FC; ++c) px[c].load_tail(x, put + (kA + c * PX::kFloats) * 4u, ldx, lane, kn);
+    } else {
+#pragma unroll
+      for (int i = 0; i < kLoadsA; ++i) PX::load_unit(a, aoff[i], put + 1024u * i);
+#pragma unroll
+      for (int c = 0; c < FC; ++c) px[c].load(x, put + (kA + c * PX::kFloats) * 4u);
+    }
+    put = put + kStage * 4u == ring_lds + NB * kStage * 4u ? ring_lds : put + kStage * 4u;
+    a += SLAB * kPackRows;
+    x += SLAB;
+    k0 += SLAB;
+    new_seg = k0 >= Ks;
+    if (new_seg) {
+      ++lseg;
+      k0 = 0;
+    }
+  };
+
+  const int total = g.slabs_per_split;
+  int issued = min(total, NB - 1);
+  for (int i = 0; i < issued; ++i) request();
+
+  // what the cell reads from memory
+  const int rl = tid % kNarrowCells, nl = tid / kNarrowCells;
+  const int r = cell0 + rl, n = n0 + nl;
+  const bool ep_ok = tid < kNarrowCells * BN && r < H && n < N;
+  float ep_add[4] = {0.f, 0.f, 0.f, 0.f}, ep_bias[4] = {0.f, 0.f, 0.f, 0.f}, ep_c = 0.f;
+  int ep_mask = 0;
+  if (ep_ok) {
+    int col = n;
+    if (g.addend_col) col = min(max(g.addend_col[n], 0), g.addend_ncols - 1);
+    const float *ad = g.C + (size_t)col * g.ldc + r;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (g.beta != 0.f) ep_add[q] = ad[(size_t)q * H];
+      ep_bias[q] = g.bias[q * H + r];
+    }
+    ep_c = g.c_prev[(size_t)n * H + r];
+    ep_mask = g.colmask[n];
+  }
+
+  floatx4 acc[FC];
+#pragma unroll
+  for (int c = 0; c < FC; ++c) acc[c] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const float *get = ring;
+  int cseg = 0, ck = 0, cK = LH_SEG(K, 0);
+  for (int s = 0; s < total; ++s) {
+    const int behind = issued - 1 - s;
+    if (NB > 3 && behind >= 2) wait_loads<kLoads * 2>();
+    else if (behind >= 1) wait_loads<kLoads>();
+    else wait_loads<0>();
+    float fa[CK / 16][4], fx[FC][CK / 16][4];
+#pragma unroll
+    for (int grp = 0; grp < CK / 16; ++grp) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) fa[grp][q] = get[(16 * grp + 4 * q + lq) * 16 + l16];
+#pragma unroll
+      for (int c = 0; c < FC; ++c) {
+        const float4 t = *reinterpret_cast<const float4 *>(
+            get + kA + c * PX::kFloats + (l16 * PX::U + ((4 * grp + lq) ^ PX::swizzle(l16))) * 4);
+        fx[c][grp][0] = t.x, fx[c][grp][1] = t.y, fx[c][grp][2] = t.z, fx[c][grp][3] = t.w;
+      }
+    }
+    if (issued < total) {
+      request();
+      ++issued;
+    }
+    const int kn = cK - ck - wk * CK;
+    if (kn < CK) {
+      LH_KEEP_BRANCH();
+#pragma unroll
+      for (int grp = 0; grp < CK / 16; ++grp)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const bool in = 16 * grp + 4 * lq + q < kn;
+          fa[grp][q] = in ? fa[grp][q] : 0.f;
+#pragma unroll
+          for (int c = 0; c < FC; ++c) fx[c][grp][q] = in ? fx[c][grp][q] : 0.f;
+        }
+    }
+#pragma unroll
+    for (int grp = 0; grp < CK / 16; ++grp)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int c = 0; c < FC; ++c)
+          acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(fx[c][grp][q], fa[grp][q], acc[c], 0, 0, 0);
+    get = get + kStage == ring + NB * kStage ? ring : get + kStage;
+    ck += SLAB;
+    if (ck >= cK) {
+      LH_KEEP_BRANCH();
+      ck = 0;
+      ++cseg;
+      if (s + 1 < total) cK = LH_SEG(K, cseg);
+    }
+  }
+#undef LH_SEG
+
+  __syncthreads();  // all wavefronts have left their rings
+#pragma unroll
+  for (int c = 0; c < FC; ++c)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) smem[(wk * BN + 16 * c + 4 * lq + j) * kNarrowLd + l16] = acc[c][j];
+  __syncthreads();
+  if (!ep_ok) return;
+  const float *src = smem + nl * kNarrowLd + rl * 4;
+  float4 sum = *reinterpret_cast<const float4 *>(src);
+#pragma unroll
+  for (int p = 1; p < 8; ++p) {
+    const float4 t = *reinterpret_cast<const float4 *>(src + p * BN * kNarrowLd);
+    sum.x += t.x, sum.y += t.y, sum.z += t.z, sum.w += t.w;
+  }
+  float pre[4] = {sum.x, sum.y, sum.z, sum.w};
+#pragma unroll
+  for (int q = 0; q < 4; ++q) pre[q] = (g.beta != 0.f ? pre[q] + ep_add[q] : pre[q]) + ep_bias[q];
+  store_cell(g, pre, ep_c, ep_mask, r, n);
+}
+
 // Several stacked gate products of one decoding step in ONE launch: everything that is known when
 // the step starts -- each layer's recurrent product W_h h_{t-1}, and the first layer's whole
 // pre-activation with its cell -- so that the GPU sees a few thousand tiles at once instead of a
@@ -1689,7 +1894,20 @@ int launch_packed_cfg(const GemmArgs &g0, hipStream_t st) {
   }
 }
 
+template <int FC>
+int launch_narrow(const GemmArgs &g0, hipStream_t st) {
+  GemmArgs g = g0;
+  g.tiles_m = (g.cell_H + kNarrowCells - 1) / kNarrowCells;
+  g.tiles_n = (g.N + 16 * FC - 1) / (16 * FC);
+  g.slabs_per_split = 0;
+  for (int s = 0; s < g.nseg; ++s) g.slabs_per_split += (g.K[s] + kNarrowSlab - 1) / kNarrowSlab;
+  return launch_kernel(gate_gemm_narrow_kernel<FC>, narrow_smem_floats<FC>() * 4, dim3(g.tiles_m * g.tiles_n),
+                       dim3(512), st, g);
+}
+
 int launch_packed_index(int c, const GemmArgs &g, hipStream_t st) {
+  if (c == kNumConfigs) return launch_narrow<1>(g, st);
+  if (c == kNumConfigs + 1) return launch_narrow<2>(g, st);
   switch (c) {
 #define LH_CFG_CASE(I, BM, BN, WM, WN, WK, BK) \
   case I: return launch_packed_cfg<BM, BN, WM, WN, WK, BK>(g, st);
@@ -1887,6 +2105,13 @@ void pick_config(int M, int N, const int *K, int nseg, bool ta, bool tx, Form fo
   e = Memo{M, N, {Kk[0], Kk[1], Kk[2]}, flags, *config, *splits, workspace_bytes, best};
 }
 
+// The narrow forms of the packed gate product, after the configurations of the table in pick_packed's
+// numbering, with rows of their own in the cost model (fitted at 256 and 1000 hidden units, weights from HBM; one
+// workgroup per CU).  They are not among the configurations that an override names.
+const Config kNarrow[] = {{16, 16, 1, 1, 8, kNarrowSlab}, {16, 32, 1, 1, 8, kNarrowSlab}};
+const Tuning kNarrowTuning[] = {{1, 3.7f, 0.0031f, 3.7f, 0.0031f}, {1, 4.2f, 0.0040f, 4.2f, 0.0040f}};
+constexpr int kNumNarrow = 2;
+
 // The packed gate product's configuration and predicted time (fifth table).
 void pick_packed(int H, int B, const int *K, int nseg, int *config, float *us) {
   static const std::vector<int> kPacked = [] {
@@ -1902,6 +2127,11 @@ void pick_packed(int H, int B, const int *K, int nseg, int *config, float *us) {
     int S;
     const float t = predict_us(kTuning[4][c], kConfigs[c], 4 * H, B, K, nseg, 1, false, &S);
     if (t < *us) *us = t, *config = c;
+  }
+  for (int i = 0; i < kNumNarrow && g_config_override < 0; ++i) {
+    int S;
+    const float t = predict_us(kNarrowTuning[i], kNarrow[i], 4 * H, B, K, nseg, 1, false, &S);
+    if (t < *us) *us = t, *config = kNumConfigs + i;
   }
 }
 
@@ -2210,8 +2440,10 @@ extern "C" int lh_gate_gemm_lstm_cell_packed_plan(int H, int B, const lh_gemm_se
   if (us > us0) return LH_OK;
   *faster = 1;
   if (name && name_cap > 0) {
-    const Config &k = kConfigs[c];
-    snprintf(name, name_cap, "gate_gemm_packed_kernel<%d, %d, %d, %d, %d, %d>", k.bm, k.bn, k.wm, k.wn, k.wk, k.bk);
+    const Config &k = kConfigs[c < kNumConfigs ? c : 0];
+    if (c < kNumConfigs)
+      snprintf(name, name_cap, "gate_gemm_packed_kernel<%d, %d, %d, %d, %d, %d>", k.bm, k.bn, k.wm, k.wn, k.wk, k.bk);
+    else snprintf(name, name_cap, "gate_gemm_narrow_kernel<%d>", c - kNumConfigs + 1);
   }
   return LH_OK;
 }

@@ -37,6 +37,19 @@ def test_pack_layout(lh, H, Ks):
         assert torch.equal(want.flatten(), p)
 
 
+@pytest.mark.parametrize("H,B,Ks,columns", [
+    (256, 16, (260,), 16), (256, 17, (292, 8), 16), (100, 32, (100, 36, 1028), 16), (1000, 1, (1000, 1000), 16),
+    (1000, 25, (1000,), 32), (996, 32, (520, 28), 32), (512, 64, (512,), 32)])
+def test_narrow_gate_product_with_cell(lh, H, B, Ks, columns):
+    """The forms of 16 rows and 16 or 32 columns: remainders of the wavefronts' 32 k, of a slab of 256, of the
+    four cells and of the columns; more slabs than the ring holds."""
+    import torch
+    any_matrix = torch.empty(4 * H * max(Ks), device="cuda")
+    name = lh.gate_gemm_lstm_cell_packed_plan(H, B, [(any_matrix, 4 * H, any_matrix, K, K) for K in Ks], True)[1]
+    assert name == f"gate_gemm_narrow_kernel<{columns // 16}>"
+    test_packed_gate_product_with_cell(lh, -1, H, B, Ks)
+
+
 @pytest.mark.parametrize("config", CONFIGS)
 @pytest.mark.parametrize("H,B,Ks", [(4, 1, (4,)), (36, 33, (36,)), (64, 32, (132, 20)), (100, 65, (16, 100, 60)),
                                     (1000, 12, (1000, 1000))])

@@ -2002,7 +2002,9 @@ struct Tuning {
 };
 #include "gemm_tuning.inc"
 constexpr int kCUs = 256;
-constexpr float kReduceFixedUs = 2.5f, kReduceBytesPerUs = 3.0e6f;
+// The pass over S partial planes: 4.3 to 4.8 us of 4 planes between other kernels of a stream (1000 x 64 to 2048 x 256),
+// 2.1, 2.6 and 3.8 us of 2, 4 and 8 planes of 1000 x 5 and 1.4 us less a launch when replayed from a graph.
+constexpr float kReduceFixedUs = 3.5f, kReducePlaneUs = 0.22f, kReduceBytesPerUs = 3.0e6f;
 constexpr float kCellFixedUs = 4.0f;  // a launch of the LSTM cell kernel behind its product
 
 float predict_us(const Tuning &t, const Config &k, int M, int N, const int *K, int nseg, int want,
@@ -2018,14 +2020,15 @@ float predict_us(const Tuning &t, const Config &k, int M, int N, const int *K, i
   // round but leaves a tail of about half a workgroup.
   const float per_cu = (float)(tiles * S) / kCUs;
   const float load = fminf(per_cu + 0.5f, ceilf(per_cu));
-  const float t1 = t.f1 + t.s1 * depth, tocc = t.focc + t.socc * depth;
+  // (both are fitted at depths of 512 and 4096: below, several workgroups could come out cheaper than one)
+  const float t1 = t.f1 + t.s1 * depth, tocc = fmaxf(t1, t.focc + t.socc * depth);
   const float rounds = floorf(load / (float)t.occ);
   const float rest = load - rounds * (float)t.occ;
   float us = rounds * tocc;
   if (rest > 1e-6f)
     us += rest <= 1.f || t.occ == 1 ? t1 : t1 + (tocc - t1) * (rest - 1.f) / (float)(t.occ - 1);
   if (S > 1 && !reduce_free)
-    us += kReduceFixedUs + (float)(S + 1) * (float)M * (float)N * 4.f / kReduceBytesPerUs;
+    us += kReduceFixedUs + kReducePlaneUs * (float)S + (float)(S + 1) * (float)M * (float)N * 4.f / kReduceBytesPerUs;
   if (S > 1 && reduce_free)  // the consumer reads S planes instead of one matrix
     us += (float)(S - 1) * (float)M * (float)N * 4.f / kReduceBytesPerUs;
   return us;

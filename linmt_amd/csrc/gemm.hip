@@ -2021,7 +2021,8 @@ float predict_us(const Tuning &t, const Config &k, int M, int N, const int *K, i
   const float per_cu = (float)(tiles * S) / kCUs;
   const float load = fminf(per_cu + 0.5f, ceilf(per_cu));
   // (both are fitted at depths of 512 and 4096: below, several workgroups could come out cheaper than one)
-  const float t1 = t.f1 + t.s1 * depth, tocc = fmaxf(t1, t.focc + t.socc * depth);
+  const float t1 = t.f1 + t.s1 * depth, full = t.focc + t.socc * depth;
+  const float tocc = t.occ > 1 ? fmaxf(t1, full) : full;
   const float rounds = floorf(load / (float)t.occ);
   const float rest = load - rounds * (float)t.occ;
   float us = rounds * tocc;

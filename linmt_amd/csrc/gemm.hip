@@ -1340,9 +1340,276 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &g, const int logical) 
   }
 }
 
+// ---- narrow form: products of at most a few 16-column blocks, packed gate products among them --------
+// A tile of 16 rows (four cells) x 16 FC columns; the eight wavefronts share its k, 32 of every slab of 256
+// each, streamed like stream_body's.  What bounds a gate product of few columns is reading the weights: 32-row
+// tiles are 125 workgroups at 1000 hidden units, which leaves half the CUs idle, and the 32x32 MFMA multiplies
+// 32 columns whatever there are; these are 250 workgroups with the 16x16x4 MFMA at the same rate per column.
+// 1000 hidden units, K = 1000 / 2000, with cell: 12 columns 9.5 / 14.7 us on 32x32 tiles, 6.8 / 9.9 (16 and 32 MB of
+// weights, 5.3 TB/s beyond the fixed part); 32 columns 10.1 / 15.3 and 8.6 / 12.3; 256 hidden units, 12 columns, K = 512
+// 6.7 and 4.5.  At 2048 hidden units both read the weights at the same rate (16.8 us, K = 2048).
+constexpr int kNarrowK = 32, kNarrowSlab = 8 * kNarrowK, kNarrowCells = 4;
+constexpr int kNarrowLd = 20;  // floats between the columns of a partial block in LDS
+template <int FC>
+constexpr int narrow_stages() {
+  return FC == 1 ? 4 : 3;
+}
+template <int FC>
+constexpr int narrow_smem_floats() {
+  return cmax(narrow_stages<FC>() * kNarrowSlab * 16 * (1 + FC), 8 * 16 * FC * kNarrowLd);
+}
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+// CELL: a packed gate product with its cell; otherwise a plain product with A as stored (TA: transposed), whose
+// share of k may be split over workgroups.  1000 x 64 is 252 of these tiles and 64 of 32x32, which were either a
+// quarter of the CUs or a split with a reduction behind it: K = 1000 / 2000 9.0 / 11.0 us there (a launch more of 4.5 us
+// between other kernels at 2000), 5.9 / 8.9 here; transposed 8.1 / 10.7 and 5.2 / 7.6; 256 x 32, K = 1024 7.9 and 4.9.
+template <int FC, bool TA, bool CELL>
+__device__ __forceinline__ void narrow_body(const GemmArgs &g, const int logical) {
+  constexpr int CK = kNarrowK, SLAB = kNarrowSlab, NB = narrow_stages<FC>(), BN = 16 * FC;
+  using PX = Piece<CK, true, 16>;
+  static_assert(!(TA && CELL), "packed gate matrices are read as stored");
+  constexpr int kA = CK * 16, kStage = kA + FC * PX::kFloats;  // floats
+  constexpr int kLoadsA = kA / 256, kLoads = kLoadsA + FC * PX::kLoads;
+  const int splits = CELL ? 1 : g.splits, tile = logical / splits, split = logical % splits;
+  const int m0 = (tile / g.tiles_n) * 16, n0 = (tile % g.tiles_n) * BN;
+  const int cell0 = m0 / 4;  // CELL
+  const int tid = threadIdx.x, lane = tid % lh::kWave;
+  const int wk = __builtin_amdgcn_readfirstlane(tid / lh::kWave);
+  const int l16 = lane % 16, lq = lane / 16;
+  float *const ring = smem + wk * NB * kStage;
+  const unsigned ring_lds = (unsigned)(size_t)(__attribute__((address_space(3))) float *)ring;
+  const int M = g.M, N = g.N, H = g.cell_H;
+  auto pick = [](int seg, auto v0, auto v1, auto v2) __attribute__((always_inline)) {
+    return seg == 0 ? v0 : (seg == 1 ? v1 : v2);
+  };
+#define LH_SEG(FIELD, SEG) pick(SEG, g.FIELD[0], g.FIELD[1], g.FIELD[2])
+
+  // A unit of the ring's A rows: row `pos` of 16 floats is k = 16 (pos / 16) + 4 (pos % 4) + pos / 4 % 4, so that the
+  // four k of one MFMA step (4 apart, one per quarter of the wavefront) are neighbouring rows.
+  auto a_k = [](int u) __attribute__((always_inline)) { return (u / 64) * 16 + 4 * (u / 4 % 4) + u / 16 % 4; };
+  unsigned aoff[kLoadsA];
+  PX pa, px[FC];  // pa: TA only
+  const int slabs0 = (g.K[0] + SLAB - 1) / SLAB;
+  const int slabs1 = g.nseg > 1 ? (g.K[1] + SLAB - 1) / SLAB : 0;
+  const int slabs2 = g.nseg > 2 ? (g.K[2] + SLAB - 1) / SLAB : 0;
+  const int first = split * g.slabs_per_split;
+  const int total = min(g.slabs_per_split, slabs0 + slabs1 + slabs2 - first);
+  int lseg = 0, k0 = first, Ks = 0, lda = 0, ldx = 0;
+  if (k0 >= slabs0) {
+    k0 -= slabs0;
+    lseg = 1;
+    if (k0 >= slabs1) {
+      k0 -= slabs1;
+      lseg = 2;
+    }
+  }
+  k0 *= SLAB;
+  int cseg = lseg, ck = k0, step_a = 0;
+  bool new_seg = true;
+  const float *a = nullptr, *x = nullptr;
+  unsigned put = ring_lds;
+  auto request = [&]() __attribute__((always_inline)) {
+    if (new_seg) {
+      LH_KEEP_BRANCH();
+      Ks = LH_SEG(K, lseg);
+      if (lda != LH_SEG(lda, lseg) || ldx != LH_SEG(ldx, lseg)) {
+        LH_KEEP_BRANCH();
+        lda = LH_SEG(lda, lseg), ldx = LH_SEG(ldx, lseg);
+        if constexpr (TA) {
+          pa.set_ld(lda, lane, 0, M - m0);
+        } else {
+#pragma unroll
+          for (int i = 0; i < kLoadsA; ++i) {
+            const int u = lane + i * 64;
+            const unsigned off = (unsigned)(a_k(u) * lda + (u % 4) * 4) * 4u;
+            aoff[i] = CELL || (u % 4) * 4 < M - m0 ? off : 0u;  // (a packed block is padded)
+          }
+        }
+        step_a = TA ? SLAB : SLAB * lda;
+#pragma unroll
+        for (int c = 0; c < FC; ++c) px[c].set_ld(ldx, lane, 16 * c, N - n0);
+      }
+      const int k = k0 + wk * CK;
+      if constexpr (CELL)
+        a = LH_SEG(A, lseg) + ((size_t)(cell0 / kPackCells) * Ks + k) * kPackRows + cell0 % kPackCells * 4;
+      else a = LH_SEG(A, lseg) + (TA ? (size_t)m0 * lda + k : (size_t)k * lda + m0);
+      x = LH_SEG(X, lseg) + (size_t)n0 * ldx + k;
+    }
+    const int kn = Ks - k0 - wk * CK;
+    if (kn < CK) {
+      LH_KEEP_BRANCH();
+      if (kn <= 0) {
+        if constexpr (CELL)
+          a = LH_SEG(A, lseg) + (size_t)(cell0 / kPackCells) * Ks * kPackRows + cell0 % kPackCells * 4;
+        else a = LH_SEG(A, lseg) + (TA ? (size_t)m0 * lda : (size_t)m0);
+        x = LH_SEG(X, lseg) + (size_t)n0 * ldx;
+      }
+      if constexpr (TA) {
+        pa.load_tail(a, put, lda, lane, kn);
+      } else {
+#pragma unroll
+        for (int i = 0; i < kLoadsA; ++i) {
+          const int k = a_k(lane + i * 64);
+          const unsigned back = (unsigned)(k * lda) * 4u;
+          PX::load_unit(a, k < kn ? aoff[i] : (aoff[i] >= back ? aoff[i] - back : 0u), put + 1024u * i);
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < FC; ++c) px[c].load_tail(x, put + (kA + c * PX::kFloats) * 4u, ldx, lane, kn);
+    } else {
+      if constexpr (TA) {
+        pa.load(a, put);
+      } else {
+#pragma unroll
+        for (int i = 0; i < kLoadsA; ++i) PX::load_unit(a, aoff[i], put + 1024u * i);
+      }
+#pragma unroll
+      for (int c = 0; c < FC; ++c) px[c].load(x, put + (kA + c * PX::kFloats) * 4u);
+    }
+    put = put + kStage * 4u == ring_lds + NB * kStage * 4u ? ring_lds : put + kStage * 4u;
+    a += step_a;
+    x += SLAB;
+    k0 += SLAB;
+    new_seg = k0 >= Ks;
+    if (new_seg) {
+      ++lseg;
+      k0 = 0;
+    }
+  };
+
+  int issued = min(total, NB - 1);
+  for (int i = 0; i < issued; ++i) request();
+
+  // what the cell reads from memory
+  const int rl = tid % kNarrowCells, nl = tid / kNarrowCells;
+  const int r = cell0 + rl, n = n0 + nl;
+  const bool ep_ok = CELL && tid < kNarrowCells * BN && r < H && n < N;
+  float ep_add[4] = {0.f, 0.f, 0.f, 0.f}, ep_bias[4] = {0.f, 0.f, 0.f, 0.f}, ep_c = 0.f;
+  int ep_mask = 0;
+  if (ep_ok) {
+    int col = n;
+    if (g.addend_col) col = min(max(g.addend_col[n], 0), g.addend_ncols - 1);
+    const float *ad = g.C + (size_t)col * g.ldc + r;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (g.beta != 0.f) ep_add[q] = ad[(size_t)q * H];
+      ep_bias[q] = g.bias[q * H + r];
+    }
+    ep_c = g.c_prev[(size_t)n * H + r];
+    ep_mask = g.colmask[n];
+  }
+
+  floatx4 acc[FC];
+#pragma unroll
+  for (int c = 0; c < FC; ++c) acc[c] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const float *get = ring;
+  int cK = LH_SEG(K, cseg);
+  for (int s = 0; s < total; ++s) {
+    const int behind = issued - 1 - s;
+    if (NB > 3 && behind >= 2) wait_loads<kLoads * 2>();
+    else if (behind >= 1) wait_loads<kLoads>();
+    else wait_loads<0>();
+    float fa[CK / 16][4], fx[FC][CK / 16][4];
+#pragma unroll
+    for (int grp = 0; grp < CK / 16; ++grp) {
+#pragma unroll
+      for (int q = 0; q < 4 && !TA; ++q) fa[grp][q] = get[(16 * grp + 4 * q + lq) * 16 + l16];
+      if constexpr (TA) {
+        const float4 t = *reinterpret_cast<const float4 *>(get + (l16 * PX::U + ((4 * grp + lq) ^ PX::swizzle(l16))) * 4);
+        fa[grp][0] = t.x, fa[grp][1] = t.y, fa[grp][2] = t.z, fa[grp][3] = t.w;
+      }
+#pragma unroll
+      for (int c = 0; c < FC; ++c) {
+        const float4 t = *reinterpret_cast<const float4 *>(
+            get + kA + c * PX::kFloats + (l16 * PX::U + ((4 * grp + lq) ^ PX::swizzle(l16))) * 4);
+        fx[c][grp][0] = t.x, fx[c][grp][1] = t.y, fx[c][grp][2] = t.z, fx[c][grp][3] = t.w;
+      }
+    }
+    if (issued < total) {
+      request();
+      ++issued;
+    }
+    const int kn = cK - ck - wk * CK;
+    if (kn < CK) {
+      LH_KEEP_BRANCH();
+#pragma unroll
+      for (int grp = 0; grp < CK / 16; ++grp)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const bool in = 16 * grp + 4 * lq + q < kn;
+          fa[grp][q] = in ? fa[grp][q] : 0.f;
+#pragma unroll
+          for (int c = 0; c < FC; ++c) fx[c][grp][q] = in ? fx[c][grp][q] : 0.f;
+        }
+    }
+#pragma unroll
+    for (int grp = 0; grp < CK / 16; ++grp)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int c = 0; c < FC; ++c)
+          acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(fx[c][grp][q], fa[grp][q], acc[c], 0, 0, 0);
+    get = get + kStage == ring + NB * kStage ? ring : get + kStage;
+    ck += SLAB;
+    if (ck >= cK) {
+      LH_KEEP_BRANCH();
+      ck = 0;
+      ++cseg;
+      if (s + 1 < total) cK = LH_SEG(K, cseg);
+    }
+  }
+#undef LH_SEG
+
+  __syncthreads();  // all wavefronts have left their rings
+#pragma unroll
+  for (int c = 0; c < FC; ++c)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) smem[(wk * BN + 16 * c + 4 * lq + j) * kNarrowLd + l16] = acc[c][j];
+  __syncthreads();
+  if constexpr (!CELL) {
+    const bool partial = splits > 1;
+    const float alpha = partial ? 1.f : g.alpha, beta = partial ? 0.f : g.beta;
+    const int *const colmask = partial ? nullptr : g.colmask;
+    const float *const bias = partial ? nullptr : g.bias;
+    const int act_rows = partial || g.act != LH_ACT_TANH ? 0 : g.act_rows;
+    float *const Cb = partial ? g.ws_part + (size_t)split * g.ws_ld * N : g.C;
+    const int ldc = partial ? g.ws_ld : g.ldc;
+    const int m = m0 + tid % 16, nn = n0 + tid / 16;
+    if (tid >= 16 * BN || m >= M || nn >= N) return;
+    const float *src = smem + (tid / 16) * kNarrowLd + tid % 16;
+    float sum = src[0];
+#pragma unroll
+    for (int p = 1; p < 8; ++p) sum += src[p * BN * kNarrowLd];
+    float *cp = Cb + (size_t)nn * ldc + m;
+    float v = alpha * sum;
+    if (beta != 0.f) v += beta * *cp;
+    if (bias) v += bias[m];
+    if (m < act_rows) v = tanhf(v);
+    if (colmask) v *= (float)colmask[nn];
+    *cp = v;
+    return;
+  }
+  if (!ep_ok) return;
+  const float *src = smem + nl * kNarrowLd + rl * 4;
+  float4 sum = *reinterpret_cast<const float4 *>(src);
+#pragma unroll
+  for (int p = 1; p < 8; ++p) {
+    const float4 t = *reinterpret_cast<const float4 *>(src + p * BN * kNarrowLd);
+    sum.x += t.x, sum.y += t.y, sum.z += t.z, sum.w += t.w;
+  }
+  float pre[4] = {sum.x, sum.y, sum.z, sum.w};
+#pragma unroll
+  for (int q = 0; q < 4; ++q) pre[q] = (g.beta != 0.f ? pre[q] + ep_add[q] : pre[q]) + ep_bias[q];
+  store_cell(g, pre, ep_c, ep_mask, r, n);
+}
+
 template <int BM, int BN, int WM, int WN, int WK, int BK, bool TA, bool TX>
 __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_kernel(const GemmArgs g) {
-  gemm_body<BM, BN, WM, WN, WK, BK, TA, TX, false, false>(g, xcd_logical_id());
+  if constexpr (BM == 16) {
+    static_assert(WM * WN == 1 && WK == 8 && BK == kNarrowSlab && !TX, "the narrow form");
+    narrow_body<BN / 16, TA, false>(g, xcd_logical_id());
+  } else gemm_body<BM, BN, WM, WN, WK, BK, TA, TX, false, false>(g, xcd_logical_id());
 }
 
 // A kernel of its own for ragged operands, told apart by name.
@@ -1400,202 +1667,10 @@ __global__ __launch_bounds__(256) void gate_pack_kernel(const PackArgs p) {
   }
 }
 
-// ---- narrow form: packed gate product of at most a few 16-column blocks ------------------------
-// A tile of 16 rows (four cells) x 16 FC columns; the eight wavefronts share its k, 32 of every slab of 256
-// each, streamed like stream_body's.  What bounds a gate product of few columns is reading the weights: 32-row
-// tiles are 125 workgroups at 1000 hidden units, which leaves half the CUs idle, and the 32x32 MFMA multiplies
-// 32 columns whatever there are; these are 250 workgroups with the 16x16x4 MFMA at the same rate per column.
-// 1000 hidden units, K = 1000 / 2000, with cell: 12 columns 9.5 / 14.7 us on 32x32 tiles, 6.8 / 9.9 (16 and 32 MB of
-// weights, 5.3 TB/s beyond the fixed part); 32 columns 10.1 / 15.3 and 8.6 / 12.3; 256 hidden units, 12 columns, K = 512
-// 6.7 and 4.5.  At 2048 hidden units both read the weights at the same rate (16.8 us, K = 2048).
-constexpr int kNarrowK = 32, kNarrowSlab = 8 * kNarrowK, kNarrowCells = 4;
-constexpr int kNarrowLd = 20;  // floats between the columns of a partial block in LDS
-template <int FC>
-constexpr int narrow_stages() {
-  return FC == 1 ? 4 : 3;
-}
-template <int FC>
-constexpr int narrow_smem_floats() {
-  return cmax(narrow_stages<FC>() * kNarrowSlab * 16 * (1 + FC), 8 * 16 * FC * kNarrowLd);
-}
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-
+// The packed gate product in its narrow form.
 template <int FC>
 __global__ __launch_bounds__(512) void gate_gemm_narrow_kernel(const GemmArgs g) {
-  constexpr int CK = kNarrowK, SLAB = kNarrowSlab, NB = narrow_stages<FC>(), BN = 16 * FC;
-  using PX = Piece<CK, true, 16>;
-  constexpr int kA = CK * 16, kStage = kA + FC * PX::kFloats;  // floats
-  constexpr int kLoadsA = kA / 256, kLoads = kLoadsA + FC * PX::kLoads;
-  const int logical = xcd_logical_id();
-  const int cell0 = (logical / g.tiles_n) * kNarrowCells, n0 = (logical % g.tiles_n) * BN;
-  const int tid = threadIdx.x, lane = tid % lh::kWave;
-  const int wk = __builtin_amdgcn_readfirstlane(tid / lh::kWave);
-  const int l16 = lane % 16, lq = lane / 16;
-  float *const ring = smem + wk * NB * kStage;
-  const unsigned ring_lds = (unsigned)(size_t)(__attribute__((address_space(3))) float *)ring;
-  const int N = g.N, H = g.cell_H;
-  auto pick = [](int seg, auto v0, auto v1, auto v2) __attribute__((always_inline)) {
-    return seg == 0 ? v0 : (seg == 1 ? v1 : v2);
-  };
-#define LH_SEG(FIELD, SEG) pick(SEG, g.FIELD[0], g.FIELD[1], g.FIELD[2])
-
-  // A unit of the ring's A rows: row `pos` of 16 floats is k = 16 (pos / 16) + 4 (pos % 4) + pos / 4 % 4, so that the
-  // four k of one MFMA step (4 apart, one per quarter of the wavefront) are neighbouring rows.
-  auto a_k = [](int u) __attribute__((always_inline)) { return (u / 64) * 16 + 4 * (u / 4 % 4) + u / 16 % 4; };
-  unsigned aoff[kLoadsA];
-#pragma unroll
-  for (int i = 0; i < kLoadsA; ++i) {
-    const int u = lane + i * 64;
-    aoff[i] = (unsigned)(a_k(u) * kPackRows + (u % 4) * 4) * 4u;
-  }
-  PX px[FC];
-  int lseg = 0, k0 = 0, Ks = 0, ldx = 0;
-  bool new_seg = true;
-  const float *a = nullptr, *x = nullptr;
-  unsigned put = ring_lds;
-  auto request = [&]() __attribute__((always_inline)) {
-    if (new_seg) {
-      LH_KEEP_BRANCH();
-      Ks = LH_SEG(K, lseg);
-      if (ldx != LH_SEG(ldx, lseg)) {
-        LH_KEEP_BRANCH();
-        ldx = LH_SEG(ldx, lseg);
-#pragma unroll
-        for (int c = 0; c < FC; ++c) px[c].set_ld(ldx, lane, 16 * c, N - n0);
-      }
-      const int k = k0 + wk * CK;
-      a = LH_SEG(A, lseg) + ((size_t)(cell0 / kPackCells) * Ks + k) * kPackRows + cell0 % kPackCells * 4;
-      x = LH_SEG(X, lseg) + (size_t)n0 * ldx + k;
-    }
-    const int kn = Ks - k0 - wk * CK;
-    if (kn < CK) {
-      LH_KEEP_BRANCH();
-      if (kn <= 0) {
-        a = LH_SEG(A, lseg) + (size_t)(cell0 / kPackCells) * Ks * kPackRows + cell0 % kPackCells * 4;
-        x = LH_SEG(X, lseg) + (size_t)n0 * ldx;
-      }
-#pragma unroll
-      for (int i = 0; i < kLoadsA; ++i) {
-        const int k = a_k(lane + i * 64);
-        PX::load_unit(a, k < kn ? aoff[i] : aoff[i] - (unsigned)(k * kPackRows) * 4u, put + 1024u * i);
-      }
-#pragma unroll
-      for (int c = 0; c < FC; ++c) px[c].load_tail(x, put + (kA + c * PX::kFloats) * 4u, ldx, lane, kn);
-    } else {
-#pragma unroll
-      for (int i = 0; i < kLoadsA; ++i) PX::load_unit(a, aoff[i], put + 1024u * i);
-#pragma unroll
-      for (int c = 0; c < FC; ++c) px[c].load(x, put + (kA + c * PX::kFloats) * 4u);
-    }
-    put = put + kStage * 4u == ring_lds + NB * kStage * 4u ? ring_lds : put + kStage * 4u;
-    a += SLAB * kPackRows;
-    x += SLAB;
-    k0 += SLAB;
-    new_seg = k0 >= Ks;
-    if (new_seg) {
-      ++lseg;
-      k0 = 0;
-    }
-  };
-
-  const int total = g.slabs_per_split;
-  int issued = min(total, NB - 1);
-  for (int i = 0; i < issued; ++i) request();
-
-  // what the cell reads from memory
-  const int rl = tid % kNarrowCells, nl = tid / kNarrowCells;
-  const int r = cell0 + rl, n = n0 + nl;
-  const bool ep_ok = tid < kNarrowCells * BN && r < H && n < N;
-  float ep_add[4] = {0.f, 0.f, 0.f, 0.f}, ep_bias[4] = {0.f, 0.f, 0.f, 0.f}, ep_c = 0.f;
-  int ep_mask = 0;
-  if (ep_ok) {
-    int col = n;
-    if (g.addend_col) col = min(max(g.addend_col[n], 0), g.addend_ncols - 1);
-    const float *ad = g.C + (size_t)col * g.ldc + r;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      if (g.beta != 0.f) ep_add[q] = ad[(size_t)q * H];
-      ep_bias[q] = g.bias[q * H + r];
-    }
-    ep_c = g.c_prev[(size_t)n * H + r];
-    ep_mask = g.colmask[n];
-  }
-
-  floatx4 acc[FC];
-#pragma unroll
-  for (int c = 0; c < FC; ++c) acc[c] = floatx4{0.f, 0.f, 0.f, 0.f};
-  const float *get = ring;
-  int cseg = 0, ck = 0, cK = LH_SEG(K, 0);
-  for (int s = 0; s < total; ++s) {
-    const int behind = issued - 1 - s;
-    if (NB > 3 && behind >= 2) wait_loads<kLoads * 2>();
-    else if (behind >= 1) wait_loads<kLoads>();
-    else wait_loads<0>();
-    float fa[CK / 16][4], fx[FC][CK / 16][4];
-#pragma unroll
-    for (int grp = 0; grp < CK / 16; ++grp) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) fa[grp][q] = get[(16 * grp + 4 * q + lq) * 16 + l16];
-#pragma unroll
-      for (int c = 0; c < FC; ++c) {
-        const float4 t = *reinterpret_cast<const float4 *>(
-            get + kA + c * PX::kFloats + (l16 * PX::U + ((4 * grp + lq) ^ PX::swizzle(l16))) * 4);
-        fx[c][grp][0] = t.x, fx[c][grp][1] = t.y, fx[c][grp][2] = t.z, fx[c][grp][3] = t.w;
-      }
-    }
-    if (issued < total) {
-      request();
-      ++issued;
-    }
-    const int kn = cK - ck - wk * CK;
-    if (kn < CK) {
-      LH_KEEP_BRANCH();
-#pragma unroll
-      for (int grp = 0; grp < CK / 16; ++grp)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const bool in = 16 * grp + 4 * lq + q < kn;
-          fa[grp][q] = in ? fa[grp][q] : 0.f;
-#pragma unroll
-          for (int c = 0; c < FC; ++c) fx[c][grp][q] = in ? fx[c][grp][q] : 0.f;
-        }
-    }
-#pragma unroll
-    for (int grp = 0; grp < CK / 16; ++grp)
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int c = 0; c < FC; ++c)
-          acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(fx[c][grp][q], fa[grp][q], acc[c], 0, 0, 0);
-    get = get + kStage == ring + NB * kStage ? ring : get + kStage;
-    ck += SLAB;
-    if (ck >= cK) {
-      LH_KEEP_BRANCH();
-      ck = 0;
-      ++cseg;
-      if (s + 1 < total) cK = LH_SEG(K, cseg);
-    }
-  }
-#undef LH_SEG
-
-  __syncthreads();  // all wavefronts have left their rings
-#pragma unroll
-  for (int c = 0; c < FC; ++c)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) smem[(wk * BN + 16 * c + 4 * lq + j) * kNarrowLd + l16] = acc[c][j];
-  __syncthreads();
-  if (!ep_ok) return;
-  const float *src = smem + nl * kNarrowLd + rl * 4;
-  float4 sum = *reinterpret_cast<const float4 *>(src);
-#pragma unroll
-  for (int p = 1; p < 8; ++p) {
-    const float4 t = *reinterpret_cast<const float4 *>(src + p * BN * kNarrowLd);
-    sum.x += t.x, sum.y += t.y, sum.z += t.z, sum.w += t.w;
-  }
-  float pre[4] = {sum.x, sum.y, sum.z, sum.w};
-#pragma unroll
-  for (int q = 0; q < 4; ++q) pre[q] = (g.beta != 0.f ? pre[q] + ep_add[q] : pre[q]) + ep_bias[q];
-  store_cell(g, pre, ep_c, ep_mask, r, n);
+  narrow_body<FC, false, true>(g, xcd_logical_id());
 }
 
 // Several stacked gate products of one decoding step in ONE launch: everything that is known when
@@ -1779,6 +1854,16 @@ int launch_kernel(KernelT kernel, int smem_bytes, dim3 grid, dim3 block, hipStre
   return lh::check_launch("lh_gemm_f32");
 }
 
+// The sum of the partial planes of a split product.
+int launch_reduce(const GemmArgs &g, hipStream_t st) {
+  // four rows per thread; small products in single-wavefront workgroups, to reach more CUs
+  const size_t total = (size_t)(g.ws_ld / 4) * g.N;
+  const unsigned nt = total < 65536 ? 64 : 256;
+  const size_t blocks = (total + nt - 1) / nt;
+  hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)(blocks < 8192 ? blocks : 8192)), dim3(nt), 0, st, g);
+  return lh::check_launch("lh_gemm_ws_f32 split reduction");
+}
+
 // What takes a product: the scalar kernel, the main kernel for aligned operands, or its form for
 // ragged ones.
 enum Form { kGeneric, kRagged, kAligned };
@@ -1818,13 +1903,7 @@ int launch_cfg(const GemmArgs &g0, bool ta, bool tx, Form form, hipStream_t st) 
 #undef LH_GEMM_LAUNCH
     }
     if (rc != LH_OK || g.splits == 1 || g.leave_partial) return rc;
-    // four rows per thread; small products in single-wavefront workgroups, to reach more CUs
-    const size_t total = (size_t)(g.ws_ld / 4) * g.N;
-    const unsigned nt = total < 65536 ? 64 : 256;
-    const size_t blocks = (total + nt - 1) / nt;
-    hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)(blocks < 8192 ? blocks : 8192)),
-                       dim3(nt), 0, st, g);
-    return lh::check_launch("lh_gemm_ws_f32 split reduction");
+    return launch_reduce(g, st);
   }
   if constexpr (ALLOW_UNALIGNED) {
     constexpr int bytes = smem_floats<BM, BN, WK, BK>() * 4;
@@ -1838,7 +1917,26 @@ int launch_cfg(const GemmArgs &g0, bool ta, bool tx, Form form, hipStream_t st) 
   return lh::fail_arg("lh_gemm_f32: internal error, unaligned operands reached an aligned-only tile");
 }
 
+template <int FC>
+int launch_narrow_gemm(const GemmArgs &g0, bool ta, hipStream_t st) {
+  GemmArgs g = g0;
+  g.tiles_m = (g.M + 15) / 16;
+  g.tiles_n = (g.N + 16 * FC - 1) / (16 * FC);
+  int slabs = 0;
+  for (int s = 0; s < g.nseg; ++s) slabs += (g.K[s] + kNarrowSlab - 1) / kNarrowSlab;
+  g.slabs_per_split = (slabs + g.splits - 1) / g.splits;
+  g.splits = (slabs + g.slabs_per_split - 1) / g.slabs_per_split;  // no empty share
+  const dim3 grid(g.tiles_m * g.tiles_n * g.splits);
+  const int rc = ta ? launch_kernel((GemmKernel)gemm_kernel<16, 16 * FC, 1, 1, 8, kNarrowSlab, true, false>,
+                                    narrow_smem_floats<FC>() * 4, grid, dim3(512), st, g)
+                    : launch_kernel((GemmKernel)gemm_kernel<16, 16 * FC, 1, 1, 8, kNarrowSlab, false, false>,
+                                    narrow_smem_floats<FC>() * 4, grid, dim3(512), st, g);
+  return rc != LH_OK || g.splits == 1 || g.leave_partial ? rc : launch_reduce(g, st);
+}
+
 int launch_index(int c, const GemmArgs &g, bool ta, bool tx, Form form, hipStream_t st) {
+  if (c == kNumConfigs) return launch_narrow_gemm<1>(g, ta, st);
+  if (c == kNumConfigs + 1) return launch_narrow_gemm<2>(g, ta, st);
   switch (c) {
 #define LH_CFG_CASE(I, BM, BN, WM, WN, WK, BK) \
   case I:                                      \
@@ -2007,6 +2105,15 @@ constexpr int kCUs = 256;
 constexpr float kReduceFixedUs = 3.5f, kReducePlaneUs = 0.22f, kReduceBytesPerUs = 3.0e6f;
 constexpr float kCellFixedUs = 4.0f;  // a launch of the LSTM cell kernel behind its product
 
+// The narrow forms, numbered behind the configurations of the table, with rows of their own in the cost model (gate
+// product: fitted at 256 and 1000 hidden units, weights from HBM; plain products: 1000 rows; one workgroup per CU).
+// They are not among the configurations that an override names.
+const Config kNarrow[] = {{16, 16, 1, 1, 8, kNarrowSlab}, {16, 32, 1, 1, 8, kNarrowSlab}};
+const Tuning kNarrowCell[] = {{1, 3.7f, 0.0031f, 3.7f, 0.0031f}, {1, 4.2f, 0.0040f, 4.2f, 0.0040f}};
+const Tuning kNarrowPlain[] = {{1, 3.2f, 0.0025f, 3.2f, 0.0025f}, {1, 4.0f, 0.0033f, 4.0f, 0.0033f}};
+constexpr int kNumNarrow = 2;
+const Config &config_at(int c) { return c < kNumConfigs ? kConfigs[c] : kNarrow[c - kNumConfigs]; }
+
 float predict_us(const Tuning &t, const Config &k, int M, int N, const int *K, int nseg, int want,
                  bool reduce_free, int *splits) {
   const long long tiles = (long long)((M + k.bm - 1) / k.bm) * ((N + k.bn - 1) / k.bn);
@@ -2083,8 +2190,10 @@ void pick_config(int M, int N, const int *K, int nseg, bool ta, bool tx, Form fo
   const Tuning *table = kTuning[only_cell ? 3 : (ta ? 1 : (tx ? 2 : 0))];
   float best = 3.0e38f;
   *config = kUnalignedConfig;
-  for (int c = 0; c < kNumConfigs; ++c) {
+  for (int c = 0; c < kNumConfigs + kNumNarrow; ++c) {
     if (g_config_override >= 0 && c != g_config_override) continue;
+    const bool narrow = c >= kNumConfigs;
+    if (narrow && (only_cell || tx || form != kAligned)) break;
     if (only_cell && !cell_capable_index(c)) continue;
     if (form == kRagged && (!ragged_config(c) || kConfigs[c].bm > max_bm || kConfigs[c].bn > max_bn)) continue;
     for (int want : kSplitChoices) {
@@ -2093,7 +2202,7 @@ void pick_config(int M, int N, const int *K, int nseg, bool ta, bool tx, Form fo
       if (max_planes > 0 && want > max_planes) want = max_planes;
       if (want > 1 && fit_splits(M, N, want, workspace_bytes) < want) break;
       int S;
-      float us = predict_us(table[c], kConfigs[c], M, N, K, nseg, want, max_planes > 0, &S);
+      float us = predict_us(narrow ? kNarrowPlain[c - kNumConfigs] : table[c], config_at(c), M, N, K, nseg, want, max_planes > 0, &S);
       // an override asks for this many shares: too few slabs for them only where no other choice has enough
       if (g_splits_override > 0 && S < want) us += 1.0e6f;
       if (us < best) {
@@ -2108,13 +2217,6 @@ void pick_config(int M, int N, const int *K, int nseg, bool ta, bool tx, Form fo
   if (us_out) *us_out = best;
   e = Memo{M, N, {Kk[0], Kk[1], Kk[2]}, flags, *config, *splits, workspace_bytes, best};
 }
-
-// The narrow forms of the packed gate product, after the configurations of the table in pick_packed's
-// numbering, with rows of their own in the cost model (fitted at 256 and 1000 hidden units, weights from HBM; one
-// workgroup per CU).  They are not among the configurations that an override names.
-const Config kNarrow[] = {{16, 16, 1, 1, 8, kNarrowSlab}, {16, 32, 1, 1, 8, kNarrowSlab}};
-const Tuning kNarrowTuning[] = {{1, 3.7f, 0.0031f, 3.7f, 0.0031f}, {1, 4.2f, 0.0040f, 4.2f, 0.0040f}};
-constexpr int kNumNarrow = 2;
 
 // The packed gate product's configuration and predicted time (fifth table).
 void pick_packed(int H, int B, const int *K, int nseg, int *config, float *us) {
@@ -2134,7 +2236,7 @@ void pick_packed(int H, int B, const int *K, int nseg, int *config, float *us) {
   }
   for (int i = 0; i < kNumNarrow && g_config_override < 0; ++i) {
     int S;
-    const float t = predict_us(kNarrowTuning[i], kNarrow[i], 4 * H, B, K, nseg, 1, false, &S);
+    const float t = predict_us(kNarrowCell[i], kNarrow[i], 4 * H, B, K, nseg, 1, false, &S);
     if (t < *us) *us = t, *config = kNumConfigs + i;
   }
 }
@@ -2252,7 +2354,7 @@ extern "C" int lh_gemm_planes_f32(int M, int N, const lh_gemm_seg *segs, int nse
                          nullptr, C, ldc, workspace, workspace_bytes, max_planes, &p);
   if (rc != LH_OK) return rc;
   // the split the launch will really use (no empty share), as launch_cfg computes it
-  const Config &k = kConfigs[p.config];
+  const Config &k = config_at(p.config);
   int slabs = 0;
   for (int s = 0; s < p.g.nseg; ++s) slabs += (p.g.K[s] + k.bk - 1) / k.bk;
   const int want = p.form != kGeneric ? p.g.splits : 1;
@@ -2309,7 +2411,7 @@ extern "C" int lh_gate_gemm_lstm_cell_plan(int H, int B, const lh_gemm_seg *segs
   if (rc != LH_OK) return rc;
   *fusable = f ? 1 : 0;
   if (name && name_cap > 0) {
-    const Config &k = kConfigs[p.config];
+    const Config &k = config_at(p.config);
     if (f) snprintf(name, name_cap, "gate_gemm_cell_kernel<%d, %d, %d, %d, %d, %d>", k.bm, k.bn, k.wm, k.wn, k.wk, k.bk);
     else name[0] = 0;
   }
@@ -2813,7 +2915,7 @@ extern "C" int lh_gemm_kernel_name(int M, int N, const lh_gemm_seg *segs, int ns
                          nullptr, &dummy, M, workspace_bytes ? (void *)(uintptr_t)256 : nullptr,
                          workspace_bytes, max_planes, &p);
   if (rc != LH_OK) return rc;
-  const Config &k = kConfigs[p.config];
+  const Config &k = config_at(p.config);
   if (p.form != kGeneric)
     snprintf(name, name_cap, "gemm_kernel<%d, %d, %d, %d, %d, %d, %s, %s%s>", k.bm, k.bn, k.wm, k.wn,
              k.wk, k.bk, p.ta ? "true" : "false", p.tx ? "true" : "false", p.form == kRagged ? ", true" : "");

@@ -25,6 +25,21 @@ def operand(torch, rows, cols, pad, seed):
     return full, full[:, :rows].T.double()
 
 
+@pytest.mark.parametrize("tA", [False, True], ids=["NN", "TN"])
+@pytest.mark.parametrize("M,N,Ks,splits", [
+    (20, 12, (260,), 1), (256, 24, (1024, 28), 1), (100, 33, (512, 36, 292), 1), (996, 64, (1000,), 1),
+    (1000, 128, (1000, 4), 1), (200, 36, (1000,), 2)])
+def test_narrow_product_matches_float64(lh, tA, M, N, Ks, splits):
+    """Tiles of 16 rows and 16 or 32 columns, which no override names: chosen at these sizes."""
+    import torch
+    lh.load().lh_gemm_set_splits_override(splits)
+    any_matrix = torch.empty(max(M, N) * 2048, device="cuda")
+    segs = [(any_matrix, 2048, any_matrix, 2048, K) for K in Ks]
+    name = lh.gemm_kernel_name(M, N, segs, tA, False, 64 * M * N)
+    assert name.startswith("gemm_kernel<16, %d," % (32 if N == 128 else 16)), name
+    test_streamed_product_matches_float64(lh, -1, tA, False, M, N, Ks, splits)
+
+
 @pytest.mark.parametrize("config", CONFIGS)
 @pytest.mark.parametrize("tA,tX", [(False, False), (True, False), (False, True)], ids=["NN", "TN", "NT"])
 @pytest.mark.parametrize("M,N,Ks,splits", [

@@ -2103,7 +2103,9 @@ constexpr int kCUs = 256;
 // The pass over S partial planes: 4.3 to 4.8 us of 4 planes between other kernels of a stream (1000 x 64 to 2048 x 256),
 // 2.1, 2.6 and 3.8 us of 2, 4 and 8 planes of 1000 x 5 and 1.4 us less a launch when replayed from a graph.
 constexpr float kReduceFixedUs = 3.5f, kReducePlaneUs = 0.22f, kReduceBytesPerUs = 3.0e6f;
-constexpr float kCellFixedUs = 4.0f;  // a launch of the LSTM cell kernel behind its product
+// A launch of the LSTM cell kernel behind its product: 4.1 to 4.7 us between other kernels at 12 columns, 7.2 and a
+// lookup of 4.6 where the addend is a column of the embedding table.
+constexpr float kCellFixedUs = 6.0f;
 
 // The narrow forms, numbered behind the configurations of the table, with rows of their own in the cost model (gate
 // product: fitted at 256 and 1000 hidden units, weights from HBM; plain products: 1000 rows; one workgroup per CU).
@@ -2152,7 +2154,7 @@ float predict_us(const Tuning &t, const Config &k, int M, int N, const int *K, i
 void pick_config(int M, int N, const int *K, int nseg, bool ta, bool tx, Form form,
                  size_t workspace_bytes, int max_planes, int *config, int *splits,
                  bool only_cell = false, float *us_out = nullptr, int max_bm = INT_MAX,
-                 int max_bn = INT_MAX) {
+                 int max_bn = INT_MAX, bool allow_narrow = true) {
   *splits = 1;
   if (us_out) *us_out = 0.f;
   if (form == kGeneric) {
@@ -2169,7 +2171,7 @@ void pick_config(int M, int N, const int *K, int nseg, bool ta, bool tx, Form fo
   const int flags = 1 + (ta ? 2 : 0) + (tx ? 4 : 0) + 8 * nseg + 64 * (g_config_override + 1) +
                     4096 * g_splits_override + 131072 * max_planes + (only_cell ? 1048576 : 0) +
                     (max_bm <= M ? 2097152 : 0) + (max_bn <= N ? 4194304 : 0) +
-                    (form == kRagged ? 8388608 : 0);
+                    (form == kRagged ? 8388608 : 0) + (allow_narrow ? 16777216 : 0);
   int Kk[LH_GEMM_MAX_SEGS] = {0, 0, 0};
   for (int s = 0; s < nseg; ++s) Kk[s] = K[s];
   // Every field into every bit of the slot: the two questions a gate product asks (any launch; an unsplit
@@ -2193,7 +2195,7 @@ void pick_config(int M, int N, const int *K, int nseg, bool ta, bool tx, Form fo
   for (int c = 0; c < kNumConfigs + kNumNarrow; ++c) {
     if (g_config_override >= 0 && c != g_config_override) continue;
     const bool narrow = c >= kNumConfigs;
-    if (narrow && (only_cell || tx || form != kAligned)) break;
+    if (narrow && (!allow_narrow || only_cell || tx || form != kAligned)) break;
     if (only_cell && !cell_capable_index(c)) continue;
     if (form == kRagged && (!ragged_config(c) || kConfigs[c].bm > max_bm || kConfigs[c].bn > max_bn)) continue;
     for (int want : kSplitChoices) {
@@ -2385,8 +2387,10 @@ int plan_cell(int H, int B, const lh_gemm_seg *segs, int nseg, bool has_addend, 
   int cfg_any, splits_any, cfg_cell, splits_cell;
   float us_any, us_cell;
   const size_t ws = workspace_bytes;
+  // (a product in the narrow form and its cell would often win here: its place is the packed gate product, which
+  // is that form with the cell inside; this plan is for callers without packed matrices, one launch a step)
   pick_config(4 * H, B, p->g.K, nseg, false, false, kAligned, ws, has_addend ? 2 : 3, &cfg_any, &splits_any,
-              false, &us_any);
+              false, &us_any, INT_MAX, INT_MAX, false);
   pick_config(4 * H, B, p->g.K, nseg, false, false, kAligned, ws, has_addend ? 2 : 3, &cfg_cell,
               &splits_cell, true, &us_cell);
   if (cfg_cell < 0) return LH_OK;

@@ -211,7 +211,8 @@ class LstmLayer {
   // stored ones: made by the first step that runs faster on it, made anew after a change of the weights.
   // M is not among them where it never is an operand of a step's product (the input layer).  A model whose
   // memory does not hold the copies runs on the stored matrices.
-  DeviceArray<float> packed_m_, packed_w_h_, packed_q_;
+  DeviceArray<float> packed_;  // one array: the copies of M, W_h and Q, null pointers where there is none
+  const float *packed_m_ = nullptr, *packed_w_h_ = nullptr, *packed_q_ = nullptr;
   bool packed_dirty_ = true, packed_possible_ = true;
   bool PackGates();  // false: no memory
   void ForwardPropInputAllSteps(int steps);

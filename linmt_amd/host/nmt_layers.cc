@@ -111,6 +111,7 @@ void LstmLayer::Init(NeuralMachineTranslation *model, bool input_layer, bool sou
 
 void LstmLayer::InitFeedInput() {
   feed_input_mode_ = true;
+  packed_dirty_ = true;  // Q joins the packed matrices
   p_device_q_stack_.Alloc(4 * (size_t)lstm_size_ * lstm_size_);
   p_device_q_stack_.Zero(p_neural_mt_->stream_);
   if (p_neural_mt_->cfg_.train_mode_ && keep_gates_) {
@@ -242,24 +243,26 @@ bool LstmLayer::PackGates() {
   if (!packed_possible_) return false;
   if (!packed_dirty_) return true;
   const int H = lstm_size_;
-  DeviceArray<float> *to[3] = {&packed_m_, &packed_w_h_, &packed_q_};
+  const float **to[3] = {&packed_m_, &packed_w_h_, &packed_q_};
   DeviceArray<float> *from[3] = {&p_device_m_stack_, &p_device_w_h_stack_, &p_device_q_stack_};
   const int K[3] = {input_layer_mode_ ? 0 : input_size_, H, feed_input_mode_ ? H : 0};
+  size_t floats = 0;
+  for (int k : K) floats += lh_gate_pack_floats(H, k);
+  if (packed_.size() != floats) {
+    try {
+      packed_.Alloc(floats);
+    } catch (const std::exception &) {
+      packed_possible_ = false;
+      return false;
+    }
+  }
   lh_gate_pack_source src[3];
   int n = 0;
+  float *at = packed_.get();
   for (int i = 0; i < 3; ++i) {
-    if (!K[i]) continue;
-    const size_t floats = lh_gate_pack_floats(H, K[i]);
-    if (to[i]->size() != floats) {
-      try {
-        to[i]->Alloc(floats);
-      } catch (const std::exception &) {
-        for (DeviceArray<float> *a : to) a->Free();
-        packed_possible_ = false;
-        return false;
-      }
-    }
-    src[n++] = lh_gate_pack_source{from[i]->get(), 4 * H, K[i], to[i]->get()};
+    *to[i] = K[i] ? at : nullptr;
+    if (K[i]) src[n++] = lh_gate_pack_source{from[i]->get(), 4 * H, K[i], at};
+    at += lh_gate_pack_floats(H, K[i]);
   }
   LhErrorWrapper(lh_gate_pack_f32(H, src, n, p_neural_mt_->stream_), "LstmLayer::PackGates");
   packed_dirty_ = false;
@@ -362,9 +365,9 @@ void LstmNode::ForwardProp() {
       double k = 0;
       for (int i = 0; i < nseg; ++i) {
         k += segs[i].K;
-        segs[i].A = segs[i].A == L.p_device_m_stack_.get()     ? L.packed_m_.get()
-                    : segs[i].A == L.p_device_w_h_stack_.get() ? L.packed_w_h_.get()
-                                                               : L.packed_q_.get();
+        segs[i].A = segs[i].A == L.p_device_m_stack_.get()     ? L.packed_m_
+                    : segs[i].A == L.p_device_w_h_stack_.get() ? L.packed_w_h_
+                                                               : L.packed_q_;
       }
       ProfileScope ps(M.profiler_, kTagGateGemm, name, 2.0 * 4 * H * (double)B * k);
       LhErrorWrapper(lh_gate_gemm_lstm_cell_packed_f32(

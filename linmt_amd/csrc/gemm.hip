@@ -17,6 +17,8 @@
 //    its epilogue, gemm_kernel<..., true> (a ninth template argument) the same body for operands at any
 //    float's address and with extents that are no multiple of 4.
 //    Tiles of eight 32x32 blocks (products of few columns) run its streamed form, stream_body.
+//    Tiles of 16 rows (narrow_body) and packed gate matrices (gate_gemm_packed_kernel, gate_gemm_narrow_kernel) are
+//    for fewer columns still.
 //  * gemm_generic_kernel (a ragged extent shorter than a copy or a tile, one slab of k): scalar loads, one
 //    tile shape.
 // WK > 1 splits every slab's k range over WK wavefront groups and reduces the partial

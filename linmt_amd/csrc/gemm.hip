@@ -2130,7 +2130,9 @@ float predict_us(const Tuning &t, const Config &k, int M, int N, const int *K, i
   // Workgroups per CU: dispatch is dynamic, so a fractional load costs less than a whole extra
   // round but leaves a tail of about half a workgroup.
   const float per_cu = (float)(tiles * S) / kCUs;
-  const float load = fminf(per_cu + 0.5f, ceilf(per_cu));
+  // Two streamed workgroups on a CU do not finish one after the other: 1400 x 192, K = 2800 (264 of them) 30.5 us, 26.1 on
+  // the 64x64 tiles that a fractional load would have passed over.
+  const float load = k.bm * k.bn == 1024 && k.bk == 64 ? ceilf(per_cu) : fminf(per_cu + 0.5f, ceilf(per_cu));
   // (both are fitted at depths of 512 and 4096: below, several workgroups could come out cheaper than one)
   const float t1 = t.f1 + t.s1 * depth, full = t.focc + t.socc * depth;
   const float tocc = t.occ > 1 ? fmaxf(t1, full) : full;
@@ -2189,6 +2191,8 @@ void pick_config(int M, int N, const int *K, int nseg, bool ta, bool tx, Form fo
     if (us_out) *us_out = e.us;
     return;
   }
+  float k_sum = 0.f;
+  for (int s = 0; s < nseg; ++s) k_sum += (float)K[s];
   static const int kSplitChoices[] = {1, 2, 3, 4, 6, 8, 12, 16};
   // the fourth table is measured on the kernel that carries the LSTM cell in its epilogue
   const Tuning *table = kTuning[only_cell ? 3 : (ta ? 1 : (tx ? 2 : 0))];
@@ -2199,6 +2203,12 @@ void pick_config(int M, int N, const int *K, int nseg, bool ta, bool tx, Form fo
     const bool narrow = c >= kNumConfigs;
     if (narrow && (!allow_narrow || only_cell || tx || form != kAligned)) break;
     if (only_cell && !cell_capable_index(c)) continue;
+    // An A beyond 48 MB comes from HBM at every use, which the table (operands in the L2s) does not show, and the
+    // streamed tiles are not the best there: transposed 2048 x 64, K = 8192 33.6 us (32x32) and 33.9 (32x64) against 30.5
+    // on staged 64x64, 2048 x 128 47.5 and 45.1; at 33 MB (K = 4096) they are ahead, 23 and 27.
+    if (!only_cell && !narrow && g_config_override < 0 && form == kAligned && N > 32 &&
+        4.f * (float)M * k_sum > 48.0e6f && packed_config(c))
+      continue;
     if (form == kRagged && (!ragged_config(c) || kConfigs[c].bm > max_bm || kConfigs[c].bn > max_bn)) continue;
     for (int want : kSplitChoices) {
       if (only_cell && want > 1) break;
@@ -2549,7 +2559,12 @@ extern "C" int lh_gate_gemm_lstm_cell_packed_plan(int H, int B, const lh_gemm_se
   if (c < 0) return LH_OK;
   pick_config(4 * H, B, p.g.K, nseg, false, false, kAligned, workspace_bytes, has_addend ? 2 : 3, &c0, &S, f, &us0);
   if (!f) us0 += kCellFixedUs + 28.f * (float)H * (float)B / kReduceBytesPerUs;
-  if (us > us0) return LH_OK;
+  // More workgroups than CUs: the rounds overlap less than the model has it, and the wider staged tiles read less.  2048
+  // hidden units, 96 / 128 / 192 columns, K = 4096: 88.6 / 92.8 / 126.6 us packed, 84.4 / 82.6 / 122.6 not; with at most one
+  // workgroup per CU the packed form is ahead (64 columns: 47.3 and 60.9).
+  const Config &pk = config_at(c);
+  const long long groups = (long long)((4 * H + pk.bm - 1) / pk.bm) * ((B + pk.bn - 1) / pk.bn);
+  if (us > us0 || groups > kCUs) return LH_OK;
   *faster = 1;
   if (name && name_cap > 0) {
     const Config &k = kConfigs[c < kNumConfigs ? c : 0];

@@ -261,8 +261,9 @@ int lh_gemm_kernel_name(int M, int N, const lh_gemm_seg *segs, int nseg, int tra
 /* Tuning and test aids (no counterpart in the reference).  Both overrides belong to the CALLING
  * THREAD: they change nothing for lh_gemm_* calls made from other host threads.
  * lh_gemm_set_config_override: forces tile configuration `config` for every later lh_gemm_* call
- * of this thread, config < 0 restores the built-in choice.  Returns the number of configurations
- * (so 0 <= config < return value), LH_ERR_ARG if config is too large.
+ * of this thread, config < 0 restores the built-in choice.  Returns the number n of configurations
+ * (so 0 <= config < n; n and n + 1 name the narrow forms of 16 x 16 and 16 x 32 tiles, which take aligned
+ * operands with X not transposed, and packed gate products), LH_ERR_ARG if config is too large.
  * lh_gemm_set_splits_override: likewise forces the K split of lh_gemm_ws_f32 (as far as the
  * workspace allows), splits <= 0 restores the built-in choice; returns the largest split.
  * lh_gemm_config_info: info = {BM, BN, WM, WN, WK, BK, workgroups resident per CU, LDS bytes} of a

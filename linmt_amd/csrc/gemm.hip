@@ -1822,6 +1822,10 @@ const Config kConfigs[] = {LH_GEMM_CONFIGS(LH_CFG_ENTRY)};
 #undef LH_CFG_ENTRY
 constexpr int kNumConfigs = sizeof(kConfigs) / sizeof(kConfigs[0]);
 constexpr int kUnalignedConfig = 7;
+// The narrow forms, numbered behind them.
+const Config kNarrow[] = {{16, 16, 1, 1, 8, kNarrowSlab}, {16, 32, 1, 1, 8, kNarrowSlab}};
+constexpr int kNumNarrow = sizeof(kNarrow) / sizeof(kNarrow[0]);
+const Config &config_at(int c) { return c < kNumConfigs ? kConfigs[c] : kNarrow[c - kNumConfigs]; }
 // Configurations built for ragged operands as well: those that the cost model gives an aligned output
 // projection and its backward products at 5 to 2560 columns of 5000 to 30000 words, or one within
 // a few per cent of them.
@@ -2037,24 +2041,11 @@ bool cell_capable_index(int c) {
   }
 }
 
-template <int BM, int BN, int WM, int WN, int WK, int BK>
-int occupancy_cfg(bool ta, bool tx, int *blocks_per_cu, int *lds_bytes) {
-  constexpr int block = 64 * WM * WN * WK;
-  hipError_t e;
-#define LH_GEMM_OCC(TA, TX)                                                                       \
-  do {                                                                                            \
-    constexpr int bytes = smem2_floats<BM, BN, WM, WN, WK, BK, TA, TX>() * 4;                     \
-    *lds_bytes = bytes;                                                                           \
-    GemmKernel kernel = gemm_kernel<BM, BN, WM, WN, WK, BK, TA, TX>;                              \
-    if (bytes > 64 * 1024)                                                                        \
-      (void)hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, \
-                                bytes);                                                           \
-    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, kernel, block, bytes);        \
-  } while (0)
-  if (!ta && !tx) LH_GEMM_OCC(false, false);
-  else if (ta) LH_GEMM_OCC(true, false);
-  else LH_GEMM_OCC(false, true);
-#undef LH_GEMM_OCC
+int occupancy(GemmKernel kernel, int block, int bytes, int *blocks_per_cu, int *lds_bytes) {
+  *lds_bytes = bytes;
+  if (bytes > 64 * 1024)
+    (void)hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, kernel, block, bytes);
   if (e != hipSuccess) {
     (void)hipGetLastError();
     return lh::fail_arg("lh_gemm_config_info: occupancy query failed: %s", hipGetErrorString(e));
@@ -2062,7 +2053,28 @@ int occupancy_cfg(bool ta, bool tx, int *blocks_per_cu, int *lds_bytes) {
   return LH_OK;
 }
 
+template <int BM, int BN, int WM, int WN, int WK, int BK>
+int occupancy_cfg(bool ta, bool tx, int *blocks_per_cu, int *lds_bytes) {
+#define LH_GEMM_OCC(TA, TX)                                                                            \
+  return occupancy(gemm_kernel<BM, BN, WM, WN, WK, BK, TA, TX>, 64 * WM * WN * WK,                     \
+                   smem2_floats<BM, BN, WM, WN, WK, BK, TA, TX>() * 4, blocks_per_cu, lds_bytes)
+  if (!ta && !tx) LH_GEMM_OCC(false, false);
+  if (ta) LH_GEMM_OCC(true, false);
+  LH_GEMM_OCC(false, true);
+#undef LH_GEMM_OCC
+}
+
+template <int FC>
+int occupancy_narrow(bool ta, bool tx, int *blocks_per_cu, int *lds_bytes) {
+  if (tx) return lh::fail_arg("lh_gemm_config_info: the narrow forms take no transposed X");
+  return occupancy(ta ? (GemmKernel)gemm_kernel<16, 16 * FC, 1, 1, 8, kNarrowSlab, true, false>
+                      : (GemmKernel)gemm_kernel<16, 16 * FC, 1, 1, 8, kNarrowSlab, false, false>,
+                   512, narrow_smem_floats<FC>() * 4, blocks_per_cu, lds_bytes);
+}
+
 int occupancy_index(int c, bool ta, bool tx, int *blocks_per_cu, int *lds_bytes) {
+  if (c == kNumConfigs) return occupancy_narrow<1>(ta, tx, blocks_per_cu, lds_bytes);
+  if (c == kNumConfigs + 1) return occupancy_narrow<2>(ta, tx, blocks_per_cu, lds_bytes);
   switch (c) {
 #define LH_CFG_CASE(I, BM, BN, WM, WN, WK, BK) \
   case I: return occupancy_cfg<BM, BN, WM, WN, WK, BK>(ta, tx, blocks_per_cu, lds_bytes);
@@ -2111,12 +2123,8 @@ constexpr float kCellFixedUs = 6.0f;
 
 // The narrow forms, numbered behind the configurations of the table, with rows of their own in the cost model (gate
 // product: fitted at 256 and 1000 hidden units, weights from HBM; plain products: 1000 rows; one workgroup per CU).
-// They are not among the configurations that an override names.
-const Config kNarrow[] = {{16, 16, 1, 1, 8, kNarrowSlab}, {16, 32, 1, 1, 8, kNarrowSlab}};
 const Tuning kNarrowCell[] = {{1, 3.7f, 0.0031f, 3.7f, 0.0031f}, {1, 4.2f, 0.0040f, 4.2f, 0.0040f}};
 const Tuning kNarrowPlain[] = {{1, 3.2f, 0.0025f, 3.2f, 0.0025f}, {1, 4.0f, 0.0033f, 4.0f, 0.0033f}};
-constexpr int kNumNarrow = 2;
-const Config &config_at(int c) { return c < kNumConfigs ? kConfigs[c] : kNarrow[c - kNumConfigs]; }
 
 float predict_us(const Tuning &t, const Config &k, int M, int N, const int *K, int nseg, int want,
                  bool reduce_free, int *splits) {
@@ -2248,7 +2256,8 @@ void pick_packed(int H, int B, const int *K, int nseg, int *config, float *us) {
     const float t = predict_us(kTuning[4][c], kConfigs[c], 4 * H, B, K, nseg, 1, false, &S);
     if (t < *us) *us = t, *config = c;
   }
-  for (int i = 0; i < kNumNarrow && g_config_override < 0; ++i) {
+  for (int i = 0; i < kNumNarrow; ++i) {
+    if (g_config_override >= 0 && kNumConfigs + i != g_config_override) continue;
     int S;
     const float t = predict_us(kNarrowCell[i], kNarrow[i], 4 * H, B, K, nseg, 1, false, &S);
     if (t < *us) *us = t, *config = kNumConfigs + i;
@@ -2903,8 +2912,8 @@ extern "C" int lh_gemm_act_rows_f32(int M, int N, const lh_gemm_seg *segs, int n
 }
 
 extern "C" int lh_gemm_set_config_override(int config) {
-  if (config >= kNumConfigs)
-    return lh::fail_arg("lh_gemm_set_config_override: %d >= %d", config, kNumConfigs);
+  if (config >= kNumConfigs + kNumNarrow)
+    return lh::fail_arg("lh_gemm_set_config_override: %d >= %d", config, kNumConfigs + kNumNarrow);
   g_config_override = config < 0 ? -1 : config;
   return kNumConfigs;
 }
@@ -2917,10 +2926,10 @@ extern "C" int lh_gemm_set_splits_override(int splits) {
 }
 
 extern "C" int lh_gemm_config_info(int config, int transA, int transX, int info[8]) {
-  if (config < 0 || config >= kNumConfigs || !info || (transA && transX))
-    return lh::fail_arg("lh_gemm_config_info: config=%d of %d, info=%p", config, kNumConfigs,
+  if (config < 0 || config >= kNumConfigs + kNumNarrow || !info || (transA && transX))
+    return lh::fail_arg("lh_gemm_config_info: config=%d of %d, info=%p", config, kNumConfigs + kNumNarrow,
                         (void *)info);
-  const Config &k = kConfigs[config];
+  const Config &k = config_at(config);
   info[0] = k.bm, info[1] = k.bn, info[2] = k.wm, info[3] = k.wn, info[4] = k.wk, info[5] = k.bk;
   return occupancy_index(config, transA != 0, transX != 0, &info[6], &info[7]);
 }

@@ -77,3 +77,51 @@ def test_streamed_product_matches_float64(lh, config, tA, tX, M, N, Ks, splits):
     # magnitudes at most
     bound = (sum(Ks) + 3) * 2.0 ** -24 * (bound + old.T.double().abs() + bias.double().abs()[:, None])
     assert bool(((out.T.double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("form", [0, 1], ids=["16x16", "16x32"])
+@pytest.mark.parametrize("tA,M,N,Ks,splits", [
+    (False, 4, 1, (4,), 1), (False, 20, 33, (32,), 1), (False, 100, 17, (288, 4), 1), (False, 64, 48, (1028, 12), 3),
+    (True, 1, 1, (4,), 1), (True, 17, 33, (36,), 1), (True, 101, 16, (260, 8, 1000), 1), (True, 33, 31, (1028,), 4),
+    (True, 1003, 5, (516, 4), 2)])
+def test_narrow_tiles_by_name(lh, form, tA, M, N, Ks, splits):
+    """The tiles of 16 rows at the edges of tiles, slabs and shares, whatever the cost model would take there; a
+    transposed A may have any number of rows."""
+    import torch
+    lib = lh.load()
+    config = lib.lh_gemm_set_config_override(-1) + form
+    lib.lh_gemm_set_config_override(config)
+    any_matrix = torch.empty(16, device="cuda")
+    info = lh.gemm_config_info(config, tA, False)
+    assert (info["BM"], info["BN"]) == (16, 16 * (form + 1)) and info["occupancy"] >= 1
+    name = lh.gemm_kernel_name(M, N, [(any_matrix, 2048, any_matrix, 2048, K) for K in Ks], tA, False, 64 * M * N)
+    assert name.startswith("gemm_kernel<16, %d," % (16 * (form + 1))), name
+    test_streamed_product_matches_float64(lh, config, tA, False, M, N, Ks, splits)
+
+
+@pytest.mark.parametrize("config", CONFIGS)
+@pytest.mark.parametrize("M,N,Ks,splits", [
+    (32, 32, (1,), 1), (36, 32, (7,), 1), (64, 36, (66, 3), 1), (100, 68, (131, 1, 513), 1), (200, 36, (1001,), 3)])
+def test_streamed_product_over_any_k(lh, config, M, N, Ks, splits):
+    """X transposed (weight gradients): both operands are contiguous along the columns, and K may be any number."""
+    import torch
+    lh.load().lh_gemm_set_config_override(config)
+    any_matrix = torch.empty(16, device="cuda")
+    name = lh.gemm_kernel_name(M, N, [(any_matrix, 2048, any_matrix, 2048, K) for K in Ks], False, True, 64 * M * N)
+    assert name.startswith("gemm_kernel<") and name.count(",") == 7, name
+    test_streamed_product_matches_float64(lh, config, False, True, M, N, Ks, splits)
+
+
+def test_narrow_tiles_named_where_they_cannot_run(lh):
+    """No such tile for a transposed X: the override falls back like any other that does not fit, and there is no
+    configuration behind the two."""
+    import torch
+    lib = lh.load()
+    n = lib.lh_gemm_set_config_override(-1)
+    with pytest.raises(lh.LinmtHipError):
+        lh.gemm_config_info(n, False, True)
+    with pytest.raises(lh.LinmtHipError):
+        lh.gemm_config_info(n + 2)
+    with pytest.raises(lh.LinmtHipError):
+        lh.check(min(0, lib.lh_gemm_set_config_override(n + 2)), "override")
+    test_streamed_product_matches_float64(lh, n, False, True, 36, 20, (64,), 1)

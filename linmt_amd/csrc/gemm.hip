@@ -592,7 +592,8 @@ constexpr int kRingStages = 4;
 template <int BM, int BN, int WM, int WN, int WK, int BK>
 constexpr bool streamed() {
   // eight wavefronts, a 32 x 32 block each, 16 k of every slab (8 where all of them share one block)
-  return BM == 32 * WM && BN == 32 * WN && WK >= 4 && WM * WN * WK == 8 && BK >= (WK == 8 ? 64 : 16 * WK);
+  return BM == 32 * WM && BN == 32 * WN && WK >= 4 && WM * WN * WK == 8 &&
+         (BK == 16 * WK || (WK == 8 && BK == 64));
 }
 // Floats from one column to the next of a partial tile in LDS: a quarter of the rows (a gate's share
 // of the tile) as padding puts the columns a wavefront reads at once on distinct banks.
@@ -1769,6 +1770,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmArgs g) {
 // ---- configurations -----------------------------------------------------------------------
 struct Config {
   int bm, bn, wm, wn, wk, bk;
+  bool streamed;
 };
 // X(index, BM, BN, WM, WN, WK, BK)
 #define LH_GEMM_CONFIGS(X)                                                     \
@@ -1815,15 +1817,16 @@ struct Config {
   X(40, 128, 96, 4, 1, 4, 64)                                                  \
   X(41, 96, 96, 3, 1, 4, 64)   /* three wavefronts along m, twelve in all (three per SIMD): 42 row tiles of the stacked gates at H = 1000 */ \
   X(42, 96, 64, 3, 1, 4, 64)                                                   \
-  X(43, 64, 160, 2, 1, 4, 64)  /* 252 tiles of the stacked gates at 580-640 columns */
+  X(43, 64, 160, 2, 1, 4, 64)  /* 252 tiles of the stacked gates at 580-640 columns */ \
+  X(44, 64, 32, 2, 1, 4, 128)  /* few columns against an A that comes from HBM */
 
-#define LH_CFG_ENTRY(I, BM, BN, WM, WN, WK, BK) {BM, BN, WM, WN, WK, BK},
+#define LH_CFG_ENTRY(I, BM, BN, WM, WN, WK, BK) {BM, BN, WM, WN, WK, BK, streamed<BM, BN, WM, WN, WK, BK>()},
 const Config kConfigs[] = {LH_GEMM_CONFIGS(LH_CFG_ENTRY)};
 #undef LH_CFG_ENTRY
 constexpr int kNumConfigs = sizeof(kConfigs) / sizeof(kConfigs[0]);
 constexpr int kUnalignedConfig = 7;
 // The narrow forms, numbered behind them.
-const Config kNarrow[] = {{16, 16, 1, 1, 8, kNarrowSlab}, {16, 32, 1, 1, 8, kNarrowSlab}};
+const Config kNarrow[] = {{16, 16, 1, 1, 8, kNarrowSlab, false}, {16, 32, 1, 1, 8, kNarrowSlab, false}};
 constexpr int kNumNarrow = sizeof(kNarrow) / sizeof(kNarrow[0]);
 const Config &config_at(int c) { return c < kNumConfigs ? kConfigs[c] : kNarrow[c - kNumConfigs]; }
 // Configurations built for ragged operands as well: those that the cost model gives an aligned output
@@ -2126,8 +2129,22 @@ constexpr float kCellFixedUs = 6.0f;
 const Tuning kNarrowCell[] = {{1, 3.7f, 0.0031f, 3.7f, 0.0031f}, {1, 4.2f, 0.0040f, 4.2f, 0.0040f}};
 const Tuning kNarrowPlain[] = {{1, 3.2f, 0.0025f, 3.2f, 0.0025f}, {1, 4.0f, 0.0033f, 4.0f, 0.0033f}};
 
+// What the K loop of a plain product costs more where its operands come from beyond the L2s, which the table does not
+// show.  A streamed wavefront takes a transposed A in 64-byte runs, one per row, and its ring covers the latency of an L2
+// but not that of HBM: from 48 MB of operands on (35 products of 400 to 2000 rows, K = 6000 to 30000) its loop takes
+// 1.28 times the time of the table at the median, 1.6 in the worst tenth; with A as stored, in runs of 128 bytes, 1.1
+// times what staged tiles take.  Staged and narrow tiles stay within 0.06 of the table, and below 16 MB so do all.
+// Transposed, 1536 x 21, K = 8460: 26.1 us on 32x32, 23.3 on staged 64x32; 996 x 109, K = 11516 47.6 and 37.9 (64x64);
+// 2048 x 64, K = 8192 33.6 and 30.5.
+float cold_share(const Config &k, bool ta, int M, int N, const int *K, int nseg) {
+  if (!k.streamed) return 0.f;
+  float mb = 0.f;
+  for (int s = 0; s < nseg; ++s) mb += 4.0e-6f * (float)K[s] * ((float)M + (float)N);
+  return fminf(fmaxf((mb - 16.f) / 32.f, 0.f), 1.f) * (ta ? 0.3f : 0.1f);
+}
+
 float predict_us(const Tuning &t, const Config &k, int M, int N, const int *K, int nseg, int want,
-                 bool reduce_free, int *splits) {
+                 bool reduce_free, int *splits, float cold = 0.f) {
   const long long tiles = (long long)((M + k.bm - 1) / k.bm) * ((N + k.bn - 1) / k.bn);
   int slabs = 0;
   for (int s = 0; s < nseg; ++s) slabs += (K[s] + k.bk - 1) / k.bk;
@@ -2149,6 +2166,7 @@ float predict_us(const Tuning &t, const Config &k, int M, int N, const int *K, i
   float us = rounds * tocc;
   if (rest > 1e-6f)
     us += rest <= 1.f || t.occ == 1 ? t1 : t1 + (tocc - t1) * (rest - 1.f) / (float)(t.occ - 1);
+  us += cold * (us - t.f1);
   if (S > 1 && !reduce_free)
     us += kReduceFixedUs + kReducePlaneUs * (float)S + (float)(S + 1) * (float)M * (float)N * 4.f / kReduceBytesPerUs;
   if (S > 1 && reduce_free)  // the consumer reads S planes instead of one matrix
@@ -2199,8 +2217,6 @@ void pick_config(int M, int N, const int *K, int nseg, bool ta, bool tx, Form fo
     if (us_out) *us_out = e.us;
     return;
   }
-  float k_sum = 0.f;
-  for (int s = 0; s < nseg; ++s) k_sum += (float)K[s];
   static const int kSplitChoices[] = {1, 2, 3, 4, 6, 8, 12, 16};
   // the fourth table is measured on the kernel that carries the LSTM cell in its epilogue
   const Tuning *table = kTuning[only_cell ? 3 : (ta ? 1 : (tx ? 2 : 0))];
@@ -2211,20 +2227,15 @@ void pick_config(int M, int N, const int *K, int nseg, bool ta, bool tx, Form fo
     const bool narrow = c >= kNumConfigs;
     if (narrow && (!allow_narrow || only_cell || tx || form != kAligned)) break;
     if (only_cell && !cell_capable_index(c)) continue;
-    // An A beyond 48 MB comes from HBM at every use, which the table (operands in the L2s) does not show, and the
-    // streamed tiles are not the best there: transposed 2048 x 64, K = 8192 33.6 us (32x32) and 33.9 (32x64) against 30.5
-    // on staged 64x64, 2048 x 128 47.5 and 45.1; at 33 MB (K = 4096) they are ahead, 23 and 27.
-    if (!only_cell && !narrow && g_config_override < 0 && form == kAligned && N > 32 &&
-        4.f * (float)M * k_sum > 48.0e6f && packed_config(c))
-      continue;
     if (form == kRagged && (!ragged_config(c) || kConfigs[c].bm > max_bm || kConfigs[c].bn > max_bn)) continue;
+    const float cold = only_cell || tx || form != kAligned ? 0.f : cold_share(config_at(c), ta, M, N, K, nseg);
     for (int want : kSplitChoices) {
       if (only_cell && want > 1) break;
       if (!only_cell && g_splits_override > 0) want = fit_splits(M, N, g_splits_override, workspace_bytes);
       if (max_planes > 0 && want > max_planes) want = max_planes;
       if (want > 1 && fit_splits(M, N, want, workspace_bytes) < want) break;
       int S;
-      float us = predict_us(narrow ? kNarrowPlain[c - kNumConfigs] : table[c], config_at(c), M, N, K, nseg, want, max_planes > 0, &S);
+      float us = predict_us(narrow ? kNarrowPlain[c - kNumConfigs] : table[c], config_at(c), M, N, K, nseg, want, max_planes > 0, &S, cold);
       // an override asks for this many shares: too few slabs for them only where no other choice has enough
       if (g_splits_override > 0 && S < want) us += 1.0e6f;
       if (us < best) {

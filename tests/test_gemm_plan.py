@@ -1,0 +1,33 @@
+"""The tile that lh_gemm takes (lh_gemm_kernel_name, no GPU needed) at sizes where one price in the cost model decides
+and the choices were timed on both sides."""
+import ctypes as C
+
+import pytest
+
+STREAMED = {(32, 32, 1, 1, 8, 64), (32, 32, 1, 1, 8, 128), (32, 64, 1, 2, 4, 64), (64, 32, 2, 1, 4, 64)}
+
+
+def tile(M, N, Ks, tA=False, tX=False, odd=0):
+    """Tile of the kernel chosen; odd: added to the leading dimensions of A (and of X where K is contiguous in both)."""
+    from linmt_amd import lib
+    segs = (lib.GemmSeg * len(Ks))()
+    for s, K in zip(segs, Ks):
+        s.A, s.lda, s.X, s.ldx, s.K = 256, (K if tA else M) + odd, 256, (N if tX else K) + (odd if tA else 0), K
+    name = C.create_string_buffer(128)
+    lib.check(lib.load().lh_gemm_kernel_name(M, N, segs, len(Ks), tA, tX, 64 << 20, 0, name, 128), "lh_gemm_kernel_name")
+    return tuple(int(v) for v in name.value.decode().split("<")[1].split(",")[:6])
+
+
+@pytest.mark.parametrize("M,N,K", [(996, 109, 11516), (1692, 20, 21312), (1644, 12, 24984), (840, 130, 11896),
+                                   (168, 391, 18740), (1916, 29, 29920), (2048, 64, 8192), (2048, 128, 8192)])
+def test_operands_beyond_the_l2s_are_not_streamed(M, N, K):
+    """Transposed A, 48 MB of operands and more: the streamed tiles took 1.1 to 1.25 times as long as a staged or
+    narrow one."""
+    assert tile(M, N, [K], tA=True) not in STREAMED
+
+
+@pytest.mark.parametrize("M,N,K", [(1000, 64, 1000), (256, 32, 1024), (512, 48, 2048)])
+def test_few_columns_of_a_small_matrix_are(M, N, K):
+    """Where the operands stay in the L2s the streamed and narrow tiles are the fastest (1000 x 64, K = 1000: 8.1 us
+    staged, 5.2)."""
+    assert tile(M, N, [K], tA=True) in STREAMED or tile(M, N, [K], tA=True)[0] == 16

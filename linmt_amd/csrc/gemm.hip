@@ -32,7 +32,6 @@
 
 #include <climits>
 #include <mutex>
-#include <vector>
 
 namespace {
 
@@ -1831,10 +1830,10 @@ constexpr int kNumNarrow = sizeof(kNarrow) / sizeof(kNarrow[0]);
 const Config &config_at(int c) { return c < kNumConfigs ? kConfigs[c] : kNarrow[c - kNumConfigs]; }
 // Configurations built for ragged operands as well: those that the cost model gives an aligned output
 // projection and its backward products at 5 to 2560 columns of 5000 to 30000 words, or one within
-// a few per cent of them.
-// Extents of 33 to 1002 choose among all of them too: 252 such products are 0.69 of the time that the
-// configurations with one chain of K take (0.47 of the scalar kernel's), 6 % behind at worst (66 x 33, K = 30:
-// 5.2 us against 5.0) and 0.31 at best (33 x 1, K = 1000: 9.0 us against 55 on the scalar kernel).
+// a few per cent of them.  All of them run the staged form, 15 too, and have rows of their own in the cost model: with
+// those of the aligned kernels (32x32: a fixed part of 3.9 us where this form takes 5.5) 340 products of 30 to 30003 rows
+// or words, 1 to 768 columns took 1.021 times the time of the best of a sweep over configurations and splits, 1.49 at
+// worst; with rows of their own 1.015 and 1.17.
 constexpr bool ragged_config(int c) {
   return c == 0 || c == 3 || c == 7 || c == 12 || c == 15 || c == 18 || c == 24 || c == 32 || c == 35 || c == 36;
 }
@@ -1973,17 +1972,6 @@ int launch_cell_cfg(const GemmArgs &g0, hipStream_t st) {
   }
 }
 
-// Configurations of the packed gate product: the streamed ones.
-bool packed_config(int c) {
-  switch (c) {
-#define LH_CFG_CASE(I, BM, BN, WM, WN, WK, BK) \
-  case I: return streamed<BM, BN, WM, WN, WK, BK>();
-    LH_GEMM_CONFIGS(LH_CFG_CASE)
-#undef LH_CFG_CASE
-    default: return false;
-  }
-}
-
 template <int BM, int BN, int WM, int WN, int WK, int BK>
 int launch_packed_cfg(const GemmArgs &g0, hipStream_t st) {
   if constexpr (streamed<BM, BN, WM, WN, WK, BK>()) {
@@ -2115,7 +2103,18 @@ struct Tuning {
   float f1, s1;      // one workgroup per CU: fixed us, us per k
   float focc, socc;  // CU full
 };
+struct TuningRow {
+  int config;
+  Tuning t;
+};
 #include "gemm_tuning.inc"
+// The row of a configuration in one of the tables that hold few of them, null where it has none.
+template <size_t N>
+const Tuning *row_of(const TuningRow (&rows)[N], int config) {
+  for (const TuningRow &r : rows)
+    if (r.config == config) return &r.t;
+  return nullptr;
+}
 constexpr int kCUs = 256;
 // The pass over S partial planes: 4.3 to 4.8 us of 4 planes between other kernels of a stream (1000 x 64 to 2048 x 256),
 // 2.1, 2.6 and 3.8 us of 2, 4 and 8 planes of 1000 x 5 and 1.4 us less a launch when replayed from a graph.
@@ -2124,10 +2123,6 @@ constexpr float kReduceFixedUs = 3.5f, kReducePlaneUs = 0.22f, kReduceBytesPerUs
 // lookup of 4.6 where the addend is a column of the embedding table.
 constexpr float kCellFixedUs = 6.0f;
 
-// The narrow forms, numbered behind the configurations of the table, with rows of their own in the cost model (gate
-// product: fitted at 256 and 1000 hidden units, weights from HBM; plain products: 1000 rows; one workgroup per CU).
-const Tuning kNarrowCell[] = {{1, 3.7f, 0.0031f, 3.7f, 0.0031f}, {1, 4.2f, 0.0040f, 4.2f, 0.0040f}};
-const Tuning kNarrowPlain[] = {{1, 3.2f, 0.0025f, 3.2f, 0.0025f}, {1, 4.0f, 0.0033f, 4.0f, 0.0033f}};
 
 // What the K loop of a plain product costs more where its operands come from beyond the L2s, which the table does not
 // show.  A streamed wavefront takes a transposed A in 64-byte runs, one per row, and its ring covers the latency of an L2
@@ -2228,6 +2223,10 @@ void pick_config(int M, int N, const int *K, int nseg, bool ta, bool tx, Form fo
     if (narrow && (!allow_narrow || only_cell || tx || form != kAligned)) break;
     if (only_cell && !cell_capable_index(c)) continue;
     if (form == kRagged && (!ragged_config(c) || kConfigs[c].bm > max_bm || kConfigs[c].bn > max_bn)) continue;
+    const Tuning *const t = form == kRagged ? row_of(kRaggedTuning[ta ? 1 : (tx ? 2 : 0)], c)
+                            : narrow        ? row_of(kNarrowTuning[ta ? 1 : 0], c)
+                                            : &table[c];
+    if (!t) continue;
     const float cold = only_cell || tx || form != kAligned ? 0.f : cold_share(config_at(c), ta, M, N, K, nseg);
     for (int want : kSplitChoices) {
       if (only_cell && want > 1) break;
@@ -2235,7 +2234,7 @@ void pick_config(int M, int N, const int *K, int nseg, bool ta, bool tx, Form fo
       if (max_planes > 0 && want > max_planes) want = max_planes;
       if (want > 1 && fit_splits(M, N, want, workspace_bytes) < want) break;
       int S;
-      float us = predict_us(narrow ? kNarrowPlain[c - kNumConfigs] : table[c], config_at(c), M, N, K, nseg, want, max_planes > 0, &S, cold);
+      float us = predict_us(*t, config_at(c), M, N, K, nseg, want, max_planes > 0, &S, cold);
       // an override asks for this many shares: too few slabs for them only where no other choice has enough
       if (g_splits_override > 0 && S < want) us += 1.0e6f;
       if (us < best) {
@@ -2251,27 +2250,15 @@ void pick_config(int M, int N, const int *K, int nseg, bool ta, bool tx, Form fo
   e = Memo{M, N, {Kk[0], Kk[1], Kk[2]}, flags, *config, *splits, workspace_bytes, best};
 }
 
-// The packed gate product's configuration and predicted time (fifth table).
+// The packed gate product's configuration and predicted time.
 void pick_packed(int H, int B, const int *K, int nseg, int *config, float *us) {
-  static const std::vector<int> kPacked = [] {
-    std::vector<int> v;
-    for (int c = 0; c < kNumConfigs; ++c)
-      if (packed_config(c)) v.push_back(c);
-    return v;
-  }();
   *config = -1;
   *us = 3.0e38f;
-  for (const int c : kPacked) {
-    if (g_config_override >= 0 && c != g_config_override) continue;
+  for (const TuningRow &r : kPackedTuning) {
+    if (g_config_override >= 0 && r.config != g_config_override) continue;
     int S;
-    const float t = predict_us(kTuning[4][c], kConfigs[c], 4 * H, B, K, nseg, 1, false, &S);
-    if (t < *us) *us = t, *config = c;
-  }
-  for (int i = 0; i < kNumNarrow; ++i) {
-    if (g_config_override >= 0 && kNumConfigs + i != g_config_override) continue;
-    int S;
-    const float t = predict_us(kNarrowCell[i], kNarrow[i], 4 * H, B, K, nseg, 1, false, &S);
-    if (t < *us) *us = t, *config = kNumConfigs + i;
+    const float t = predict_us(r.t, config_at(r.config), 4 * H, B, K, nseg, 1, false, &S);
+    if (t < *us) *us = t, *config = r.config;
   }
 }
 

@@ -2150,9 +2150,10 @@ float predict_us(const Tuning &t, const Config &k, int M, int N, const int *K, i
   // Workgroups per CU: dispatch is dynamic, so a fractional load costs less than a whole extra
   // round but leaves a tail of about half a workgroup.
   const float per_cu = (float)(tiles * S) / kCUs;
-  // Two streamed workgroups on a CU do not finish one after the other: 1400 x 192, K = 2800 (264 of them) 30.5 us, 26.1 on
-  // the 64x64 tiles that a fractional load would have passed over.
-  const float load = k.bm * k.bn == 1024 && k.bk == 64 ? ceilf(per_cu) : fminf(per_cu + 0.5f, ceilf(per_cu));
+  // Not so on streamed tiles: two of their workgroups on a CU do not finish one after the other (and where only one fits,
+  // a last round takes as long as any).  1400 x 192, K = 2800 (264 workgroups of 32x32, two to a CU) 30.5 us, 26.1 on the
+  // 64x64 tiles that a fractional load would have passed over.
+  const float load = k.streamed ? ceilf(per_cu) : fminf(per_cu + 0.5f, ceilf(per_cu));
   // (both are fitted at depths of 512 and 4096: below, several workgroups could come out cheaper than one)
   const float t1 = t.f1 + t.s1 * depth, full = t.focc + t.socc * depth;
   const float tocc = t.occ > 1 ? fmaxf(t1, full) : full;
@@ -2566,12 +2567,7 @@ extern "C" int lh_gate_gemm_lstm_cell_packed_plan(int H, int B, const lh_gemm_se
   if (c < 0) return LH_OK;
   pick_config(4 * H, B, p.g.K, nseg, false, false, kAligned, workspace_bytes, has_addend ? 2 : 3, &c0, &S, f, &us0);
   if (!f) us0 += kCellFixedUs + 28.f * (float)H * (float)B / kReduceBytesPerUs;
-  // More workgroups than CUs: the rounds overlap less than the model has it, and the wider staged tiles read less.  2048
-  // hidden units, 96 / 128 / 192 columns, K = 4096: 88.6 / 92.8 / 126.6 us packed, 84.4 / 82.6 / 122.6 not; with at most one
-  // workgroup per CU the packed form is ahead (64 columns: 47.3 and 60.9).
-  const Config &pk = config_at(c);
-  const long long groups = (long long)((4 * H + pk.bm - 1) / pk.bm) * ((B + pk.bn - 1) / pk.bn);
-  if (us > us0 || groups > kCUs) return LH_OK;
+  if (us > us0) return LH_OK;
   *faster = 1;
   if (name && name_cap > 0) {
     const Config &k = kConfigs[c < kNumConfigs ? c : 0];

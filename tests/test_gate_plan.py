@@ -23,3 +23,22 @@ def test_few_columns_take_one_shape(segments, widest, B):
     from linmt_amd import lib
     names = {_plan(lib, H, B, (H,) * segments) for H in range(64, widest + 1, 4)}
     assert names <= {"gate_gemm_cell_kernel<32, 32, 1, 1, 8, 64>", "gate_gemm_cell_kernel<32, 32, 1, 1, 8, 128>"}, names
+
+
+def _packed_plan(lib, H, B, Ks):
+    segs = (lib.GemmSeg * 3)()
+    for s, K in zip(segs, Ks):
+        s.A, s.lda, s.X, s.ldx, s.K = 256, 4 * H, 256, K, K
+    faster, name = C.c_int(), C.create_string_buffer(128)
+    lib.check(lib.load().lh_gate_gemm_lstm_cell_packed_plan(H, B, segs, len(Ks), 1, 64 << 20, C.byref(faster), name, 128),
+              "lh_gate_gemm_lstm_cell_packed_plan")
+    return name.value.decode() if faster.value else None
+
+
+@pytest.mark.parametrize("H,B,Ks,packed", [(1084, 134, (1084, 1084), True), (1000, 64, (1000, 1000), True),
+                                           (2048, 128, (2048, 2048), False), (2048, 192, (2048, 2048), False)])
+def test_packed_matrices_by_time_not_by_workgroups(H, B, Ks, packed):
+    """More workgroups than CUs are no reason by themselves: the first of these is 544 and took 43.8 us packed, 46.5 from
+    the stored matrix; the last two took 92.8 and 82.6, 126.6 and 122.6."""
+    from linmt_amd import lib
+    assert (_packed_plan(lib, H, B, Ks) is not None) == packed

@@ -2119,23 +2119,30 @@ constexpr int kCUs = 256;
 // The pass over S partial planes: 4.3 to 4.8 us of 4 planes between other kernels of a stream (1000 x 64 to 2048 x 256),
 // 2.1, 2.6 and 3.8 us of 2, 4 and 8 planes of 1000 x 5 and 1.4 us less a launch when replayed from a graph.
 constexpr float kReduceFixedUs = 3.5f, kReducePlaneUs = 0.22f, kReduceBytesPerUs = 3.0e6f;
-// A launch of the LSTM cell kernel behind its product: 4.1 to 4.7 us between other kernels at 12 columns, 7.2 and a
-// lookup of 4.6 where the addend is a column of the embedding table.
-constexpr float kCellFixedUs = 6.0f;
+// The LSTM cell as a launch of its own behind its product (us): 4.1 to 4.7 us between other kernels at 12 columns, and 7.2
+// and a lookup of 4.6 where the addend is a column of the embedding table.  Behind a short product the dearer price holds
+// (the host, which issues two launches for one, is no faster than they are); behind a longer one it made 15 of 240 gate
+// products of 64 to 2048 hidden units, 1 to 256 columns 5 % slower or more than the split product they had been, 16 % at
+// worst, all of 26 us or longer; now 1 of them, 6 %.
+float cell_launch_us(float product_us, int H, int B) {
+  return (product_us < 16.f ? 6.f : 4.f) + 28.f * (float)H * (float)B / kReduceBytesPerUs;
+}
 
-
-// What the K loop of a plain product costs more where its operands come from beyond the L2s, which the table does not
+// What the K loop costs more where its operands come from beyond the L2s, which the table does not
 // show.  A streamed wavefront takes a transposed A in 64-byte runs, one per row, and its ring covers the latency of an L2
 // but not that of HBM: from 48 MB of operands on (35 products of 400 to 2000 rows, K = 6000 to 30000) its loop takes
 // 1.28 times the time of the table at the median, 1.6 in the worst tenth; with A as stored, in runs of 128 bytes, 1.1
 // times what staged tiles take.  Staged and narrow tiles stay within 0.06 of the table, and below 16 MB so do all.
 // Transposed, 1536 x 21, K = 8460: 26.1 us on 32x32, 23.3 on staged 64x32; 996 x 109, K = 11516 47.6 and 37.9 (64x64);
 // 2048 x 64, K = 8192 33.6 and 30.5.
-float cold_share(const Config &k, bool ta, int M, int N, const int *K, int nseg) {
+// The stored gate matrix of a product with its cell is runs of 32 bytes (8 rows of a gate) and costs the same: 1.36 at
+// the median of 78 products of at most a workgroup per CU, where staged tiles take 1.06 and packed matrices 1.12 (no
+// price for those).  1956 hidden units, 58 columns, K = 3912: 69 us on streamed 64x32, 60 on the staged one, 51 split with a cell kernel behind.
+float cold_share(const Config &k, bool short_runs, int M, int N, const int *K, int nseg) {
   if (!k.streamed) return 0.f;
   float mb = 0.f;
   for (int s = 0; s < nseg; ++s) mb += 4.0e-6f * (float)K[s] * ((float)M + (float)N);
-  return fminf(fmaxf((mb - 16.f) / 32.f, 0.f), 1.f) * (ta ? 0.3f : 0.1f);
+  return fminf(fmaxf((mb - 16.f) / 32.f, 0.f), 1.f) * (short_runs ? 0.3f : 0.1f);
 }
 
 float predict_us(const Tuning &t, const Config &k, int M, int N, const int *K, int nseg, int want,
@@ -2228,7 +2235,7 @@ void pick_config(int M, int N, const int *K, int nseg, bool ta, bool tx, Form fo
                             : narrow        ? row_of(kNarrowTuning[ta ? 1 : 0], c)
                                             : &table[c];
     if (!t) continue;
-    const float cold = only_cell || tx || form != kAligned ? 0.f : cold_share(config_at(c), ta, M, N, K, nseg);
+    const float cold = tx || form != kAligned ? 0.f : cold_share(config_at(c), ta || only_cell, M, N, K, nseg);
     for (int want : kSplitChoices) {
       if (only_cell && want > 1) break;
       if (!only_cell && g_splits_override > 0) want = fit_splits(M, N, g_splits_override, workspace_bytes);
@@ -2414,9 +2421,8 @@ int plan_cell(int H, int B, const lh_gemm_seg *segs, int nseg, bool has_addend, 
   pick_config(4 * H, B, p->g.K, nseg, false, false, kAligned, ws, has_addend ? 2 : 3, &cfg_cell,
               &splits_cell, true, &us_cell);
   if (cfg_cell < 0) return LH_OK;
-  const float cell_us = kCellFixedUs + 28.f * (float)H * (float)B / kReduceBytesPerUs;
   // a configuration override (tuning, tests) asks for the fused form whenever the tile can hold it
-  if (g_config_override >= 0 || us_cell <= us_any + cell_us) {
+  if (g_config_override >= 0 || us_cell <= us_any + cell_launch_us(us_any, H, B)) {
     *fusable = true;
     p->config = cfg_cell;
     p->g.splits = 1;
@@ -2566,7 +2572,7 @@ extern "C" int lh_gate_gemm_lstm_cell_packed_plan(int H, int B, const lh_gemm_se
   pick_packed(H, B, p.g.K, nseg, &c, &us);
   if (c < 0) return LH_OK;
   pick_config(4 * H, B, p.g.K, nseg, false, false, kAligned, workspace_bytes, has_addend ? 2 : 3, &c0, &S, f, &us0);
-  if (!f) us0 += kCellFixedUs + 28.f * (float)H * (float)B / kReduceBytesPerUs;
+  if (!f) us0 += cell_launch_us(us0, H, B);
   if (us > us0) return LH_OK;
   *faster = 1;
   if (name && name_cap > 0) {

@@ -42,3 +42,11 @@ def test_packed_matrices_by_time_not_by_workgroups(H, B, Ks, packed):
     the stored matrix; the last two took 92.8 and 82.6, 126.6 and 122.6."""
     from linmt_amd import lib
     assert (_packed_plan(lib, H, B, Ks) is not None) == packed
+
+
+@pytest.mark.parametrize("H,B,Ks", [(1956, 58, (1956, 1956)), (1364, 60, (1364, 1364, 1364)), (1740, 44, (1740, 1740, 1740))])
+def test_large_stored_matrices_are_not_streamed(H, B, Ks):
+    """A tile's share of a stored gate matrix is 32-byte runs: streamed from HBM it took 1.36 times the time of the L2s (the
+    first of these 69 us, 51 as a split product with the cell kernel behind it)."""
+    from linmt_amd import lib
+    assert _plan(lib, H, B, Ks) != "gate_gemm_cell_kernel<64, 32, 2, 1, 4, 64>"

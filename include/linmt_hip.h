@@ -191,8 +191,9 @@ int lh_gate_gemm_lstm_cell_train_f32(int H, int B, const lh_gemm_seg *segs, int 
  * lh_gate_pack_f32 writes a copy in which they are one run: for every 8 cells (the last block padded with
  * zeros) K rows of 32 floats, float 4r + q of row k = gate q of cell r.  A caller packs once per change of
  * the weights, and uses the copy where lh_gate_gemm_lstm_cell_packed_plan says that it is the faster way
- * (*faster; segs, workspace_bytes and has_addend as for lh_gate_gemm_lstm_cell_plan, with the matrices as
- * stored; few columns, H and K multiples of 4, 16-byte aligned operands).
+ * (*faster: 0, or by how many nanoseconds a call; segs, workspace_bytes and has_addend as for
+ * lh_gate_gemm_lstm_cell_plan, with the matrices as stored; few columns, H and K multiples of 4, 16-byte
+ * aligned operands).
  * lh_gate_gemm_lstm_cell_packed_f32: A of a segment is a packed matrix (16-byte aligned; lda is not read);
  * everything else as for lh_gate_gemm_lstm_cell_f32 and, with gates / h_drop (both optional),
  * lh_gate_gemm_lstm_cell_train_f32.  It does not look at the plan's advice: any B runs. */

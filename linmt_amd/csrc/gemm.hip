@@ -2574,7 +2574,7 @@ extern "C" int lh_gate_gemm_lstm_cell_packed_plan(int H, int B, const lh_gemm_se
   pick_config(4 * H, B, p.g.K, nseg, false, false, kAligned, workspace_bytes, has_addend ? 2 : 3, &c0, &S, f, &us0);
   if (!f) us0 += cell_launch_us(us0, H, B);
   if (us > us0) return LH_OK;
-  *faster = 1;
+  *faster = 1 + (int)(1000.f * fminf(us0 - us, 1.0e6f));
   if (name && name_cap > 0) {
     const Config &k = kConfigs[c < kNumConfigs ? c : 0];
     if (c < kNumConfigs)

@@ -207,14 +207,30 @@ class LstmLayer {
   int split_kgroups_ = 0;  // k-groups of both operands, padding included
   bool split_dirty_ = true;
   void BuildSplitWeights();
-  // The stacked gate matrices as the packed gate product reads them (lh_gate_pack_f32), a copy beside the
-  // stored ones: made by the first step that runs faster on it, made anew after a change of the weights.
-  // M is not among them where it never is an operand of a step's product (the input layer).  A model whose
-  // memory does not hold the copies runs on the stored matrices.
-  DeviceArray<float> packed_;  // one array: the copies of M, W_h and Q, null pointers where there is none
-  const float *packed_m_ = nullptr, *packed_w_h_ = nullptr, *packed_q_ = nullptr;
-  bool packed_dirty_ = true, packed_possible_ = true;
-  bool PackGates();  // false: no memory
+  // Stacked gate matrices as the packed gate product reads them (lh_gate_pack_f32), a copy beside the stored
+  // one: of the matrices that are operands of a step's product (M is not where the input product is hoisted), made
+  // by the first step that runs faster on it, made anew after a change of the weights.  While training that is
+  // every minibatch, so there it has to pay within the pass.  A model whose memory does not hold the copies runs
+  // on the stored matrices.
+  struct PackedGates {
+    DeviceArray<float> copy;
+    bool dirty = true;
+  };
+  PackedGates packed_[3];  // M, W_h, Q
+  bool packed_possible_ = true;
+  int pass_steps_ = 0;     // steps of the pass that is running (teacher-forced passes and the encoder)
+  void WeightsChanged() {
+    for (PackedGates &p : packed_) p.dirty = true;
+  }
+  // Puts the copies into segs; false: stays with the stored matrices.  saved_ns: what a step saves by the plan,
+  // steps: how many are left of the pass.
+  bool PackGates(lh_gemm_seg *segs, int nseg, int saved_ns, int steps);
+  // Whether copies of this many floats are worth making for these steps.  A launch reads and writes them at
+  // 3.1 TB/s (20.5 us for two 4000 x 1000 matrices) and costs 4 us more: W_h of 1000 hidden units alone, whose steps
+  // save 2.4 us at 64 columns, pays from 6 steps on.
+  static bool PackingPays(size_t floats, int saved_ns, int steps) {
+    return 4000.0 + 8.0 * (double)floats / 3.1e3 < (double)saved_ns * steps;
+  }
   void ForwardPropInputAllSteps(int steps);
   void ForwardPropInputSteps(int first, int steps);
   void BuildEmbeddingFold();

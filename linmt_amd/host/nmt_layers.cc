@@ -111,7 +111,6 @@ void LstmLayer::Init(NeuralMachineTranslation *model, bool input_layer, bool sou
 
 void LstmLayer::InitFeedInput() {
   feed_input_mode_ = true;
-  packed_dirty_ = true;  // Q joins the packed matrices
   p_device_q_stack_.Alloc(4 * (size_t)lstm_size_ * lstm_size_);
   p_device_q_stack_.Zero(p_neural_mt_->stream_);
   if (p_neural_mt_->cfg_.train_mode_ && keep_gates_) {
@@ -138,7 +137,8 @@ bool LstmLayer::SetParam(const std::string &name, const float *host, size_t n) {
   hipStream_t s = p_neural_mt_->stream_;
   const int H = lstm_size_;
   if (name == "W" || name[0] == 'M') mw_fold_dirty_ = true;
-  split_dirty_ = packed_dirty_ = true;
+  split_dirty_ = true;
+  WeightsChanged();
   if (name == "W") return input_layer_mode_ && SetFlat(p_device_w_, host, n, s);
   if (name.size() == 3 && name[0] == 'M' && name[1] == '_') {
     const int g = GateIndex(name[2]);
@@ -239,33 +239,39 @@ void LstmLayer::BuildSplitWeights() {
   split_dirty_ = false;
 }
 
-bool LstmLayer::PackGates() {
+bool LstmLayer::PackGates(lh_gemm_seg *segs, int nseg, int saved_ns, int steps) {
   if (!packed_possible_) return false;
-  if (!packed_dirty_) return true;
   const int H = lstm_size_;
-  const float **to[3] = {&packed_m_, &packed_w_h_, &packed_q_};
-  DeviceArray<float> *from[3] = {&p_device_m_stack_, &p_device_w_h_stack_, &p_device_q_stack_};
-  const int K[3] = {input_layer_mode_ ? 0 : input_size_, H, feed_input_mode_ ? H : 0};
-  size_t floats = 0;
-  for (int k : K) floats += lh_gate_pack_floats(H, k);
-  if (packed_.size() != floats) {
-    try {
-      packed_.Alloc(floats);
-    } catch (const std::exception &) {
-      packed_possible_ = false;
-      return false;
+  const DeviceArray<float> *const stored[3] = {&p_device_m_stack_, &p_device_w_h_stack_, &p_device_q_stack_};
+  const int K[3] = {input_size_, H, H};
+  int of[LH_GEMM_MAX_SEGS] = {0, 0, 0};
+  bool wanted[3] = {false, false, feed_input_mode_};  // (Q is an operand from the second step on)
+  for (int i = 0; i < nseg; ++i) {
+    while (of[i] < 2 && segs[i].A != stored[of[i]]->get()) ++of[i];
+    wanted[of[i]] = true;
+  }
+  size_t stale = 0;
+  for (int m = 0; m < 3; ++m)
+    if (wanted[m] && packed_[m].dirty) stale += lh_gate_pack_floats(H, K[m]);
+  if (stale) {
+    if (p_neural_mt_->cfg_.train_mode_ && !PackingPays(stale, saved_ns, steps)) return false;
+    lh_gate_pack_source src[3];
+    int n = 0;
+    for (int m = 0; m < 3; ++m) {
+      if (!wanted[m] || !packed_[m].dirty) continue;
+      try {
+        packed_[m].copy.Reserve(lh_gate_pack_floats(H, K[m]));
+      } catch (const std::exception &) {
+        packed_possible_ = false;
+        return false;
+      }
+      src[n++] = lh_gate_pack_source{stored[m]->get(), 4 * H, K[m], packed_[m].copy.get()};
     }
+    LhErrorWrapper(lh_gate_pack_f32(H, src, n, p_neural_mt_->stream_), "LstmLayer::PackGates");
+    for (int m = 0; m < 3; ++m)
+      if (wanted[m]) packed_[m].dirty = false;
   }
-  lh_gate_pack_source src[3];
-  int n = 0;
-  float *at = packed_.get();
-  for (int i = 0; i < 3; ++i) {
-    *to[i] = K[i] ? at : nullptr;
-    if (K[i]) src[n++] = lh_gate_pack_source{from[i]->get(), 4 * H, K[i], at};
-    at += lh_gate_pack_floats(H, K[i]);
-  }
-  LhErrorWrapper(lh_gate_pack_f32(H, src, n, p_neural_mt_->stream_), "LstmLayer::PackGates");
-  packed_dirty_ = false;
+  for (int i = 0; i < nseg; ++i) segs[i].A = packed_[of[i]].copy.get();
   return true;
 }
 
@@ -361,14 +367,10 @@ void LstmNode::ForwardProp() {
     LhErrorWrapper(lh_gate_gemm_lstm_cell_packed_plan(H, B, segs, nseg, beta != 0.f, M.gemm_ws_bytes_, &faster,
                                                       name, sizeof(name)),
                    "lh_gate_gemm_lstm_cell_packed_plan");
-    if (faster && !(folded && (p_device_gates_ || drop_out)) && L.PackGates()) {
+    if (faster && !(folded && (p_device_gates_ || drop_out)) &&
+        L.PackGates(segs, nseg, faster, L.pass_steps_ - index_)) {
       double k = 0;
-      for (int i = 0; i < nseg; ++i) {
-        k += segs[i].K;
-        segs[i].A = segs[i].A == L.p_device_m_stack_.get()     ? L.packed_m_
-                    : segs[i].A == L.p_device_w_h_stack_.get() ? L.packed_w_h_
-                                                               : L.packed_q_;
-      }
+      for (int i = 0; i < nseg; ++i) k += segs[i].K;
       ProfileScope ps(M.profiler_, kTagGateGemm, name, 2.0 * 4 * H * (double)B * k);
       LhErrorWrapper(lh_gate_gemm_lstm_cell_packed_f32(
                          H, B, segs, nseg, beta != 0.f ? (folded ? L.mw_fold_.get() : pre) : nullptr, 4 * H,

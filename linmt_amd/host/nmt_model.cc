@@ -366,6 +366,7 @@ void NeuralMachineTranslation::ForwardTeacherForced(const int *p_host_source, in
   const bool all_steps_loss = per_step_loss && B == cfg_.minibatch_size_;
 
   if (seq2seq) RunSourceSide(source_length, B);
+  for (int l = 0; l < L; ++l) TargetLayer(l).pass_steps_ = target_length;
   {
     LstmLayer &L0 = input_layer_target_;
     L0.input_hoisted_ = L0.input_hoistable_ && B == L0.minibatch_size_;
@@ -524,6 +525,7 @@ void NeuralMachineTranslation::ForwardPropSource(const int *p_host_source, int s
 void NeuralMachineTranslation::RunSourceSide(int source_length, int B) {
   const int L = cfg_.num_layers_;
   const bool lanes_off = Debug().no_lanes != 0;  // measurement and test aid
+  for (int l = 0; l < L; ++l) SourceLayer(l).pass_steps_ = source_length;
   bool lanes = !lanes_off && decode_mode_ && L > 1 && L <= 4 && profiler_.level_ < 2 &&
                source_length > kLaneChunkSteps;
   for (int l = 0; l < L && lanes; ++l)

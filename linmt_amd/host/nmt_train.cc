@@ -736,7 +736,7 @@ void NeuralMachineTranslation::UpdateWeights() {
   // (src/layer_input_to_hidden.h:1154,1257,1263, src/layer_hidden_to_hidden.h:765,831)
   auto add_layer = [&](LstmLayer &Ly, bool source_side) {
     const bool rnn_frozen = source_side ? !cfg_.train_source_rnn_mode_ : !cfg_.train_target_rnn_mode_;
-    if (!rnn_frozen) Ly.packed_dirty_ = true;
+    if (!rnn_frozen) Ly.WeightsChanged();
     const bool emb_frozen = source_side ? !cfg_.train_source_input_embedding_mode_
                                         : !cfg_.train_target_input_embedding_mode_;
     add_stack(Ly.p_device_w_h_stack_, Ly.p_device_w_h_grad_, H, rnn_frozen);

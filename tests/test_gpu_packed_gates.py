@@ -120,3 +120,35 @@ def test_weights_set_between_passes_reach_the_packed_copy(lh, B):
     assert abs(first - second) > 1e-2
     assert_close(second, want, "loss with the weights as they are now", rtol=1e-6, atol=1e-4)
     m.close(), fresh.close()
+
+
+def _training_model(host, rng, H, V, B, longest, layers=2):
+    m = host.Model(layers, H, V, V, longest_sentence=longest, attention_mode=0, minibatch_size=B,
+                   training=dict(learning_rate=0.1, grad_clip_mode=0))
+    u = lambda *s: rng.uniform(-0.1, 0.1, size=s).astype(np.float32)  # noqa: E731
+    P = {"softmax.D": u(V, H), "softmax.b_d": u(V)}
+    for side in ("src", "tgt"):
+        P[side + ".0.W"] = u(H, V)
+        for layer in range(layers):
+            for g in "ifco":
+                P[f"{side}.{layer}.W_h{g}"], P[f"{side}.{layer}.M_{g}"], P[f"{side}.{layer}.b_{g}"] = u(H, H), u(H, H), u(H)
+    m.set_params(P)
+    return m
+
+
+def test_training_packs_where_the_pass_is_long_enough(lh):
+    """The weights are packed anew for every minibatch: one step does not save what that costs, 24 do."""
+    from linmt_amd import host
+    rng = np.random.default_rng(5)
+    H, V, B = 512, 60, 32
+    m = _training_model(host, rng, H, V, B, 28)
+    for steps, packed in ((1, False), (24, True)):
+        src, ti, to = (rng.integers(0, V, (B, steps)).astype(np.int32) for _ in range(3))
+        info = np.concatenate([np.full(B, steps), np.zeros(B)]).astype(np.int32)
+        m.profile(2)
+        m.compute_gradients(src, ti, to, info, *(np.unique(a).astype(np.int32) for a in (src, ti)))
+        names = list(m.profile_totals())
+        m.profile(0)
+        m.update_weights()
+        assert any("gate_gemm_packed_kernel" in n or "gate_gemm_narrow_kernel" in n for n in names) == packed, (steps, names)
+    m.close()

@@ -220,7 +220,9 @@ int lnmt_set_split_products(lnmt_model *m, int on, int min_columns);
  *   "no_lanes"                the encoder of a decoding batch runs on the model's one stream;
  *   "grouped_gates"           what the previous step fixes of every layer's gate product runs as
  *                             one grouped launch (lh_gate_gemm_group_f32);
- *   "separate_beam_launches"  beam merge and state gather as two launches instead of one.
+ *   "separate_beam_launches"  beam merge and state gather as two launches instead of one;
+ *   "no_packed_gates"         gate products of few columns run on the stored matrices, as they do
+ *                             where the card is short of memory for packed copies.
  * An unknown name is an error.  Set them before a model is created or between calls, not while
  * another thread decodes. */
 int lnmt_set_debug_option(const char *name, int value);

@@ -432,6 +432,7 @@ extern "C" int lnmt_set_debug_option(const char *name, int value) {
     else if (n == "no_lanes") d.no_lanes = value;
     else if (n == "grouped_gates") d.grouped_gates = value;
     else if (n == "separate_beam_launches") d.separate_beam_launches = value;
+    else if (n == "no_packed_gates") d.no_packed_gates = value;
     else throw LinmtError("lnmt_set_debug_option: unknown option " + n);
   });
 }

@@ -73,18 +73,25 @@ class DeviceArray {
   void Reserve(size_t n) {
     if (n > n_) Alloc(n);
   }
-  // The same for memory the caller can do without: false (and an empty array) when there is none.
+  // The same for memory the caller can do without: false (and an empty array) when there is none.  Any
+  // other failure is reported like everywhere else: an error of an earlier kernel can surface here.
   bool TryReserve(size_t n) {
     if (n <= n_) return true;
     Free();
     if (n > SIZE_MAX / sizeof(T)) return false;
-    if (hipMalloc(reinterpret_cast<void **>(&p_), n * sizeof(T)) != hipSuccess) {
+    const hipError_t e = hipMalloc(reinterpret_cast<void **>(&p_), n * sizeof(T));
+    if (e != hipSuccess) {
       p_ = nullptr;
       (void)hipGetLastError();
+      if (!NoMemory(e)) HipErrorWrapper(e, "GPU memory allocation failed");
       return false;
     }
     n_ = n;
     return true;
+  }
+  // A machine without a device has no memory either; a size beyond what the driver takes is none there is.
+  static bool NoMemory(hipError_t e) {
+    return e == hipErrorOutOfMemory || e == hipErrorNoDevice || e == hipErrorInvalidValue;
   }
   void Free() {
     if (p_) (void)hipFree(p_);

@@ -77,6 +77,7 @@ struct DebugOptions {
   int no_lanes = 0;                // the encoder of a decoding batch runs on the model's one stream
   int grouped_gates = 0;           // what the previous step fixes of every layer's gate product in one grouped launch
   int separate_beam_launches = 0;  // beam merge and state gather as the two launches the fused one replaces
+  int no_packed_gates = 0;         // gate products of few columns on the stored matrices (as where memory is short)
 };
 DebugOptions &Debug();
 class LstmLayer;
@@ -210,8 +211,8 @@ class LstmLayer {
   // Stacked gate matrices as the packed gate product reads them (lh_gate_pack_f32), a copy beside the stored
   // one: of the matrices that are operands of a step's product (M is not where the input product is hoisted), made
   // by the first step that runs faster on it, made anew after a change of the weights.  While training that is
-  // every minibatch, so there it has to pay within the pass.  A model whose memory does not hold the copies runs
-  // on the stored matrices.
+  // every minibatch, so there it has to pay within the pass.  Where the card is short of memory for them the layer
+  // runs on the stored matrices, for the rest of its life.
   struct PackedGates {
     DeviceArray<float> copy;
     bool dirty = true;
@@ -221,6 +222,12 @@ class LstmLayer {
   int pass_steps_ = 0;     // steps of the pass that is running (teacher-forced passes and the encoder)
   void WeightsChanged() {
     for (PackedGates &p : packed_) p.dirty = true;
+  }
+  // Memory that a model cannot do without is taken after the copies too (attention memories, the embedding fold, the
+  // histories of a stream, other models), and must find what it found without them: the copies are made only where a
+  // quarter of the card's memory stays free behind them.
+  static bool PackedCopiesFit(size_t bytes, size_t free, size_t total) {
+    return bytes <= free && free - bytes >= total / 4;
   }
   // Puts the copies into segs; false: stays with the stored matrices.  saved_ns: what a step saves by the plan,
   // steps: how many are left of the pass.

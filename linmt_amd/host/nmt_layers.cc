@@ -240,7 +240,7 @@ void LstmLayer::BuildSplitWeights() {
 }
 
 bool LstmLayer::PackGates(lh_gemm_seg *segs, int nseg, int saved_ns, int steps) {
-  if (!packed_possible_) return false;
+  if (!packed_possible_ || Debug().no_packed_gates) return false;
   const int H = lstm_size_;
   const DeviceArray<float> *const stored[3] = {&p_device_m_stack_, &p_device_w_h_stack_, &p_device_q_stack_};
   const int K[3] = {input_size_, H, H};
@@ -255,16 +255,24 @@ bool LstmLayer::PackGates(lh_gemm_seg *segs, int nseg, int saved_ns, int steps) 
     if (wanted[m] && packed_[m].dirty) stale += lh_gate_pack_floats(H, K[m]);
   if (stale) {
     if (p_neural_mt_->cfg_.train_mode_ && !PackingPays(stale, saved_ns, steps)) return false;
+    size_t missing = 0;
+    for (int m = 0; m < 3; ++m)
+      if (wanted[m] && !packed_[m].copy.size()) missing += lh_gate_pack_floats(H, K[m]);
+    if (missing) {
+      size_t free = 0, total = 0;
+      HipErrorWrapper(hipMemGetInfo(&free, &total), "LstmLayer::PackGates: free memory");
+      packed_possible_ = PackedCopiesFit(missing * sizeof(float), free, total);
+      for (int m = 0; m < 3 && packed_possible_; ++m)
+        if (wanted[m]) packed_possible_ = packed_[m].copy.TryReserve(lh_gate_pack_floats(H, K[m]));
+      if (!packed_possible_) {
+        for (PackedGates &p : packed_) p.copy.Free();
+        return false;
+      }
+    }
     lh_gate_pack_source src[3];
     int n = 0;
     for (int m = 0; m < 3; ++m) {
       if (!wanted[m] || !packed_[m].dirty) continue;
-      try {
-        packed_[m].copy.Reserve(lh_gate_pack_floats(H, K[m]));
-      } catch (const std::exception &) {
-        packed_possible_ = false;
-        return false;
-      }
       src[n++] = lh_gate_pack_source{stored[m]->get(), 4 * H, K[m], packed_[m].copy.get()};
     }
     LhErrorWrapper(lh_gate_pack_f32(H, src, n, p_neural_mt_->stream_), "LstmLayer::PackGates");

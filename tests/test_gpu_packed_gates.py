@@ -152,3 +152,35 @@ def test_training_packs_where_the_pass_is_long_enough(lh):
         m.update_weights()
         assert any("gate_gemm_packed_kernel" in n or "gate_gemm_narrow_kernel" in n for n in names) == packed, (steps, names)
     m.close()
+
+
+def test_without_packed_copies_the_stored_matrices_are_used(lh):
+    """What a layer does where the card has no memory to spare: the same results to the rounding of the sums, and copies
+    made before are not used."""
+    from linmt_amd import host
+    rng = np.random.default_rng(9)
+    H, V, B, steps = 512, 60, 32, 24
+    src, ti, to = (rng.integers(0, V, (B, steps)).astype(np.int32) for _ in range(3))
+    info = np.concatenate([np.full(B, steps), np.zeros(B)]).astype(np.int32)
+    unique = [np.unique(a).astype(np.int32) for a in (src, ti)]
+    m = _training_model(host, rng, H, V, B, 28)
+    watched = {n: (H, H) for n in ("src.0.W_hf", "src.1.M_i", "tgt.1.W_ho", "tgt.1.M_c")}
+    results = []
+    try:
+        for off in (0, 1, 0):
+            host.set_debug_option("no_packed_gates", off)
+            m.profile(2)
+            loss = m.compute_gradients(src, ti, to, info, *unique)
+            packed = any("gate_gemm_packed_kernel" in n or "gate_gemm_narrow_kernel" in n for n in m.profile_totals())
+            m.profile(0)
+            assert packed == (off == 0)
+            # (gradients add up until the next update)
+            results.append((loss, {n: m.get_grad(n, s) / (len(results) + 1) for n, s in watched.items()}))
+    finally:
+        host.set_debug_option("no_packed_gates", 0)
+    for loss, grads in results[1:]:
+        assert_close(loss, results[0][0], "loss", rtol=1e-6, atol=1e-4)
+        for n in watched:
+            # (2-norm; products whose sums are cut at other places give up to 1e-5 in a gradient of this size)
+            assert np.linalg.norm(grads[n] - results[0][1][n]) <= 4e-5 * np.linalg.norm(results[0][1][n]), n
+    m.close()

@@ -54,7 +54,7 @@ def test_narrow_gate_product_with_cell(lh, H, B, Ks, columns):
 @pytest.mark.parametrize("H,B,Ks", [(4, 1, (4,)), (36, 33, (36,)), (64, 32, (132, 20)), (100, 65, (16, 100, 60)),
                                     (1000, 12, (1000, 1000))])
 def test_packed_gate_product_with_cell(lh, config, H, B, Ks):
-    """All of the cell's forms: an addend by column, gate values and the dropped copy kept."""
+    """With an addend by column, gate values and the dropped copy kept."""
     import torch
     torch.manual_seed(H + B)
     dev = dict(device="cuda")
@@ -184,3 +184,55 @@ def test_without_packed_copies_the_stored_matrices_are_used(lh):
             # (2-norm; products whose sums are cut at other places give up to 1e-5 in a gradient of this size)
             assert np.linalg.norm(grads[n] - results[0][1][n]) <= 4e-5 * np.linalg.norm(results[0][1][n]), n
     m.close()
+
+
+@pytest.mark.parametrize("config", [-1, 13, 14, 15, 19, 45, 46])  # 45 and 46: the narrow forms
+@pytest.mark.parametrize("f64,clip,addend,kept", [
+    (False, 0.0, None, False), (True, 0.0, "column", False),  # scoring without feed input; a decoding step with it
+    (True, 0.3, "dense", True), (False, 0.3, "dense", False), (True, 0.0, None, True), (False, 0.0, "column", True)])
+@pytest.mark.parametrize("H,B,Ks", [(36, 33, (36,)), (100, 12, (100, 260))])
+def test_packed_cell_forms(lh, orc, config, f64, clip, addend, kept, H, B, Ks):
+    """Every argument that changes the cell or what it leaves: double sigmoids, columns that take the fp32 ones all the
+    same (mask 3: the first step of a streamed sentence), clipping, an addend per column, through a column index or none,
+    gate values and the dropped copy kept or not, the cell state in place."""
+    import torch
+    n = lh.load().lh_gemm_set_config_override(-1)
+    assert n == 45
+    rng = np.random.default_rng(H + B + 2 * int(f64) + int(kept))
+    uni = lambda *s: rng.uniform(-1, 1, s).astype(np.float32)  # noqa: E731
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    W, X = [uni(K, 4 * H) * np.float32(0.3) for K in Ks], [uni(B, K) for K in Ks]  # column-major 4H x K and K x B
+    table, col = uni(7, 4 * H), rng.integers(0, 7, B).astype(np.int32)
+    bias, c_prev, drop = uni(4 * H), uni(B, H), rng.random((B, H)).astype(np.float32)
+    mask = rng.choice(np.array([0, 1, 3], np.int32), B)
+    add = {None: None, "column": table[col], "dense": uni(B, 4 * H)}[addend]
+    pre = sum(x.astype(np.float64) @ w for x, w in zip(X, W)) + (0 if add is None else add)
+    want = [orc.lstm_cell_fwd(pre.T.astype(np.float32), bias, c_prev.T, mask & 1, feed=form, cell_clip=clip)
+            for form in (False, f64)]
+    gates_want, c_want, h_want = (np.where(mask >= 2, a, b).T for a, b in zip(*want))  # per column
+    segs = [(p, 32, dev(x), x.shape[1], x.shape[1]) for p, x in zip(_packed(lh, torch, H, [dev(w) for w in W], Ks), X)]
+
+    def cell(sigmoid_f64):
+        c, h = dev(c_prev), torch.full((B, H), float("nan"), device="cuda")
+        g, d = (torch.full((B, k * H), float("nan"), device="cuda") for k in (4, 1))
+        args = {}
+        if addend == "column":
+            args = dict(addend=dev(table), ld_addend=4 * H, addend_col=dev(col), addend_ncols=7)
+        elif addend == "dense":
+            args = dict(addend=dev(add), ld_addend=4 * H)
+        keep = dict(gates=g, next_drop_mask=dev(drop), keep=0.8, h_drop=d) if kept else {}
+        lh.load().lh_gemm_set_config_override(config)
+        lh.gate_gemm_lstm_cell_packed(H, B, segs, dev(bias), c, dev(mask), c, h, sigmoid_f64=sigmoid_f64, cell_clip=clip,
+                                      **args, **keep)
+        torch.cuda.synchronize()
+        return [t.cpu().numpy() for t in (c, h, g, d)]
+
+    c, h, g, d = cell(f64)
+    assert_close(c, c_want, "c")
+    assert_close(h, h_want, "h")
+    if kept:
+        assert_close(g, gates_want, "gates")
+        assert np.array_equal(d, (drop < np.float32(0.8)) * (np.float32(1) / np.float32(0.8)) * h)
+    if f64:
+        for a, b in zip((c, h) + ((g,) if kept else ()), cell(False)):
+            assert np.array_equal(a[mask >= 2], b[mask >= 2])

@@ -2209,9 +2209,11 @@ void pick_config(int M, int N, const int *K, int nseg, bool ta, bool tx, Form fo
   for (int s = 0; s < nseg; ++s) Kk[s] = K[s];
   // Every field into every bit of the slot: the two questions a gate product asks (any launch; an unsplit
   // one that can carry the cell) once shared a slot, each overwrote the other's answer, and a plan took 5.7 us of
-  // host time; it takes 0.2.
+  // host time; it takes 0.2.  The workspace is among them: an encoder lane and the main stream ask for the same
+  // products with unlike ones.
   unsigned h = 2166136261u;
-  for (const int v : {M, N, Kk[0], Kk[1], Kk[2], flags}) h = (h ^ (unsigned)v) * 2654435761u, h ^= h >> 15;
+  for (const int v : {M, N, Kk[0], Kk[1], Kk[2], flags, (int)(workspace_bytes >> 8)})
+    h = (h ^ (unsigned)v) * 2654435761u, h ^= h >> 15;
   Memo &e = memo[h % 64];
   if (e.flags == flags && e.M == M && e.N == N && e.K[0] == Kk[0] && e.K[1] == Kk[1] &&
       e.K[2] == Kk[2] && e.workspace_bytes == workspace_bytes) {

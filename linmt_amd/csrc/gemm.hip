@@ -1872,6 +1872,18 @@ int launch_reduce(const GemmArgs &g, hipStream_t st) {
   return lh::check_launch("lh_gemm_ws_f32 split reduction");
 }
 
+// Shares of the K slabs of a product (bk deep, none across two segments) that is to be split `want` ways: slabs of a
+// share, and how many shares hold any.
+struct Shares {
+  int slabs, n;
+};
+Shares shares_of(const int *K, int nseg, int bk, int want) {
+  int slabs = 0;
+  for (int s = 0; s < nseg; ++s) slabs += (K[s] + bk - 1) / bk;
+  const int share = (slabs + want - 1) / want;
+  return {share, (slabs + share - 1) / share};
+}
+
 // What takes a product: the scalar kernel, the main kernel for aligned operands, or its form for
 // ragged ones.
 enum Form { kGeneric, kRagged, kAligned };
@@ -1882,10 +1894,8 @@ int launch_cfg(const GemmArgs &g0, bool ta, bool tx, Form form, hipStream_t st) 
   g.tiles_m = (g.M + BM - 1) / BM;
   g.tiles_n = (g.N + BN - 1) / BN;
   if (form == kGeneric) g.splits = 1;
-  int slabs = 0;
-  for (int s = 0; s < g.nseg; ++s) slabs += (g.K[s] + BK - 1) / BK;
-  g.slabs_per_split = (slabs + g.splits - 1) / g.splits;
-  g.splits = (slabs + g.slabs_per_split - 1) / g.slabs_per_split;  // no empty share
+  const Shares shares = shares_of(g.K, g.nseg, BK, g.splits);
+  g.slabs_per_split = shares.slabs, g.splits = shares.n;
   const dim3 grid(g.tiles_m * g.tiles_n * g.splits), block(64 * WM * WN * WK);
   if (form != kGeneric) {
     int rc = LH_OK;
@@ -1930,10 +1940,8 @@ int launch_narrow_gemm(const GemmArgs &g0, bool ta, hipStream_t st) {
   GemmArgs g = g0;
   g.tiles_m = (g.M + 15) / 16;
   g.tiles_n = (g.N + 16 * FC - 1) / (16 * FC);
-  int slabs = 0;
-  for (int s = 0; s < g.nseg; ++s) slabs += (g.K[s] + kNarrowSlab - 1) / kNarrowSlab;
-  g.slabs_per_split = (slabs + g.splits - 1) / g.splits;
-  g.splits = (slabs + g.slabs_per_split - 1) / g.slabs_per_split;  // no empty share
+  const Shares shares = shares_of(g.K, g.nseg, kNarrowSlab, g.splits);
+  g.slabs_per_split = shares.slabs, g.splits = shares.n;
   const dim3 grid(g.tiles_m * g.tiles_n * g.splits);
   const int rc = ta ? launch_kernel((GemmKernel)gemm_kernel<16, 16 * FC, 1, 1, 8, kNarrowSlab, true, false>,
                                     narrow_smem_floats<FC>() * 4, grid, dim3(512), st, g)
@@ -2148,12 +2156,10 @@ float cold_share(const Config &k, bool short_runs, int M, int N, const int *K, i
 float predict_us(const Tuning &t, const Config &k, int M, int N, const int *K, int nseg, int want,
                  bool reduce_free, int *splits, float cold = 0.f) {
   const long long tiles = (long long)((M + k.bm - 1) / k.bm) * ((N + k.bn - 1) / k.bn);
-  int slabs = 0;
-  for (int s = 0; s < nseg; ++s) slabs += (K[s] + k.bk - 1) / k.bk;
-  const int share = (slabs + want - 1) / want;
-  const int S = (slabs + share - 1) / share;
+  const Shares shares = shares_of(K, nseg, k.bk, want);
+  const int S = shares.n;
   *splits = S;
-  const float depth = (float)share * k.bk;
+  const float depth = (float)shares.slabs * k.bk;
   // Workgroups per CU: dispatch is dynamic, so a fractional load costs less than a whole extra
   // round but leaves a tail of about half a workgroup.
   const float per_cu = (float)(tiles * S) / kCUs;
@@ -2178,7 +2184,6 @@ float predict_us(const Tuning &t, const Config &k, int M, int N, const int *K, i
 }
 
 // max_planes > 0: the caller consumes up to that many partial planes itself (no reduction pass).
-
 // only_cell: restrict the choice to unsplit launches of configurations whose LDS holds a whole
 // tile (what the gate product with the cell in its epilogue can use).  *us (optional) receives
 // the predicted time of the choice.
@@ -2384,13 +2389,8 @@ extern "C" int lh_gemm_planes_f32(int M, int N, const lh_gemm_seg *segs, int nse
   const int rc = prepare(M, N, segs, nseg, transA, transX, 1.f, beta, nullptr, LH_ACT_NONE, M,
                          nullptr, C, ldc, workspace, workspace_bytes, max_planes, &p);
   if (rc != LH_OK) return rc;
-  // the split the launch will really use (no empty share), as launch_cfg computes it
-  const Config &k = config_at(p.config);
-  int slabs = 0;
-  for (int s = 0; s < p.g.nseg; ++s) slabs += (p.g.K[s] + k.bk - 1) / k.bk;
-  const int want = p.form != kGeneric ? p.g.splits : 1;
-  const int share = (slabs + want - 1) / want;
-  *planes = (slabs + share - 1) / share;
+  // the split the launch will really use (no empty share)
+  *planes = shares_of(p.g.K, p.g.nseg, config_at(p.config).bk, p.form != kGeneric ? p.g.splits : 1).n;
   return launch_index(p.config, p.g, p.ta, p.tx, p.form, lh::as_stream(stream));
 }
 

@@ -1349,7 +1349,9 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &g, const int logical) 
 // 32 columns whatever there are; these are 250 workgroups with the 16x16x4 MFMA at the same rate per column.
 // 1000 hidden units, K = 1000 / 2000, with cell: 12 columns 9.5 / 14.7 us on 32x32 tiles, 6.8 / 9.9 (16 and 32 MB of
 // weights, 5.3 TB/s beyond the fixed part); 32 columns 10.1 / 15.3 and 8.6 / 12.3; 256 hidden units, 12 columns, K = 512
-// 6.7 and 4.5.  At 2048 hidden units both read the weights at the same rate (16.8 us, K = 2048).
+// 6.7 and 4.5.  From 1025 hidden units on it would be a second round of workgroups: at 1100 to 1800 units, 1 to 32 columns
+// 32-row tiles on part of the CUs take 0.7 to 0.93 of its time (1200 units, 16 columns, K = 2400: 18.8 us and 23.2), at
+// 2048 both read the weights at the same rate (16.8 us, K = 2048).
 constexpr int kNarrowK = 32, kNarrowSlab = 8 * kNarrowK, kNarrowCells = 4;
 constexpr int kNarrowLd = 20;  // floats between the columns of a partial block in LDS
 template <int FC>
@@ -2136,21 +2138,26 @@ float cell_launch_us(float product_us, int H, int B) {
   return (product_us < 16.f ? 6.f : 4.f) + 28.f * (float)H * (float)B / kReduceBytesPerUs;
 }
 
-// What the K loop costs more where its operands come from beyond the L2s, which the table does not
-// show.  A streamed wavefront takes a transposed A in 64-byte runs, one per row, and its ring covers the latency of an L2
-// but not that of HBM: from 48 MB of operands on (35 products of 400 to 2000 rows, K = 6000 to 30000) its loop takes
-// 1.28 times the time of the table at the median, 1.6 in the worst tenth; with A as stored, in runs of 128 bytes, 1.1
-// times what staged tiles take.  Staged and narrow tiles stay within 0.06 of the table, and below 16 MB so do all.
+// What the K loop costs more where its operands come from beyond the L2s, which the table does not show.  A streamed
+// wavefront takes a transposed A in 64-byte runs, one per row, and its ring covers the latency of an L2 but not that of
+// HBM: from 48 MB of operands on (35 products of 400 to 2000 rows, K = 6000 to 30000) its loop takes 1.28 times the time
+// of the table at the median, 1.6 in the worst tenth; with A as stored, in runs of 128 bytes, 1.1 times what staged tiles
+// take.  Staged tiles stay within 0.06 of the table, and below 8 MB so do all.
 // Transposed, 1536 x 21, K = 8460: 26.1 us on 32x32, 23.3 on staged 64x32; 996 x 109, K = 11516 47.6 and 37.9 (64x64);
 // 2048 x 64, K = 8192 33.6 and 30.5.
-// The stored gate matrix of a product with its cell is runs of 32 bytes (8 rows of a gate) and costs the same: 1.36 at
-// the median of 78 products of at most a workgroup per CU, where staged tiles take 1.06 and packed matrices 1.12 (no
-// price for those).  1956 hidden units, 58 columns, K = 3912: 69 us on streamed 64x32, 60 on the staged one, 51 split with a cell kernel behind.
+// The narrow tiles lose the most: a workgroup per CU reads 16 rows and nothing hides it.  Transposed, 1000 x 64, K = 4000
+// takes 10.2 us on 16x16 where one matrix is read again and again and 12.3 where twenty take turns (32x32 split in four:
+// 12.0 and 14.7), 2000 x 64, K = 8000 29.6 and 39.1 (64x64: 24.2 and 30.0).
+// The stored gate matrix of a product with its cell is runs of 32 bytes (8 rows of a gate) and costs what a transposed A
+// does: 1.36 at the median of 78 products of at most a workgroup per CU, where staged tiles take 1.06 and packed matrices
+// 1.12 (no price for those).  1956 hidden units, 58 columns, K = 3912: 69 us on streamed 64x32, 60 on the staged one, 51
+// split with a cell kernel behind.
 float cold_share(const Config &k, bool short_runs, int M, int N, const int *K, int nseg) {
-  if (!k.streamed) return 0.f;
+  const bool narrow = k.bm == 16;
+  if (!k.streamed && !narrow) return 0.f;
   float mb = 0.f;
   for (int s = 0; s < nseg; ++s) mb += 4.0e-6f * (float)K[s] * ((float)M + (float)N);
-  return fminf(fmaxf((mb - 16.f) / 32.f, 0.f), 1.f) * (short_runs ? 0.3f : 0.1f);
+  return fminf(fmaxf((mb - 8.f) / 24.f, 0.f), 1.f) * (narrow ? 0.5f : (short_runs ? 0.3f : 0.1f));
 }
 
 float predict_us(const Tuning &t, const Config &k, int M, int N, const int *K, int nseg, int want,

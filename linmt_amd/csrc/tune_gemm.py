@@ -106,8 +106,8 @@ class Tuner:
         fits = []
         for per_cu in (1, occ):
             tm, tn = 16 * per_cu, 16
-            if info["BM"] == 16:  # few columns are what the narrow tiles are for
-                tm, tn = CUS * per_cu, 1
+            if info["BM"] == 16:  # the few columns that the narrow tiles are for
+                tm, tn = (CUS * per_cu, 1) if block == "packed" else (CUS // 4 * per_cu, 4)
             while tm * info["BM"] > 12288:
                 tm //= 2
                 tn *= 2

@@ -1832,10 +1832,12 @@ constexpr int kNumNarrow = sizeof(kNarrow) / sizeof(kNarrow[0]);
 const Config &config_at(int c) { return c < kNumConfigs ? kConfigs[c] : kNarrow[c - kNumConfigs]; }
 // Configurations built for ragged operands as well: those that the cost model gives an aligned output
 // projection and its backward products at 5 to 2560 columns of 5000 to 30000 words, or one within
-// a few per cent of them.  All of them run the staged form, 15 too, and have rows of their own in the cost model: with
-// those of the aligned kernels (32x32: a fixed part of 3.9 us where this form takes 5.5) 340 products of 30 to 30003 rows
-// or words, 1 to 768 columns took 1.021 times the time of the best of a sweep over configurations and splits, 1.49 at
-// worst; with rows of their own 1.015 and 1.17.
+// a few per cent of them.  All of them run the staged form, 15 too, whose aligned
+// form is streamed.  In the cost model 12, 15 and 18 have rows of their own: loads that start at any float cost these most
+// (32x64: 0.0197 us per k where aligned operands take 0.0115).  With the rows of the aligned kernels 340 products of 30 to
+// 30003 rows or words, 1 to 768 columns took 1.021 times the time of the best of a sweep over configurations and splits,
+// 1.49 at worst; with these 1.008 and 1.17.  Rows for all ten are no better there, and put 64x64 behind 128x64 where a
+// large result has a short K (8830 x 1538, K = 24: 21.4 us and 26.2).
 constexpr bool ragged_config(int c) {
   return c == 0 || c == 3 || c == 7 || c == 12 || c == 15 || c == 18 || c == 24 || c == 32 || c == 35 || c == 36;
 }
@@ -2245,10 +2247,11 @@ void pick_config(int M, int N, const int *K, int nseg, bool ta, bool tx, Form fo
     if (narrow && (!allow_narrow || only_cell || tx || form != kAligned)) break;
     if (only_cell && !cell_capable_index(c)) continue;
     if (form == kRagged && (!ragged_config(c) || kConfigs[c].bm > max_bm || kConfigs[c].bn > max_bn)) continue;
-    const Tuning *const t = form == kRagged ? row_of(kRaggedTuning[ta ? 1 : (tx ? 2 : 0)], c)
-                            : narrow        ? row_of(kNarrowTuning[ta ? 1 : 0], c)
-                                            : &table[c];
-    if (!t) continue;
+    const Tuning *t = form == kRagged ? row_of(kRaggedTuning[ta ? 1 : (tx ? 2 : 0)], c)
+                      : narrow        ? row_of(kNarrowTuning[ta ? 1 : 0], c)
+                                      : nullptr;
+    if (!t && narrow) break;
+    if (!t) t = &table[c];
     const float cold = tx || form != kAligned ? 0.f : cold_share(config_at(c), ta || only_cell, M, N, K, nseg);
     for (int want : kSplitChoices) {
       if (only_cell && want > 1) break;

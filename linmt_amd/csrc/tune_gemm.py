@@ -11,7 +11,7 @@ file as it is.  For every row it times a product whose tiles give each CU exactl
 one that gives each CU as many as fit at once, at two depths K; the table holds the fixed and per-k
 cost of both, which is all the cost model in gemm.hip uses.  Blocks: the operand layouts NN, TN and
 NT; "cell", the stacked gate product that ends in the LSTM cell; "ragged-NN", "ragged-TN" and
-"ragged-NT", the same products where no row of an operand is 16-byte aligned; "narrow-NN" and
+"ragged-NT", products of a few configurations where no row of an operand is 16-byte aligned; "narrow-NN" and
 "narrow-TN", the tiles of 16 rows; "packed", the gate product with its cell on packed gate matrices.
 """
 import os
@@ -26,7 +26,8 @@ from linmt_amd import lib as lh  # noqa: E402
 
 CUS = 256
 KS = (512, 4096)
-KS_RAGGED = (256, 2048)  # (rows that share cache lines cost the more the deeper K: no line over more than this)
+RAGGED_ROWS = (12, 15, 18)  # configurations whose form for ragged operands costs other than that for aligned ones
+KS_RAGGED = (128, 2048)  # (no line holds from one slab of k to 4096: rows that share cache lines cost the more the deeper)
 LAYOUTS = {"NN": (False, False), "TN": (True, False), "NT": (False, True)}
 PLAIN = list(LAYOUTS)
 BLOCKS = PLAIN + ["cell"] + ["ragged-" + lay for lay in PLAIN] + ["narrow-NN", "narrow-TN", "packed"]
@@ -122,6 +123,8 @@ class Tuner:
         return (occ, *fits)
 
     def configs(self, block):
+        if block.startswith("ragged"):
+            return RAGGED_ROWS
         if block.startswith("narrow"):
             return range(self.n_cfg, self.n_cfg + 2)
         return range(self.n_cfg + 2) if block == "packed" else range(self.n_cfg)

@@ -39,3 +39,15 @@ def test_ragged_products_are_priced_as_staged(M, N, K, tA, tX):
     """Ragged operands take the staged form of the 32x32 tile, whose fixed part is 1.5 us more than that of the streamed
     one: 5.6 us against 5.0 at 246 x 22, K = 31; 40.9 against 36.2 at the last of these."""
     assert tile(M, N, [K], tA, tX) != (32, 32, 1, 1, 8, 128)
+
+
+@pytest.mark.parametrize("M,N,K,tX", [(8830, 1538, 24, True), (22565, 673, 43, False), (21910, 298, 104, False)])
+def test_large_ragged_results_of_a_short_k(M, N, K, tX):
+    """64x64 tiles, 21.4, 26.8 and 22.8 us; 128x64 took 26.2, 31.1 and 25.4."""
+    assert tile(M, N, [K], tX=tX) == (64, 64, 2, 2, 1, 16)
+
+
+@pytest.mark.parametrize("M,N,K", [(443, 2, 120), (4567, 1, 130), (58, 47, 127)])
+def test_few_ragged_columns_of_one_deep_slab(M, N, K):
+    """32x32 tiles, 4.4, 5.5 and 5.9 us; 32x64, whose loads at any float's address cost it the most, 5.2, 6.4 and 6.9."""
+    assert tile(M, N, [K]) == (32, 32, 1, 1, 8, 128)
